@@ -191,14 +191,6 @@ bool pipe_on(std::initializer_list<const void *> ptrs)
     return true;
 }
 
-// The pipelined fused step stores each stage's primitives from the stage kernel
-// (no ctoprim pass in stages 2 and 3); CNS_STAGE_Q=0 selects a ctoprim pass per stage.
-bool stage_q_on()
-{
-    const char *e = getenv("CNS_STAGE_Q");
-    return !(e && atoi(e) == 0);
-}
-
 hipError_t stencil_hypterm(const Geom &g, const double *cons, const double *q, double *flux,
                            const double dxi[3], hipStream_t s)
 {
@@ -546,59 +538,31 @@ int cns_advance_async(cns_ctx *ctx, double *U, double *Unew, double *Q, double *
     hipStream_t s = t_stream;
     double *dt = dt_dev ? dt_dev : ctx->d_dt;
     if (ctx->d_stage) {
-        // Fused composition: each stage is fill, ctoprim, diffterm, and hypterm with the
-        // RK update of its cell applied in the same pass (F is still written).  Stage
-        // results go to a buffer the stage does not read with halos:
+        // Fused composition.  Stage results go to a buffer the stage does not read with halos:
         //   stage 1: U -> stage (U^{1/3});  stage 2: stage -> Unew (U^{2/3});
         //   stage 3: Unew -> U (U^{n+1}).
         // Every ABI array ends as the reference leaves it (cpu/advance.cpp:13-154).
         double *T = ctx->d_stage;
-        if (pipe_on({U, Unew, Q, D, F, T, ctx->d_wz})) {
-            // q is ctoprim(state) here, so the stage kernel derives u, v, w, p from the
-            // conserved fields itself, and the first two stages' ctoprim stores only the
-            // u, v, w, T that diffterm reads; the third stores all of Q, as the
-            // reference leaves it.
-            // ctoprim also writes the wz field diffterm reads (one z-marching pass).
+        if (pipe_on({U, Unew, Q, D, F, T}) && stage_fits(g)) {
+            // One kernel per stage (cns_stage.hip): it derives the primitives, D and F of its
+            // cells itself, so a stage is the ghost fill of the state and that kernel.  The
+            // Courant number needs the whole state before any update, in a pass that stores
+            // nothing.  Stage 2 also stores the primitives of its result, the Q the
+            // reference leaves; the last fill copies their ghosts with the state's.
             const double *dxi = ctx->dxi;
-            double *WZ = ctx->d_wz;
-            if (stage_q_on()) {
-                // Stages 1 and 2 also store ctoprim of their result (interior cells) into
-                // Q, so stages 2 and 3 skip the ctoprim pass: the periodic fill copies
-                // those cells' Q into the ghosts with the state's, and a wz pass reads w.
-                // diffterm's rho row (0.0) is stored by stage 3 only; nothing reads it.
-                const unsigned uvwt = (1u << QU) | (1u << QV) | (1u << QW) | (1u << QTEMP);
-                TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, s));
-                HIPCHK(launch_courno_reset(ctx->d_acc, 1.0E-50, s));
-                TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim_wz(g, U, Q, WZ, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], dxi[2], false, s));
-                HIPCHK(launch_courno_to_dt(ctx->d_acc, ctx->cfl, dt, courno_dev ? courno_dev : ctx->d_courno, s));
-                TIMED(ctx, CNS_PROF_DIFFTERM, s, launch_diffterm_pipe(g, Q, WZ, D, dxi[0], dxi[1], dxi[2], ctx->eta, ctx->alam, s, false));
-                TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_hypterm_cons(g, U, F, dxi[0], dxi[1], dxi[2], D, U, T, dt, 1, false, Q, 1, s));
-                TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary_q(g, T, Q, uvwt, s));
-                TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_wz(g, Q, WZ, dxi[2], s));
-                TIMED(ctx, CNS_PROF_DIFFTERM, s, launch_diffterm_pipe(g, Q, WZ, D, dxi[0], dxi[1], dxi[2], ctx->eta, ctx->alam, s, false));
-                TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_hypterm_cons(g, T, F, dxi[0], dxi[1], dxi[2], D, U, Unew, dt, 2, false, Q, 2, s));
-                TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary_q(g, Unew, Q, (1u << NQ) - 1u, s));
-                TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_wz(g, Q, WZ, dxi[2], s));
-                TIMED(ctx, CNS_PROF_DIFFTERM, s, launch_diffterm_pipe(g, Q, WZ, D, dxi[0], dxi[1], dxi[2], ctx->eta, ctx->alam, s, true));
-                TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_hypterm_cons(g, Unew, F, dxi[0], dxi[1], dxi[2], D, U, U, dt, 3, true, nullptr, 0, s));
-                return CNS_OK;
-            }
             TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, s));
             HIPCHK(launch_courno_reset(ctx->d_acc, 1.0E-50, s));
-            TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim_wz(g, U, Q, WZ, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], dxi[2], false, s));
+            TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_courno(g, U, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
             HIPCHK(launch_courno_to_dt(ctx->d_acc, ctx->cfl, dt, courno_dev ? courno_dev : ctx->d_courno, s));
-            TIMED(ctx, CNS_PROF_DIFFTERM, s, launch_diffterm_pipe(g, Q, WZ, D, dxi[0], dxi[1], dxi[2], ctx->eta, ctx->alam, s));
-            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_hypterm_cons(g, U, F, ctx->dxi[0], ctx->dxi[1], ctx->dxi[2], D, U, T, dt, 1, false, nullptr, 0, s));
+            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, U, U, T, Q, D, F, dt, dxi, ctx->eta, ctx->alam, 1, s));
             TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, T, s));
-            TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim_wz(g, T, Q, WZ, nullptr, 0.0, 0.0, 0.0, dxi[2], false, s));
-            TIMED(ctx, CNS_PROF_DIFFTERM, s, launch_diffterm_pipe(g, Q, WZ, D, dxi[0], dxi[1], dxi[2], ctx->eta, ctx->alam, s));
-            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_hypterm_cons(g, T, F, ctx->dxi[0], ctx->dxi[1], ctx->dxi[2], D, U, Unew, dt, 2, false, nullptr, 0, s));
-            TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, s));
-            TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim_wz(g, Unew, Q, WZ, nullptr, 0.0, 0.0, 0.0, dxi[2], true, s));
-            TIMED(ctx, CNS_PROF_DIFFTERM, s, launch_diffterm_pipe(g, Q, WZ, D, dxi[0], dxi[1], dxi[2], ctx->eta, ctx->alam, s));
-            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_hypterm_cons(g, Unew, F, ctx->dxi[0], ctx->dxi[1], ctx->dxi[2], D, U, U, dt, 3, true, nullptr, 0, s));
+            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, T, U, Unew, Q, D, F, dt, dxi, ctx->eta, ctx->alam, 2, s));
+            TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary_q(g, Unew, Q, (1u << NQ) - 1u, s));
+            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, Unew, U, U, Q, D, F, dt, dxi, ctx->eta, ctx->alam, 3, s));
             return CNS_OK;
         }
+        // Arrays that are not 16-byte aligned, or too large for its offsets: fill, ctoprim,
+        // diffterm, and hypterm with the RK update of its cell applied in the same pass.
         TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, s));
         HIPCHK(launch_courno_reset(ctx->d_acc, 1.0E-50, s));
         TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, U, Q, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));

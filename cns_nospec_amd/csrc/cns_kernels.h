@@ -45,6 +45,10 @@ hipError_t launch_courno_reset(unsigned long long *acc, double init, hipStream_t
 hipError_t launch_ctoprim(const Geom &g, const double *u, double *q, unsigned long long *acc,
                           double dx0, double dx1, double dx2, hipStream_t s, bool full = true);
 
+// The Courant maximum of the interior cells of u alone, into acc.
+hipError_t launch_courno(const Geom &g, const double *u, unsigned long long *acc, double dx0, double dx1,
+                         double dx2, hipStream_t s, const BoxSet &bs = BoxSet());
+
 // dt = cfl / max(acc, 1e-50) into dt_dev (and the Courant number into courno_dev).
 hipError_t launch_courno_to_dt(const unsigned long long *acc, double cfl, double *dt_dev,
                                double *courno_dev, hipStream_t s);
@@ -106,5 +110,14 @@ hipError_t launch_ctoprim_wz(const Geom &g, const double *u, double *q, double *
 hipError_t launch_diffterm_pipe(const Geom &g, const double *q, const double *wz, double *difflux,
                                 double dxi0, double dxi1, double dxi2, double eta, double alam,
                                 hipStream_t s, bool write_rho = true, const BoxSet &bs = BoxSet());
+
+// One RK stage in one kernel (cns_stage.hip): out = the SSP-RK3 update of phase 1..3 of the
+// ghosted state cons with base U^n (phases 2 and 3), its primitives into q (phase 2), D and
+// F stored by phase 3.  Every array must be 16-byte aligned; out must not alias cons; the
+// geometry must satisfy stage_fits (planes below 4 GiB, pitches below 2^24).
+bool stage_fits(const Geom &g);
+hipError_t launch_stage(const Geom &g, const double *cons, const double *base, double *out, double *q, double *d,
+                        double *f, const double *dt_dev, const double dxi[3], double eta, double alam, int phase,
+                        hipStream_t s, const BoxSet &bs = BoxSet());
 
 }  // namespace cns

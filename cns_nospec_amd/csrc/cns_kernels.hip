@@ -262,6 +262,47 @@ rk_update_kernel(Geom g, int phase, double *__restrict__ u, double *__restrict__
     }
 }
 
+// ---------------------------------------------------------------- Courant number
+// The Courant maximum of a state's interior cells (cpu/ctoprim.cpp:42-69), without storing
+// its primitives, into acc (one 64-bit atomicMax per block).  A thread takes every
+// (grid size)-th cell of the interior, so a wave reads 64 consecutive cells of a row but for
+// the row ends: HBM-bound at large boxes (512^3 1.05 ms, 5.4 TB/s).
+__global__ void __launch_bounds__(kStreamBlock)
+courno_kernel(Geom g, const double *__restrict__ u, unsigned long long *__restrict__ acc, double dx0, double dx1,
+              double dx2, FastDiv by_n0, FastDiv by_n1, unsigned cells, BoxSet bs)
+{
+    u += blockIdx.y * bs.su;  // box of a box set
+    const int64_t cg = g.cg;
+    unsigned long long cmax = 0ull;
+    for (unsigned n = blockIdx.x * kStreamBlock + threadIdx.x; n < cells; n += gridDim.x * kStreamBlock) {
+        const unsigned r = by_n0.div(n), k = by_n1.div(r);
+        const int64_t e = gidx(g, (int)(n - r * g.n0) + NG, (int)(r - k * g.n1) + NG, (int)k + NG);
+        const double rho = u[e];
+        double qu, qv, qw, eint, p;
+        ctoprim_cell(rho, u[e + cg], u[e + 2 * cg], u[e + 3 * cg], u[e + 4 * cg], qu, qv, qw, eint, p);
+        const double c = sqrt(GAMMA * p / rho);
+        unsigned long long b = courno_bits((c + fabs(qu)) / dx0);
+        const unsigned long long by = courno_bits((c + fabs(qv)) / dx1);
+        const unsigned long long bz = courno_bits((c + fabs(qw)) / dx2);
+        b = b > by ? b : by;
+        b = b > bz ? b : bz;
+        cmax = cmax > b ? cmax : b;
+    }
+    __shared__ unsigned long long wmax[kStreamBlock / 64];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long o = __shfl_xor(cmax, off);
+        cmax = cmax > o ? cmax : o;
+    }
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = cmax;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long m = wmax[0];
+        for (int w = 1; w < kStreamBlock / 64; w++) m = m > wmax[w] ? m : wmax[w];
+        atomicMax(acc, m);
+    }
+}
+
 // ------------------------------------------------- direct-load stencils
 __device__ __forceinline__ double d1(const double *__restrict__ f, int64_t o, int64_t s)
 {
@@ -450,6 +491,26 @@ hipError_t launch_domain_fill(const Geom &g, const BoxSet &bs, const int nb[3], 
 hipError_t launch_courno_reset(unsigned long long *acc, double init, hipStream_t s)
 {
     courno_reset_kernel<<<1, 1, 0, s>>>(acc, init);
+    return hipGetLastError();
+}
+
+hipError_t launch_courno(const Geom &g, const double *u, unsigned long long *acc, double dx0, double dx1,
+                         double dx2, hipStream_t s, const BoxSet &bs)
+{
+    if (bs.n < 1 || bs.n > 65535) return hipErrorInvalidValue;
+    // Each block ends in an atomic on one address, about 20 ns apiece one after the other, so
+    // small boxes take 256 blocks (128^3: 57 us with 4096 blocks, 26 with 512) and large ones up
+    // to 1024, which their bandwidth needs (512^3: 1.76 / 1.13 / 1.00 / 1.02 ms with 256 / 512 /
+    // 1024 / 2048): 16 cells a thread or more in between.
+    const int64_t cells = (int64_t)g.n0 * g.n1 * g.n2, all = cells * bs.n;
+    if (cells > 0xffffffffll - 1024ll * kStreamBlock) return hipErrorInvalidValue;
+    int64_t most = all / (16 * kStreamBlock);
+    most = (most < 256 ? 256 : (most > 1024 ? 1024 : most)) / bs.n;
+    int64_t gx = (cells + kStreamBlock - 1) / kStreamBlock;
+    if (gx > most) gx = most;
+    if (gx < 1) gx = 1;
+    courno_kernel<<<dim3((unsigned)gx, (unsigned)bs.n), kStreamBlock, 0, s>>>(
+        g, u, acc, dx0, dx1, dx2, fast_div(g.n0), fast_div(g.n1), (unsigned)cells, bs);
     return hipGetLastError();
 }
 

@@ -1,0 +1,721 @@
+// cns_stage.hip -- one RK stage of the step in a single z-marching kernel (gfx950).
+//
+// From the ghosted conserved state alone a workgroup produces, for its 32 x 16 column tile
+// and run of planes, the viscous and inviscid terms of each cell (cpu/diffterm.cpp,
+// cpu/hypterm.cpp) and its SSP-RK3 update.  Primitives, their derivatives, D and F live in
+// LDS and registers only: a stage reads the five conserved fields (and the stage base) and
+// writes the result, where separate kernels pass Q, wz and D through memory.
+//
+// Storage.  512 threads, one workgroup per CU, two waves per SIMD of 256 registers each.
+// Registers: 9-plane z windows of mx, my, mz, E, 1/rho, p, T and of the computed ux, vy of
+// the lane's own column (u, v, w of a window plane are one product with 1/rho: ctoprim's
+// own), 144 registers between planes.  LDS, 158 KB: the centre plane's raw fields as
+// 24 x 40 tiles and the leading plane's own and halo cells, both loaded by direct-to-LDS
+// DMA; the derived u, v, w, T, p tiles; the leading plane's u rows and v columns; an 8-plane
+// ring of w on the tile's halo columns; ux, vy, wz of the centre plane with the halos
+// their mixed derivatives need.
+//
+// Plane k (leading plane k+4):
+//   1  primitives of the leading own cell into the windows, of the leading halo cells into
+//      the lead tiles and the ring, of the centre plane's halo cells into the derived tiles
+//      (the own cells come from the windows);
+//   B
+//   2  DMA of the next leading plane; ux, vy of the leading plane into the windows; ux, vy, wz
+//      of the centre plane into LDS; every z term, from the windows; hypterm's x and y
+//      terms, from the tiles;
+//   C
+//   3  DMA of the next centre plane; diffterm's x and y terms; the update and the stores;
+//   A
+// Before the first centre plane eight shorter iterations fill the windows and the ring.
+//
+// What bounds it: the vector arithmetic, about 1020 FP64 and 250 other instructions per
+// cell and plane at 4.5 cycles each (two waves per SIMD: 64 % of the cycles of a plane; the
+// rest is the latency of phase 1's divisions and the three barriers).  The time of a plane is
+// the same for one workgroup alone on the GPU and for 256.  512^3: 7.8 / 8.5 / 8.9 ms for stages
+// 1 / 2 / 3 against 11.4 / 12.8 / 11.4 ms of the fill-to-update chain of separate kernels;
+// 256^3 1.03 / 1.07 / 1.14 ms against 1.6 / 1.8 / 1.7 ms.
+//   A register spilled in the loop costs far more than its instructions: the reload waits for
+// every DMA issued before it (stages 2 and 3 ran 13 ms at 512^3 with ten reloads per plane).
+// Hence one-plane products instead of u, v, w windows, indices formed anew where they are used,
+// and pin() and FENCE().  One wave per SIMD with 512 registers (32 x 8 tiles) ran
+// 12.4 ms per stage at 512^3, opposite order of the z and the x, y parts in the two waves of a
+// SIMD 7 % slower, LDS reads issued half a tap pair ahead no faster.
+//   Every value is computed by the reference's expression (-ffp-contract=off), so results are
+// bit-identical to the reference cpu/ path.
+#include <type_traits>
+
+#include "cns_pipe_tile.h"
+
+namespace cns {
+
+namespace {
+
+// Tile geometry; sizes are in doubles unless they say otherwise.
+constexpr int TX = 32, BY = 16, PX = TX + 8, R = BY + 8, NT = TX * BY, NW = NT / 64;
+constexpr int TILE = R * PX;             // a haloed plane
+constexpr int YH = 8 * TX, XH = 8 * BY;  // y-halo and x-halo cells of its cross
+constexpr int HALO = YH + XH;
+constexpr int OB = NT / 128;             // 1 KB DMA blocks of the own cells of a plane
+static_assert(NW == 8 && OB == 4 && TILE <= 128 * NW, "the wave shares below are for 8 waves");
+constexpr int LHY = 5 * NT, LHX = LHY + 3 * YH, LEAD = LHX + 3 * XH;  // staged leading plane
+static_assert(LEAD <= 5 * TILE, "the window fill stages every second plane in the centre tile");
+enum { RRHO = 0, RMX, RMY, RMZ, RE, RNF };
+enum { VU = 0, VV, VW, VT, VP, VNF };
+
+struct StageArgs {
+    const double *base;  // U^n (stages 2 and 3)
+    double *out;         // result (ghosted); must not alias cons
+    double *q;           // primitives of the result (QOUT)
+    double *d, *f;       // D and F (LAST)
+    const double *dt;    // device dt
+    int phase;
+};
+
+typedef __attribute__((address_space(3))) double lds_double;
+// Taps are read one by one: the compiler otherwise pairs them into ds_read2_b64, which moves
+// 128 bytes per cycle where ds_read_b64 moves 240 (measured, eight waves).
+typedef const volatile __attribute__((address_space(3))) double lds_tap;
+
+__device__ __forceinline__ void dma16(const double *src, unsigned off, lds_double *lds)
+{
+    __builtin_amdgcn_global_load_lds((const void *)((const char *)src + off), (lds_void *)lds, 16, 0, 0);
+}
+
+// A lane's element of a plane: uniform plane pointer, 32-bit byte offset (a plane is below
+// 4 GiB), so that the access is one scalar-base instruction.
+#define GAS __attribute__((address_space(1)))
+template <typename T>
+__device__ __forceinline__ T GAS &at(T *p, unsigned off)
+{
+    asm volatile("" : "+s"(p));  // kept scalar: folded with the offset it would take a register pair per array
+    return *(T GAS *)((const char GAS *)p + off);
+}
+
+// Keeps the scheduler from hoisting the LDS reads of later groups above earlier ones, which
+// bounds the live registers.
+#define FENCE() __builtin_amdgcn_sched_barrier(0)
+// Has the values computed where it stands: the compiler would otherwise move arithmetic that
+// is used later past the barriers, and keep its operands live instead.
+template <typename... T>
+__device__ __forceinline__ void pin(T &...v)
+{
+    (..., [](auto &x) { asm volatile("" : "+v"(x)); }(v));
+}
+// A thread index that the compiler cannot see through: what is formed from it is formed
+// anew where it stands.  Held across the plane loop, the lane's places and offsets would
+// push window entries into scratch.
+__device__ __forceinline__ unsigned opaque_tid()
+{
+    unsigned t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t & (NT - 1);
+}
+// Products of indices and pitches, all below 2^24 (a full 32-bit product takes four times
+// the time of a 24-bit one).
+__device__ __forceinline__ unsigned mul24(unsigned a, unsigned b) { return __umul24(a, b); }
+
+// One tap pair (+m, -m) of a sum of differences, in the reference's order: the sum of a term
+// begins with its first tap pair.
+template <bool FIRST>
+__device__ __forceinline__ void tap(double &s, double t)
+{
+    s = FIRST ? t : s + t;
+}
+
+// hypterm's tap pair in one direction: n the momentum along it, a and b the others, v the
+// velocity along it; sums s of rho, n, a, b, E (cpu/hypterm.cpp:43-90).
+template <bool FIRST>
+__device__ __forceinline__ void hyp_tap(double c, double n1, double n0, double a1, double a0, double b1, double b0,
+                                        double e1, double e0, double p1, double p0, double v1, double v0,
+                                        double (&s)[5])
+{
+    tap<FIRST>(s[0], c * (n1 - n0));
+    tap<FIRST>(s[1], c * (n1 * v1 - n0 * v0 + (p1 - p0)));
+    tap<FIRST>(s[2], c * (a1 * v1 - a0 * v0));
+    tap<FIRST>(s[3], c * (b1 * v1 - b0 * v0));
+    tap<FIRST>(s[4], c * (e1 * v1 - e0 * v0 + (p1 * v1 - p0 * v0)));
+}
+
+template <bool STAGE1, bool LAST, bool QOUT>
+__global__ void __launch_bounds__(NT, 2)
+stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, double dxi1, double dxi2,
+             double eta, double alam, int kz, int ntx, int nty, BoxSet bs, int nbpb)
+{
+    __shared__ __align__(16) double raw[RNF * TILE];   // centre plane, raw
+    // leading plane, raw: own cells; y halo's rho, my, mz (at LHY); x halo's rho, mx, mz (at LHX)
+    __shared__ __align__(16) double s_lead[LEAD];
+    __shared__ double der[VNF * TILE];                 // centre plane, derived
+    __shared__ double s_lu[BY * PX];                   // leading u: own rows, column c (0..39)
+    __shared__ double s_lv[R * TX];                    // leading v: row r (0..R-1), column 4+c
+    __shared__ double s_ring[8 * HALO];                // w of plane p on the halo columns, slot p % 8
+    __shared__ double s_ux[R * TX];                    // row r (0..R-1), column 4+c
+    __shared__ double s_vy[BY * PX];                   // own rows, column c (0..39)
+    __shared__ double s_wz[TILE];
+
+    int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int box = t / nbpb;
+    t -= box * nbpb;
+    cons += box * bs.su;
+    const double *base = a.base + box * bs.su;
+    double *out = a.out + box * bs.su;
+    double *q = a.q + box * bs.sq, *dif = a.d + box * bs.sc, *flux = a.f + box * bs.sc;
+    const int bx = t % ntx, by = (t / ntx) % nty, bz = t / (ntx * nty);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int gi0 = bx * TX, gj0 = by * BY;  // ghosted coordinates of tile cell (0, 0)
+    const int kbeg = bz * kz, kend = min(kbeg + kz, g.n2);
+    const int64_t cg = g.cg, pg = g.pg;
+    const double dt = a.dt[0];
+    const double ra = a.phase == 1 ? 0.0E0 : (a.phase == 2 ? ThreeQuarters : OneThird);
+    const double rb = a.phase == 1 ? 1.0E0 : (a.phase == 2 ? OneQuarter : TwoThirds);
+    const double dxi0s = dxi0 * dxi0, dxi1s = dxi1 * dxi1, dxi2s = dxi2 * dxi2;
+    const unsigned xg = (unsigned)g.xg;
+
+    // Shares of the halo cells, in units of one cell per lane: leading y halo, its ring and
+    // wz on waves 0..3; leading x halo, its ring and wz on waves 4, 5; centre y halo and its
+    // ux on waves 4..7; centre x halo on waves 0, 1; corners on wave 2; vy's x halo on 6, 7.
+    const bool w_yl = wave < 4, w_xl = wave == 4 || wave == 5, w_xc = wave < 2, w_c = wave == 2, w_vx = wave >= 6;
+
+    // In-plane byte offset of tile cell (r, c)'s 16-byte pair, clamped into the array: cells
+    // past the box feed discarded outputs only.
+    auto pair_off = [&](int r, int c) {
+        return (mul24(min(gj0 + r, g.g1 - 1), xg) + (unsigned)min(gi0 + c, g.xg - 2)) * 8u;
+    };
+    // the lane's cell in ghosted coordinates, whether it lies in the box, and its byte offset
+    // within a ghosted plane
+    struct Cell {
+        int i, j;
+        bool active;
+        unsigned own8;
+    };
+    auto cell = [&]() {
+        const unsigned tid = opaque_tid();
+        Cell c;
+        c.i = gi0 + (tid & (TX - 1)) + 4;
+        c.j = gj0 + tid / TX + 4;
+        c.active = c.i < g.n0 + NG && c.j < g.n1 + NG;
+        c.own8 = (mul24(c.j, xg) + (unsigned)c.i) * 8u;
+        return c;
+    };
+    auto issue_raw = [&](int k) {  // centre plane k: block `wave` of every field
+        const double *p = cons + (int64_t)(k + NG) * pg;
+        const unsigned lane = opaque_tid() & 63, e = 128 * wave + 2 * lane;
+        const unsigned off = pair_off(e / PX, e % PX);
+        if (e < TILE) {
+#pragma unroll
+            for (int f = 0; f < RNF; f++) dma16(p + f * cg, off, (lds_double *)raw + f * TILE + 128 * wave);
+        }
+    };
+    // leading plane of centre plane k: own block wave % 4 of fields 0..2 (waves 0..3) or 3, 4;
+    // the y halo's two blocks and the x halo's one on waves 4, 5, 6
+    auto issue_lead = [&](int k, double *area) {
+        const double *p = cons + (int64_t)(k + 2 * NG) * pg;
+        const unsigned lane = opaque_tid() & 63, ob = wave & (OB - 1);
+        const unsigned ooff = pair_off(4 + 4 * ob + (lane >> 4), 4 + 2 * (lane & 15));
+        lds_double *l = (lds_double *)area + 128 * ob;
+        if (wave < OB) {
+            dma16(p, ooff, l);
+            dma16(p + cg, ooff, l + NT);
+            dma16(p + 2 * cg, ooff, l + 2 * NT);
+        } else {
+            dma16(p + 3 * cg, ooff, l + 3 * NT);
+            dma16(p + 4 * cg, ooff, l + 4 * NT);
+            if (wave < 6) {  // rows 0..3 or BY+4..BY+7
+                const unsigned hoff = pair_off((wave == 4 ? 0 : BY + 4) + (lane >> 4), 4 + 2 * (lane & 15));
+                lds_double *h = (lds_double *)area + LHY + 128 * (wave - 4);
+                dma16(p, hoff, h);
+                dma16(p + IMY * cg, hoff, h + YH);
+                dma16(p + IMZ * cg, hoff, h + 2 * YH);
+            } else if (wave == 6) {  // columns 0..3 and TX+4..TX+7 of the own rows
+                const int pr = lane & 3;
+                const unsigned hoff = pair_off(4 + (lane >> 2), pr < 2 ? 2 * pr : 2 * pr + TX);
+                lds_double *h = (lds_double *)area + LHX;
+                dma16(p, hoff, h);
+                dma16(p + IMX * cg, hoff, h + XH);
+                dma16(p + IMZ * cg, hoff, h + 2 * XH);
+            }
+        }
+    };
+
+    // Windows: plane k+m of the own column at [4+m].  wri is 1/rho, from which u, v, w of a
+    // window plane are one product (ctoprim's own).
+    double wmx[9], wmy[9], wmz[9], wE[9], wri[9], wp[9], wT[9], wux[9], wvy[9];
+#pragma unroll
+    for (int m = 0; m < 9; m++)
+        wmx[m] = wmy[m] = wmz[m] = wE[m] = wri[m] = wp[m] = wT[m] = wux[m] = wvy[m] = 0.0;
+
+    // primitives of the leading plane: own cell into the windows' entry 8, u and v with their
+    // halos into the lead tiles, w of the halo columns
+    auto lead = [&](const double *area) {
+        const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
+        const double lr = area[tid];
+        wmx[8] = area[RMX * NT + tid];
+        wmy[8] = area[RMY * NT + tid];
+        wmz[8] = area[RMZ * NT + tid];
+        wE[8] = area[RE * NT + tid];
+        double u_, v_, w_, eint;
+        ctoprim_cell(lr, wmx[8], wmy[8], wmz[8], wE[8], u_, v_, w_, eint, wp[8]);
+        wri[8] = 1.0E0 / lr;
+        wT[8] = eint / CV;
+        pin(wri[8], wp[8], wT[8]);
+        s_lu[mul24(row, PX) + col + 4] = u_;
+        s_lv[(row + 4) * TX + col] = v_;
+        if (w_yl) {
+            const unsigned yr = row < 4 ? row : row + BY;  // waves 0..3: rows 0..7
+            const double hinv = 1.0E0 / area[LHY + tid];
+            s_lv[yr * TX + col] = area[LHY + YH + tid] * hinv;
+            s_wz[mul24(yr, PX) + col + 4] = area[LHY + 2 * YH + tid] * hinv;
+        }
+        if (w_xl) {
+            const unsigned xid = tid & 127, c8 = xid & 7;
+            const double hinv = 1.0E0 / area[LHX + xid];
+            const unsigned l = mul24(xid >> 3, PX) + (c8 < 4 ? c8 : c8 + TX);
+            s_lu[l] = area[LHX + XH + xid] * hinv;
+            s_wz[l + 4 * PX] = area[LHX + 2 * XH + xid] * hinv;
+        }
+    };
+    auto shift = [&]() {
+#pragma unroll
+        for (int m = 0; m < 8; m++) {
+            wmx[m] = wmx[m + 1]; wmy[m] = wmy[m + 1]; wmz[m] = wmz[m + 1]; wE[m] = wE[m + 1];
+            wri[m] = wri[m + 1]; wp[m] = wp[m + 1]; wT[m] = wT[m + 1];
+            wux[m] = wux[m + 1]; wvy[m] = wvy[m + 1];
+        }
+    };
+
+    // ux, vy of the leading plane into the windows; w of the halo columns: planes k .. k+7 are
+    // in the ring, k+8 where lead() left it, which gives wz there (when the plane is a centre)
+    // and then takes the place of plane k
+    auto lead_grads = [&](int k, auto centre) {
+        const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
+        const unsigned mlu = mul24(row, PX) + col + 4, mlv = (row + 4) * TX + col;
+        lds_tap *p_lu = (lds_tap *)s_lu + mlu, *p_lv = (lds_tap *)s_lv + mlv;
+#define LUX(mm) p_lu[mm]
+#define LVY(mm) p_lv[(mm) * TX]
+        wux[8] = D1(LUX) * dxi0;
+        wvy[8] = D1(LVY) * dxi1;
+#undef LUX
+#undef LVY
+        pin(wux[8], wvy[8]);
+        if (w_yl || w_xl) {
+            const unsigned xid = tid & 127, c8 = xid & 7;
+            const unsigned rc = w_yl ? tid : YH + xid;
+            const unsigned l = w_yl ? mul24(row < 4 ? row : row + BY, PX) + col + 4
+                               : mul24((xid >> 3) + 4, PX) + (c8 < 4 ? c8 : c8 + TX);
+            const double hw = s_wz[l];  // w of plane k+8, left here by lead()
+#define RW(mm) ((mm) == 4 ? hw : s_ring[((k + 4 + (mm)) & 7) * HALO + rc])
+            if (centre.value) s_wz[l] = D1(RW) * dxi2;
+#undef RW
+            s_ring[(k & 7) * HALO + rc] = hw;
+        }
+    };
+
+    // Fill the windows and the ring with planes kbeg .. kbeg+7, staged two ahead in turn in the
+    // leading and the (still unused) centre tile.  A wave waits for the older plane only: the
+    // younger one's loads are 3, 5 or 2 of its own (issue_lead).
+    auto fill_plane = [&](int k, double *area) {
+        if (wave < 4)
+            __builtin_amdgcn_s_waitcnt(0xF73);
+        else if (wave < 7)
+            __builtin_amdgcn_s_waitcnt(0xF75);
+        else
+            __builtin_amdgcn_s_waitcnt(0xF72);
+        __syncthreads();
+        lead(area);
+        __syncthreads();
+        lead_grads(k, std::false_type());
+        shift();
+    };
+    issue_lead(kbeg - 8, s_lead);
+    issue_lead(kbeg - 7, raw);
+#pragma unroll 1
+    for (int k = kbeg - 8; k < kbeg; k += 2) {
+        fill_plane(k, s_lead);
+        issue_lead(k + 2, s_lead);
+        fill_plane(k + 1, raw);
+        if (k + 3 < kbeg) issue_lead(k + 3, raw);
+    }
+    issue_raw(kbeg);
+    __builtin_amdgcn_s_waitcnt(0xF70);
+    __syncthreads();
+
+#pragma unroll 1
+    for (int k = kbeg; k < kend; k++) {
+        const double *d_u = der + VU * TILE, *d_v = der + VV * TILE, *d_w = der + VW * TILE, *d_t = der + VT * TILE,
+                     *d_p = der + VP * TILE;
+        // ---------------- phase 1: primitives of the leading plane, derived tiles of the centre plane
+        lead(s_lead);
+        {
+            const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX, lane = tid & 63;
+            const unsigned me = mul24(row + 4, PX) + col + 4;
+            der[VU * TILE + me] = wmx[4] * wri[4];
+            der[VV * TILE + me] = wmy[4] * wri[4];
+            der[VW * TILE + me] = wmz[4] * wri[4];
+            der[VT * TILE + me] = wT[4];
+            der[VP * TILE + me] = wp[4];
+            auto halo_prim = [&](unsigned l) {
+                double u_, v_, w_, eint, p_;
+                ctoprim_cell(raw[RRHO * TILE + l], raw[RMX * TILE + l], raw[RMY * TILE + l], raw[RMZ * TILE + l],
+                             raw[RE * TILE + l], u_, v_, w_, eint, p_);
+                der[VU * TILE + l] = u_;
+                der[VV * TILE + l] = v_;
+                der[VW * TILE + l] = w_;
+                der[VT * TILE + l] = eint / CV;
+                der[VP * TILE + l] = p_;
+            };
+            if (!w_yl) {
+                const unsigned yrow = row - 8;
+                halo_prim(mul24(yrow < 4 ? yrow : yrow + BY, PX) + col + 4);
+            }
+            if (w_xc) {
+                const unsigned c8 = tid & 7;
+                halo_prim(mul24((tid >> 3) + 4, PX) + (c8 < 4 ? c8 : c8 + TX));
+            }
+            if (w_c) {  // u and v only
+                const unsigned r8 = lane >> 3, c8 = lane & 7;
+                const unsigned l = mul24(r8 < 4 ? r8 : r8 + BY, PX) + (c8 < 4 ? c8 : c8 + TX);
+                const double cinv = 1.0E0 / raw[RRHO * TILE + l];
+                der[VU * TILE + l] = raw[RMX * TILE + l] * cinv;
+                der[VV * TILE + l] = raw[RMY * TILE + l] * cinv;
+            }
+        }
+        __syncthreads();  // B
+
+        // ---------------- phase 2
+        if (k + 1 < kend) issue_lead(k + 1, s_lead);
+        double F[5], zf[5], rho_c;
+        lead_grads(k, std::true_type());
+        {
+            const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
+            const unsigned me = mul24(row + 4, PX) + col + 4;
+            {
+                // ux, vy, wz of the centre plane: own cells from the windows, the halos the mixed
+                // derivatives read from the derived tiles (cpu/diffterm.cpp:77-151)
+                s_ux[(row + 4) * TX + col] = wux[4];
+                if (!w_yl) {
+                    const unsigned yrow = row - 8, yr = yrow < 4 ? yrow : yrow + BY, l = mul24(yr, PX) + col + 4;
+                    lds_tap *p_u = (lds_tap *)d_u + l;
+#define CUX(mm) p_u[mm]
+                    s_ux[yr * TX + col] = D1(CUX) * dxi0;
+#undef CUX
+                }
+                s_vy[mul24(row, PX) + col + 4] = wvy[4];
+                if (w_vx) {
+                    const unsigned xid = tid & 127, c8 = xid & 7, c = c8 < 4 ? c8 : c8 + TX;
+                    const unsigned l = mul24((xid >> 3) + 4, PX) + c;
+                    lds_tap *p_v = (lds_tap *)d_v + l;
+#define CVY(mm) p_v[(mm) * PX]
+                    s_vy[mul24(xid >> 3, PX) + c] = D1(CVY) * dxi1;
+#undef CVY
+                }
+                rho_c = raw[RRHO * TILE + me];
+            }
+            FENCE();
+        }
+        double zx = 0.0, zy = 0.0, zz = 0.0, zt = 0.0, uz = 0.0, vz = 0.0, mz = 0.0;
+        {
+            // every z term of the cell, from the windows
+            double hs[5], uxz, vyz, wzc;
+            zx = CENTER * (wmx[4] * wri[4]);
+            zy = CENTER * (wmy[4] * wri[4]);
+            zz = CENTER * (wmz[4] * wri[4]);
+            zt = CENTER * wT[4];
+#define ZTAP(m, C1, C2, FIRST)                                                                                   \
+    {                                                                                                            \
+        const double w1 = wmz[4 + m] * wri[4 + m], w0 = wmz[4 - m] * wri[4 - m];                                 \
+        hyp_tap<FIRST>(C1, wmz[4 + m], wmz[4 - m], wmx[4 + m], wmx[4 - m], wmy[4 + m], wmy[4 - m], wE[4 + m],     \
+                       wE[4 - m], wp[4 + m], wp[4 - m], w1, w0, hs);                                             \
+        tap<FIRST>(wzc, C1 * (w1 - w0));                                                                         \
+        tap<false>(zz, C2 * (w1 + w0));                                                                          \
+        const double u1 = wmx[4 + m] * wri[4 + m], u0 = wmx[4 - m] * wri[4 - m];                                 \
+        tap<FIRST>(uz, C1 * (u1 - u0));                                                                          \
+        tap<false>(zx, C2 * (u1 + u0));                                                                          \
+        const double v1 = wmy[4 + m] * wri[4 + m], v0 = wmy[4 - m] * wri[4 - m];                                 \
+        tap<FIRST>(vz, C1 * (v1 - v0));                                                                          \
+        tap<false>(zy, C2 * (v1 + v0));                                                                          \
+        tap<false>(zt, C2 * (wT[4 + m] + wT[4 - m]));                                                            \
+        tap<FIRST>(uxz, C1 * (wux[4 + m] - wux[4 - m]));                                                         \
+        tap<FIRST>(vyz, C1 * (wvy[4 + m] - wvy[4 - m]));                                                         \
+        pin(hs[0], hs[1], hs[2], hs[3], hs[4], wzc, zz, uz, zx, vz, zy, zt, uxz, vyz);                            \
+        FENCE();                                                                                                 \
+    }
+            ZTAP(1, ALP, OFF1, true)
+            ZTAP(2, BET, OFF2, false)
+            ZTAP(3, GAM, OFF3, false)
+            ZTAP(4, DEL, OFF4, false)
+#undef ZTAP
+            zf[IRHO] = hs[0] * dxi2;
+            zf[IMZ] = hs[1] * dxi2;
+            zf[IMX] = hs[2] * dxi2;
+            zf[IMY] = hs[3] * dxi2;
+            zf[IENE] = hs[4] * dxi2;
+            wzc = wzc * dxi2;
+            uz = uz * dxi2;
+            vz = vz * dxi2;
+            zx = zx * dxi2s;
+            zy = zy * dxi2s;
+            zz = zz * dxi2s;
+            zt = zt * dxi2s;
+            mz = uxz * dxi2 + vyz * dxi2;
+            pin(zf[0], zf[1], zf[2], zf[3], zf[4], uz, vz, zx, zy, zz, zt, mz);
+            FENCE();
+            const unsigned tid = opaque_tid();
+            s_wz[mul24(tid / TX + 4, PX) + (tid & (TX - 1)) + 4] = wzc;
+        }
+        shift();  // the centre plane is window entry 3 from here
+        {
+            const unsigned tid = opaque_tid(), me = mul24(tid / TX + 4, PX) + (tid & (TX - 1)) + 4;
+            lds_tap *s_c = (lds_tap *)raw + me, *s_d = (lds_tap *)der + me;
+            double hs[5], A[12];
+            // fields n, a, b, E of the raw tile, p and v of the derived one at taps +o and -o
+            auto load = [&](double (&T)[12], int n, int a_, int b_, int v, int o) {
+                T[0] = s_c[n * TILE + o]; T[1] = s_c[n * TILE - o];
+                T[2] = s_c[a_ * TILE + o]; T[3] = s_c[a_ * TILE - o];
+                T[4] = s_c[b_ * TILE + o]; T[5] = s_c[b_ * TILE - o];
+                T[6] = s_c[RE * TILE + o]; T[7] = s_c[RE * TILE - o];
+                T[8] = s_d[VP * TILE + o]; T[9] = s_d[VP * TILE - o];
+                T[10] = s_d[v * TILE + o]; T[11] = s_d[v * TILE - o];
+            };
+#define HT(FIRST, C, T) \
+    hyp_tap<FIRST>(C, T[0], T[1], T[2], T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11], hs); \
+    pin(hs[0], hs[1], hs[2], hs[3], hs[4]); FENCE()
+            load(A, RMX, RMY, RMZ, VU, 1); FENCE();
+            HT(true, ALP, A);
+            load(A, RMX, RMY, RMZ, VU, 2); FENCE();
+            HT(false, BET, A);
+            load(A, RMX, RMY, RMZ, VU, 3); FENCE();
+            HT(false, GAM, A);
+            load(A, RMX, RMY, RMZ, VU, 4); FENCE();
+            HT(false, DEL, A);
+            F[IRHO] = -(hs[0]) * dxi0;
+            F[IMX] = -(hs[1]) * dxi0;
+            F[IMY] = -(hs[2]) * dxi0;
+            F[IMZ] = -(hs[3]) * dxi0;
+            F[IENE] = -(hs[4]) * dxi0;
+            load(A, RMY, RMX, RMZ, VV, PX); FENCE();
+            HT(true, ALP, A);
+            load(A, RMY, RMX, RMZ, VV, 2 * PX); FENCE();
+            HT(false, BET, A);
+            load(A, RMY, RMX, RMZ, VV, 3 * PX); FENCE();
+            HT(false, GAM, A);
+            load(A, RMY, RMX, RMZ, VV, 4 * PX); FENCE();
+            HT(false, DEL, A);
+#undef HT
+            F[IRHO] = F[IRHO] - hs[0] * dxi1;
+            F[IMY] = F[IMY] - hs[1] * dxi1;
+            F[IMX] = F[IMX] - hs[2] * dxi1;
+            F[IMZ] = F[IMZ] - hs[3] * dxi1;
+            F[IENE] = F[IENE] - hs[4] * dxi1;
+#pragma unroll
+            for (int l = 0; l < NC; l++) F[l] = F[l] - zf[l];
+            pin(F[0], F[1], F[2], F[3], F[4], rho_c);
+        }
+        __syncthreads();  // C
+
+        // ---------------- phase 3
+        const int64_t zk = (int64_t)(k + NG) * pg;
+        if (k + 1 < kend) issue_raw(k + 1);
+        {   // held in the lead tiles' own cells (read by the neighbours before C) until the update
+            const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
+            s_lu[mul24(row, PX) + col + 4] = rho_c;
+            s_lv[(row + 4) * TX + col] = F[IENE];
+        }
+        {
+            // diffterm's x and y terms, from the tiles, then its sums as the reference forms them
+            // (cpu/diffterm.cpp:159-311)
+            const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
+            const unsigned me = mul24(row + 4, PX) + col + 4;
+            lds_tap *s_d = (lds_tap *)der + me, *s_z = (lds_tap *)s_wz + me, *s_m = (lds_tap *)s_vy + mul24(row, PX) + col + 4,
+                    *s_n = (lds_tap *)s_ux + (row + 4) * TX + col;
+            double A[12], xu, xv, xw, xt, d2v, d2w, m1, m2;
+            // u, v, w, T of the derived tile, wz, and vy or ux at taps +o and -o
+            auto load = [&](double (&T)[12], int o, lds_tap *m, int om) {
+                T[0] = s_d[VU * TILE + o]; T[1] = s_d[VU * TILE - o];
+                T[2] = s_d[VV * TILE + o]; T[3] = s_d[VV * TILE - o];
+                T[4] = s_d[VW * TILE + o]; T[5] = s_d[VW * TILE - o];
+                T[6] = s_d[VT * TILE + o]; T[7] = s_d[VT * TILE - o];
+                T[8] = s_z[o]; T[9] = s_z[-o];
+                T[10] = m[om]; T[11] = m[-om];
+            };
+            // second differences of u, v, w, T; first of T[2 * f] (d2v), w (d2w), and of the two mixed terms
+#define DT(FIRST, C1, C2, T, f)                  \
+    tap<false>(xu, C2 * (T[0] + T[1]));          \
+    tap<false>(xv, C2 * (T[2] + T[3]));          \
+    tap<false>(xw, C2 * (T[4] + T[5]));          \
+    tap<false>(xt, C2 * (T[6] + T[7]));          \
+    tap<FIRST>(d2v, C1 * (T[2 * f] - T[2 * f + 1])); \
+    tap<FIRST>(d2w, C1 * (T[4] - T[5]));         \
+    tap<FIRST>(m1, C1 * (T[10] - T[11]));        \
+    tap<FIRST>(m2, C1 * (T[8] - T[9]));          \
+    pin(xu, xv, xw, xt, d2v, d2w, m1, m2);       \
+    FENCE()
+            xu = CENTER * (wmx[3] * wri[3]); xv = CENTER * (wmy[3] * wri[3]);
+            xw = CENTER * (wmz[3] * wri[3]); xt = CENTER * wT[3];
+            load(A, 1, s_m, 1); FENCE();
+            DT(true, ALP, OFF1, A, 1);
+            load(A, 2, s_m, 2); FENCE();
+            DT(false, BET, OFF2, A, 1);
+            load(A, 3, s_m, 3); FENCE();
+            DT(false, GAM, OFF3, A, 1);
+            load(A, 4, s_m, 4); FENCE();
+            DT(false, DEL, OFF4, A, 1);
+            double sx = FourThirds * (xu * dxi0s), sy = xv * dxi0s, sz = xw * dxi0s, st = xt * dxi0s;
+            const double vx = d2v * dxi0, wx = d2w * dxi0, mx = m1 * dxi0 + m2 * dxi0;
+            pin(sx, sy, sz, st);
+            double rkb[5];
+            if (!STAGE1) {  // (cells past the box read clamped, for nothing: no divergent branch here)
+                const unsigned t3 = opaque_tid();
+                const unsigned off = (mul24(min(gj0 + (int)(t3 / TX) + 4, g.g1 - 1), xg)
+                                      + (unsigned)min(gi0 + (int)(t3 & (TX - 1)) + 4, g.g0 - 1)) * 8u;
+#pragma unroll
+                for (int l = 0; l < NC; l++) rkb[l] = at(base + l * cg + zk, off);
+            }
+            xu = CENTER * (wmx[3] * wri[3]); xv = CENTER * (wmy[3] * wri[3]);
+            xw = CENTER * (wmz[3] * wri[3]); xt = CENTER * wT[3];
+            auto ytap = [&](auto first, double c1, double c2, int o, int on) {
+                constexpr bool FI = decltype(first)::value;
+                {
+                    const double u1 = s_d[VU * TILE + o], u0 = s_d[VU * TILE - o], v1 = s_d[VV * TILE + o],
+                                 v0 = s_d[VV * TILE - o], w1 = s_d[VW * TILE + o], w0 = s_d[VW * TILE - o];
+                    FENCE();
+                    tap<false>(xu, c2 * (u1 + u0));
+                    tap<false>(xv, c2 * (v1 + v0));
+                    tap<false>(xw, c2 * (w1 + w0));
+                    tap<FI>(d2v, c1 * (u1 - u0));
+                    tap<FI>(d2w, c1 * (w1 - w0));
+                    pin(xu, xv, xw, d2v, d2w);
+                    FENCE();
+                }
+                {
+                    const double t1 = s_d[VT * TILE + o], t0 = s_d[VT * TILE - o], z1 = s_z[o], z0 = s_z[-o],
+                                 n1 = s_n[on], n0 = s_n[-on];
+                    FENCE();
+                    tap<false>(xt, c2 * (t1 + t0));
+                    tap<FI>(m1, c1 * (n1 - n0));
+                    tap<FI>(m2, c1 * (z1 - z0));
+                    pin(xt, m1, m2);
+                    FENCE();
+                }
+            };
+            ytap(std::true_type(), ALP, OFF1, PX, TX);
+            ytap(std::false_type(), BET, OFF2, 2 * PX, 2 * TX);
+            ytap(std::false_type(), GAM, OFF3, 3 * PX, 3 * TX);
+            ytap(std::false_type(), DEL, OFF4, 4 * PX, 4 * TX);
+#undef DT
+            sx = sx + xu * dxi1s;
+            sy = sy + FourThirds * (xv * dxi1s);
+            sz = sz + xw * dxi1s;
+            st = st + xt * dxi1s;
+            const double tauxy = d2v * dxi1 + vx, wy = d2w * dxi1, my = m1 * dxi1 + m2 * dxi1;
+            const double uzz = zx, vzz = zy, wzz = zz, tzz = zt;
+            double D[5];
+            D[IRHO] = 0.0E0;
+            D[IMX] = eta * (sx + uzz + OneThird * mx);
+            D[IMY] = eta * (sy + vzz + OneThird * my);
+            D[IMZ] = eta * (sz + FourThirds * wzz + OneThird * mz);
+            {
+                const double ux = wux[3], vy = wvy[3], wz = *s_z;
+                const double divu = TwoThirds * (ux + vy + wz);
+                const double tauxx = 2.E0 * ux - divu;
+                const double tauyy = 2.E0 * vy - divu;
+                const double tauzz = 2.E0 * wz - divu;
+                const double tauxz = uz + wx;
+                const double tauyz = vz + wy;
+                double mechwork = tauxx * ux + tauyy * vy + tauzz * wz + (tauxy * tauxy) + (tauxz * tauxz)
+                                  + (tauyz * tauyz);
+                mechwork = eta * mechwork + D[IMX] * (wmx[3] * wri[3]) + D[IMY] * (wmy[3] * wri[3])
+                           + D[IMZ] * (wmz[3] * wri[3]);
+                D[IENE] = alam * (st + tzz) + mechwork;
+            }
+            rho_c = s_lu[mul24(row, PX) + col + 4];
+            F[IENE] = s_lv[(row + 4) * TX + col];
+            const double uc[5] = {rho_c, wmx[3], wmy[3], wmz[3], wE[3]};
+            // the centre plane's DMA has landed before the stores join the queue, so the barrier
+            // that ends the phase need not wait for them
+            __builtin_amdgcn_s_waitcnt(0xF70);
+            const Cell c = cell();
+            if (c.active) {
+                const unsigned own8 = c.own8,
+                               int8 = (mul24(c.j - NG, g.x) + (unsigned)(c.i - NG)) * 8u;
+                const int64_t fk = (int64_t)k * g.p;
+                double o[5];
+#pragma unroll
+                for (int l = 0; l < NC; l++) {
+                    if (LAST) {
+                        at(dif + l * g.c + fk, int8) = D[l];
+                        at(flux + l * g.c + fk, int8) = F[l];
+                    }
+                    // STAGE1: cons + dt(D+F) (cpu/advance.cpp:82); then ra*base + rb*(cons + dt(D+F))
+                    // (:114-116, :148-150)
+                    o[l] = STAGE1 ? uc[l] + dt * (D[l] + F[l]) : ra * rkb[l] + rb * (uc[l] + dt * (D[l] + F[l]));
+                    at(out + l * cg + zk, own8) = o[l];
+                }
+                if (QOUT) {  // cpu/ctoprim.cpp:23-38
+                    double u, v, w, eint, p;
+                    ctoprim_cell(o[IRHO], o[IMX], o[IMY], o[IMZ], o[IENE], u, v, w, eint, p);
+                    double *qk = q + zk;
+                    at(qk, own8) = o[IRHO];
+                    at(qk + QU * cg, own8) = u;
+                    at(qk + QV * cg, own8) = v;
+                    at(qk + QW * cg, own8) = w;
+                    at(qk + QPRES * cg, own8) = p;
+                    at(qk + QTEMP * cg, own8) = eint / CV;
+                }
+            }
+        }
+        __syncthreads();  // A
+    }
+}
+
+// z runs.  A CU holds one workgroup, so a launch takes ceil(workgroups / 256) rounds of
+// (planes + the window fill, which costs about kFill planes: 18 us of 6.7 us a plane); the run
+// length that makes this smallest is taken.
+constexpr int kCUs = 256;
+constexpr double kFill = 2.5;
+
+int stage_kz(const Geom &g, int64_t tiles)
+{
+    int best = g.n2;
+    double cost = 1e300;
+    for (int nz = 1; nz <= g.n2; nz++) {
+        const int kz = (g.n2 + nz - 1) / nz, runs = (g.n2 + kz - 1) / kz;
+        const int64_t rounds = (tiles * runs + kCUs - 1) / kCUs;
+        const double c = (double)rounds * (kz + kFill);
+        if (c < cost) {
+            cost = c;
+            best = kz;
+        }
+    }
+    return best;
+}
+
+}  // namespace
+
+bool stage_fits(const Geom &g)
+{
+    return g.pg < (1 << 29) && g.xg < (1 << 24) && g.g1 < (1 << 24);
+}
+
+hipError_t launch_stage(const Geom &g, const double *cons, const double *base, double *out, double *q, double *d,
+                        double *f, const double *dt_dev, const double dxi[3], double eta, double alam, int phase,
+                        hipStream_t s, const BoxSet &bs)
+{
+    if (bs.n < 1 || !stage_fits(g)) return hipErrorInvalidValue;
+    const StageArgs a{base, out, q, d, f, dt_dev, phase};
+    const int ntx = (g.n0 + TX - 1) / TX, nty = (g.n1 + BY - 1) / BY;
+    const int kz = stage_kz(g, (int64_t)ntx * nty * bs.n);
+    const int64_t nbpb = (int64_t)ntx * nty * ((g.n2 + kz - 1) / kz);
+    if (nbpb * bs.n > 0x7fffffff) return hipErrorInvalidValue;
+    const int nb = (int)(nbpb * bs.n);
+#define STAGE(S1, L, QO) \
+    stage_kernel<S1, L, QO><<<nb, NT, 0, s>>>(g, cons, a, dxi[0], dxi[1], dxi[2], eta, alam, kz, ntx, nty, bs, (int)nbpb)
+    switch (phase) {
+    case 1: STAGE(true, false, false); break;
+    case 2: STAGE(false, false, true); break;
+    case 3: STAGE(false, true, false); break;
+    default: return hipErrorInvalidValue;
+    }
+#undef STAGE
+    return hipGetLastError();
+}
+
+}  // namespace cns
