@@ -1,13 +1,12 @@
 // cns_domain.hip -- multi-box periodic domains (include/cns_domain.h).
 //
 // A domain's boxes all have one geometry and sit back to back in each array, so
-// every kernel of the step covers every box in one launch: the pipelined stencil
-// kernels take the box as the leading part of their workgroup index, the column
-// kernels (ctoprim + wz, wz) as their third grid dimension, and the fill copies
-// ghost cells across boxes.  The step is the fused composition of cns_advance
-// (cns_abi.hip) with the box fill in place of the single-box fill; the Courant
-// maxima of all boxes meet in one accumulator, as BoxLib's parallel_reduce does
-// (fortran90/advance.f90:139).
+// every kernel of the step covers every box in one launch: the stage kernel takes the
+// box as the leading part of its workgroup index, the Courant pass as its second grid
+// dimension, and the fill copies ghost cells across boxes.  The step is the fused
+// composition of cns_advance (cns_abi.hip) with the box fill in place of the single-box
+// fill; the Courant maxima of all boxes meet in one accumulator, as BoxLib's
+// parallel_reduce does (fortran90/advance.f90:139).
 #include <cmath>
 #include <new>
 
@@ -27,7 +26,6 @@ struct cns_domain {
     unsigned long long *d_acc;  // [0] Courant bits, [1] dt, [2] courno
     double *d_dt, *d_courno;
     double *d_stage;  // U^{1/3} of every box (5 ghosted comps per box)
-    double *d_wz;     // wz field of every box
 };
 
 extern "C" {
@@ -71,15 +69,12 @@ int cns_domain_create(cns_domain **out, const int ncell[3], int max_grid_size, c
     D->d_acc = (unsigned long long *)blk;
     D->d_dt = (double *)blk + 1;
     D->d_courno = (double *)blk + 2;
-    const size_t stage = (size_t)nbox * D->bs.su, wz = (size_t)nbox * D->bs.sw;
-    if (hipMalloc((void **)&D->d_stage, stage * sizeof(double)) != hipSuccess ||
-        hipMalloc((void **)&D->d_wz, wz * sizeof(double)) != hipSuccess) {
+    const size_t stage = (size_t)nbox * D->bs.su;
+    if (hipMalloc((void **)&D->d_stage, stage * sizeof(double)) != hipSuccess) {
         (void)hipGetLastError();
-        if (D->d_stage) (void)hipFree(D->d_stage);
         (void)hipFree(blk);
         delete D;
-        return fail(CNS_ENOMEM, "hipMalloc of the %zu-byte stage and wz buffers failed",
-                    (stage + wz) * sizeof(double));
+        return fail(CNS_ENOMEM, "hipMalloc of the %zu-byte stage buffer failed", stage * sizeof(double));
     }
     *out = D;
     return CNS_OK;
@@ -90,7 +85,6 @@ int cns_domain_destroy(cns_domain *D)
     if (!D) return CNS_OK;
     (void)hipFree(D->d_acc);
     (void)hipFree(D->d_stage);
-    (void)hipFree(D->d_wz);
     delete D;
     return CNS_OK;
 }
@@ -137,27 +131,20 @@ int cns_domain_advance(cns_domain *D, double *U, double *Unew, double *Q, double
     const Geom &g = D->g;
     const BoxSet &bs = D->bs;
     const double *dxi = D->dxi;
-    double *T = D->d_stage, *WZ = D->d_wz;
+    double *T = D->d_stage;
     hipStream_t s = current_stream();
-    const unsigned uvwt = (1u << QU) | (1u << QV) | (1u << QW) | (1u << QTEMP);
-    // stage 1 (fortran90/advance.f90:81-262): box fill, ctoprim + Courant over every box
+    // stage 1 (fortran90/advance.f90:81-262): box fill, the Courant number over every box
     CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, U, nullptr, 0u, s));
     CNS_HIPCHK(launch_courno_reset(D->d_acc, 1.0E-50, s));
-    CNS_HIPCHK(launch_ctoprim_wz(g, U, Q, WZ, D->d_acc, D->dx[0], D->dx[1], D->dx[2], dxi[2], false, s, bs));
+    CNS_HIPCHK(launch_courno(g, U, D->d_acc, D->dx[0], D->dx[1], D->dx[2], s, bs));
     CNS_HIPCHK(launch_courno_to_dt(D->d_acc, D->cfl, D->d_dt, D->d_courno, s));
-    CNS_HIPCHK(launch_diffterm_pipe(g, Q, WZ, Dd, dxi[0], dxi[1], dxi[2], D->eta, D->alam, s, false, bs));
-    CNS_HIPCHK(launch_hypterm_cons(g, U, F, dxi[0], dxi[1], dxi[2], Dd, U, T, D->d_dt, 1, false, Q, 1, s, bs));
-    // stage 2 (:264-336): the stage kernel stored u, v, w, T of U^{1/3}; the fill
-    // takes them across boxes with the state
-    CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, T, Q, uvwt, s));
-    CNS_HIPCHK(launch_wz(g, Q, WZ, dxi[2], s, bs));
-    CNS_HIPCHK(launch_diffterm_pipe(g, Q, WZ, Dd, dxi[0], dxi[1], dxi[2], D->eta, D->alam, s, false, bs));
-    CNS_HIPCHK(launch_hypterm_cons(g, T, F, dxi[0], dxi[1], dxi[2], Dd, U, Unew, D->d_dt, 2, false, Q, 2, s, bs));
+    CNS_HIPCHK(launch_stage(g, U, U, T, Q, Dd, F, D->d_dt, dxi, D->eta, D->alam, 1, s, bs));
+    // stage 2 (:264-336), which also stores the primitives of its result
+    CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, T, nullptr, 0u, s));
+    CNS_HIPCHK(launch_stage(g, T, U, Unew, Q, Dd, F, D->d_dt, dxi, D->eta, D->alam, 2, s, bs));
     // stage 3 (:338-410)
     CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, Unew, Q, (1u << NQ) - 1u, s));
-    CNS_HIPCHK(launch_wz(g, Q, WZ, dxi[2], s, bs));
-    CNS_HIPCHK(launch_diffterm_pipe(g, Q, WZ, Dd, dxi[0], dxi[1], dxi[2], D->eta, D->alam, s, true, bs));
-    CNS_HIPCHK(launch_hypterm_cons(g, Unew, F, dxi[0], dxi[1], dxi[2], Dd, U, U, D->d_dt, 3, true, nullptr, 0, s, bs));
+    CNS_HIPCHK(launch_stage(g, Unew, U, U, Q, Dd, F, D->d_dt, dxi, D->eta, D->alam, 3, s, bs));
     double h[2];
     CNS_HIPCHK(hipMemcpyAsync(h, D->d_dt, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
     CNS_HIPCHK(hipStreamSynchronize(s));

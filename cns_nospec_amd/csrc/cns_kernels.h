@@ -7,11 +7,11 @@ namespace cns {
 
 // A set of n boxes of one geometry stored back to back: box b of an array starts
 // b * stride doubles after box 0, with stride su for 5-component ghosted arrays (U),
-// sq for 6-component ghosted ones (Q), sc for 5-component interior ones (D, F) and
-// sw for the one-component ghosted wz field.  The default is a single box.
+// sq for 6-component ghosted ones (Q), sc for 5-component interior ones (D, F).  The
+// default is a single box.
 struct BoxSet {
     int n = 1;
-    int64_t su = 0, sq = 0, sc = 0, sw = 0;
+    int64_t su = 0, sq = 0, sc = 0;
 };
 inline BoxSet box_set(const Geom &g, int n)
 {
@@ -20,7 +20,6 @@ inline BoxSet box_set(const Geom &g, int n)
     b.su = NC * g.cg;
     b.sq = NQ * g.cg;
     b.sc = NC * g.c;
-    b.sw = g.cg;
     return b;
 }
 
@@ -84,32 +83,14 @@ hipError_t launch_diffterm_tiled(const Geom &g, const double *q, double *difflux
 // later).  diffterm reads wz, a one-component ghosted array filled by launch_wz from
 // the same q.
 bool pipe_aligned(const void *p);
-
-
 hipError_t launch_hypterm_pipe(const Geom &g, const double *cons, const double *q, double *flux,
                                double dxi0, double dxi1, double dxi2, const double *d,
                                const double *base, double *out, const double *dt_dev, int phase,
                                bool write_f, hipStream_t s);
-// The same fused stage reading only cons (phases 1..3): u, v, w, p are derived from it
-// with ctoprim's arithmetic, so it equals launch_hypterm_pipe with q = ctoprim(cons).
-// qout (with write_f false): ctoprim of the result on interior cells into qout, u, v,
-// w and T (qout_kind 1) or all six components (2); 0 or a null qout stores none.
-hipError_t launch_hypterm_cons(const Geom &g, const double *cons, double *flux, double dxi0,
-                               double dxi1, double dxi2, const double *d, const double *base,
-                               double *out, const double *dt_dev, int phase, bool write_f,
-                               double *qout, int qout_kind, hipStream_t s, const BoxSet &bs = BoxSet());
-hipError_t launch_wz(const Geom &g, const double *q, double *wz, double dxi2, hipStream_t s,
-                     const BoxSet &bs = BoxSet());
-// ctoprim (as launch_ctoprim, full or u, v, w, T only) that also writes the wz field of
-// launch_wz from the same state, in one z-marching pass.
-hipError_t launch_ctoprim_wz(const Geom &g, const double *u, double *q, double *wz,
-                             unsigned long long *acc, double dx0, double dx1, double dx2, double dxi2,
-                             bool full, hipStream_t s, const BoxSet &bs = BoxSet());
-// write_rho = false leaves difflux's rho row (always 0.0) unwritten, for a caller that
-// stores it once and never reads it in between.
+hipError_t launch_wz(const Geom &g, const double *q, double *wz, double dxi2, hipStream_t s);
 hipError_t launch_diffterm_pipe(const Geom &g, const double *q, const double *wz, double *difflux,
                                 double dxi0, double dxi1, double dxi2, double eta, double alam,
-                                hipStream_t s, bool write_rho = true, const BoxSet &bs = BoxSet());
+                                hipStream_t s);
 
 // One RK stage in one kernel (cns_stage.hip): out = the SSP-RK3 update of phase 1..3 of the
 // ghosted state cons with base U^n (phases 2 and 3), its primitives into q (phase 2), D and
