@@ -363,7 +363,7 @@ int cns_fill_boundary(double *u, const int dim[3], const int dim_g[3])
             return fail(CNS_EINVAL, "dim_g[%d] = %d, expected %d", d, dim_g[d], dim[d] + 2 * NG);
     }
     Geom g = make_geom(dim[0], dim[1], dim[2]);
-    HIPCHK(launch_fill_boundary(g, u, t_stream));
+    HIPCHK(launch_fill_boundary(g, u, nullptr, t_stream));
     return CNS_OK;
 }
 
@@ -550,32 +550,32 @@ int cns_advance_async(cns_ctx *ctx, double *U, double *Unew, double *Q, double *
             // nothing.  Stage 2 also stores the primitives of its result, the Q the
             // reference leaves; the last fill copies their ghosts with the state's.
             const double *dxi = ctx->dxi;
-            TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, s));
+            TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, nullptr, s));
             HIPCHK(launch_courno_reset(ctx->d_acc, 1.0E-50, s));
             TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_courno(g, U, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
             HIPCHK(launch_courno_to_dt(ctx->d_acc, ctx->cfl, dt, courno_dev ? courno_dev : ctx->d_courno, s));
             TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, U, U, T, Q, D, F, dt, dxi, ctx->eta, ctx->alam, 1, s));
-            TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, T, s));
+            TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, T, nullptr, s));
             TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, T, U, Unew, Q, D, F, dt, dxi, ctx->eta, ctx->alam, 2, s));
-            TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary_q(g, Unew, Q, (1u << NQ) - 1u, s));
+            TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, Q, s));
             TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, Unew, U, U, Q, D, F, dt, dxi, ctx->eta, ctx->alam, 3, s));
             return CNS_OK;
         }
         // Arrays that are not 16-byte aligned, or too large for its offsets: fill, ctoprim,
         // diffterm, and hypterm with the RK update of its cell applied in the same pass.
-        TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, s));
+        TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, nullptr, s));
         HIPCHK(launch_courno_reset(ctx->d_acc, 1.0E-50, s));
         TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, U, Q, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
         HIPCHK(launch_courno_to_dt(ctx->d_acc, ctx->cfl, dt, courno_dev ? courno_dev : ctx->d_courno, s));
         TIMED(ctx, CNS_PROF_DIFFTERM, s, stencil_diffterm(g, Q, D, ctx->dxi, ctx->eta, ctx->alam, ctx->d_wz, s));
         TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, U, Q, F, ctx->dxi, D, U, T, dt, 1, false, s));
 
-        TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, T, s));
+        TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, T, nullptr, s));
         TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, T, Q, nullptr, 0.0, 0.0, 0.0, s));
         TIMED(ctx, CNS_PROF_DIFFTERM, s, stencil_diffterm(g, Q, D, ctx->dxi, ctx->eta, ctx->alam, ctx->d_wz, s));
         TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, T, Q, F, ctx->dxi, D, U, Unew, dt, 2, false, s));
 
-        TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, s));
+        TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, nullptr, s));
         TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, Unew, Q, nullptr, 0.0, 0.0, 0.0, s));
         TIMED(ctx, CNS_PROF_DIFFTERM, s, stencil_diffterm(g, Q, D, ctx->dxi, ctx->eta, ctx->alam, ctx->d_wz, s));
         TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, Unew, Q, F, ctx->dxi, D, U, U, dt, 3, true, s));
@@ -583,7 +583,7 @@ int cns_advance_async(cns_ctx *ctx, double *U, double *Unew, double *Q, double *
     }
     // Unfused composition, kernel for kernel as the reference.
     // cpu/advance.cpp:45-85: stage 1
-    TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, s));
+    TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, nullptr, s));
     HIPCHK(launch_courno_reset(ctx->d_acc, 1.0E-50, s));
     TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, U, Q, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
     HIPCHK(launch_courno_to_dt(ctx->d_acc, ctx->cfl, dt, courno_dev ? courno_dev : ctx->d_courno, s));
@@ -591,13 +591,13 @@ int cns_advance_async(cns_ctx *ctx, double *U, double *Unew, double *Q, double *
     TIMED(ctx, CNS_PROF_HYPTERM, s, stencil_hypterm(g, U, Q, F, ctx->dxi, s));
     TIMED(ctx, CNS_PROF_RK, s, launch_rk_update(g, 1, U, Unew, D, F, dt, 0.0, s));
     // :90-119: stage 2
-    TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, s));
+    TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, nullptr, s));
     TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, Unew, Q, nullptr, 0.0, 0.0, 0.0, s));
     TIMED(ctx, CNS_PROF_DIFFTERM, s, stencil_diffterm(g, Q, D, ctx->dxi, ctx->eta, ctx->alam, ctx->d_wz, s));
     TIMED(ctx, CNS_PROF_HYPTERM, s, stencil_hypterm(g, Unew, Q, F, ctx->dxi, s));
     TIMED(ctx, CNS_PROF_RK, s, launch_rk_update(g, 2, U, Unew, D, F, dt, 0.0, s));
     // :124-153: stage 3
-    TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, s));
+    TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, nullptr, s));
     TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, Unew, Q, nullptr, 0.0, 0.0, 0.0, s));
     TIMED(ctx, CNS_PROF_DIFFTERM, s, stencil_diffterm(g, Q, D, ctx->dxi, ctx->eta, ctx->alam, ctx->d_wz, s));
     TIMED(ctx, CNS_PROF_HYPTERM, s, stencil_hypterm(g, Unew, Q, F, ctx->dxi, s));

@@ -118,7 +118,7 @@ size_t cns_domain_array_len(const cns_domain *D, int ncomp, int ghosted)
 int cns_domain_fill_boundary(cns_domain *D, double *U)
 {
     if (!D || !U) return fail(CNS_EINVAL, "NULL argument");
-    CNS_HIPCHK(launch_domain_fill(D->g, D->bs, D->nb, U, nullptr, 0u, current_stream()));
+    CNS_HIPCHK(launch_domain_fill(D->g, D->bs, D->nb, U, nullptr, current_stream()));
     return CNS_OK;
 }
 
@@ -134,16 +134,16 @@ int cns_domain_advance(cns_domain *D, double *U, double *Unew, double *Q, double
     double *T = D->d_stage;
     hipStream_t s = current_stream();
     // stage 1 (fortran90/advance.f90:81-262): box fill, the Courant number over every box
-    CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, U, nullptr, 0u, s));
+    CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, U, nullptr, s));
     CNS_HIPCHK(launch_courno_reset(D->d_acc, 1.0E-50, s));
     CNS_HIPCHK(launch_courno(g, U, D->d_acc, D->dx[0], D->dx[1], D->dx[2], s, bs));
     CNS_HIPCHK(launch_courno_to_dt(D->d_acc, D->cfl, D->d_dt, D->d_courno, s));
     CNS_HIPCHK(launch_stage(g, U, U, T, Q, Dd, F, D->d_dt, dxi, D->eta, D->alam, 1, s, bs));
     // stage 2 (:264-336), which also stores the primitives of its result
-    CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, T, nullptr, 0u, s));
+    CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, T, nullptr, s));
     CNS_HIPCHK(launch_stage(g, T, U, Unew, Q, Dd, F, D->d_dt, dxi, D->eta, D->alam, 2, s, bs));
     // stage 3 (:338-410)
-    CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, Unew, Q, (1u << NQ) - 1u, s));
+    CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, Unew, Q, s));
     CNS_HIPCHK(launch_stage(g, Unew, U, U, Q, Dd, F, D->d_dt, dxi, D->eta, D->alam, 3, s, bs));
     double h[2];
     CNS_HIPCHK(hipMemcpyAsync(h, D->d_dt, 2 * sizeof(double), hipMemcpyDeviceToHost, s));

@@ -23,18 +23,15 @@ inline BoxSet box_set(const Geom &g, int n)
     return b;
 }
 
-// Ghost shell, closed-form periodic image (cns_kernels.hip).
-hipError_t launch_fill_boundary(const Geom &g, double *u, hipStream_t s);
-// The same periodic fill of u's NC components and of the components of q selected by
-// qmask (bit l for component l), in one pass.
-hipError_t launch_fill_boundary_q(const Geom &g, double *u, double *q, unsigned qmask, hipStream_t s);
+// Ghost shell of u (5 components) and, when not null, of q (6), closed-form periodic image
+// (cns_kernels.hip).
+hipError_t launch_fill_boundary(const Geom &g, double *u, double *q, hipStream_t s);
 // The periodic fill of a domain of nb[0] x nb[1] x nb[2] boxes (box b = I + nb[0]*(J +
 // nb[1]*K) at cell origin (I*n0, J*n1, K*n2)): each ghost cell of each box gets the
 // domain cell at the periodic image of its global index, from whichever box holds
-// it (multifab_fill_boundary, fortran90/advance.f90:81); u and the qmask components
-// of q, as launch_fill_boundary_q.  With one box it equals launch_fill_boundary_q.
-hipError_t launch_domain_fill(const Geom &g, const BoxSet &bs, const int nb[3], double *u, double *q,
-                              unsigned qmask, hipStream_t s);
+// it (multifab_fill_boundary, fortran90/advance.f90:81).  With one box it equals
+// launch_fill_boundary.
+hipError_t launch_domain_fill(const Geom &g, const BoxSet &bs, const int nb[3], double *u, double *q, hipStream_t s);
 
 // Resets a Courant accumulator slot to the bits of max(init, 0) (cns_kernels.hip).
 hipError_t launch_courno_reset(unsigned long long *acc, double init, hipStream_t s);

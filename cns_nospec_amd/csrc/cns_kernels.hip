@@ -22,11 +22,6 @@ inline int stream_grid(int64_t work, int per_thread = 4)
     return (int)blocks;
 }
 
-__device__ __forceinline__ int wrap_ghost(int a, int n)
-{
-    return a < NG ? a + n : (a >= n + NG ? a - n : a);
-}
-
 // ------------------------------------------------------------------ ghost fill
 // The reference fills the ghost shell in three ordered copy passes (z planes over
 // interior i,j; y planes over interior i and all k; x columns over all j,k:
@@ -35,117 +30,100 @@ __device__ __forceinline__ int wrap_ghost(int a, int n)
 // of all three of its indices, so one pass over the shell copies exactly the same
 // values.  The shell is enumerated compactly: first the full rows whose j or k is
 // a ghost index (g0 cells each), then the 2*NG ghost cells of each interior row.
-__global__ void __launch_bounds__(kStreamBlock)
-fill_boundary_kernel(Geom g, double *__restrict__ u, double *__restrict__ q, unsigned qmask,
-                     int64_t n_rows_a, int64_t total)
+//
+// One thread per ghost cell, its components' loads all in flight before the first store.
+// What bounds it: at small boxes latency, so the index arithmetic is 32-bit with
+// precomputed quotients; at large ones the x ghosts, whose four-cell pieces touch
+// two 128-byte lines per row and component.
+struct Shell {
+    FastDiv g0, g1, n1, nbx, nby;
+    unsigned plane_rows, elems_a, total;  // rows of the ghost planes; cells of the full rows; all cells
+};
+
+Shell make_shell(const Geom &g, const int nb[3])
 {
-    const int64_t plane_rows = (int64_t)2 * NG * g.g1;
-    const int64_t elems_a = n_rows_a * g.g0;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        int i, j, k;
-        if (e < elems_a) {
-            int64_t r = e / g.g0;
-            i = (int)(e - r * g.g0);
-            if (r < plane_rows) {
-                int kk = (int)(r / g.g1);
-                j = (int)(r - (int64_t)kk * g.g1);
-                k = kk < NG ? kk : g.n2 + kk;
-            } else {
-                r -= plane_rows;
-                int kk = (int)(r / (2 * NG));
-                int jj = (int)(r - (int64_t)kk * 2 * NG);
-                k = NG + kk;
-                j = jj < NG ? jj : g.n1 + jj;
-            }
-        } else {
-            int64_t e2 = e - elems_a;
-            int64_t row = e2 / (2 * NG);
-            int ii = (int)(e2 - row * 2 * NG);
-            i = ii < NG ? ii : g.n0 + ii;
-            int kk = (int)(row / g.n1);
-            k = NG + kk;
-            j = NG + (int)(row - (int64_t)kk * g.n1);
-        }
-        const int64_t dst = gidx(g, i, j, k);
-        const int64_t src = gidx(g, wrap_ghost(i, g.n0), wrap_ghost(j, g.n1), wrap_ghost(k, g.n2));
-#pragma unroll
-        for (int l = 0; l < NC; l++) u[l * g.cg + dst] = u[l * g.cg + src];
-#pragma unroll
-        for (int l = 0; l < NQ; l++)
-            if (qmask & (1u << l)) q[l * g.cg + dst] = q[l * g.cg + src];
-    }
+    Shell h;
+    h.g0 = fast_div(g.g0);
+    h.g1 = fast_div(g.g1);
+    h.n1 = fast_div(g.n1);
+    h.nbx = fast_div(nb[0]);
+    h.nby = fast_div(nb[1]);
+    h.plane_rows = 2u * NG * g.g1;
+    h.elems_a = (h.plane_rows + 2u * NG * g.n2) * g.g0;
+    h.total = h.elems_a + 2u * NG * (unsigned)g.n1 * g.n2;
+    return h;
 }
 
-// Ghost cell h of the compact shell enumeration of fill_boundary_kernel, as (i, j, k).
-__device__ __forceinline__ void shell_cell(const Geom &g, int64_t e, int64_t elems_a, int &i, int &j, int &k)
+int64_t shell_cells(const Geom &g)
 {
-    const int64_t plane_rows = (int64_t)2 * NG * g.g1;
-    if (e < elems_a) {
-        int64_t r = e / g.g0;
+    return ((int64_t)2 * NG * g.g1 + (int64_t)2 * NG * g.n2) * g.g0 + (int64_t)2 * NG * g.n1 * g.n2;
+}
+
+// Ghost cell e of the enumeration, as (i, j, k).
+__device__ __forceinline__ void shell_cell(const Geom &g, const Shell &h, unsigned e, int &i, int &j, int &k)
+{
+    if (e < h.elems_a) {
+        unsigned r = h.g0.div(e);
         i = (int)(e - r * g.g0);
-        if (r < plane_rows) {
-            const int kk = (int)(r / g.g1);
-            j = (int)(r - (int64_t)kk * g.g1);
+        if (r < h.plane_rows) {
+            const int kk = (int)h.g1.div(r);
+            j = (int)r - kk * g.g1;
             k = kk < NG ? kk : g.n2 + kk;
         } else {
-            r -= plane_rows;
-            const int kk = (int)(r / (2 * NG));
-            const int jj = (int)(r - (int64_t)kk * 2 * NG);
-            k = NG + kk;
+            r -= h.plane_rows;
+            const int jj = (int)(r & (2 * NG - 1));
+            k = NG + (int)(r / (2 * NG));
             j = jj < NG ? jj : g.n1 + jj;
         }
     } else {
-        const int64_t e2 = e - elems_a;
-        const int64_t row = e2 / (2 * NG);
-        const int ii = (int)(e2 - row * 2 * NG);
+        const unsigned e2 = e - h.elems_a, row = e2 / (2 * NG), kk = h.n1.div(row);
+        const int ii = (int)(e2 & (2 * NG - 1));
         i = ii < NG ? ii : g.n0 + ii;
-        const int kk = (int)(row / g.n1);
-        k = NG + kk;
-        j = NG + (int)(row - (int64_t)kk * g.n1);
+        k = NG + (int)kk;
+        j = NG + (int)(row - kk * g.n1);
     }
 }
 
-// One axis of the domain fill: ghost index a (0 <= a < n + 2 NG) of box I of nb
-// boxes of n cells -> the box I' and ghosted index a' holding the periodic image.
-__device__ __forceinline__ void domain_image(int a, int I, int n, int nb, int &Is, int &as)
+// One axis of a ghost cell at index a of box I of nb boxes of n cells: the box (relative
+// step dI) and the index there of the cell it is the periodic image of.  Extents are at
+// least NG, so that is the neighbouring box.
+__device__ __forceinline__ int image(int a, int I, int n, int nb, int &dI)
 {
-    const int N = n * nb;
-    int G = I * n + a - NG;  // global cell index, in [-NG, N + NG)
-    G = G < 0 ? G + N : (G >= N ? G - N : G);
-    Is = G / n;
-    as = G - Is * n + NG;
+    dI = a < NG ? (I == 0 ? nb - 1 : -1) : (a >= n + NG ? (I == nb - 1 ? 1 - nb : 1) : 0);
+    return a < NG ? a + n : (a >= n + NG ? a - n : a);
 }
 
-// Domain fill: one y-row of the grid per box (blockIdx.y), grid-stride over its shell.
+// Box blockIdx.y of a set of nb[0] x nb[1] x nb[2] boxes (one box: its own images).  Q: the
+// components of q as well.
+template <bool Q>
 __global__ void __launch_bounds__(kStreamBlock)
-domain_fill_kernel(Geom g, BoxSet bs, int nbx, int nby, int nbz, double *__restrict__ u,
-                   double *__restrict__ q, unsigned qmask, int64_t n_rows_a, int64_t total)
+fill_kernel(Geom g, Shell h, BoxSet bs, int nbx, int nby, int nbz, double *__restrict__ u, double *__restrict__ q)
 {
-    const int b = blockIdx.y;
-    const int I = b % nbx, J = (b / nbx) % nby, K = b / (nbx * nby);
-    const int64_t elems_a = n_rows_a * g.g0;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        int i, j, k;
-        shell_cell(g, e, elems_a, i, j, k);
-        int Is, Js, Ks, is, js, ks;
-        domain_image(i, I, g.n0, nbx, Is, is);
-        domain_image(j, J, g.n1, nby, Js, js);
-        domain_image(k, K, g.n2, nbz, Ks, ks);
-        const int bsrc = Is + nbx * (Js + nby * Ks);
-        const int64_t dst = gidx(g, i, j, k), src = gidx(g, is, js, ks);
-        double *ud = u + b * bs.su;
-        const double *us = u + bsrc * bs.su;
+    const unsigned e = blockIdx.x * kStreamBlock + threadIdx.x;
+    if (e >= h.total) return;
+    const unsigned b = blockIdx.y, r = h.nbx.div(b);
+    const int K = (int)h.nby.div(r), J = (int)r - K * nby, I = (int)b - (int)r * nbx;
+    int i, j, k, dI, dJ, dK;
+    shell_cell(g, h, e, i, j, k);
+    const int is = image(i, I, g.n0, nbx, dI), js = image(j, J, g.n1, nby, dJ), ks = image(k, K, g.n2, nbz, dK);
+    const int64_t bsrc = (int64_t)b + dI + (int64_t)nbx * (dJ + (int64_t)nby * dK);
+    const int64_t dst = gidx(g, i, j, k), src = gidx(g, is, js, ks);
+    const double *us = u + bsrc * bs.su + src;
+    double *ud = u + b * bs.su + dst;
+    double v[NC], w[NQ];
 #pragma unroll
-        for (int l = 0; l < NC; l++) ud[l * g.cg + dst] = us[l * g.cg + src];
-        if (qmask) {
-            double *qd = q + b * bs.sq;
-            const double *qs = q + bsrc * bs.sq;
+    for (int l = 0; l < NC; l++) v[l] = us[l * g.cg];
+    if (Q) {
+        const double *qs = q + bsrc * bs.sq + src;
 #pragma unroll
-            for (int l = 0; l < NQ; l++)
-                if (qmask & (1u << l)) qd[l * g.cg + dst] = qs[l * g.cg + src];
-        }
+        for (int l = 0; l < NQ; l++) w[l] = qs[l * g.cg];
+    }
+#pragma unroll
+    for (int l = 0; l < NC; l++) ud[l * g.cg] = v[l];
+    if (Q) {
+        double *qd = q + b * bs.sq + dst;
+#pragma unroll
+        for (int l = 0; l < NQ; l++) qd[l * g.cg] = w[l];
     }
 }
 
@@ -455,37 +433,24 @@ diffterm_direct_kernel(Geom g, const double *__restrict__ q, double *__restrict_
 }  // namespace
 
 // ------------------------------------------------------------------ launchers
-hipError_t launch_fill_boundary(const Geom &g, double *u, hipStream_t s)
+hipError_t launch_domain_fill(const Geom &g, const BoxSet &bs, const int nb[3], double *u, double *q, hipStream_t s)
 {
-    const int64_t rows_a = (int64_t)2 * NG * g.g1 + (int64_t)g.n2 * 2 * NG;
-    const int64_t total = rows_a * g.g0 + (int64_t)g.n1 * g.n2 * 2 * NG;
-    fill_boundary_kernel<<<stream_grid(total, 2), kStreamBlock, 0, s>>>(g, u, nullptr, 0u, rows_a, total);
+    const int64_t total = shell_cells(g);
+    if (bs.n != nb[0] * nb[1] * nb[2] || bs.n < 1 || bs.n > 65535 || total > 0xffffffffll - kStreamBlock)
+        return hipErrorInvalidValue;
+    const Shell h = make_shell(g, nb);
+    const dim3 grid((unsigned)((total + kStreamBlock - 1) / kStreamBlock), (unsigned)bs.n);
+    if (q)
+        fill_kernel<true><<<grid, kStreamBlock, 0, s>>>(g, h, bs, nb[0], nb[1], nb[2], u, q);
+    else
+        fill_kernel<false><<<grid, kStreamBlock, 0, s>>>(g, h, bs, nb[0], nb[1], nb[2], u, nullptr);
     return hipGetLastError();
 }
 
-hipError_t launch_fill_boundary_q(const Geom &g, double *u, double *q, unsigned qmask, hipStream_t s)
+hipError_t launch_fill_boundary(const Geom &g, double *u, double *q, hipStream_t s)
 {
-    if (!q) qmask = 0;
-    const int64_t rows_a = (int64_t)2 * NG * g.g1 + (int64_t)g.n2 * 2 * NG;
-    const int64_t total = rows_a * g.g0 + (int64_t)g.n1 * g.n2 * 2 * NG;
-    fill_boundary_kernel<<<stream_grid(total, 2), kStreamBlock, 0, s>>>(g, u, q, qmask & 63u, rows_a, total);
-    return hipGetLastError();
-}
-
-hipError_t launch_domain_fill(const Geom &g, const BoxSet &bs, const int nb[3], double *u, double *q,
-                              unsigned qmask, hipStream_t s)
-{
-    if (!q) qmask = 0;
-    if (bs.n != nb[0] * nb[1] * nb[2] || bs.n < 1 || bs.n > 65535) return hipErrorInvalidValue;
-    const int64_t rows_a = (int64_t)2 * NG * g.g1 + (int64_t)g.n2 * 2 * NG;
-    const int64_t total = rows_a * g.g0 + (int64_t)g.n1 * g.n2 * 2 * NG;
-    int gx = stream_grid(total, 2);
-    // a few waves per box keep the whole grid resident on small boxes
-    const int64_t want = (int64_t)(gx + bs.n - 1) / bs.n;
-    gx = (int)(want < 1 ? 1 : want);
-    const dim3 grid((unsigned)gx, (unsigned)bs.n);
-    domain_fill_kernel<<<grid, kStreamBlock, 0, s>>>(g, bs, nb[0], nb[1], nb[2], u, q, qmask & 63u, rows_a, total);
-    return hipGetLastError();
+    const int one[3] = {1, 1, 1};
+    return launch_domain_fill(g, BoxSet(), one, u, q, s);
 }
 
 hipError_t launch_courno_reset(unsigned long long *acc, double init, hipStream_t s)
