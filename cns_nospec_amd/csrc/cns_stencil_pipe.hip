@@ -401,24 +401,31 @@ diffterm_pipe_kernel(Geom g, const double *__restrict__ q, const double *__restr
     }
 }
 
-// z runs: enough workgroups to fill 256 CUs several times over, with runs long enough
-// that the 8-plane window warm-up stays a small overhead; small boxes then shorten the
-// runs down to 4 planes until a launch has 256 workgroups (64^3 step 0.60 -> 0.40 ms,
-// 32^3 0.55 -> 0.35 ms; at 128^3, with 512 workgroups at runs of 16, shorter runs are
-// slower).
+// z runs.  A launch takes ceil(workgroups / slots) rounds of (planes + the window fill, which
+// costs `warm` planes: its prologue differences u and v of eight planes for diffterm, 3,
+// and only loads for hypterm, 1); the run length that makes this smallest is taken, and of
+// runs within 1 % the shortest, which start their neighbours' planes closer in time.  Halving
+// until 2048 workgroups, as before, left a last round nearly empty or the runs at twice
+// the fill: diffterm 324 -> 272 us at 200x180x160, 76 -> 54 us at 130x97x61, 712 -> 655 us at
+// 256^3; hypterm 58 -> 39 us at 130x97x61.
 // CNS_PIPE_KZ in the environment caps the run length (for measurements).
-int pipe_kz(const Geom &g, int tiles_xy)
+int pipe_kz(const Geom &g, int64_t tiles, int slots, int warm)
 {
-    int kz = g.n2;
     static const int cap = [] {
         const char *e = getenv("CNS_PIPE_KZ");
         return e ? atoi(e) : 0;
     }();
-    if (cap >= 4 && kz > cap) kz = cap;
-    auto blocks = [&](int z) { return (int64_t)tiles_xy * ((g.n2 + z - 1) / z); };
-    while (kz > 16 && blocks(kz) < 2048) kz = (kz + 1) / 2;
-    while (kz > 4 && blocks(kz) < 256) kz = (kz + 1) / 2;
-    return kz;
+    const int most = cap >= 4 && cap < g.n2 ? cap : g.n2;
+    int best = most;
+    int64_t cost = INT64_MAX / 2;
+    for (int nz = (g.n2 + most - 1) / most; nz <= g.n2; nz++) {
+        const int kz = (g.n2 + nz - 1) / nz, runs = (g.n2 + kz - 1) / kz;
+        const int64_t c = (tiles * runs + slots - 1) / slots * (kz + warm);
+        if (c > cost + cost / 100) continue;
+        best = kz;
+        if (c < cost) cost = c;
+    }
+    return best;
 }
 
 // The stencils run on 32 x 8 tiles, two workgroups per CU (512^3: diffterm
@@ -436,7 +443,7 @@ hipError_t launch_hyp_pipe_shape(const Geom &g, const double *cons, const double
                                  const double *dt_dev, int phase, bool write_f, hipStream_t s)
 {
     const int ntx = (g.n0 + S::TX - 1) / S::TX, nty = (g.n1 + S::BY - 1) / S::BY;
-    const int kz = pipe_kz(g, ntx * nty);
+    const int kz = pipe_kz(g, (int64_t)ntx * nty, S::TX == 32 ? 512 : 256, 1);
     const int nb = ntx * nty * ((g.n2 + kz - 1) / kz);
     PipeRk rk{d, base, out, dt_dev, phase};
     const bool stage1 = phase == 1 && base == cons;
@@ -459,7 +466,7 @@ hipError_t launch_diffterm_shape(const Geom &g, const double *q, const double *w
                                  hipStream_t s)
 {
     const int ntx = (g.n0 + S::TX - 1) / S::TX, nty = (g.n1 + S::BY - 1) / S::BY;
-    const int kz = pipe_kz(g, ntx * nty);
+    const int kz = pipe_kz(g, (int64_t)ntx * nty, S::TX == 32 ? 512 : 256, 3);
     const int nb = ntx * nty * ((g.n2 + kz - 1) / kz);
     diffterm_pipe_kernel<S><<<nb, S::NT, 0, s>>>(g, q, wz, difflux, dxi0, dxi1, dxi2, eta, alam, kz, ntx, nty);
     return hipGetLastError();
