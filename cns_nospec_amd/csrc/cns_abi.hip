@@ -290,9 +290,10 @@ struct cns_ctx {
     double dx[3], dxi[3];
     double cfl, eta, alam;
     int device;
-    // one device block: [0] Courant accumulator bits, [1] dt, [2] courno
+    // one device block: [0] Courant accumulator bits (zero between steps), [1] dt, [2] courno
     unsigned long long *d_acc;
     double *d_dt, *d_courno;
+    double *h_dt;  // dt and courno of cns_advance, written by the device (pinned)
     // Stage buffer of the fused step (ghosted, 5 comps): holds U^{1/3}, so that the
     // fused hypterm+update never writes an array it reads with halos.  Null when the
     // unfused composition is selected.
@@ -480,21 +481,17 @@ int cns_ctx_create(cns_ctx **ctx, const int ncells[3], const double dx[3], doubl
         delete c;
         return fail(CNS_EHIP, "hipGetDevice failed");
     }
-    void *blk = nullptr;
-    if (hipMalloc(&blk, 4 * sizeof(double)) != hipSuccess) {
+    if (step_dt_alloc(&c->d_acc, &c->d_dt, &c->d_courno, &c->h_dt)) {
         delete c;
-        return fail(CNS_ENOMEM, "hipMalloc of the context block failed");
+        return fail(CNS_ENOMEM, "allocation of the context block failed");
     }
-    c->d_acc = (unsigned long long *)blk;
-    c->d_dt = (double *)blk + 1;
-    c->d_courno = (double *)blk + 2;
     c->d_stage = nullptr;
     c->d_wz = nullptr;
     if (hipMalloc((void **)&c->d_stage, (size_t)NC * c->g.cg * sizeof(double)) != hipSuccess ||
         hipMalloc((void **)&c->d_wz, (size_t)c->g.cg * sizeof(double)) != hipSuccess) {
         (void)hipGetLastError();
         if (c->d_stage) (void)hipFree(c->d_stage);
-        (void)hipFree(blk);
+        step_dt_free(c->d_acc, c->h_dt);
         delete c;
         return fail(CNS_ENOMEM, "hipMalloc of the %zu-byte stage and wz buffers failed",
                     (size_t)(NC + 1) * c->g.cg * sizeof(double));
@@ -523,20 +520,21 @@ int cns_ctx_set_fused(cns_ctx *ctx, int fused)
 int cns_ctx_destroy(cns_ctx *ctx)
 {
     if (!ctx) return CNS_OK;
-    (void)hipFree(ctx->d_acc);
+    step_dt_free(ctx->d_acc, ctx->h_dt);
     if (ctx->d_stage) (void)hipFree(ctx->d_stage);
     if (ctx->d_wz) (void)hipFree(ctx->d_wz);
     delete ctx;
     return CNS_OK;
 }
 
-int cns_advance_async(cns_ctx *ctx, double *U, double *Unew, double *Q, double *D, double *F,
-                      double *dt_dev, double *courno_dev)
+}  // extern "C"
+
+// Enqueues one step; sd.acc is zero before it and after it.
+static int enqueue_step(cns_ctx *ctx, double *U, double *Unew, double *Q, double *D, double *F, const StepDt &sd,
+                        hipStream_t s)
 {
-    if (!ctx || !U || !Unew || !Q || !D || !F) return fail(CNS_EINVAL, "NULL argument");
     const Geom &g = ctx->g;
-    hipStream_t s = t_stream;
-    double *dt = dt_dev ? dt_dev : ctx->d_dt;
+    const double *dt = sd.dt;
     if (ctx->d_stage) {
         // Fused composition.  Stage results go to a buffer the stage does not read with halos:
         //   stage 1: U -> stage (U^{1/3});  stage 2: stage -> Unew (U^{2/3});
@@ -550,23 +548,19 @@ int cns_advance_async(cns_ctx *ctx, double *U, double *Unew, double *Q, double *
             // nothing.  Stage 2 also stores the primitives of its result, the Q the
             // reference leaves; the last fill copies their ghosts with the state's.
             const double *dxi = ctx->dxi;
-            TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, nullptr, s));
-            HIPCHK(launch_courno_reset(ctx->d_acc, 1.0E-50, s));
-            TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_courno(g, U, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
-            HIPCHK(launch_courno_to_dt(ctx->d_acc, ctx->cfl, dt, courno_dev ? courno_dev : ctx->d_courno, s));
-            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, U, U, T, Q, D, F, dt, dxi, ctx->eta, ctx->alam, 1, s));
+            TIMED(ctx, CNS_PROF_FILL_CTOPRIM, s, launch_fill_courno(g, U, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
+            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, U, U, T, Q, D, F, sd, dxi, ctx->eta, ctx->alam, 1, s));
             TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, T, nullptr, s));
-            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, T, U, Unew, Q, D, F, dt, dxi, ctx->eta, ctx->alam, 2, s));
+            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, T, U, Unew, Q, D, F, sd, dxi, ctx->eta, ctx->alam, 2, s));
             TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, Q, s));
-            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, Unew, U, U, Q, D, F, dt, dxi, ctx->eta, ctx->alam, 3, s));
+            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, Unew, U, U, Q, D, F, sd, dxi, ctx->eta, ctx->alam, 3, s));
             return CNS_OK;
         }
         // Arrays that are not 16-byte aligned, or too large for its offsets: fill, ctoprim,
         // diffterm, and hypterm with the RK update of its cell applied in the same pass.
         TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, nullptr, s));
-        HIPCHK(launch_courno_reset(ctx->d_acc, 1.0E-50, s));
-        TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, U, Q, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
-        HIPCHK(launch_courno_to_dt(ctx->d_acc, ctx->cfl, dt, courno_dev ? courno_dev : ctx->d_courno, s));
+            TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, U, Q, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
+        HIPCHK(launch_courno_to_dt(sd, s));
         TIMED(ctx, CNS_PROF_DIFFTERM, s, stencil_diffterm(g, Q, D, ctx->dxi, ctx->eta, ctx->alam, ctx->d_wz, s));
         TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, U, Q, F, ctx->dxi, D, U, T, dt, 1, false, s));
 
@@ -584,9 +578,8 @@ int cns_advance_async(cns_ctx *ctx, double *U, double *Unew, double *Q, double *
     // Unfused composition, kernel for kernel as the reference.
     // cpu/advance.cpp:45-85: stage 1
     TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, nullptr, s));
-    HIPCHK(launch_courno_reset(ctx->d_acc, 1.0E-50, s));
     TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, U, Q, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
-    HIPCHK(launch_courno_to_dt(ctx->d_acc, ctx->cfl, dt, courno_dev ? courno_dev : ctx->d_courno, s));
+    HIPCHK(launch_courno_to_dt(sd, s));
     TIMED(ctx, CNS_PROF_DIFFTERM, s, stencil_diffterm(g, Q, D, ctx->dxi, ctx->eta, ctx->alam, ctx->d_wz, s));
     TIMED(ctx, CNS_PROF_HYPTERM, s, stencil_hypterm(g, U, Q, F, ctx->dxi, s));
     TIMED(ctx, CNS_PROF_RK, s, launch_rk_update(g, 1, U, Unew, D, F, dt, 0.0, s));
@@ -605,14 +598,32 @@ int cns_advance_async(cns_ctx *ctx, double *U, double *Unew, double *Q, double *
     return CNS_OK;
 }
 
+static int advance(cns_ctx *ctx, double *U, double *Unew, double *Q, double *D, double *F, double *dt_dev,
+                   double *courno_dev, double *host)
+{
+    if (!ctx || !U || !Unew || !Q || !D || !F) return fail(CNS_EINVAL, "NULL argument");
+    const StepDt sd{ctx->d_acc, ctx->cfl, dt_dev ? dt_dev : ctx->d_dt, courno_dev ? courno_dev : ctx->d_courno, host};
+    const int rc = enqueue_step(ctx, U, Unew, Q, D, F, sd, t_stream);
+    // A step cut short may leave its maximum behind.
+    if (rc) (void)launch_courno_reset(ctx->d_acc, 0.0, t_stream);
+    return rc;
+}
+
+extern "C" {
+
+int cns_advance_async(cns_ctx *ctx, double *U, double *Unew, double *Q, double *D, double *F,
+                      double *dt_dev, double *courno_dev)
+{
+    return advance(ctx, U, Unew, Q, D, F, dt_dev, courno_dev, nullptr);
+}
+
 int cns_advance(cns_ctx *ctx, double *U, double *Unew, double *Q, double *D, double *F, double *dt)
 {
     if (!dt) return fail(CNS_EINVAL, "NULL dt");
-    int rc = cns_advance_async(ctx, U, Unew, Q, D, F, nullptr, nullptr);
+    int rc = advance(ctx, U, Unew, Q, D, F, nullptr, nullptr, ctx ? ctx->h_dt : nullptr);
     if (rc) return rc;
-    double h[2];
-    HIPCHK(hipMemcpyAsync(h, ctx->d_dt, 2 * sizeof(double), hipMemcpyDeviceToHost, t_stream));
     HIPCHK(hipStreamSynchronize(t_stream));
+    const double h[2] = {ctx->h_dt[0], ctx->h_dt[1]};
     *dt = h[0];
     if (!std::isfinite(h[1]) || !std::isfinite(h[0]))
         return fail(CNS_ENUMERIC, "non-finite Courant number %g (dt %g)", h[1], h[0]);

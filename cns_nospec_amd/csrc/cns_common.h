@@ -127,4 +127,32 @@ __device__ __forceinline__ unsigned long long courno_bits(double v)
     return b;
 }
 
+// Where a step's dt is: the Courant maximum (bits; zero when a step begins and again when it
+// has ended, so that no launch clears it), dt and the Courant number on the device, and both
+// again in host memory (or null).
+struct StepDt {
+    unsigned long long *acc;
+    double cfl;
+    double *dt, *courno, *host;
+};
+__device__ __forceinline__ void step_dt_store(const StepDt &sd, double dt, double courno)
+{
+    sd.dt[0] = dt;
+    sd.courno[0] = courno;
+    if (sd.host) {
+        sd.host[0] = dt;
+        sd.host[1] = courno;
+    }
+}
+
+// courno = MAX(MAX(courmx,courmy), MAX(courmz, courno_in)) (cpu/ctoprim.cpp:69) with
+// courno_in = 1e-50 (cpu/advance.cpp:52); dt = cfl/courno (cpu/advance.cpp:57-58).
+__device__ __forceinline__ double courno_dt(const unsigned long long *acc, double cfl, double &courno)
+{
+    const double c = __longlong_as_double((long long)acc[0]);
+    courno = c > 1.0E-50 ? c : 1.0E-50;
+    if (!(c == c)) courno = c;
+    return cfl / courno;
+}
+
 }  // namespace cns

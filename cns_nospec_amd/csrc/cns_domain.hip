@@ -23,8 +23,9 @@ struct cns_domain {
     int m;           // max_grid_size
     double dx[3], dxi[3];
     double cfl, eta, alam;
-    unsigned long long *d_acc;  // [0] Courant bits, [1] dt, [2] courno
+    unsigned long long *d_acc;  // Courant bits, zero between steps
     double *d_dt, *d_courno;
+    double *h_dt;               // dt and courno, written by the device (pinned)
     double *d_stage;  // U^{1/3} of every box (5 ghosted comps per box)
 };
 
@@ -60,19 +61,14 @@ int cns_domain_create(cns_domain **out, const int ncell[3], int max_grid_size, c
     D->cfl = cfl;
     D->eta = eta;
     D->alam = alam;
-    void *blk = nullptr;
-    if (hipMalloc(&blk, 4 * sizeof(double)) != hipSuccess) {
-        (void)hipGetLastError();
+    if (step_dt_alloc(&D->d_acc, &D->d_dt, &D->d_courno, &D->h_dt)) {
         delete D;
-        return fail(CNS_ENOMEM, "hipMalloc of the domain block failed");
+        return fail(CNS_ENOMEM, "allocation of the domain block failed");
     }
-    D->d_acc = (unsigned long long *)blk;
-    D->d_dt = (double *)blk + 1;
-    D->d_courno = (double *)blk + 2;
     const size_t stage = (size_t)nbox * D->bs.su;
     if (hipMalloc((void **)&D->d_stage, stage * sizeof(double)) != hipSuccess) {
         (void)hipGetLastError();
-        (void)hipFree(blk);
+        step_dt_free(D->d_acc, D->h_dt);
         delete D;
         return fail(CNS_ENOMEM, "hipMalloc of the %zu-byte stage buffer failed", stage * sizeof(double));
     }
@@ -83,7 +79,7 @@ int cns_domain_create(cns_domain **out, const int ncell[3], int max_grid_size, c
 int cns_domain_destroy(cns_domain *D)
 {
     if (!D) return CNS_OK;
-    (void)hipFree(D->d_acc);
+    step_dt_free(D->d_acc, D->h_dt);
     (void)hipFree(D->d_stage);
     delete D;
     return CNS_OK;
@@ -122,32 +118,44 @@ int cns_domain_fill_boundary(cns_domain *D, double *U)
     return CNS_OK;
 }
 
+}  // extern "C"
+
+static hipError_t enqueue_step(cns_domain *D, double *U, double *Unew, double *Q, double *Dd, double *F, hipStream_t s)
+{
+    const Geom &g = D->g;
+    const BoxSet &bs = D->bs;
+    const double *dxi = D->dxi;
+    double *T = D->d_stage;
+    const StepDt sd{D->d_acc, D->cfl, D->d_dt, D->d_courno, D->h_dt};
+    hipError_t e;
+    // stage 1 (fortran90/advance.f90:81-262): box fill, the Courant number over every box
+    if ((e = launch_fill_courno(g, U, D->d_acc, D->dx[0], D->dx[1], D->dx[2], s, bs, D->nb))) return e;
+    if ((e = launch_stage(g, U, U, T, Q, Dd, F, sd, dxi, D->eta, D->alam, 1, s, bs))) return e;
+    // stage 2 (:264-336), which also stores the primitives of its result
+    if ((e = launch_domain_fill(g, bs, D->nb, T, nullptr, s))) return e;
+    if ((e = launch_stage(g, T, U, Unew, Q, Dd, F, sd, dxi, D->eta, D->alam, 2, s, bs))) return e;
+    // stage 3 (:338-410)
+    if ((e = launch_domain_fill(g, bs, D->nb, Unew, Q, s))) return e;
+    return launch_stage(g, Unew, U, U, Q, Dd, F, sd, dxi, D->eta, D->alam, 3, s, bs);
+}
+
+extern "C" {
+
 int cns_domain_advance(cns_domain *D, double *U, double *Unew, double *Q, double *Dd, double *F,
                        double *dt)
 {
     if (!D || !U || !Unew || !Q || !Dd || !F || !dt) return fail(CNS_EINVAL, "NULL argument");
     for (const void *p : {(const void *)U, (const void *)Unew, (const void *)Q, (const void *)Dd, (const void *)F})
         if (!pipe_aligned(p)) return fail(CNS_EINVAL, "domain arrays must be 16-byte aligned");
-    const Geom &g = D->g;
-    const BoxSet &bs = D->bs;
-    const double *dxi = D->dxi;
-    double *T = D->d_stage;
     hipStream_t s = current_stream();
-    // stage 1 (fortran90/advance.f90:81-262): box fill, the Courant number over every box
-    CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, U, nullptr, s));
-    CNS_HIPCHK(launch_courno_reset(D->d_acc, 1.0E-50, s));
-    CNS_HIPCHK(launch_courno(g, U, D->d_acc, D->dx[0], D->dx[1], D->dx[2], s, bs));
-    CNS_HIPCHK(launch_courno_to_dt(D->d_acc, D->cfl, D->d_dt, D->d_courno, s));
-    CNS_HIPCHK(launch_stage(g, U, U, T, Q, Dd, F, D->d_dt, dxi, D->eta, D->alam, 1, s, bs));
-    // stage 2 (:264-336), which also stores the primitives of its result
-    CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, T, nullptr, s));
-    CNS_HIPCHK(launch_stage(g, T, U, Unew, Q, Dd, F, D->d_dt, dxi, D->eta, D->alam, 2, s, bs));
-    // stage 3 (:338-410)
-    CNS_HIPCHK(launch_domain_fill(g, bs, D->nb, Unew, Q, s));
-    CNS_HIPCHK(launch_stage(g, Unew, U, U, Q, Dd, F, D->d_dt, dxi, D->eta, D->alam, 3, s, bs));
-    double h[2];
-    CNS_HIPCHK(hipMemcpyAsync(h, D->d_dt, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+    const hipError_t e = enqueue_step(D, U, Unew, Q, Dd, F, s);
+    if (e != hipSuccess) {
+        // A step cut short may leave its maximum behind.
+        (void)launch_courno_reset(D->d_acc, 0.0, s);
+        CNS_HIPCHK(e);
+    }
     CNS_HIPCHK(hipStreamSynchronize(s));
+    const double h[2] = {D->h_dt[0], D->h_dt[1]};
     *dt = h[0];
     if (!std::isfinite(h[1]) || !std::isfinite(h[0]))
         return fail(CNS_ENUMERIC, "non-finite Courant number %g (dt %g)", h[1], h[0]);

@@ -13,6 +13,7 @@ struct BoxSet {
     int n = 1;
     int64_t su = 0, sq = 0, sc = 0;
 };
+constexpr int kOneBox[3] = {1, 1, 1};
 inline BoxSet box_set(const Geom &g, int n)
 {
     BoxSet b;
@@ -41,13 +42,11 @@ hipError_t launch_courno_reset(unsigned long long *acc, double init, hipStream_t
 hipError_t launch_ctoprim(const Geom &g, const double *u, double *q, unsigned long long *acc,
                           double dx0, double dx1, double dx2, hipStream_t s, bool full = true);
 
-// The Courant maximum of the interior cells of u alone, into acc.
-hipError_t launch_courno(const Geom &g, const double *u, unsigned long long *acc, double dx0, double dx1,
-                         double dx2, hipStream_t s, const BoxSet &bs = BoxSet());
-
-// dt = cfl / max(acc, 1e-50) into dt_dev (and the Courant number into courno_dev).
-hipError_t launch_courno_to_dt(const unsigned long long *acc, double cfl, double *dt_dev,
-                               double *courno_dev, hipStream_t s);
+// The device words and the pinned host words of a StepDt, acc zero.
+hipError_t step_dt_alloc(unsigned long long **acc, double **dt, double **courno, double **host);
+void step_dt_free(unsigned long long *acc, double *host);
+// sd.dt = cfl / max(acc, 1e-50) and the Courant number; acc back to zero.
+hipError_t launch_courno_to_dt(const StepDt &sd, hipStream_t s);
 
 // RK3 stage update; dt from dt_dev when non-null, else dt_host.
 hipError_t launch_rk_update(const Geom &g, int phase, double *u, double *unew, const double *d,
@@ -89,13 +88,17 @@ hipError_t launch_diffterm_pipe(const Geom &g, const double *q, const double *wz
                                 double dxi0, double dxi1, double dxi2, double eta, double alam,
                                 hipStream_t s);
 
+// The start of a fused step in one launch: the periodic ghosts of u (every box of the set) and
+// the Courant maximum of its interior into acc.  The two touch different cells.
+hipError_t launch_fill_courno(const Geom &g, double *u, unsigned long long *acc, double dx0, double dx1,
+                              double dx2, hipStream_t s, const BoxSet &bs = BoxSet(), const int nb[3] = kOneBox);
 // One RK stage in one kernel (cns_stage.hip): out = the SSP-RK3 update of phase 1..3 of the
 // ghosted state cons with base U^n (phases 2 and 3), its primitives into q (phase 2), D and
 // F stored by phase 3.  Every array must be 16-byte aligned; out must not alias cons; the
 // geometry must satisfy stage_fits (planes below 4 GiB, pitches below 2^24).
 bool stage_fits(const Geom &g);
 hipError_t launch_stage(const Geom &g, const double *cons, const double *base, double *out, double *q, double *d,
-                        double *f, const double *dt_dev, const double dxi[3], double eta, double alam, int phase,
+                        double *f, const StepDt &sd, const double dxi[3], double eta, double alam, int phase,
                         hipStream_t s, const BoxSet &bs = BoxSet());
 
 }  // namespace cns

@@ -93,15 +93,13 @@ __device__ __forceinline__ int image(int a, int I, int n, int nb, int &dI)
     return a < NG ? a + n : (a >= n + NG ? a - n : a);
 }
 
-// Box blockIdx.y of a set of nb[0] x nb[1] x nb[2] boxes (one box: its own images).  Q: the
-// components of q as well.
+// Ghost cell e of box b of a set of nb[0] x nb[1] x nb[2] boxes (one box: its own images).  Q:
+// the components of q as well.
 template <bool Q>
-__global__ void __launch_bounds__(kStreamBlock)
-fill_kernel(Geom g, Shell h, BoxSet bs, int nbx, int nby, int nbz, double *__restrict__ u, double *__restrict__ q)
+__device__ __forceinline__ void fill_cell(const Geom &g, const Shell &h, const BoxSet &bs, int nbx, int nby, int nbz,
+                                          unsigned e, unsigned b, double *u, double *q)
 {
-    const unsigned e = blockIdx.x * kStreamBlock + threadIdx.x;
-    if (e >= h.total) return;
-    const unsigned b = blockIdx.y, r = h.nbx.div(b);
+    const unsigned r = h.nbx.div(b);
     const int K = (int)h.nby.div(r), J = (int)r - K * nby, I = (int)b - (int)r * nbx;
     int i, j, k, dI, dJ, dK;
     shell_cell(g, h, e, i, j, k);
@@ -127,22 +125,26 @@ fill_kernel(Geom g, Shell h, BoxSet bs, int nbx, int nby, int nbz, double *__res
     }
 }
 
+template <bool Q>
+__global__ void __launch_bounds__(kStreamBlock)
+fill_kernel(Geom g, Shell h, BoxSet bs, int nbx, int nby, int nbz, double *__restrict__ u, double *__restrict__ q)
+{
+    const unsigned e = blockIdx.x * kStreamBlock + threadIdx.x;
+    if (e < h.total) fill_cell<Q>(g, h, bs, nbx, nby, nbz, e, blockIdx.y, u, q);
+}
+
 // -------------------------------------------------------------------- courno
 __global__ void courno_reset_kernel(unsigned long long *acc, double init)
 {
     acc[0] = init > 0.0 ? (unsigned long long)__double_as_longlong(init) : 0ull;
 }
 
-// courno = MAX(MAX(courmx,courmy), MAX(courmz, courno_in)) (cpu/ctoprim.cpp:69) with
-// courno_in = 1e-50 (cpu/advance.cpp:52); dt = cfl/courno (cpu/advance.cpp:57-58).
-__global__ void courno_to_dt_kernel(const unsigned long long *acc, double cfl, double *dt,
-                                    double *courno_out)
+__global__ void courno_to_dt_kernel(StepDt sd)
 {
-    double c = __longlong_as_double((long long)acc[0]);
-    double courno = c > 1.0E-50 ? c : 1.0E-50;
-    if (!(c == c)) courno = c;
-    dt[0] = cfl / courno;
-    if (courno_out) courno_out[0] = courno;
+    double courno;
+    const double dt = courno_dt(sd.acc, sd.cfl, courno);
+    step_dt_store(sd, dt, courno);
+    sd.acc[0] = 0ull;
 }
 
 // ------------------------------------------------------------------- ctoprim
@@ -244,15 +246,23 @@ rk_update_kernel(Geom g, int phase, double *__restrict__ u, double *__restrict__
 // The Courant maximum of a state's interior cells (cpu/ctoprim.cpp:42-69), without storing
 // its primitives, into acc (one 64-bit atomicMax per block).  A thread takes every
 // (grid size)-th cell of the interior, so a wave reads 64 consecutive cells of a row but for
-// the row ends: HBM-bound at large boxes (512^3 1.05 ms, 5.4 TB/s).
+// the row ends: HBM-bound at large boxes (512^3 1.0 ms, 5.4 TB/s).
+// The first `cb` blocks of a box do this; the others fill u's ghosts, one cell a thread: the two
+// touch different cells, and a step of a small box is a few launches long.
 __global__ void __launch_bounds__(kStreamBlock)
-courno_kernel(Geom g, const double *__restrict__ u, unsigned long long *__restrict__ acc, double dx0, double dx1,
-              double dx2, FastDiv by_n0, FastDiv by_n1, unsigned cells, BoxSet bs)
+fill_courno_kernel(Geom g, double *__restrict__ u, unsigned long long *__restrict__ acc, double dx0, double dx1,
+                   double dx2, FastDiv by_n0, FastDiv by_n1, unsigned cells, unsigned cb, Shell h, BoxSet bs, int nbx,
+                   int nby, int nbz)
 {
+    if (blockIdx.x >= cb) {
+        const unsigned e = (blockIdx.x - cb) * kStreamBlock + threadIdx.x;
+        if (e < h.total) fill_cell<false>(g, h, bs, nbx, nby, nbz, e, blockIdx.y, u, nullptr);
+        return;
+    }
     u += blockIdx.y * bs.su;  // box of a box set
     const int64_t cg = g.cg;
     unsigned long long cmax = 0ull;
-    for (unsigned n = blockIdx.x * kStreamBlock + threadIdx.x; n < cells; n += gridDim.x * kStreamBlock) {
+    for (unsigned n = blockIdx.x * kStreamBlock + threadIdx.x; n < cells; n += cb * kStreamBlock) {
         const unsigned r = by_n0.div(n), k = by_n1.div(r);
         const int64_t e = gidx(g, (int)(n - r * g.n0) + NG, (int)(r - k * g.n1) + NG, (int)k + NG);
         const double rho = u[e];
@@ -449,8 +459,7 @@ hipError_t launch_domain_fill(const Geom &g, const BoxSet &bs, const int nb[3], 
 
 hipError_t launch_fill_boundary(const Geom &g, double *u, double *q, hipStream_t s)
 {
-    const int one[3] = {1, 1, 1};
-    return launch_domain_fill(g, BoxSet(), one, u, q, s);
+    return launch_domain_fill(g, BoxSet(), kOneBox, u, q, s);
 }
 
 hipError_t launch_courno_reset(unsigned long long *acc, double init, hipStream_t s)
@@ -459,23 +468,26 @@ hipError_t launch_courno_reset(unsigned long long *acc, double init, hipStream_t
     return hipGetLastError();
 }
 
-hipError_t launch_courno(const Geom &g, const double *u, unsigned long long *acc, double dx0, double dx1,
-                         double dx2, hipStream_t s, const BoxSet &bs)
+hipError_t launch_fill_courno(const Geom &g, double *u, unsigned long long *acc, double dx0, double dx1,
+                              double dx2, hipStream_t s, const BoxSet &bs, const int nb[3])
 {
-    if (bs.n < 1 || bs.n > 65535) return hipErrorInvalidValue;
+    if (bs.n != nb[0] * nb[1] * nb[2] || bs.n < 1 || bs.n > 65535) return hipErrorInvalidValue;
     // Each block ends in an atomic on one address, about 20 ns apiece one after the other, so
     // small boxes take 256 blocks (128^3: 57 us with 4096 blocks, 26 with 512) and large ones up
     // to 1024, which their bandwidth needs (512^3: 1.76 / 1.13 / 1.00 / 1.02 ms with 256 / 512 /
     // 1024 / 2048): 16 cells a thread or more in between.
     const int64_t cells = (int64_t)g.n0 * g.n1 * g.n2, all = cells * bs.n;
-    if (cells > 0xffffffffll - 1024ll * kStreamBlock) return hipErrorInvalidValue;
+    const int64_t total = shell_cells(g);
+    if (cells > 0xffffffffll - 1024ll * kStreamBlock || total > 0xffffffffll - kStreamBlock) return hipErrorInvalidValue;
     int64_t most = all / (16 * kStreamBlock);
     most = (most < 256 ? 256 : (most > 1024 ? 1024 : most)) / bs.n;
     int64_t gx = (cells + kStreamBlock - 1) / kStreamBlock;
     if (gx > most) gx = most;
     if (gx < 1) gx = 1;
-    courno_kernel<<<dim3((unsigned)gx, (unsigned)bs.n), kStreamBlock, 0, s>>>(
-        g, u, acc, dx0, dx1, dx2, fast_div(g.n0), fast_div(g.n1), (unsigned)cells, bs);
+    const unsigned fb = (unsigned)((total + kStreamBlock - 1) / kStreamBlock);
+    fill_courno_kernel<<<dim3((unsigned)gx + fb, (unsigned)bs.n), kStreamBlock, 0, s>>>(
+        g, u, acc, dx0, dx1, dx2, fast_div(g.n0), fast_div(g.n1), (unsigned)cells, (unsigned)gx, make_shell(g, nb), bs,
+        nb[0], nb[1], nb[2]);
     return hipGetLastError();
 }
 
@@ -491,11 +503,39 @@ hipError_t launch_ctoprim(const Geom &g, const double *u, double *q, unsigned lo
     return hipGetLastError();
 }
 
-hipError_t launch_courno_to_dt(const unsigned long long *acc, double cfl, double *dt_dev,
-                               double *courno_dev, hipStream_t s)
+hipError_t launch_courno_to_dt(const StepDt &sd, hipStream_t s)
 {
-    courno_to_dt_kernel<<<1, 1, 0, s>>>(acc, cfl, dt_dev, courno_dev);
+    courno_to_dt_kernel<<<1, 1, 0, s>>>(sd);
     return hipGetLastError();
+}
+
+hipError_t step_dt_alloc(unsigned long long **acc, double **dt, double **courno, double **host)
+{
+    *host = nullptr;
+    unsigned long long *blk = nullptr;
+    hipStream_t s = nullptr;
+    hipError_t e = hipMalloc((void **)&blk, 4 * sizeof(double));
+    if (!e) e = hipHostMalloc((void **)host, 2 * sizeof(double), hipHostMallocDefault);
+    // A stream of its own: no other stream is waited for or made to wait.
+    if (!e) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+    if (!e) e = launch_courno_reset(blk, 0.0, s);
+    if (!e) e = hipStreamSynchronize(s);
+    if (s) (void)hipStreamDestroy(s);
+    if (e) {
+        (void)hipGetLastError();
+        step_dt_free(blk, *host);
+        return e;
+    }
+    *acc = blk;
+    *dt = (double *)blk + 1;
+    *courno = (double *)blk + 2;
+    return hipSuccess;
+}
+
+void step_dt_free(unsigned long long *acc, double *host)
+{
+    if (acc) (void)hipFree(acc);
+    if (host) (void)hipHostFree(host);
 }
 
 hipError_t launch_rk_update(const Geom &g, int phase, double *u, double *unew, const double *d,

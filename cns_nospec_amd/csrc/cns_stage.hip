@@ -67,8 +67,7 @@ struct StageArgs {
     double *out;         // result (ghosted); must not alias cons
     double *q;           // primitives of the result (QOUT)
     double *d, *f;       // D and F (LAST)
-    const double *dt;    // device dt
-    int phase;
+    StepDt sd;           // the step's dt, made by stage 1 from the Courant maximum
 };
 
 typedef __attribute__((address_space(3))) double lds_double;
@@ -164,9 +163,19 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     const int gi0 = bx * TX, gj0 = by * BY;  // ghosted coordinates of tile cell (0, 0)
     const int kbeg = bz * kz, kend = min(kbeg + kz, g.n2);
     const int64_t cg = g.cg, pg = g.pg;
-    const double dt = a.dt[0];
-    const double ra = a.phase == 1 ? 0.0E0 : (a.phase == 2 ? ThreeQuarters : OneThird);
-    const double rb = a.phase == 1 ? 1.0E0 : (a.phase == 2 ? OneQuarter : TwoThirds);
+    // Stage 1 forms dt from the maximum (every workgroup for itself, the first one also for the
+    // later stages and the host); stage 2 clears the maximum for the next step.
+    double dt;
+    if (STAGE1) {
+        double courno;
+        dt = courno_dt(a.sd.acc, a.sd.cfl, courno);
+        if (blockIdx.x == 0 && threadIdx.x == 0) step_dt_store(a.sd, dt, courno);
+    } else {
+        dt = a.sd.dt[0];
+        if (!LAST && blockIdx.x == 0 && threadIdx.x == 0) a.sd.acc[0] = 0ull;
+    }
+    const double ra = STAGE1 ? 0.0E0 : (LAST ? OneThird : ThreeQuarters);
+    const double rb = STAGE1 ? 1.0E0 : (LAST ? TwoThirds : OneQuarter);
     const double dxi0s = dxi0 * dxi0, dxi1s = dxi1 * dxi1, dxi2s = dxi2 * dxi2;
     const unsigned xg = (unsigned)g.xg;
 
@@ -696,11 +705,11 @@ bool stage_fits(const Geom &g)
 }
 
 hipError_t launch_stage(const Geom &g, const double *cons, const double *base, double *out, double *q, double *d,
-                        double *f, const double *dt_dev, const double dxi[3], double eta, double alam, int phase,
+                        double *f, const StepDt &sd, const double dxi[3], double eta, double alam, int phase,
                         hipStream_t s, const BoxSet &bs)
 {
     if (bs.n < 1 || !stage_fits(g)) return hipErrorInvalidValue;
-    const StageArgs a{base, out, q, d, f, dt_dev, phase};
+    const StageArgs a{base, out, q, d, f, sd};
     const int ntx = (g.n0 + TX - 1) / TX, nty = (g.n1 + BY - 1) / BY;
     const int kz = stage_kz(g, (int64_t)ntx * nty * bs.n);
     const int64_t nbpb = (int64_t)ntx * nty * ((g.n2 + kz - 1) / kz);

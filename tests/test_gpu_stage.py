@@ -37,3 +37,40 @@ def test_stage_kernel_equals_direct_kernels(device, n):
     assert dts == rdts
     for a, b, name in zip(arrays, rarrays, ("U", "Unew", "Q", "D", "F")):
         assert np.array_equal(a, b), name
+
+
+@pytest.mark.parametrize("first", ["stage", "direct", "unfused"])
+def test_courant_maximum_does_not_outlive_a_step(device, first):
+    """A step leaves its context's Courant maximum at zero on every route, so a slower flow
+    stepped after a faster one, in any composition, gets its own dt."""
+    import torch
+    lay = BoxLayout((20, 18, 9))
+
+    def fresh(mach):
+        arrays = ops.allocate_variables(lay, device)
+        arrays[0].copy_(torch.from_numpy(sinusoid_state(lay, 5, mach=mach, kmax=2)).to(device))
+        return arrays
+
+    def step(st, route, arrays):
+        print(f"courant maximum route={route}", flush=True)
+        ops.set_stencil_impl(_lib.CNS_IMPL_DIRECT if route == "direct" else _lib.CNS_IMPL_TILED)
+        st.set_fused(route != "unfused")
+        try:
+            return st.new_advance(*arrays)
+        finally:
+            ops.set_stencil_impl(_lib.CNS_IMPL_TILED)
+
+    ref = ops.Stepper(lay)
+    want_fast, want_slow = ref.new_advance(*fresh(0.9)), ref.new_advance(*fresh(0.01))
+    ref.close()
+    alone = ops.Stepper(lay)
+    assert alone.new_advance(*fresh(0.01)) == want_slow and want_slow > want_fast
+    alone.close()
+
+    st = ops.Stepper(lay)
+    for route in (first, "stage", "direct", "unfused", "stage"):
+        assert step(st, route, fresh(0.9)) == want_fast
+        assert step(st, "stage", fresh(0.01)) == want_slow
+        assert step(st, first, fresh(0.9)) == want_fast
+        assert step(st, route, fresh(0.01)) == want_slow
+    st.close()
