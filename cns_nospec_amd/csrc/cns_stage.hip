@@ -26,7 +26,7 @@
 //   C
 //   3  DMA of the next centre plane; diffterm's x and y terms; the update and the stores;
 //   A
-// Before the first centre plane eight shorter iterations fill the windows and the ring.
+// Before the first centre plane the windows and the ring are filled with eight planes at once.
 //
 // What bounds it: the vector arithmetic, about 1020 FP64 and 250 other instructions per
 // cell and plane at 4.5 cycles each (two waves per SIMD: 64 % of the cycles of a plane; the
@@ -58,7 +58,8 @@ constexpr int HALO = YH + XH;
 constexpr int OB = NT / 128;             // 1 KB DMA blocks of the own cells of a plane
 static_assert(NW == 8 && OB == 4 && TILE <= 128 * NW, "the wave shares below are for 8 waves");
 constexpr int LHY = 5 * NT, LHX = LHY + 3 * YH, LEAD = LHX + 3 * XH;  // staged leading plane
-static_assert(LEAD <= 5 * TILE, "the window fill stages every second plane in the centre tile");
+constexpr int LU = BY * PX, LV = R * TX; // u rows and v columns of a plane
+static_assert(LEAD >= 4 * LU + LV && 5 * TILE >= 6 * LV && TILE >= LU && LV >= LU, "places of the window fill");
 enum { RRHO = 0, RMX, RMY, RMZ, RE, RNF };
 enum { VU = 0, VV, VW, VT, VP, VNF };
 
@@ -144,8 +145,8 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     // leading plane, raw: own cells; y halo's rho, my, mz (at LHY); x halo's rho, mx, mz (at LHX)
     __shared__ __align__(16) double s_lead[LEAD];
     __shared__ double der[VNF * TILE];                 // centre plane, derived
-    __shared__ double s_lu[BY * PX];                   // leading u: own rows, column c (0..39)
-    __shared__ double s_lv[R * TX];                    // leading v: row r (0..R-1), column 4+c
+    __shared__ double s_lu[LU];                   // leading u: own rows, column c (0..39)
+    __shared__ double s_lv[LV];                    // leading v: row r (0..R-1), column 4+c
     __shared__ double s_ring[8 * HALO];                // w of plane p on the halo columns, slot p % 8
     __shared__ double s_ux[R * TX];                    // row r (0..R-1), column 4+c
     __shared__ double s_vy[BY * PX];                   // own rows, column c (0..39)
@@ -216,11 +217,11 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     };
     // leading plane of centre plane k: own block wave % 4 of fields 0..2 (waves 0..3) or 3, 4;
     // the y halo's two blocks and the x halo's one on waves 4, 5, 6
-    auto issue_lead = [&](int k, double *area) {
+    auto issue_lead = [&](int k) {
         const double *p = cons + (int64_t)(k + 2 * NG) * pg;
         const unsigned lane = opaque_tid() & 63, ob = wave & (OB - 1);
         const unsigned ooff = pair_off(4 + 4 * ob + (lane >> 4), 4 + 2 * (lane & 15));
-        lds_double *l = (lds_double *)area + 128 * ob;
+        lds_double *l = (lds_double *)s_lead + 128 * ob;
         if (wave < OB) {
             dma16(p, ooff, l);
             dma16(p + cg, ooff, l + NT);
@@ -230,14 +231,14 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
             dma16(p + 4 * cg, ooff, l + 4 * NT);
             if (wave < 6) {  // rows 0..3 or BY+4..BY+7
                 const unsigned hoff = pair_off((wave == 4 ? 0 : BY + 4) + (lane >> 4), 4 + 2 * (lane & 15));
-                lds_double *h = (lds_double *)area + LHY + 128 * (wave - 4);
+                lds_double *h = (lds_double *)s_lead + LHY + 128 * (wave - 4);
                 dma16(p, hoff, h);
                 dma16(p + IMY * cg, hoff, h + YH);
                 dma16(p + IMZ * cg, hoff, h + 2 * YH);
             } else if (wave == 6) {  // columns 0..3 and TX+4..TX+7 of the own rows
                 const int pr = lane & 3;
                 const unsigned hoff = pair_off(4 + (lane >> 2), pr < 2 ? 2 * pr : 2 * pr + TX);
-                lds_double *h = (lds_double *)area + LHX;
+                lds_double *h = (lds_double *)s_lead + LHX;
                 dma16(p, hoff, h);
                 dma16(p + IMX * cg, hoff, h + XH);
                 dma16(p + IMZ * cg, hoff, h + 2 * XH);
@@ -248,13 +249,11 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     // Windows: plane k+m of the own column at [4+m].  wri is 1/rho, from which u, v, w of a
     // window plane are one product (ctoprim's own).
     double wmx[9], wmy[9], wmz[9], wE[9], wri[9], wp[9], wT[9], wux[9], wvy[9];
-#pragma unroll
-    for (int m = 0; m < 9; m++)
-        wmx[m] = wmy[m] = wmz[m] = wE[m] = wri[m] = wp[m] = wT[m] = wux[m] = wvy[m] = 0.0;
 
     // primitives of the leading plane: own cell into the windows' entry 8, u and v with their
     // halos into the lead tiles, w of the halo columns
-    auto lead = [&](const double *area) {
+    auto lead = [&]() {
+        const double *area = s_lead;
         const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
         const double lr = area[tid];
         wmx[8] = area[RMX * NT + tid];
@@ -292,9 +291,8 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     };
 
     // ux, vy of the leading plane into the windows; w of the halo columns: planes k .. k+7 are
-    // in the ring, k+8 where lead() left it, which gives wz there (when the plane is a centre)
-    // and then takes the place of plane k
-    auto lead_grads = [&](int k, auto centre) {
+    // in the ring, k+8 where lead() left it, which gives wz there and then takes the place of plane k
+    auto lead_grads = [&](int k) {
         const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
         const unsigned mlu = mul24(row, PX) + col + 4, mlv = (row + 4) * TX + col;
         lds_tap *p_lu = (lds_tap *)s_lu + mlu, *p_lv = (lds_tap *)s_lv + mlv;
@@ -312,47 +310,98 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
                                : mul24((xid >> 3) + 4, PX) + (c8 < 4 ? c8 : c8 + TX);
             const double hw = s_wz[l];  // w of plane k+8, left here by lead()
 #define RW(mm) ((mm) == 4 ? hw : s_ring[((k + 4 + (mm)) & 7) * HALO + rc])
-            if (centre.value) s_wz[l] = D1(RW) * dxi2;
+            s_wz[l] = D1(RW) * dxi2;
 #undef RW
             s_ring[(k & 7) * HALO + rc] = hw;
         }
     };
 
-    // Fill the windows and the ring with planes kbeg .. kbeg+7, staged two ahead in turn in the
-    // leading and the (still unused) centre tile.  A wave waits for the older plane only: the
-    // younger one's loads are 3, 5 or 2 of its own (issue_lead).
-    auto fill_plane = [&](int k, double *area) {
-        if (wave < 4)
-            __builtin_amdgcn_s_waitcnt(0xF73);
-        else if (wave < 7)
-            __builtin_amdgcn_s_waitcnt(0xF75);
-        else
-            __builtin_amdgcn_s_waitcnt(0xF72);
+    // Fill the windows and the ring with planes kbeg .. kbeg+7: all their loads at once, into
+    // the windows' own registers, then the primitives of all eight planes with their u and v
+    // rows and columns in LDS (the centre plane's DMA meanwhile has the raw tile), then ux and vy.
+    // Its time is the loads' latency and the arithmetic of eight planes of primitives, about 9 us;
+    // plane by plane through the staged tile, with sixteen barriers, it took 15 (a stage of 16^3
+    // 23 -> 18 us, of 64^3 42 -> 32 us, of 130 x 97 x 61 95 -> 85 us).
+    {
+        // where plane kbeg+m's u rows and v columns are until ux and vy are formed
+        double *const lu[8] = {s_lead, s_lead + LU, s_lead + 2 * LU, s_lead + 3 * LU, s_lu, s_ux, s_vy, s_wz};
+        double *const lv[8] = {s_lead + 4 * LU, s_lv, der, der + LV, der + 2 * LV, der + 3 * LV, der + 4 * LV,
+                               der + 5 * LV};
+        const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
+        const unsigned xid = tid & 127, c8 = xid & 7, xcol = c8 < 4 ? c8 : c8 + TX, yrow = row < 4 ? row : row + BY;
+        const bool halo = w_yl || w_xl;
+        double hr[8], hm[8], hz[8];
+        {
+            auto off8 = [&](unsigned r, unsigned c) {
+                return (mul24(min(gj0 + (int)r, g.g1 - 1), xg) + (unsigned)min(gi0 + (int)c, g.xg - 1)) * 8u;
+            };
+            const unsigned own8 = off8(row + 4, col + 4), h8 = w_yl ? off8(yrow, col + 4) : off8((xid >> 3) + 4, xcol);
+            const double *p = cons + (int64_t)kbeg * pg, *pm = p + (w_yl ? IMY : IMX) * cg;
+#pragma unroll
+            for (int m = 0; m < 8; m++) {
+                wri[m] = at(p + m * pg, own8);
+                wmx[m] = at(p + m * pg + IMX * cg, own8);
+                wmy[m] = at(p + m * pg + IMY * cg, own8);
+                wmz[m] = at(p + m * pg + IMZ * cg, own8);
+                wE[m] = at(p + m * pg + IENE * cg, own8);
+                hr[m] = hm[m] = hz[m] = 1.0;
+                if (halo) {
+                    hr[m] = at(p + m * pg, h8);
+                    hm[m] = at(pm + m * pg, h8);
+                    hz[m] = at(p + m * pg + IMZ * cg, h8);
+                }
+            }
+        }
+        issue_raw(kbeg);
+        FENCE();
+#pragma unroll
+        for (int m = 0; m < 8; m++) {
+            double u_, v_, w_, eint;
+            const double rho = wri[m];
+            ctoprim_cell(rho, wmx[m], wmy[m], wmz[m], wE[m], u_, v_, w_, eint, wp[m]);
+            wri[m] = 1.0E0 / rho;
+            wT[m] = eint / CV;
+            pin(wri[m], wp[m], wT[m]);
+            lu[m][mul24(row, PX) + col + 4] = u_;
+            lv[m][(row + 4) * TX + col] = v_;
+            if (halo) {
+                const double hinv = 1.0E0 / hr[m];
+                if (w_yl)
+                    lv[m][yrow * TX + col] = hm[m] * hinv;
+                else
+                    lu[m][mul24(xid >> 3, PX) + xcol] = hm[m] * hinv;
+                s_ring[((kbeg + m) & 7) * HALO + (w_yl ? tid : YH + xid)] = hz[m] * hinv;
+            }
+            FENCE();
+        }
         __syncthreads();
-        lead(area);
+        auto grads = [&](int m) {
+            lds_tap *p_lu = (lds_tap *)lu[m] + mul24(row, PX) + col + 4, *p_lv = (lds_tap *)lv[m] + (row + 4) * TX + col;
+#define LUX(mm) p_lu[mm]
+#define LVY(mm) p_lv[(mm) * TX]
+            wux[m] = D1(LUX) * dxi0;
+            wvy[m] = D1(LVY) * dxi1;
+#undef LUX
+#undef LVY
+            pin(wux[m], wvy[m]);
+            FENCE();
+        };
+#pragma unroll
+        for (int m = 0; m < 4; m++) grads(m);
+        __syncthreads();  // the planes in s_lead are used
+        issue_lead(kbeg);
+#pragma unroll
+        for (int m = 4; m < 8; m++) grads(m);
+        __builtin_amdgcn_s_waitcnt(0xF70);
         __syncthreads();
-        lead_grads(k, std::false_type());
-        shift();
-    };
-    issue_lead(kbeg - 8, s_lead);
-    issue_lead(kbeg - 7, raw);
-#pragma unroll 1
-    for (int k = kbeg - 8; k < kbeg; k += 2) {
-        fill_plane(k, s_lead);
-        issue_lead(k + 2, s_lead);
-        fill_plane(k + 1, raw);
-        if (k + 3 < kbeg) issue_lead(k + 3, raw);
     }
-    issue_raw(kbeg);
-    __builtin_amdgcn_s_waitcnt(0xF70);
-    __syncthreads();
 
 #pragma unroll 1
     for (int k = kbeg; k < kend; k++) {
         const double *d_u = der + VU * TILE, *d_v = der + VV * TILE, *d_w = der + VW * TILE, *d_t = der + VT * TILE,
                      *d_p = der + VP * TILE;
         // ---------------- phase 1: primitives of the leading plane, derived tiles of the centre plane
-        lead(s_lead);
+        lead();
         {
             const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX, lane = tid & 63;
             const unsigned me = mul24(row + 4, PX) + col + 4;
@@ -390,9 +439,9 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
         __syncthreads();  // B
 
         // ---------------- phase 2
-        if (k + 1 < kend) issue_lead(k + 1, s_lead);
+        if (k + 1 < kend) issue_lead(k + 1);
         double F[5], zf[5], rho_c;
-        lead_grads(k, std::true_type());
+        lead_grads(k);
         {
             const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
             const unsigned me = mul24(row + 4, PX) + col + 4;
@@ -676,10 +725,10 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
 }
 
 // z runs.  A CU holds one workgroup, so a launch takes ceil(workgroups / 256) rounds of
-// (planes + the window fill, which costs about kFill planes: 18 us of 6.7 us a plane); the run
+// (planes + the window fill and launch, which cost about kFill planes: 11 us of 6.7 us a plane); the run
 // length that makes this smallest is taken.
 constexpr int kCUs = 256;
-constexpr double kFill = 2.5;
+constexpr double kFill = 1.6;
 
 int stage_kz(const Geom &g, int64_t tiles)
 {
