@@ -63,6 +63,11 @@ static_assert(LEAD >= 4 * LU + LV && 5 * TILE >= 6 * LV && TILE >= LU && LV >= L
 enum { RRHO = 0, RMX, RMY, RMZ, RE, RNF };
 enum { VU = 0, VV, VW, VT, VP, VNF };
 
+// where the arrays lie in LDS (the compiler's order, largest first)
+constexpr int AT_DER = 0, AT_RAW = AT_DER + VNF * TILE * 8, AT_LEAD = AT_RAW + RNF * TILE * 8,
+              AT_RING = AT_LEAD + LEAD * 8, AT_WZ = AT_RING + 8 * HALO * 8, AT_LV = AT_WZ + TILE * 8,
+              AT_UX = AT_LV + LV * 8, AT_LU = AT_UX + LV * 8, AT_VY = AT_LU + LU * 8;
+
 struct StageArgs {
     const double *base;  // U^n (stages 2 and 3)
     double *out;         // result (ghosted); must not alias cons
@@ -114,6 +119,24 @@ __device__ __forceinline__ unsigned opaque_tid()
 // the time of a 24-bit one).
 __device__ __forceinline__ unsigned mul24(unsigned a, unsigned b) { return __umul24(a, b); }
 
+// The taps of a lane around cell i of an array in LDS.  The lane's byte offset is formed once,
+// with the array's place in LDS in it, so that every tap is a constant of at most 64 KB away,
+// which an LDS instruction holds; left to itself the compiler forms an address per tap.
+// (The index is hidden and not the pointer: a pointer of unknown origin might read what the
+// DMA in flight writes, and would wait for it.)  at: where the array lies, a matter of speed
+// alone.
+template <int at>
+struct Taps {
+    const __attribute__((address_space(3))) char *a;
+    unsigned off;
+    __device__ __forceinline__ Taps(const double *array, unsigned i)
+        : a((const __attribute__((address_space(3))) char *)array), off(i * 8u + at)
+    {
+        asm volatile("" : "+v"(off));
+    }
+    __device__ __forceinline__ double operator[](int i) const { return *(lds_tap *)(a + (off + (unsigned)(8 * i - at))); }
+};
+
 // One tap pair (+m, -m) of a sum of differences, in the reference's order: the sum of a term
 // begins with its first tap pair.
 template <bool FIRST>
@@ -145,12 +168,12 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     // leading plane, raw: own cells; y halo's rho, my, mz (at LHY); x halo's rho, mx, mz (at LHX)
     __shared__ __align__(16) double s_lead[LEAD];
     __shared__ double der[VNF * TILE];                 // centre plane, derived
-    __shared__ double s_lu[LU];                   // leading u: own rows, column c (0..39)
-    __shared__ double s_lv[LV];                    // leading v: row r (0..R-1), column 4+c
-    __shared__ double s_ring[8 * HALO];                // w of plane p on the halo columns, slot p % 8
-    __shared__ double s_ux[R * TX];                    // row r (0..R-1), column 4+c
-    __shared__ double s_vy[BY * PX];                   // own rows, column c (0..39)
+    __shared__ double s_lu[LU];                        // leading u: own rows, column c (0..39)
+    __shared__ double s_lv[LV];                        // leading v: row r (0..R-1), column 4+c
+    __shared__ double s_ux[LV];                        // row r (0..R-1), column 4+c
+    __shared__ double s_vy[LU];                        // own rows, column c (0..39)
     __shared__ double s_wz[TILE];
+    __shared__ double s_ring[8 * HALO];                // w of plane p on the halo columns, slot p % 8
 
     int t = xcd_tile(blockIdx.x, gridDim.x);
     const int box = t / nbpb;
@@ -183,7 +206,13 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     // Shares of the halo cells, in units of one cell per lane: leading y halo, its ring and
     // wz on waves 0..3; leading x halo, its ring and wz on waves 4, 5; centre y halo and its
     // ux on waves 4..7; centre x halo on waves 0, 1; corners on wave 2; vy's x halo on 6, 7.
-    const bool w_yl = wave < 4, w_xl = wave == 4 || wave == 5, w_xc = wave < 2, w_c = wave == 2, w_vx = wave >= 6;
+    // (The wave index is hidden at each use: the conditions, held across the loop, would be more
+    // scalar registers than there are.)
+    auto wv = [&]() {
+        int w = wave;
+        asm volatile("" : "+s"(w));
+        return w;
+    };
 
     // In-plane byte offset of tile cell (r, c)'s 16-byte pair, clamped into the array: cells
     // past the box feed discarded outputs only.
@@ -208,34 +237,36 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     };
     auto issue_raw = [&](int k) {  // centre plane k: block `wave` of every field
         const double *p = cons + (int64_t)(k + NG) * pg;
-        const unsigned lane = opaque_tid() & 63, e = 128 * wave + 2 * lane;
+        const int w = wv();
+        const unsigned lane = opaque_tid() & 63, e = 128 * w + 2 * lane;
         const unsigned off = pair_off(e / PX, e % PX);
         if (e < TILE) {
 #pragma unroll
-            for (int f = 0; f < RNF; f++) dma16(p + f * cg, off, (lds_double *)raw + f * TILE + 128 * wave);
+            for (int f = 0; f < RNF; f++) dma16(p + f * cg, off, (lds_double *)raw + f * TILE + 128 * w);
         }
     };
     // leading plane of centre plane k: own block wave % 4 of fields 0..2 (waves 0..3) or 3, 4;
     // the y halo's two blocks and the x halo's one on waves 4, 5, 6
     auto issue_lead = [&](int k) {
         const double *p = cons + (int64_t)(k + 2 * NG) * pg;
-        const unsigned lane = opaque_tid() & 63, ob = wave & (OB - 1);
+        const int w = wv();
+        const unsigned lane = opaque_tid() & 63, ob = w & (OB - 1);
         const unsigned ooff = pair_off(4 + 4 * ob + (lane >> 4), 4 + 2 * (lane & 15));
         lds_double *l = (lds_double *)s_lead + 128 * ob;
-        if (wave < OB) {
+        if (w < OB) {
             dma16(p, ooff, l);
             dma16(p + cg, ooff, l + NT);
             dma16(p + 2 * cg, ooff, l + 2 * NT);
         } else {
             dma16(p + 3 * cg, ooff, l + 3 * NT);
             dma16(p + 4 * cg, ooff, l + 4 * NT);
-            if (wave < 6) {  // rows 0..3 or BY+4..BY+7
-                const unsigned hoff = pair_off((wave == 4 ? 0 : BY + 4) + (lane >> 4), 4 + 2 * (lane & 15));
-                lds_double *h = (lds_double *)s_lead + LHY + 128 * (wave - 4);
+            if (w < 6) {  // rows 0..3 or BY+4..BY+7
+                const unsigned hoff = pair_off((w == 4 ? 0 : BY + 4) + (lane >> 4), 4 + 2 * (lane & 15));
+                lds_double *h = (lds_double *)s_lead + LHY + 128 * (w - 4);
                 dma16(p, hoff, h);
                 dma16(p + IMY * cg, hoff, h + YH);
                 dma16(p + IMZ * cg, hoff, h + 2 * YH);
-            } else if (wave == 6) {  // columns 0..3 and TX+4..TX+7 of the own rows
+            } else if (w == 6) {  // columns 0..3 and TX+4..TX+7 of the own rows
                 const int pr = lane & 3;
                 const unsigned hoff = pair_off(4 + (lane >> 2), pr < 2 ? 2 * pr : 2 * pr + TX);
                 lds_double *h = (lds_double *)s_lead + LHX;
@@ -267,13 +298,14 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
         pin(wri[8], wp[8], wT[8]);
         s_lu[mul24(row, PX) + col + 4] = u_;
         s_lv[(row + 4) * TX + col] = v_;
-        if (w_yl) {
+        const int w = wv();
+        if (w < 4) {
             const unsigned yr = row < 4 ? row : row + BY;  // waves 0..3: rows 0..7
             const double hinv = 1.0E0 / area[LHY + tid];
             s_lv[yr * TX + col] = area[LHY + YH + tid] * hinv;
             s_wz[mul24(yr, PX) + col + 4] = area[LHY + 2 * YH + tid] * hinv;
         }
-        if (w_xl) {
+        if (w == 4 || w == 5) {
             const unsigned xid = tid & 127, c8 = xid & 7;
             const double hinv = 1.0E0 / area[LHX + xid];
             const unsigned l = mul24(xid >> 3, PX) + (c8 < 4 ? c8 : c8 + TX);
@@ -294,25 +326,42 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     // in the ring, k+8 where lead() left it, which gives wz there and then takes the place of plane k
     auto lead_grads = [&](int k) {
         const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
-        const unsigned mlu = mul24(row, PX) + col + 4, mlv = (row + 4) * TX + col;
-        lds_tap *p_lu = (lds_tap *)s_lu + mlu, *p_lv = (lds_tap *)s_lv + mlv;
-#define LUX(mm) p_lu[mm]
-#define LVY(mm) p_lv[(mm) * TX]
+        double a[9], b[9];
+        {
+            const Taps<AT_LU> p_lu(s_lu, mul24(row, PX) + col);
+            const Taps<AT_LV> p_lv(s_lv, tid);
+#pragma unroll
+            for (int m = 0; m < 9; m++)
+                if (m != 4) {
+                    a[m] = p_lu[m];
+                    b[m] = p_lv[m * TX];
+                }
+            FENCE();
+        }
+#define LUX(mm) a[4 + (mm)]
+#define LVY(mm) b[4 + (mm)]
         wux[8] = D1(LUX) * dxi0;
         wvy[8] = D1(LVY) * dxi1;
 #undef LUX
 #undef LVY
         pin(wux[8], wvy[8]);
-        if (w_yl || w_xl) {
+        FENCE();
+        const int w = wv();
+        if (w < 6) {
             const unsigned xid = tid & 127, c8 = xid & 7;
-            const unsigned rc = w_yl ? tid : YH + xid;
-            const unsigned l = w_yl ? mul24(row < 4 ? row : row + BY, PX) + col + 4
+            const unsigned rc = w < 4 ? tid : YH + xid;
+            const unsigned l = w < 4 ? mul24(row < 4 ? row : row + BY, PX) + col + 4
                                : mul24((xid >> 3) + 4, PX) + (c8 < 4 ? c8 : c8 + TX);
-            const double hw = s_wz[l];  // w of plane k+8, left here by lead()
-#define RW(mm) ((mm) == 4 ? hw : s_ring[((k + 4 + (mm)) & 7) * HALO + rc])
+            const Taps<0> p_r(s_ring, rc);  // (slots are scalars: the place goes with them)
+            a[8] = s_wz[l];  // w of plane k+8, left here by lead()
+#pragma unroll
+            for (int m = 0; m < 8; m++)
+                if (m != 4) a[m] = p_r[((k + m) & 7) * HALO];
+            FENCE();
+#define RW(mm) a[4 + (mm)]
             s_wz[l] = D1(RW) * dxi2;
 #undef RW
-            s_ring[(k & 7) * HALO + rc] = hw;
+            s_ring[(k & 7) * HALO + rc] = a[8];
         }
     };
 
@@ -329,14 +378,14 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
                                der + 5 * LV};
         const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
         const unsigned xid = tid & 127, c8 = xid & 7, xcol = c8 < 4 ? c8 : c8 + TX, yrow = row < 4 ? row : row + BY;
-        const bool halo = w_yl || w_xl;
+        const bool yl = wave < 4, halo = wave < 6;
         double hr[8], hm[8], hz[8];
         {
             auto off8 = [&](unsigned r, unsigned c) {
                 return (mul24(min(gj0 + (int)r, g.g1 - 1), xg) + (unsigned)min(gi0 + (int)c, g.xg - 1)) * 8u;
             };
-            const unsigned own8 = off8(row + 4, col + 4), h8 = w_yl ? off8(yrow, col + 4) : off8((xid >> 3) + 4, xcol);
-            const double *p = cons + (int64_t)kbeg * pg, *pm = p + (w_yl ? IMY : IMX) * cg;
+            const unsigned own8 = off8(row + 4, col + 4), h8 = yl ? off8(yrow, col + 4) : off8((xid >> 3) + 4, xcol);
+            const double *p = cons + (int64_t)kbeg * pg, *pm = p + (yl ? IMY : IMX) * cg;
 #pragma unroll
             for (int m = 0; m < 8; m++) {
                 wri[m] = at(p + m * pg, own8);
@@ -366,11 +415,11 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
             lv[m][(row + 4) * TX + col] = v_;
             if (halo) {
                 const double hinv = 1.0E0 / hr[m];
-                if (w_yl)
+                if (yl)
                     lv[m][yrow * TX + col] = hm[m] * hinv;
                 else
                     lu[m][mul24(xid >> 3, PX) + xcol] = hm[m] * hinv;
-                s_ring[((kbeg + m) & 7) * HALO + (w_yl ? tid : YH + xid)] = hz[m] * hinv;
+                s_ring[((kbeg + m) & 7) * HALO + (yl ? tid : YH + xid)] = hz[m] * hinv;
             }
             FENCE();
         }
@@ -420,15 +469,16 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
                 der[VT * TILE + l] = eint / CV;
                 der[VP * TILE + l] = p_;
             };
-            if (!w_yl) {
+            const int w = wv();
+            if (w >= 4) {
                 const unsigned yrow = row - 8;
                 halo_prim(mul24(yrow < 4 ? yrow : yrow + BY, PX) + col + 4);
             }
-            if (w_xc) {
+            if (w < 2) {
                 const unsigned c8 = tid & 7;
                 halo_prim(mul24((tid >> 3) + 4, PX) + (c8 < 4 ? c8 : c8 + TX));
             }
-            if (w_c) {  // u and v only
+            if (w == 2) {  // u and v only
                 const unsigned r8 = lane >> 3, c8 = lane & 7;
                 const unsigned l = mul24(r8 < 4 ? r8 : r8 + BY, PX) + (c8 < 4 ? c8 : c8 + TX);
                 const double cinv = 1.0E0 / raw[RRHO * TILE + l];
@@ -449,20 +499,30 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
                 // ux, vy, wz of the centre plane: own cells from the windows, the halos the mixed
                 // derivatives read from the derived tiles (cpu/diffterm.cpp:77-151)
                 s_ux[(row + 4) * TX + col] = wux[4];
-                if (!w_yl) {
-                    const unsigned yrow = row - 8, yr = yrow < 4 ? yrow : yrow + BY, l = mul24(yr, PX) + col + 4;
-                    lds_tap *p_u = (lds_tap *)d_u + l;
-#define CUX(mm) p_u[mm]
+                const int w = wv();
+                if (w >= 4) {
+                    const unsigned yrow = row - 8, yr = yrow < 4 ? yrow : yrow + BY;
+                    const Taps<AT_DER> p_u(d_u, mul24(yr, PX) + col);
+                    double a[9];
+#pragma unroll
+                    for (int m = 0; m < 9; m++)
+                        if (m != 4) a[m] = p_u[m];
+                    FENCE();
+#define CUX(mm) a[4 + (mm)]
                     s_ux[yr * TX + col] = D1(CUX) * dxi0;
 #undef CUX
                 }
                 s_vy[mul24(row, PX) + col + 4] = wvy[4];
-                if (w_vx) {
-                    const unsigned xid = tid & 127, c8 = xid & 7, c = c8 < 4 ? c8 : c8 + TX;
-                    const unsigned l = mul24((xid >> 3) + 4, PX) + c;
-                    lds_tap *p_v = (lds_tap *)d_v + l;
-#define CVY(mm) p_v[(mm) * PX]
-                    s_vy[mul24(xid >> 3, PX) + c] = D1(CVY) * dxi1;
+                if (w >= 6) {
+                    const unsigned xid = tid & 127, c8 = xid & 7, l = mul24(xid >> 3, PX) + (c8 < 4 ? c8 : c8 + TX);
+                    const Taps<AT_DER> p_v(d_v, l);
+                    double a[9];
+#pragma unroll
+                    for (int m = 0; m < 9; m++)
+                        if (m != 4) a[m] = p_v[m * PX];
+                    FENCE();
+#define CVY(mm) a[4 + (mm)]
+                    s_vy[l] = D1(CVY) * dxi1;
 #undef CVY
                 }
                 rho_c = raw[RRHO * TILE + me];
@@ -521,17 +581,20 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
         }
         shift();  // the centre plane is window entry 3 from here
         {
-            const unsigned tid = opaque_tid(), me = mul24(tid / TX + 4, PX) + (tid & (TX - 1)) + 4;
-            lds_tap *s_c = (lds_tap *)raw + me, *s_d = (lds_tap *)der + me;
+            // from four rows above the own cell: every tap is a non-negative constant away
+            const unsigned tid = opaque_tid(), me4 = mul24(tid / TX, PX) + (tid & (TX - 1)) + 4;
+            const Taps<AT_RAW> s_c(raw, me4);
+            const Taps<AT_DER> s_d(der, me4);
             double hs[5], A[12];
             // fields n, a, b, E of the raw tile, p and v of the derived one at taps +o and -o
+            constexpr int Z = 4 * PX;
             auto load = [&](double (&T)[12], int n, int a_, int b_, int v, int o) {
-                T[0] = s_c[n * TILE + o]; T[1] = s_c[n * TILE - o];
-                T[2] = s_c[a_ * TILE + o]; T[3] = s_c[a_ * TILE - o];
-                T[4] = s_c[b_ * TILE + o]; T[5] = s_c[b_ * TILE - o];
-                T[6] = s_c[RE * TILE + o]; T[7] = s_c[RE * TILE - o];
-                T[8] = s_d[VP * TILE + o]; T[9] = s_d[VP * TILE - o];
-                T[10] = s_d[v * TILE + o]; T[11] = s_d[v * TILE - o];
+                T[0] = s_c[n * TILE + Z + o]; T[1] = s_c[n * TILE + Z - o];
+                T[2] = s_c[a_ * TILE + Z + o]; T[3] = s_c[a_ * TILE + Z - o];
+                T[4] = s_c[b_ * TILE + Z + o]; T[5] = s_c[b_ * TILE + Z - o];
+                T[6] = s_c[RE * TILE + Z + o]; T[7] = s_c[RE * TILE + Z - o];
+                T[8] = s_d[VP * TILE + Z + o]; T[9] = s_d[VP * TILE + Z - o];
+                T[10] = s_d[v * TILE + Z + o]; T[11] = s_d[v * TILE + Z - o];
             };
 #define HT(FIRST, C, T) \
     hyp_tap<FIRST>(C, T[0], T[1], T[2], T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11], hs); \
@@ -581,18 +644,20 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
             // diffterm's x and y terms, from the tiles, then its sums as the reference forms them
             // (cpu/diffterm.cpp:159-311)
             const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
-            const unsigned me = mul24(row + 4, PX) + col + 4;
-            lds_tap *s_d = (lds_tap *)der + me, *s_z = (lds_tap *)s_wz + me, *s_m = (lds_tap *)s_vy + mul24(row, PX) + col + 4,
-                    *s_n = (lds_tap *)s_ux + (row + 4) * TX + col;
+            const unsigned me4 = mul24(row, PX) + col + 4;  // as above
+            const Taps<AT_DER> s_d(der, me4);
+            const Taps<AT_WZ> s_z(s_wz, me4);
+            constexpr int Z = 4 * PX;
             double A[12], xu, xv, xw, xt, d2v, d2w, m1, m2;
-            // u, v, w, T of the derived tile, wz, and vy or ux at taps +o and -o
-            auto load = [&](double (&T)[12], int o, lds_tap *m, int om) {
-                T[0] = s_d[VU * TILE + o]; T[1] = s_d[VU * TILE - o];
-                T[2] = s_d[VV * TILE + o]; T[3] = s_d[VV * TILE - o];
-                T[4] = s_d[VW * TILE + o]; T[5] = s_d[VW * TILE - o];
-                T[6] = s_d[VT * TILE + o]; T[7] = s_d[VT * TILE - o];
-                T[8] = s_z[o]; T[9] = s_z[-o];
-                T[10] = m[om]; T[11] = m[-om];
+            // u, v, w, T of the derived tile, wz and vy at taps +o and -o in x
+            const Taps<AT_VY> s_m4(s_vy, me4 - 4);
+            auto load = [&](double (&T)[12], int o) {
+                T[0] = s_d[VU * TILE + Z + o]; T[1] = s_d[VU * TILE + Z - o];
+                T[2] = s_d[VV * TILE + Z + o]; T[3] = s_d[VV * TILE + Z - o];
+                T[4] = s_d[VW * TILE + Z + o]; T[5] = s_d[VW * TILE + Z - o];
+                T[6] = s_d[VT * TILE + Z + o]; T[7] = s_d[VT * TILE + Z - o];
+                T[8] = s_z[Z + o]; T[9] = s_z[Z - o];
+                T[10] = s_m4[4 + o]; T[11] = s_m4[4 - o];
             };
             // second differences of u, v, w, T; first of T[2 * f] (d2v), w (d2w), and of the two mixed terms
 #define DT(FIRST, C1, C2, T, f)                  \
@@ -608,13 +673,13 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     FENCE()
             xu = CENTER * (wmx[3] * wri[3]); xv = CENTER * (wmy[3] * wri[3]);
             xw = CENTER * (wmz[3] * wri[3]); xt = CENTER * wT[3];
-            load(A, 1, s_m, 1); FENCE();
+            load(A, 1); FENCE();
             DT(true, ALP, OFF1, A, 1);
-            load(A, 2, s_m, 2); FENCE();
+            load(A, 2); FENCE();
             DT(false, BET, OFF2, A, 1);
-            load(A, 3, s_m, 3); FENCE();
+            load(A, 3); FENCE();
             DT(false, GAM, OFF3, A, 1);
-            load(A, 4, s_m, 4); FENCE();
+            load(A, 4); FENCE();
             DT(false, DEL, OFF4, A, 1);
             double sx = FourThirds * (xu * dxi0s), sy = xv * dxi0s, sz = xw * dxi0s, st = xt * dxi0s;
             const double vx = d2v * dxi0, wx = d2w * dxi0, mx = m1 * dxi0 + m2 * dxi0;
@@ -629,11 +694,12 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
             }
             xu = CENTER * (wmx[3] * wri[3]); xv = CENTER * (wmy[3] * wri[3]);
             xw = CENTER * (wmz[3] * wri[3]); xt = CENTER * wT[3];
+            const Taps<AT_UX> s_n(s_ux, tid);
             auto ytap = [&](auto first, double c1, double c2, int o, int on) {
                 constexpr bool FI = decltype(first)::value;
                 {
-                    const double u1 = s_d[VU * TILE + o], u0 = s_d[VU * TILE - o], v1 = s_d[VV * TILE + o],
-                                 v0 = s_d[VV * TILE - o], w1 = s_d[VW * TILE + o], w0 = s_d[VW * TILE - o];
+                    const double u1 = s_d[VU * TILE + Z + o], u0 = s_d[VU * TILE + Z - o], v1 = s_d[VV * TILE + Z + o],
+                                 v0 = s_d[VV * TILE + Z - o], w1 = s_d[VW * TILE + Z + o], w0 = s_d[VW * TILE + Z - o];
                     FENCE();
                     tap<false>(xu, c2 * (u1 + u0));
                     tap<false>(xv, c2 * (v1 + v0));
@@ -644,8 +710,8 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
                     FENCE();
                 }
                 {
-                    const double t1 = s_d[VT * TILE + o], t0 = s_d[VT * TILE - o], z1 = s_z[o], z0 = s_z[-o],
-                                 n1 = s_n[on], n0 = s_n[-on];
+                    const double t1 = s_d[VT * TILE + Z + o], t0 = s_d[VT * TILE + Z - o], z1 = s_z[Z + o], z0 = s_z[Z - o],
+                                 n1 = s_n[4 * TX + on], n0 = s_n[4 * TX - on];
                     FENCE();
                     tap<false>(xt, c2 * (t1 + t0));
                     tap<FI>(m1, c1 * (n1 - n0));
@@ -671,7 +737,7 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
             D[IMY] = eta * (sy + vzz + OneThird * my);
             D[IMZ] = eta * (sz + FourThirds * wzz + OneThird * mz);
             {
-                const double ux = wux[3], vy = wvy[3], wz = *s_z;
+                const double ux = wux[3], vy = wvy[3], wz = s_z[Z];
                 const double divu = TwoThirds * (ux + vy + wz);
                 const double tauxx = 2.E0 * ux - divu;
                 const double tauyy = 2.E0 * vy - divu;
