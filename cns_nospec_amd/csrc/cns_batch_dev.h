@@ -35,7 +35,7 @@ __host__ __device__ inline bool box_stopped(const BoxDev &b) { return b.target >
 struct TileDev {
     int box;
     short x0, y0, z0, nz;  // tile origin (cells) and z run
-    short ltx;             // log2 of the tile width (4, 5 or 6); height = 256 >> ltx
+    short ltx;             // log2 of the tile width (4, 5 or 6)
     short pad;
 };
 
@@ -44,19 +44,22 @@ constexpr int kTileClasses = 3;
 
 constexpr int kBatchThreads = 256;
 
-hipError_t launch_batch_init(BoxDev *boxes, int box, int e, bool fp32, hipStream_t s);
+// Primitives of the box's U into Q[0]; fresh (admission): its Courant maximum and pref too.
+hipError_t launch_batch_init(BoxDev *boxes, int box, int e, bool fp32, bool fresh, hipStream_t s);
 hipError_t launch_batch_finalize(BoxDev *boxes, const int *box_ids, int nbox, int count_step,
                                  hipStream_t s);
 // One RK stage over the tile list: the list holds class 0, 1, 2 tiles in the
-// ranges [start[c], start[c]+count[c]); each class gets a diffterm launch, then a
-// hypterm + update launch, of one workgroup per tile.  staged_diff selects the
-// diffterm whose planes are staged by direct-to-LDS loads, preceded by a wz-field
-// launch per class; keep_centre the FP32 hypterm + update of stages 2 and 3 that keeps
-// its window's FP64 leading values for the centre plane; staged_hyp (FP32 flux) and
-// staged_hyp64 (FP64) the hypterm + update of 32-wide tiles whose planes are staged by
-// direct-to-LDS loads.
+// ranges [start[c], start[c]+count[c]).  fused: class 1 takes one launch of the fused stage
+// kernel, and its tiles are kFusedHeight rows high; it neither reads nor writes Q.  Every
+// other class gets a diffterm launch, then a hypterm + update launch, of one workgroup per
+// tile.  staged_diff selects the diffterm whose planes are staged by direct-to-LDS loads,
+// preceded by a wz-field launch per class; keep_centre the FP32 hypterm + update of stages 2
+// and 3 that keeps its window's FP64 leading values for the centre plane.
 hipError_t launch_batch_stage(BoxDev *boxes, const TileDev *tiles, const int start[3],
-                              const int count[3], int stage, bool fp32, bool staged_diff,
-                              bool keep_centre, bool staged_hyp, bool staged_hyp64, hipStream_t s);
+                              const int count[3], int stage, bool fp32, bool fused, bool staged_diff,
+                              bool keep_centre, hipStream_t s);
+// Its class-1 launch (cns_batch_stage.hip).
+constexpr int kFusedHeight = 16;
+hipError_t launch_batch_fused(BoxDev *boxes, const TileDev *tiles, int n, int stage, bool fp32, hipStream_t s);
 
 }  // namespace cns

@@ -78,6 +78,7 @@ struct Pool {
 
 struct BoxHost {
     bool live = false;
+    bool fused = false;  // in the fused class of the last work list: Q[0] is not kept
     int e = 0;
     size_t off = 0, bytes = 0;
 };
@@ -121,16 +122,16 @@ struct cns_batch {
     // which cost more than the 32 bytes per cell it saves: 4.66 vs 4.73 G cell-steps/s
     // on the request mix).
     bool keep_centre = false;
-    // 32-wide tiles: the hypterm + update tile staged by direct-to-LDS loads, FP32 flux
-    // and FP64 (CNS_BATCH_HYP=0, CNS_BATCH_HYP64=0 select the tile that gathers its halos
-    // through registers; the same bits either way).
-    bool staged_hyp = true;
-    bool staged_hyp64 = true;
+    // 32-wide tiles: a stage is one kernel (cns_batch_stage.hip).  CNS_BATCH_HYP=0 (FP32 flux)
+    // and CNS_BATCH_HYP64=0 (FP64) select the separate kernels, as CNS_BATCH_DIFF=0 and
+    // CNS_BATCH_KEEP=1 do; the same bits either way.
+    bool fused_stage = true;
     bool dirty = true;
     hipStream_t cap_stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
 
+    bool fused() const { return fused_stage && staged_diff && !(fp32 && keep_centre); }
     std::pair<int, int> tile_of(int e) const
     {
         auto it = tune.find(e);
@@ -164,12 +165,15 @@ int rebuild(cns_batch *b, hipStream_t s)
     std::vector<TileDev> cls[kTileClasses];
     b->hids.clear();
     for (int id = 0; id < (int)b->hb.size(); id++) {
-        const BoxHost &h = b->hb[id];
+        BoxHost &h = b->hb[id];
         if (!h.live) continue;
         b->hids.push_back(id);
         const auto t = b->tile_of(h.e);
         const int w = t.first, c = width_class(w), kz = std::max(1, std::min(t.second, h.e));
-        const int hgt = kBatchThreads / w, ltx = c + 4;
+        const bool fused = b->fused() && c == 1;
+        if (h.fused && !fused) CNS_HIPCHK(launch_batch_init(b->d_boxes, id, h.e, b->fp32, false, s));
+        h.fused = fused;
+        const int hgt = fused ? kFusedHeight : kBatchThreads / w, ltx = c + 4;
         for (int z0 = 0; z0 < h.e; z0 += kz)
             for (int y0 = 0; y0 < h.e; y0 += hgt)
                 for (int x0 = 0; x0 < h.e; x0 += w) {
@@ -217,8 +221,7 @@ int rebuild(cns_batch *b, hipStream_t s)
         hipError_t e = hipSuccess;
         for (int stage = 1; stage <= 3 && e == hipSuccess; stage++)
             e = launch_batch_stage(b->d_boxes, b->d_tiles, b->cls_start, b->cls_count, stage, b->fp32,
-                                   b->staged_diff, b->keep_centre, b->staged_hyp, b->staged_hyp64,
-                                   b->cap_stream);
+                                   b->fused(), b->staged_diff, b->keep_centre, b->cap_stream);
         if (e == hipSuccess) e = launch_batch_finalize(b->d_boxes, b->d_ids, b->nresident, 1, b->cap_stream);
         hipGraph_t g = nullptr;
         const hipError_t e2 = hipStreamEndCapture(b->cap_stream, &g);
@@ -259,8 +262,7 @@ int cns_batch_create(cns_batch **out, size_t hbm_budget, int flux_fp32, int max_
     b->max_boxes = max_boxes;
     if (const char *env = getenv("CNS_BATCH_DIFF")) b->staged_diff = atoi(env) != 0;
     if (const char *env = getenv("CNS_BATCH_KEEP")) b->keep_centre = atoi(env) != 0;
-    if (const char *env = getenv("CNS_BATCH_HYP")) b->staged_hyp = atoi(env) != 0;
-    if (const char *env = getenv("CNS_BATCH_HYP64")) b->staged_hyp64 = atoi(env) != 0;
+    if (const char *env = getenv(b->fp32 ? "CNS_BATCH_HYP" : "CNS_BATCH_HYP64")) b->fused_stage = atoi(env) != 0;
     int rc = CNS_OK;
     if (hipGetDevice(&b->device) != hipSuccess) rc = fail(CNS_EHIP, "hipGetDevice failed");
     if (!rc && hbm_budget && hipMalloc((void **)&b->pool_mem, hbm_budget) != hipSuccess) {
@@ -359,7 +361,7 @@ int cns_batch_add(cns_batch *b, int edge, double dx, double cfl, double eta, dou
     int rc = CNS_OK;
     if (hipMemcpyAsync(b->d_boxes + id, &r, sizeof r, hipMemcpyHostToDevice, s) != hipSuccess ||
         hipMemcpyAsync(r.U, u0, 5 * e3 * sizeof(double), hipMemcpyDeviceToDevice, s) != hipSuccess ||
-        launch_batch_init(b->d_boxes, id, edge, b->fp32, s) != hipSuccess ||
+        launch_batch_init(b->d_boxes, id, edge, b->fp32, true, s) != hipSuccess ||
         launch_batch_finalize(b->d_boxes, b->d_iota + id, 1, 0, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
         rc = fail(CNS_EHIP, "initialising box %d failed: %s", id, hipGetErrorString(hipGetLastError()));
@@ -369,6 +371,7 @@ int cns_batch_add(cns_batch *b, int edge, double dx, double cfl, double eta, dou
     }
     BoxHost &h = b->hb[id];
     h.live = true;
+    h.fused = false;
     h.e = edge;
     h.off = off;
     h.bytes = bytes;

@@ -44,24 +44,11 @@
 // bit-identical to the reference cpu/ path.
 #include <type_traits>
 
-#include "cns_pipe_tile.h"
+#include "cns_stage_tile.h"
 
 namespace cns {
 
 namespace {
-
-// Tile geometry; sizes are in doubles unless they say otherwise.
-constexpr int TX = 32, BY = 16, PX = TX + 8, R = BY + 8, NT = TX * BY, NW = NT / 64;
-constexpr int TILE = R * PX;             // a haloed plane
-constexpr int YH = 8 * TX, XH = 8 * BY;  // y-halo and x-halo cells of its cross
-constexpr int HALO = YH + XH;
-constexpr int OB = NT / 128;             // 1 KB DMA blocks of the own cells of a plane
-static_assert(NW == 8 && OB == 4 && TILE <= 128 * NW, "the wave shares below are for 8 waves");
-constexpr int LHY = 5 * NT, LHX = LHY + 3 * YH, LEAD = LHX + 3 * XH;  // staged leading plane
-constexpr int LU = BY * PX, LV = R * TX; // u rows and v columns of a plane
-static_assert(LEAD >= 4 * LU + LV && 5 * TILE >= 6 * LV && TILE >= LU && LV >= LU, "places of the window fill");
-enum { RRHO = 0, RMX, RMY, RMZ, RE, RNF };
-enum { VU = 0, VV, VW, VT, VP, VNF };
 
 // where the arrays lie in LDS (the compiler's order, largest first)
 constexpr int AT_DER = 0, AT_RAW = AT_DER + VNF * TILE * 8, AT_LEAD = AT_RAW + RNF * TILE * 8,
@@ -75,89 +62,6 @@ struct StageArgs {
     double *d, *f;       // D and F (LAST)
     StepDt sd;           // the step's dt, made by stage 1 from the Courant maximum
 };
-
-typedef __attribute__((address_space(3))) double lds_double;
-// Taps are read one by one: the compiler otherwise pairs them into ds_read2_b64, which moves
-// 128 bytes per cycle where ds_read_b64 moves 240 (measured, eight waves).
-typedef const volatile __attribute__((address_space(3))) double lds_tap;
-
-__device__ __forceinline__ void dma16(const double *src, unsigned off, lds_double *lds)
-{
-    __builtin_amdgcn_global_load_lds((const void *)((const char *)src + off), (lds_void *)lds, 16, 0, 0);
-}
-
-// A lane's element of a plane: uniform plane pointer, 32-bit byte offset (a plane is below
-// 4 GiB), so that the access is one scalar-base instruction.
-#define GAS __attribute__((address_space(1)))
-template <typename T>
-__device__ __forceinline__ T GAS &at(T *p, unsigned off)
-{
-    asm volatile("" : "+s"(p));  // kept scalar: folded with the offset it would take a register pair per array
-    return *(T GAS *)((const char GAS *)p + off);
-}
-
-// Keeps the scheduler from hoisting the LDS reads of later groups above earlier ones, which
-// bounds the live registers.
-#define FENCE() __builtin_amdgcn_sched_barrier(0)
-// Has the values computed where it stands: the compiler would otherwise move arithmetic that
-// is used later past the barriers, and keep its operands live instead.
-template <typename... T>
-__device__ __forceinline__ void pin(T &...v)
-{
-    (..., [](auto &x) { asm volatile("" : "+v"(x)); }(v));
-}
-// A thread index that the compiler cannot see through: what is formed from it is formed
-// anew where it stands.  Held across the plane loop, the lane's places and offsets would
-// push window entries into scratch.
-__device__ __forceinline__ unsigned opaque_tid()
-{
-    unsigned t = threadIdx.x;
-    asm volatile("" : "+v"(t));
-    return t & (NT - 1);
-}
-// Products of indices and pitches, all below 2^24 (a full 32-bit product takes four times
-// the time of a 24-bit one).
-__device__ __forceinline__ unsigned mul24(unsigned a, unsigned b) { return __umul24(a, b); }
-
-// The taps of a lane around cell i of an array in LDS.  The lane's byte offset is formed once,
-// with the array's place in LDS in it, so that every tap is a constant of at most 64 KB away,
-// which an LDS instruction holds; left to itself the compiler forms an address per tap.
-// (The index is hidden and not the pointer: a pointer of unknown origin might read what the
-// DMA in flight writes, and would wait for it.)  at: where the array lies, a matter of speed
-// alone.
-template <int at>
-struct Taps {
-    const __attribute__((address_space(3))) char *a;
-    unsigned off;
-    __device__ __forceinline__ Taps(const double *array, unsigned i)
-        : a((const __attribute__((address_space(3))) char *)array), off(i * 8u + at)
-    {
-        asm volatile("" : "+v"(off));
-    }
-    __device__ __forceinline__ double operator[](int i) const { return *(lds_tap *)(a + (off + (unsigned)(8 * i - at))); }
-};
-
-// One tap pair (+m, -m) of a sum of differences, in the reference's order: the sum of a term
-// begins with its first tap pair.
-template <bool FIRST>
-__device__ __forceinline__ void tap(double &s, double t)
-{
-    s = FIRST ? t : s + t;
-}
-
-// hypterm's tap pair in one direction: n the momentum along it, a and b the others, v the
-// velocity along it; sums s of rho, n, a, b, E (cpu/hypterm.cpp:43-90).
-template <bool FIRST>
-__device__ __forceinline__ void hyp_tap(double c, double n1, double n0, double a1, double a0, double b1, double b0,
-                                        double e1, double e0, double p1, double p0, double v1, double v0,
-                                        double (&s)[5])
-{
-    tap<FIRST>(s[0], c * (n1 - n0));
-    tap<FIRST>(s[1], c * (n1 * v1 - n0 * v0 + (p1 - p0)));
-    tap<FIRST>(s[2], c * (a1 * v1 - a0 * v0));
-    tap<FIRST>(s[3], c * (b1 * v1 - b0 * v0));
-    tap<FIRST>(s[4], c * (e1 * v1 - e0 * v0 + (p1 * v1 - p0 * v0)));
-}
 
 template <bool STAGE1, bool LAST, bool QOUT>
 __global__ void __launch_bounds__(NT, 2)
@@ -425,7 +329,7 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
         }
         __syncthreads();
         auto grads = [&](int m) {
-            lds_tap *p_lu = (lds_tap *)lu[m] + mul24(row, PX) + col + 4, *p_lv = (lds_tap *)lv[m] + (row + 4) * TX + col;
+            lds_tap<double> *p_lu = (lds_tap<double> *)lu[m] + mul24(row, PX) + col + 4, *p_lv = (lds_tap<double> *)lv[m] + (row + 4) * TX + col;
 #define LUX(mm) p_lu[mm]
 #define LVY(mm) p_lv[(mm) * TX]
             wux[m] = D1(LUX) * dxi0;
@@ -541,7 +445,7 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     {                                                                                                            \
         const double w1 = wmz[4 + m] * wri[4 + m], w0 = wmz[4 - m] * wri[4 - m];                                 \
         hyp_tap<FIRST>(C1, wmz[4 + m], wmz[4 - m], wmx[4 + m], wmx[4 - m], wmy[4 + m], wmy[4 - m], wE[4 + m],     \
-                       wE[4 - m], wp[4 + m], wp[4 - m], w1, w0, hs);                                             \
+                       wE[4 - m], wp[4 + m], wp[4 - m], wp[4 + m], wp[4 - m], w1, w0, hs);                                             \
         tap<FIRST>(wzc, C1 * (w1 - w0));                                                                         \
         tap<false>(zz, C2 * (w1 + w0));                                                                          \
         const double u1 = wmx[4 + m] * wri[4 + m], u0 = wmx[4 - m] * wri[4 - m];                                 \
@@ -597,7 +501,7 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
                 T[10] = s_d[v * TILE + Z + o]; T[11] = s_d[v * TILE + Z - o];
             };
 #define HT(FIRST, C, T) \
-    hyp_tap<FIRST>(C, T[0], T[1], T[2], T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11], hs); \
+    hyp_tap<FIRST>(C, T[0], T[1], T[2], T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[8], T[9], T[10], T[11], hs); \
     pin(hs[0], hs[1], hs[2], hs[3], hs[4]); FENCE()
             load(A, RMX, RMY, RMZ, VU, 1); FENCE();
             HT(true, ALP, A);
