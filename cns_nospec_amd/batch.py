@@ -12,7 +12,8 @@ The tile shape of each box edge comes from ``tuning_gfx950.json``, which the
 autotuner below (:func:`autotune`, ``python -m cns_nospec_amd.batch``) writes: it
 times whole tile tables on the served request mix resident in one engine (one width
 for every edge, so each RK stage stays one launch per kernel, and a z run per edge
-bucket).  Edges the table does not list get 32-wide tiles and z runs of min(edge, 16).
+bucket; of 32-wide tiles the longest run, which the engine's work list splits further).
+Edges the table does not list get 32-wide tiles and z runs as the work list chooses.
 """
 from __future__ import annotations
 
@@ -175,7 +176,7 @@ def compact_sinusoid(edge: int, seed: int, mach: float = 0.085, kmax: int = 2, d
 
 # ---------------------------------------------------------------- autotuner
 WIDTHS = (16, 32, 64)
-KZS = (8, 16, 32, 64)
+KZS = (16, 32, 64, 512)
 # edge ranges whose z run the tuner chooses separately (the engine admits edges 8..512)
 EDGE_BUCKETS = ((8, 31), (32, 47), (48, 63), (64, 95), (96, 512))
 
@@ -205,7 +206,9 @@ def autotune(requests, fp32: bool, widths=WIDTHS, kzs=KZS, buckets=EDGE_BUCKETS,
     one engine, which is what the server runs.  Stage 1: every (width, kz) applied to every
     edge (one width class, so each RK stage stays one launch per kernel); the fastest is the
     base.  Stage 2: for each edge bucket in turn, every kz with the base width for the
-    bucket's edges, kept when the whole mix steps faster.  Tables are judged by the mix's
+    bucket's edges, kept when the whole mix steps faster.  Longer runs are tried first and a
+    later trial has to be 1 % faster, more than two windows of one table differ by.  Tables
+    are judged by the mix's
     aggregate cell-steps/s; tiling never changes results (each cell's arithmetic is the
     same whichever lane computes it).
 
@@ -232,9 +235,9 @@ def autotune(requests, fp32: bool, widths=WIDTHS, kzs=KZS, buckets=EDGE_BUCKETS,
 
     best, base = 0.0, None
     for w in widths:
-        for kz in kzs:
+        for kz in sorted(kzs, reverse=True):
             rate = trial(lambda e, w=w, kz=kz: (w, kz), f"all edges {w} x {kz}")
-            if rate > best:
+            if rate > 1.01 * best:
                 best, base = rate, (w, kz)
     choice = {bk: base[1] for bk in buckets}
 
@@ -251,7 +254,7 @@ def autotune(requests, fp32: bool, widths=WIDTHS, kzs=KZS, buckets=EDGE_BUCKETS,
             trial_choice[bk] = kz
             rate = trial(lambda e, c=trial_choice: (base[0], c.get(bucket_of(e), base[1])),
                          f"edges {bk[0]}-{bk[1]} kz {kz}")
-            if rate > best:
+            if rate > 1.01 * best:
                 best, choice = rate, trial_choice
     eng.close()
     del eng

@@ -14,6 +14,7 @@
 #include <cstring>
 #include <map>
 #include <new>
+#include <queue>
 #include <vector>
 
 #include "cns_batch.h"
@@ -85,12 +86,9 @@ struct BoxHost {
 
 int width_class(int w) { return w == 16 ? 0 : (w == 32 ? 1 : (w == 64 ? 2 : -1)); }
 
-// Default tile: 32 x 8 columns for every edge, so all boxes share one width class and
-// an RK stage is two launches; z runs of 16 planes.  On the mixed request stream (edges
-// 24-128) this steps 8 % faster in FP32 than per-edge widths chosen by lane efficiency
-// or by timing each edge alone (4.58 vs 4.24 G cell-steps/s; FP64 2.46 vs 2.44 G), and
-// runs of 16 planes beat runs of 8 or 32 by 2-3 %.
-std::pair<int, int> default_tile(int e) { return {32, std::min(e, 16)}; }
+// Default tile: 32-wide columns, so that all boxes share one width class and an RK stage is
+// one launch of the fused kernel, whose work list chooses the z runs.
+std::pair<int, int> default_tile(int e) { return {32, e}; }
 
 }  // namespace
 
@@ -158,11 +156,124 @@ void destroy_graph(cns_batch *b)
     b->graph = nullptr;
 }
 
+// The fused class's work list.  A CU holds one workgroup of the stage kernel, which takes
+// about planes + 1.5 plane times, and XCD x runs the x-th eighth of the list in order on its
+// 32 CUs.  So the list is made of eight equally long parts (dummy tiles fill them up): the z
+// runs of all boxes, longest first, each go whole (its tiles share halos) to the part with the
+// least work.  Long runs fill their windows less often, short ones end together: the boxes are
+// split in one of a few ways, the one whose slowest part is predicted to end first.
+//   Predicted / measured, 64 boxes of edges 16..96 (the work alone: 125 plane times of every
+// CU): runs of 16 planes 140 / 2.86 ms a step (FP64), of 32 151 / 3.17, this list 134 / 2.80;
+// 40 boxes of 24..128 (233): runs of 16 in the boxes' order 5.12 ms (FP32 flux), of 32 longest
+// first 260 / 4.86, this list 248 / 4.64.
+constexpr int kXcds = 8, kCusPerXcd = 32;
+constexpr size_t kMostSimulated = 1 << 14;  // tiles; a longer list's tail is short however it is split
+
+struct Split {
+    int run, last, eighths;  // runs of `run` planes, and of `last` for so many eighths:
+    bool boxes;              // of the work, the smallest boxes (or the last planes of every box)
+};
+constexpr Split kSplits[] = {{24, 0, 0, false}, {16, 0, 0, false}, {32, 0, 0, false}, {48, 0, 0, false},
+                             {64, 0, 0, false}, {48, 16, 3, true}, {32, 16, 2, true}, {24, 16, 2, true},
+                             {40, 8, 2, true},  {64, 12, 1, false}, {48, 8, 1, false}, {24, 8, 4, false}};
+
+struct FusedBox {
+    int id, e, kz, xy;  // kz: longest run allowed; xy: tiles of a plane
+};
+struct Unit {
+    int box, z0, nz;  // index of the FusedBox
+};
+struct FusedPlan {
+    std::vector<Unit> part[kXcds];
+    int64_t end = 0;  // of the slowest part, in half plane times
+    size_t tiles = 0;
+};
+
+// `boxes`: largest first
+FusedPlan plan_runs(const std::vector<FusedBox> &boxes, const Split &sp, bool simulate)
+{
+    FusedPlan p;
+    std::vector<Unit> units;
+    int64_t all = 0, done = 0;
+    for (const FusedBox &b : boxes) all += (int64_t)b.xy * b.e;
+    // planes z0 .. z1-1 of box b in even runs of about `run`, at most the box's kz
+    auto runs = [&](int b, int z0, int z1, int run) {
+        const int len = z1 - z0;
+        if (len <= 0) return;
+        const int n = std::max({1, (len + run / 2) / run, (len + boxes[b].kz - 1) / boxes[b].kz});
+        const int nz = (len + n - 1) / n;
+        for (int z = z0; z < z1; z += nz) units.push_back({b, z, std::min(nz, z1 - z)});
+    };
+    for (int b = 0; b < (int)boxes.size(); b++) {
+        const int e = boxes[b].e;
+        if (sp.boxes) {
+            runs(b, 0, e, 8 * done < (8 - sp.eighths) * all ? sp.run : sp.last);
+            done += (int64_t)boxes[b].xy * e;
+        } else {
+            const int first = e - e * sp.eighths / 8;
+            runs(b, 0, first, sp.run);
+            runs(b, first, e, sp.last);
+        }
+    }
+    std::stable_sort(units.begin(), units.end(), [](const Unit &a, const Unit &b) { return a.nz > b.nz; });
+    int64_t load[kXcds] = {};
+    for (const Unit &u : units) {
+        const int x = (int)(std::min_element(load, load + kXcds) - load);
+        load[x] += (int64_t)boxes[u.box].xy * (2 * u.nz + 3);
+        p.part[x].push_back(u);
+        p.tiles += (size_t)boxes[u.box].xy;
+    }
+    for (int x = 0; simulate && x < kXcds; x++) {
+        std::priority_queue<int64_t, std::vector<int64_t>, std::greater<int64_t>> cu;
+        for (int i = 0; i < kCusPerXcd; i++) cu.push(0);
+        for (const Unit &u : p.part[x])
+            for (int t = 0; t < boxes[u.box].xy; t++) {
+                const int64_t end = cu.top() + 2 * u.nz + 3;
+                cu.pop();
+                cu.push(end);
+                p.end = std::max(p.end, end);
+            }
+    }
+    return p;
+}
+
+// Appends the list; returns the number of its real tiles.
+size_t fused_list(std::vector<FusedBox> &boxes, std::vector<TileDev> &out)
+{
+    std::stable_sort(boxes.begin(), boxes.end(), [](const FusedBox &a, const FusedBox &b) { return a.e > b.e; });
+    size_t most = 0;
+    for (const FusedBox &b : boxes) most += (size_t)b.xy * ((b.e + 11) / 12);
+    const bool simulate = most <= kMostSimulated;
+    FusedPlan best;
+    for (const Split &sp : kSplits) {
+        FusedPlan p = plan_runs(boxes, sp, simulate);
+        if (&sp == kSplits || p.end < best.end) best = std::move(p);
+        if (!simulate) break;
+    }
+    std::vector<TileDev> part[kXcds];
+    most = 0;
+    for (int x = 0; x < kXcds; x++) {
+        for (const Unit &u : best.part[x]) {
+            const FusedBox &b = boxes[u.box];
+            for (int y0 = 0; y0 < b.e; y0 += kFusedHeight)
+                for (int x0 = 0; x0 < b.e; x0 += 32)
+                    part[x].push_back({b.id, (short)x0, (short)y0, (short)u.z0, (short)u.nz, 5, 0});
+        }
+        most = std::max(most, part[x].size());
+    }
+    for (int x = 0; x < kXcds; x++) {
+        part[x].resize(most, {boxes[0].id, 0, 0, 0, 0, 5, 0});  // no planes: ends at once
+        out.insert(out.end(), part[x].begin(), part[x].end());
+    }
+    return best.tiles;
+}
+
 // Rebuild the work list and re-capture the step graph.
 int rebuild(cns_batch *b, hipStream_t s)
 {
     CNS_HIPCHK(hipStreamSynchronize(s));  // host staging is about to change
     std::vector<TileDev> cls[kTileClasses];
+    std::vector<FusedBox> fboxes;
     b->hids.clear();
     for (int id = 0; id < (int)b->hb.size(); id++) {
         BoxHost &h = b->hb[id];
@@ -173,7 +284,11 @@ int rebuild(cns_batch *b, hipStream_t s)
         const bool fused = b->fused() && c == 1;
         if (h.fused && !fused) CNS_HIPCHK(launch_batch_init(b->d_boxes, id, h.e, b->fp32, false, s));
         h.fused = fused;
-        const int hgt = fused ? kFusedHeight : kBatchThreads / w, ltx = c + 4;
+        if (fused) {
+            fboxes.push_back({id, h.e, kz, ((h.e + 31) / 32) * ((h.e + kFusedHeight - 1) / kFusedHeight)});
+            continue;
+        }
+        const int hgt = kBatchThreads / w, ltx = c + 4;
         for (int z0 = 0; z0 < h.e; z0 += kz)
             for (int y0 = 0; y0 < h.e; y0 += hgt)
                 for (int x0 = 0; x0 < h.e; x0 += w) {
@@ -188,6 +303,9 @@ int rebuild(cns_batch *b, hipStream_t s)
                     cls[c].push_back(td);
                 }
     }
+    b->ntiles = 0;
+    for (int c = 0; c < kTileClasses; c++) b->ntiles += (int)cls[c].size();
+    if (!fboxes.empty()) b->ntiles += (int)fused_list(fboxes, cls[1]);
     b->htiles.clear();
     for (int c = 0; c < kTileClasses; c++) {
         b->cls_start[c] = (int)b->htiles.size();
@@ -195,11 +313,11 @@ int rebuild(cns_batch *b, hipStream_t s)
         b->htiles.insert(b->htiles.end(), cls[c].begin(), cls[c].end());
     }
     b->nresident = (int)b->hids.size();
-    b->ntiles = (int)b->htiles.size();
-    if ((size_t)b->ntiles > b->tile_cap) {
+    const size_t listed = b->htiles.size();
+    if (listed > b->tile_cap) {
         if (b->d_tiles) CNS_HIPCHK(hipFree(b->d_tiles));
         b->d_tiles = nullptr;
-        size_t cap = std::max<size_t>((size_t)b->ntiles * 2, 1024);
+        size_t cap = std::max<size_t>(listed * 2, 1024);
         if (hipMalloc((void **)&b->d_tiles, cap * sizeof(TileDev)) != hipSuccess) {
             (void)hipGetLastError();
             b->tile_cap = 0;
@@ -207,8 +325,8 @@ int rebuild(cns_batch *b, hipStream_t s)
         }
         b->tile_cap = cap;
     }
-    if (b->ntiles)
-        CNS_HIPCHK(hipMemcpyAsync(b->d_tiles, b->htiles.data(), b->ntiles * sizeof(TileDev),
+    if (listed)
+        CNS_HIPCHK(hipMemcpyAsync(b->d_tiles, b->htiles.data(), listed * sizeof(TileDev),
                                   hipMemcpyHostToDevice, s));
     if (b->nresident)
         CNS_HIPCHK(hipMemcpyAsync(b->d_ids, b->hids.data(), b->nresident * sizeof(int),

@@ -79,6 +79,7 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
     const int ti = xcd_tile(blockIdx.x, gridDim.x);
     if (ti >= ntiles) return;
     const TileDev tl = tiles[ti];
+    if (tl.nz == 0) return;  // filler of an XCD's part of the list
     BoxDev &B = boxes[__builtin_amdgcn_readfirstlane(tl.box)];
     if (box_stopped(B)) return;  // uniform over the workgroup
     const int x0 = __builtin_amdgcn_readfirstlane(tl.x0), y0 = __builtin_amdgcn_readfirstlane(tl.y0);

@@ -74,10 +74,11 @@ int cns_batch_set_target(cns_batch *b, int box_id, long long target);
 int cns_batch_query(cns_batch *b, int n, const int *ids, long long *steps, double *dt,
                     double *courno, int *err);
 
-/* Tile shape used for boxes of a given edge: width 16, 32 or 64 cells (height
- * 256/width) and z run kz (1..edge).  Applies to boxes admitted afterwards and
- * rebuilds the work list.  The table starts from built-in defaults; the
- * package's autotuner measures and sets it. */
+/* Tile shape used for boxes of a given edge: width 16, 32 or 64 cells and z run kz
+ * (1..edge).  Tiles are 256/width cells high, 32-wide ones 16, whose kz is the longest run:
+ * the work list splits every box so that the GPU's CUs end together.  Applies to boxes
+ * admitted afterwards and rebuilds the work list; results do not depend on it.  The table
+ * starts from built-in defaults; the package's autotuner measures and sets it. */
 int cns_batch_set_tile(cns_batch *b, int edge, int tile_width, int kz);
 int cns_batch_get_tile(cns_batch *b, int edge, int *tile_width, int *kz);
 
