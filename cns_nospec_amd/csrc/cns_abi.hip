@@ -542,18 +542,24 @@ static int enqueue_step(cns_ctx *ctx, double *U, double *Unew, double *Q, double
         // Every ABI array ends as the reference leaves it (cpu/advance.cpp:13-154).
         double *T = ctx->d_stage;
         if (pipe_on({U, Unew, Q, D, F, T}) && stage_fits(g)) {
-            // One kernel per stage (cns_stage.hip): it derives the primitives, D and F of its
-            // cells itself, so a stage is the ghost fill of the state and that kernel.  The
-            // Courant number needs the whole state before any update, in a pass that stores
-            // nothing.  Stage 2 also stores the primitives of its result, the Q the
-            // reference leaves; the last fill copies their ghosts with the state's.
+            // The ghosts of U with the Courant number, which needs the whole state before any
+            // update, then a kernel per stage, which derives the primitives, D and F of its cells
+            // itself (cns_stage.hip).  Stage 2 also stores the primitives of its result, the Q
+            // the reference leaves.  Where the stages wrap, they read their state at periodic
+            // addresses and stage 3 fills the ghosts of Unew and Q beside its own work.
             const double *dxi = ctx->dxi;
+            const BoxSet one;
+            const bool wraps = stage_wraps(g);
+            auto stage = [&](int phase, const double *cons, double *out, double *wrapped) {
+                return launch_stage(g, cons, U, out, Q, D, F, sd, dxi, ctx->eta, ctx->alam, phase, s, one,
+                                    wraps ? wrapped : nullptr);
+            };
             TIMED(ctx, CNS_PROF_FILL_CTOPRIM, s, launch_fill_courno(g, U, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
-            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, U, U, T, Q, D, F, sd, dxi, ctx->eta, ctx->alam, 1, s));
-            TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, T, nullptr, s));
-            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, T, U, Unew, Q, D, F, sd, dxi, ctx->eta, ctx->alam, 2, s));
-            TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, Q, s));
-            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, launch_stage(g, Unew, U, U, Q, D, F, sd, dxi, ctx->eta, ctx->alam, 3, s));
+            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stage(1, U, T, U));
+            if (!wraps) TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, T, nullptr, s));
+            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stage(2, T, Unew, T));
+            if (!wraps) TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, Q, s));
+            TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stage(3, Unew, U, Unew));
             return CNS_OK;
         }
         // Arrays that are not 16-byte aligned, or too large for its offsets: fill, ctoprim,

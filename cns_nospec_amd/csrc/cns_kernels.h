@@ -96,9 +96,14 @@ hipError_t launch_fill_courno(const Geom &g, double *u, unsigned long long *acc,
 // ghosted state cons with base U^n (phases 2 and 3), its primitives into q (phase 2), D and
 // F stored by phase 3.  Every array must be 16-byte aligned; out must not alias cons; the
 // geometry must satisfy stage_fits (planes below 4 GiB, pitches below 2^24).
+// wrapped (one box; the same array as cons in phases 2 and 3, any in phase 1): the periodic
+// box needs no fill between its stages.  Phases 1 and 2 store the x ghosts of out beside its
+// interior, phases 2 and 3 read cons at wrapped rows and planes, and phase 3 fills the ghosts
+// of cons (which is not const then) and q.  Null: cons has its ghosts filled.
 bool stage_fits(const Geom &g);
+bool stage_wraps(const Geom &g);  // whether a periodic box is stepped without fills between its stages
 hipError_t launch_stage(const Geom &g, const double *cons, const double *base, double *out, double *q, double *d,
                         double *f, const StepDt &sd, const double dxi[3], double eta, double alam, int phase,
-                        hipStream_t s, const BoxSet &bs = BoxSet());
+                        hipStream_t s, const BoxSet &bs = BoxSet(), double *wrapped = nullptr);
 
 }  // namespace cns

@@ -7,6 +7,7 @@
 // compiled with -ffp-contract=off, so results are bit-identical to the
 // reference cpu/ path (which g++ -O2 builds without FMA).
 #include "cns_kernels.h"
+#include "cns_fill.h"
 
 namespace cns {
 
@@ -22,109 +23,7 @@ inline int stream_grid(int64_t work, int per_thread = 4)
     return (int)blocks;
 }
 
-// ------------------------------------------------------------------ ghost fill
-// The reference fills the ghost shell in three ordered copy passes (z planes over
-// interior i,j; y planes over interior i and all k; x columns over all j,k:
-// cpu/helper_functions.cpp:226-262, gpu/util.cu:53-127).  For extents >= NG their
-// composition maps every ghost cell to the interior cell at the periodic image
-// of all three of its indices, so one pass over the shell copies exactly the same
-// values.  The shell is enumerated compactly: first the full rows whose j or k is
-// a ghost index (g0 cells each), then the 2*NG ghost cells of each interior row.
-//
-// One thread per ghost cell, its components' loads all in flight before the first store.
-// What bounds it: at small boxes latency, so the index arithmetic is 32-bit with
-// precomputed quotients; at large ones the x ghosts, whose four-cell pieces touch
-// two 128-byte lines per row and component.
-struct Shell {
-    FastDiv g0, g1, n1, nbx, nby;
-    unsigned plane_rows, elems_a, total;  // rows of the ghost planes; cells of the full rows; all cells
-};
-
-Shell make_shell(const Geom &g, const int nb[3])
-{
-    Shell h;
-    h.g0 = fast_div(g.g0);
-    h.g1 = fast_div(g.g1);
-    h.n1 = fast_div(g.n1);
-    h.nbx = fast_div(nb[0]);
-    h.nby = fast_div(nb[1]);
-    h.plane_rows = 2u * NG * g.g1;
-    h.elems_a = (h.plane_rows + 2u * NG * g.n2) * g.g0;
-    h.total = h.elems_a + 2u * NG * (unsigned)g.n1 * g.n2;
-    return h;
-}
-
-int64_t shell_cells(const Geom &g)
-{
-    return ((int64_t)2 * NG * g.g1 + (int64_t)2 * NG * g.n2) * g.g0 + (int64_t)2 * NG * g.n1 * g.n2;
-}
-
-// Ghost cell e of the enumeration, as (i, j, k).
-__device__ __forceinline__ void shell_cell(const Geom &g, const Shell &h, unsigned e, int &i, int &j, int &k)
-{
-    if (e < h.elems_a) {
-        unsigned r = h.g0.div(e);
-        i = (int)(e - r * g.g0);
-        if (r < h.plane_rows) {
-            const int kk = (int)h.g1.div(r);
-            j = (int)r - kk * g.g1;
-            k = kk < NG ? kk : g.n2 + kk;
-        } else {
-            r -= h.plane_rows;
-            const int jj = (int)(r & (2 * NG - 1));
-            k = NG + (int)(r / (2 * NG));
-            j = jj < NG ? jj : g.n1 + jj;
-        }
-    } else {
-        const unsigned e2 = e - h.elems_a, row = e2 / (2 * NG), kk = h.n1.div(row);
-        const int ii = (int)(e2 & (2 * NG - 1));
-        i = ii < NG ? ii : g.n0 + ii;
-        k = NG + (int)kk;
-        j = NG + (int)(row - kk * g.n1);
-    }
-}
-
-// One axis of a ghost cell at index a of box I of nb boxes of n cells: the box (relative
-// step dI) and the index there of the cell it is the periodic image of.  Extents are at
-// least NG, so that is the neighbouring box.
-__device__ __forceinline__ int image(int a, int I, int n, int nb, int &dI)
-{
-    dI = a < NG ? (I == 0 ? nb - 1 : -1) : (a >= n + NG ? (I == nb - 1 ? 1 - nb : 1) : 0);
-    return a < NG ? a + n : (a >= n + NG ? a - n : a);
-}
-
-// Ghost cell e of box b of a set of nb[0] x nb[1] x nb[2] boxes (one box: its own images).  Q:
-// the components of q as well.
-template <bool Q>
-__device__ __forceinline__ void fill_cell(const Geom &g, const Shell &h, const BoxSet &bs, int nbx, int nby, int nbz,
-                                          unsigned e, unsigned b, double *u, double *q)
-{
-    const unsigned r = h.nbx.div(b);
-    const int K = (int)h.nby.div(r), J = (int)r - K * nby, I = (int)b - (int)r * nbx;
-    int i, j, k, dI, dJ, dK;
-    shell_cell(g, h, e, i, j, k);
-    const int is = image(i, I, g.n0, nbx, dI), js = image(j, J, g.n1, nby, dJ), ks = image(k, K, g.n2, nbz, dK);
-    const int64_t bsrc = (int64_t)b + dI + (int64_t)nbx * (dJ + (int64_t)nby * dK);
-    const int64_t dst = gidx(g, i, j, k), src = gidx(g, is, js, ks);
-    const double *us = u + bsrc * bs.su + src;
-    double *ud = u + b * bs.su + dst;
-    double v[NC], w[NQ];
-#pragma unroll
-    for (int l = 0; l < NC; l++) v[l] = us[l * g.cg];
-    if (Q) {
-        const double *qs = q + bsrc * bs.sq + src;
-#pragma unroll
-        for (int l = 0; l < NQ; l++) w[l] = qs[l * g.cg];
-    }
-#pragma unroll
-    for (int l = 0; l < NC; l++) ud[l * g.cg] = v[l];
-    if (Q) {
-        double *qd = q + b * bs.sq + dst;
-#pragma unroll
-        for (int l = 0; l < NQ; l++) qd[l * g.cg] = w[l];
-    }
-}
-
+// ------------------------------------------------------------------ ghost fill (cns_fill.h)
 template <bool Q>
 __global__ void __launch_bounds__(kStreamBlock)
 fill_kernel(Geom g, Shell h, BoxSet bs, int nbx, int nby, int nbz, double *__restrict__ u, double *__restrict__ q)

@@ -42,8 +42,10 @@
 // SIMD 7 % slower, LDS reads issued half a tap pair ahead no faster.
 //   Every value is computed by the reference's expression (-ffp-contract=off), so results are
 // bit-identical to the reference cpu/ path.
+#include <algorithm>
 #include <type_traits>
 
+#include "cns_fill.h"
 #include "cns_stage_tile.h"
 
 namespace cns {
@@ -61,9 +63,15 @@ struct StageArgs {
     double *q;           // primitives of the result (QOUT)
     double *d, *f;       // D and F (LAST)
     StepDt sd;           // the step's dt, made by stage 1 from the Courant maximum
+    // WRAP, the box is its own periodic neighbour: stages 2 and 3 read cons at wrapped rows and planes,
+    // of which stages 1 and 2 store the x ghosts with the result.  Stage 3 then also fills the
+    // ghosts of cons and q: workgroups nt and above.
+    int nt;
+    Shell shell;
+    double *fill_u;
 };
 
-template <bool STAGE1, bool LAST, bool QOUT>
+template <bool STAGE1, bool LAST, bool QOUT, bool WRAP>
 __global__ void __launch_bounds__(NT, 2)
 stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, double dxi1, double dxi2,
              double eta, double alam, int kz, int ntx, int nty, BoxSet bs, int nbpb)
@@ -79,7 +87,13 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     __shared__ double s_wz[TILE];
     __shared__ double s_ring[8 * HALO];                // w of plane p on the halo columns, slot p % 8
 
-    int t = xcd_tile(blockIdx.x, gridDim.x);
+    if (LAST && WRAP && (int)blockIdx.x >= a.nt) {
+        const unsigned stride = (gridDim.x - a.nt) * NT;
+        for (unsigned e = (blockIdx.x - a.nt) * NT + threadIdx.x; e < a.shell.total; e += stride)
+            fill_cell<true>(g, a.shell, bs, 1, 1, 1, e, 0, a.fill_u, a.q, false);
+        return;
+    }
+    int t = xcd_tile(blockIdx.x, a.nt);
     const int box = t / nbpb;
     t -= box * nbpb;
     cons += box * bs.su;
@@ -120,8 +134,30 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
 
     // In-plane byte offset of tile cell (r, c)'s 16-byte pair, clamped into the array: cells
     // past the box feed discarded outputs only.
+    // Row r of the tile in the array: clamped, and of a box that wraps the periodic image (a few
+    // instructions that only the tiles at the box's y ends take; the conditions are formed where
+    // they are used, like the wave's).
+    auto row_of = [&](int r) {
+        int j = min(gj0 + r, g.g1 - 1);
+        if (WRAP && !STAGE1) {
+            int j0 = gj0;
+            asm volatile("" : "+s"(j0));
+            if (j0 == 0 || j0 + R > g.g1 - NG) {
+                j += j < NG ? g.n1 : 0;
+                j -= j >= g.g1 - NG ? g.n1 : 0;
+            }
+        }
+        return j;
+    };
+    auto plane_of = [&](int k) {  // ghosted plane index
+        if (WRAP && !STAGE1) {
+            k += k < NG ? g.n2 : 0;
+            k -= k >= g.n2 + NG ? g.n2 : 0;
+        }
+        return (int64_t)k * pg;
+    };
     auto pair_off = [&](int r, int c) {
-        return (mul24(min(gj0 + r, g.g1 - 1), xg) + (unsigned)min(gi0 + c, g.xg - 2)) * 8u;
+        return (mul24(row_of(r), xg) + (unsigned)min(gi0 + c, g.xg - 2)) * 8u;
     };
     // the lane's cell in ghosted coordinates, whether it lies in the box, and its byte offset
     // within a ghosted plane
@@ -140,7 +176,7 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
         return c;
     };
     auto issue_raw = [&](int k) {  // centre plane k: block `wave` of every field
-        const double *p = cons + (int64_t)(k + NG) * pg;
+        const double *p = cons + (int64_t)(k + NG) * pg;  // an interior plane
         const int w = wv();
         const unsigned lane = opaque_tid() & 63, e = 128 * w + 2 * lane;
         const unsigned off = pair_off(e / PX, e % PX);
@@ -152,7 +188,7 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
     // leading plane of centre plane k: own block wave % 4 of fields 0..2 (waves 0..3) or 3, 4;
     // the y halo's two blocks and the x halo's one on waves 4, 5, 6
     auto issue_lead = [&](int k) {
-        const double *p = cons + (int64_t)(k + 2 * NG) * pg;
+        const double *p = cons + plane_of(k + 2 * NG);
         const int w = wv();
         const unsigned lane = opaque_tid() & 63, ob = w & (OB - 1);
         const unsigned ooff = pair_off(4 + 4 * ob + (lane >> 4), 4 + 2 * (lane & 15));
@@ -286,22 +322,22 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
         double hr[8], hm[8], hz[8];
         {
             auto off8 = [&](unsigned r, unsigned c) {
-                return (mul24(min(gj0 + (int)r, g.g1 - 1), xg) + (unsigned)min(gi0 + (int)c, g.xg - 1)) * 8u;
+                return (mul24(row_of((int)r), xg) + (unsigned)min(gi0 + (int)c, g.xg - 1)) * 8u;
             };
             const unsigned own8 = off8(row + 4, col + 4), h8 = yl ? off8(yrow, col + 4) : off8((xid >> 3) + 4, xcol);
-            const double *p = cons + (int64_t)kbeg * pg, *pm = p + (yl ? IMY : IMX) * cg;
 #pragma unroll
             for (int m = 0; m < 8; m++) {
-                wri[m] = at(p + m * pg, own8);
-                wmx[m] = at(p + m * pg + IMX * cg, own8);
-                wmy[m] = at(p + m * pg + IMY * cg, own8);
-                wmz[m] = at(p + m * pg + IMZ * cg, own8);
-                wE[m] = at(p + m * pg + IENE * cg, own8);
+                const double *p = cons + plane_of(kbeg + m);
+                wri[m] = at(p, own8);
+                wmx[m] = at(p + IMX * cg, own8);
+                wmy[m] = at(p + IMY * cg, own8);
+                wmz[m] = at(p + IMZ * cg, own8);
+                wE[m] = at(p + IENE * cg, own8);
                 hr[m] = hm[m] = hz[m] = 1.0;
                 if (halo) {
-                    hr[m] = at(p + m * pg, h8);
-                    hm[m] = at(pm + m * pg, h8);
-                    hz[m] = at(p + m * pg + IMZ * cg, h8);
+                    hr[m] = at(p, h8);
+                    hm[m] = at(p + (yl ? IMY : IMX) * cg, h8);
+                    hz[m] = at(p + IMZ * cg, h8);
                 }
             }
         }
@@ -677,6 +713,20 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
                     o[l] = STAGE1 ? uc[l] + dt * (D[l] + F[l]) : ra * rkb[l] + rb * (uc[l] + dt * (D[l] + F[l]));
                     at(out + l * cg + zk, own8) = o[l];
                 }
+                // the x ghosts that are images of the cell
+                int i0 = gi0;
+                asm volatile("" : "+s"(i0));
+                if (WRAP && !LAST && (i0 == 0 || i0 + TX + NG > g.n0)) {
+                    const unsigned n8 = (unsigned)g.n0 * 8u;
+                    if (c.i < 2 * NG) {
+#pragma unroll
+                        for (int l = 0; l < NC; l++) at(out + l * cg + zk, own8 + n8) = o[l];
+                    }
+                    if (c.i >= g.n0) {
+#pragma unroll
+                        for (int l = 0; l < NC; l++) at(out + l * cg + zk, own8 - n8) = o[l];
+                    }
+                }
                 if (QOUT) {  // cpu/ctoprim.cpp:23-38
                     double u, v, w, eint, p;
                     ctoprim_cell(o[IRHO], o[IMX], o[IMY], o[IMZ], o[IENE], u, v, w, eint, p);
@@ -723,19 +773,41 @@ bool stage_fits(const Geom &g)
     return g.pg < (1 << 29) && g.xg < (1 << 24) && g.g1 < (1 << 24);
 }
 
+// Reading at wrapped addresses and storing the x ghosts beside the result costs a plane about
+// 1.5 % (scalar registers that no longer fit), two fill launches their time and two gaps: a step
+// with / without them takes 73 / 80 us at 16^3, 113 / 120 at 64^3, 466 / 480 at 128^3, 3.24 / 3.26
+// ms at 256^3 (128 planes a CU), 6.53 / 6.58 at 320^3 (250), 25.9 / 25.6 at 512^3 (1024).
+bool stage_wraps(const Geom &g)
+{
+    return (int64_t)((g.n0 + TX - 1) / TX) * ((g.n1 + BY - 1) / BY) * g.n2 <= 512 * kCUs;
+}
+
 hipError_t launch_stage(const Geom &g, const double *cons, const double *base, double *out, double *q, double *d,
                         double *f, const StepDt &sd, const double dxi[3], double eta, double alam, int phase,
-                        hipStream_t s, const BoxSet &bs)
+                        hipStream_t s, const BoxSet &bs, double *wrapped)
 {
-    if (bs.n < 1 || !stage_fits(g)) return hipErrorInvalidValue;
-    const StageArgs a{base, out, q, d, f, sd};
+    if (bs.n < 1 || !stage_fits(g) || (wrapped && bs.n != 1)) return hipErrorInvalidValue;
     const int ntx = (g.n0 + TX - 1) / TX, nty = (g.n1 + BY - 1) / BY;
     const int kz = stage_kz(g, (int64_t)ntx * nty * bs.n);
     const int64_t nbpb = (int64_t)ntx * nty * ((g.n2 + kz - 1) / kz);
     if (nbpb * bs.n > 0x7fffffff) return hipErrorInvalidValue;
-    const int nb = (int)(nbpb * bs.n);
-#define STAGE(S1, L, QO) \
-    stage_kernel<S1, L, QO><<<nb, NT, 0, s>>>(g, cons, a, dxi[0], dxi[1], dxi[2], eta, alam, kz, ntx, nty, bs, (int)nbpb)
+    const int nt = (int)(nbpb * bs.n);
+    const StageArgs a{base, out, q, d, f, sd, nt, make_shell(g, kOneBox), wrapped};
+    // Ghost cells of stage 3, about one a thread in a small box, whose fill workgroups take the
+    // CUs that the stage leaves idle; at most one workgroup a CU.
+    int nb = nt;
+    if (wrapped && phase == 3) {
+        const int64_t total = shell_cells(g);
+        if (total > 0xffffffffll - kCUs * NT) return hipErrorInvalidValue;
+        nb += (int)std::min<int64_t>((total + NT - 1) / NT, kCUs);
+    }
+#define STAGE(S1, L, QO)                                                                                           \
+    if (wrapped)                                                                                                   \
+        stage_kernel<S1, L, QO, true><<<nb, NT, 0, s>>>(g, cons, a, dxi[0], dxi[1], dxi[2], eta, alam, kz, ntx, nty, \
+                                                        bs, (int)nbpb);                                            \
+    else                                                                                                           \
+        stage_kernel<S1, L, QO, false><<<nb, NT, 0, s>>>(g, cons, a, dxi[0], dxi[1], dxi[2], eta, alam, kz, ntx,     \
+                                                         nty, bs, (int)nbpb)
     switch (phase) {
     case 1: STAGE(true, false, false); break;
     case 2: STAGE(false, false, true); break;
