@@ -414,6 +414,9 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
         __syncthreads();  // B
 
         // ---------------- phase 2
+        // Of the two waves of a SIMD the older wins every choice, and would wait at C while the
+        // younger (4..7) runs alone: the younger goes first up to the end of the z terms.
+        if (wave >= 4) __builtin_amdgcn_s_setprio(1);
         if (k + 1 < kend) issue_lead(k + 1);
         FT F[5], zf[5];
         lead_grads(k);
@@ -498,6 +501,7 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
             const unsigned tid = opaque_tid();
             s_wz[mul24(tid / TX + 4, PX) + (tid & (TX - 1)) + 4] = wzc;
         }
+        __builtin_amdgcn_s_setprio(0);
         shift();  // the centre plane is window entry 3 from here
         constexpr int Z = 4 * PX;
         {

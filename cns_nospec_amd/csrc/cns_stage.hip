@@ -40,6 +40,10 @@
 // and pin() and FENCE().  One wave per SIMD with 512 registers (32 x 8 tiles) ran
 // 12.4 ms per stage at 512^3, opposite order of the z and the x, y parts in the two waves of a
 // SIMD 7 % slower, LDS reads issued half a tap pair ahead no faster.
+//   Wave priorities (phase 2) took 930 / 1040 / 1095 us for stages 1 / 2 / 3 at 256^3 where equal ones
+// took 943 / 1051 / 1136; the younger wave first in phase 3 too, or always, was no faster.  LDS reads of the
+// x taps issued a z tap ahead, lead() in phase 3, and the stage base loaded at the start of phase 3 were not
+// faster either.  With the full chip running on a real flow the clock is at 2.05 GHz (2.35 on constant data).
 //   Every value is computed by the reference's expression (-ffp-contract=off), so results are
 // bit-identical to the reference cpu/ path.
 #include <algorithm>
@@ -429,6 +433,9 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
         __syncthreads();  // B
 
         // ---------------- phase 2
+        // Of the two waves of a SIMD the older wins every choice, and would wait at C while the
+        // younger (4..7) runs alone: the younger goes first up to the end of the z terms.
+        if (wave >= 4) __builtin_amdgcn_s_setprio(1);
         if (k + 1 < kend) issue_lead(k + 1);
         double F[5], zf[5], rho_c;
         lead_grads(k);
@@ -519,6 +526,7 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
             const unsigned tid = opaque_tid();
             s_wz[mul24(tid / TX + 4, PX) + (tid & (TX - 1)) + 4] = wzc;
         }
+        __builtin_amdgcn_s_setprio(0);
         shift();  // the centre plane is window entry 3 from here
         {
             // from four rows above the own cell: every tap is a non-negative constant away
