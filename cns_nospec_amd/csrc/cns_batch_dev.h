@@ -36,7 +36,7 @@ struct TileDev {
     int box;
     short x0, y0, z0, nz;  // tile origin (cells) and z run
     short ltx;             // log2 of the tile width (4, 5 or 6)
-    short pad;
+    short rows;            // of a tile of the fused kernel
 };
 
 // Tile widths 16, 32, 64 (class 0, 1, 2); a box's tiles all have one width.
@@ -50,7 +50,7 @@ hipError_t launch_batch_finalize(BoxDev *boxes, const int *box_ids, int nbox, in
                                  hipStream_t s);
 // One RK stage over the tile list: the list holds class 0, 1, 2 tiles in the
 // ranges [start[c], start[c]+count[c]).  fused: class 1 takes one launch of the fused stage
-// kernel, and its tiles are kFusedHeight rows high; it neither reads nor writes Q.  Every
+// kernel, and its tiles are kShortRows or (FP32 flux only) kTallRows high; it neither reads nor writes Q.  Every
 // other class gets a diffterm launch, then a hypterm + update launch, of one workgroup per
 // tile.  staged_diff selects the diffterm whose planes are staged by direct-to-LDS loads,
 // preceded by a wz-field launch per class; keep_centre the FP32 hypterm + update of stages 2
@@ -59,7 +59,7 @@ hipError_t launch_batch_stage(BoxDev *boxes, const TileDev *tiles, const int sta
                               const int count[3], int stage, bool fp32, bool fused, bool staged_diff,
                               bool keep_centre, hipStream_t s);
 // Its class-1 launch (cns_batch_stage.hip).
-constexpr int kFusedHeight = 16;
+constexpr int kShortRows = 16, kTallRows = 24;
 hipError_t launch_batch_fused(BoxDev *boxes, const TileDev *tiles, int n, int stage, bool fp32, hipStream_t s);
 
 }  // namespace cns

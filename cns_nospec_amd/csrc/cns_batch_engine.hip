@@ -9,6 +9,7 @@
 // the dt finalize) is captured once into a hipGraph and replayed until the
 // resident set or the tile table changes.
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -162,11 +163,12 @@ void destroy_graph(cns_batch *b)
 // runs of all boxes, longest first, each go whole (its tiles share halos) to the part with the
 // least work.  Long runs fill their windows less often, short ones end together: the boxes are
 // split in one of a few ways, the one whose slowest part is predicted to end first.
-//   Predicted / measured, 64 boxes of edges 16..96 (the work alone: 125 plane times of every
-// CU): runs of 16 planes 140 / 2.86 ms a step (FP64), of 32 151 / 3.17, this list 134 / 2.80;
-// 40 boxes of 24..128 (233): runs of 16 in the boxes' order 5.12 ms (FP32 flux), of 32 longest
-// first 260 / 4.86, this list 248 / 4.64.
+//   Predicted / measured with 16-row tiles alone, 64 boxes of edges 16..96 (the work alone: 125
+// plane times of every CU): runs of 16 planes 140 / 2.86 ms a step (FP64), of 32 151 / 3.17, this
+// list 134 / 2.80; 40 boxes of 24..128 (233): runs of 16 in the boxes' order 5.12 ms (FP32 flux), of
+// 32 longest first 260 / 4.86, this list 248 / 4.64.
 constexpr int kXcds = 8, kCusPerXcd = 32;
+constexpr int kTallCost = 4, kShortCost = 3;  // of a plane
 constexpr size_t kMostSimulated = 1 << 14;  // tiles; a longer list's tail is short however it is split
 
 struct Split {
@@ -178,14 +180,35 @@ constexpr Split kSplits[] = {{24, 0, 0, false}, {16, 0, 0, false}, {32, 0, 0, fa
                              {40, 8, 2, true},  {64, 12, 1, false}, {48, 8, 1, false}, {24, 8, 4, false}};
 
 struct FusedBox {
-    int id, e, kz, xy;  // kz: longest run allowed; xy: tiles of a plane
+    int id, e, kz;      // kz: longest run allowed
+    int nx, tall, low;  // tiles of a plane: nx times so many of kTallRows and of kShortRows rows
+    int cost() const { return nx * (kTallCost * tall + kShortCost * low); }
+    int tiles() const { return nx * (tall + low); }
 };
+
+// A box's rows in the fewest plane times: of FP32 flux a tall tile's plane takes 1.35 times a
+// short one's (cns_batch_stage.hip; edges 96 and 64 measured), e.g. 16 rows one short tile, 24 one
+// tall, 32 two short, 40 one of each.
+void tile_rows(FusedBox &b, bool fp32)
+{
+    int best = INT_MAX;
+    for (int tall = 0; tall <= (fp32 ? (b.e + kTallRows - 1) / kTallRows : 0); tall++) {
+        const int low = std::max(0, (b.e - tall * kTallRows + kShortRows - 1) / kShortRows);
+        const int cost = kTallCost * tall + kShortCost * low;
+        if (cost < best) {
+            best = cost;
+            b.tall = tall;
+            b.low = low;
+        }
+    }
+}
+
 struct Unit {
     int box, z0, nz;  // index of the FusedBox
 };
 struct FusedPlan {
     std::vector<Unit> part[kXcds];
-    int64_t end = 0;  // of the slowest part, in half plane times
+    int64_t end = 0;  // of the slowest part, in sixths of a short tile's plane time
     size_t tiles = 0;
 };
 
@@ -195,7 +218,7 @@ FusedPlan plan_runs(const std::vector<FusedBox> &boxes, const Split &sp, bool si
     FusedPlan p;
     std::vector<Unit> units;
     int64_t all = 0, done = 0;
-    for (const FusedBox &b : boxes) all += (int64_t)b.xy * b.e;
+    for (const FusedBox &b : boxes) all += (int64_t)b.cost() * b.e;
     // planes z0 .. z1-1 of box b in even runs of about `run`, at most the box's kz
     auto runs = [&](int b, int z0, int z1, int run) {
         const int len = z1 - z0;
@@ -208,7 +231,7 @@ FusedPlan plan_runs(const std::vector<FusedBox> &boxes, const Split &sp, bool si
         const int e = boxes[b].e;
         if (sp.boxes) {
             runs(b, 0, e, 8 * done < (8 - sp.eighths) * all ? sp.run : sp.last);
-            done += (int64_t)boxes[b].xy * e;
+            done += (int64_t)boxes[b].cost() * e;
         } else {
             const int first = e - e * sp.eighths / 8;
             runs(b, 0, first, sp.run);
@@ -219,16 +242,17 @@ FusedPlan plan_runs(const std::vector<FusedBox> &boxes, const Split &sp, bool si
     int64_t load[kXcds] = {};
     for (const Unit &u : units) {
         const int x = (int)(std::min_element(load, load + kXcds) - load);
-        load[x] += (int64_t)boxes[u.box].xy * (2 * u.nz + 3);
+        load[x] += (int64_t)boxes[u.box].cost() * (2 * u.nz + 3);
         p.part[x].push_back(u);
-        p.tiles += (size_t)boxes[u.box].xy;
+        p.tiles += (size_t)boxes[u.box].tiles();
     }
     for (int x = 0; simulate && x < kXcds; x++) {
         std::priority_queue<int64_t, std::vector<int64_t>, std::greater<int64_t>> cu;
         for (int i = 0; i < kCusPerXcd; i++) cu.push(0);
         for (const Unit &u : p.part[x])
-            for (int t = 0; t < boxes[u.box].xy; t++) {
-                const int64_t end = cu.top() + 2 * u.nz + 3;
+            for (int t = 0; t < boxes[u.box].tiles(); t++) {
+                const int c = t < boxes[u.box].nx * boxes[u.box].tall ? kTallCost : kShortCost;
+                const int64_t end = cu.top() + c * (2 * u.nz + 3);
                 cu.pop();
                 cu.push(end);
                 p.end = std::max(p.end, end);
@@ -242,7 +266,7 @@ size_t fused_list(std::vector<FusedBox> &boxes, std::vector<TileDev> &out)
 {
     std::stable_sort(boxes.begin(), boxes.end(), [](const FusedBox &a, const FusedBox &b) { return a.e > b.e; });
     size_t most = 0;
-    for (const FusedBox &b : boxes) most += (size_t)b.xy * ((b.e + 11) / 12);
+    for (const FusedBox &b : boxes) most += (size_t)b.tiles() * ((b.e + 11) / 12);
     const bool simulate = most <= kMostSimulated;
     FusedPlan best;
     for (const Split &sp : kSplits) {
@@ -255,9 +279,12 @@ size_t fused_list(std::vector<FusedBox> &boxes, std::vector<TileDev> &out)
     for (int x = 0; x < kXcds; x++) {
         for (const Unit &u : best.part[x]) {
             const FusedBox &b = boxes[u.box];
-            for (int y0 = 0; y0 < b.e; y0 += kFusedHeight)
+            for (int y0 = 0, r = 0; r < b.tall + b.low; r++) {
+                const short rows = r < b.tall ? kTallRows : kShortRows;
                 for (int x0 = 0; x0 < b.e; x0 += 32)
-                    part[x].push_back({b.id, (short)x0, (short)y0, (short)u.z0, (short)u.nz, 5, 0});
+                    part[x].push_back({b.id, (short)x0, (short)y0, (short)u.z0, (short)u.nz, 5, rows});
+                y0 += rows;
+            }
         }
         most = std::max(most, part[x].size());
     }
@@ -285,7 +312,9 @@ int rebuild(cns_batch *b, hipStream_t s)
         if (h.fused && !fused) CNS_HIPCHK(launch_batch_init(b->d_boxes, id, h.e, b->fp32, false, s));
         h.fused = fused;
         if (fused) {
-            fboxes.push_back({id, h.e, kz, ((h.e + 31) / 32) * ((h.e + kFusedHeight - 1) / kFusedHeight)});
+            FusedBox fb{id, h.e, kz, (h.e + 31) / 32, 0, 0};
+            tile_rows(fb, b->fp32);
+            fboxes.push_back(fb);
             continue;
         }
         const int hgt = kBatchThreads / w, ltx = c + 4;
@@ -299,7 +328,7 @@ int rebuild(cns_batch *b, hipStream_t s)
                     td.z0 = (short)z0;
                     td.nz = (short)std::min(kz, h.e - z0);
                     td.ltx = (short)ltx;
-                    td.pad = 0;
+                    td.rows = 0;
                     cls[c].push_back(td);
                 }
     }

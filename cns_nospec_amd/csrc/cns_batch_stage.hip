@@ -3,7 +3,7 @@
 //
 // The stage kernel of the plain step (cns_stage.hip: its windows, tiles, phases and LDS
 // staging) for ghost-free boxes and both flux types: a workgroup takes a 32 x 16 column tile
-// and a run of planes of one box and produces, from the five conserved fields alone, the
+// (FP32 flux: or 32 x 24) and a run of planes of one box and produces, from the five conserved fields alone, the
 // result of the stage; in stage 3 also the Courant maximum of the result.  The separate
 // kernels (cns_batch.hip) pass Q, wz and D through memory between a wz, a diffterm and a
 // hypterm launch.
@@ -17,6 +17,13 @@
 //   Flux type FT.  Primitives, the update and the Courant number are FP64 in both modes; with
 // FT = float the windows and tiles hold the rounded values (u, v, w too, which FP64 recomputes
 // as one product) and the pressure less the box's reference, as the separate kernels' fields.
+//   FP32 flux: tall tiles.  A wave issues an instruction every four cycles at best and waits half
+// its time, whatever the type, so a plane of FP32 took as long as one of FP64.  Its windows are
+// half the size, though: 168 registers a lane and 143 KB of LDS hold three waves a SIMD, 32 x 24
+// cells a plane at 1.35 times the time of 32 x 16 (G cell-steps/s, one height for all: edge 96 6.5
+// -> 7.3, 48 5.1 -> 6.0, 24 3.7 -> 5.6).  A box's rows are covered by both heights (fused_list()),
+// for which the kernel holds both bodies; waves 8..11 end at once in a short tile.  64 boxes x4
+// 10.4 -> 9.35 ms, serving 40 boxes x8 40.1 -> 36.4 ms; 24 rows alone gave 9.7 and 37.7.
 //   Every value is the separate kernels' expression: the same bits, and in FP64 the reference's.
 #include "cns_batch_dev.h"
 #include "cns_stage_tile.h"
@@ -28,19 +35,38 @@ namespace {
 
 constexpr int CORN = 64;  // corner cells of a tile
 
-template <typename FT>
-struct Lay {
+// A tile of BY rows: cns_stage_tile.h's sizes for them, and who does what.
+template <typename FT, int BY_>
+struct Rows {
     static constexpr bool F32 = sizeof(FT) == 4;
-    static constexpr int B = (int)sizeof(FT);
+    static constexpr int BY = BY_, R = BY + 8, NT = TX * BY, NW = NT / 64;
+    static constexpr int TILE = R * PX, XH = 8 * BY, HALO = YH + XH;
+    static constexpr int LHY = 5 * NT, LHX = LHY + 3 * YH, LEAD = LHX + 3 * XH, LU = BY * PX, LV = R * TX;
+    static_assert(LEAD * 8 >= (4 * LU + LV) * (int)sizeof(FT) && 5 * TILE >= 6 * LV && TILE >= LU && LV >= LU,
+                  "places of the window fill");
+    // Shares of the halo cells, one cell per lane, as first waves: leading y halo, its ring and wz
+    // on waves 0..3; leading x halo, its ring and wz on XW waves from 4; centre y halo and its ux on
+    // four from YC; centre x halo on XW from XC; corners on wave CC; vy's x halo on XW from VX.
+    static constexpr int XW = XH / 64, YC = NW - 4, XC = BY == 16 ? 0 : 5, CC = BY == 16 ? 2 : 4, VX = BY == 16 ? 6 : 5;
+    // staged x halo: XS waves of 32 cells, then two of corners
+    static constexpr int XS = XH / 32;
+    static_assert(XH % 64 == 0 && NW >= 8 && 4 + XW <= NW && XC + XW <= NW && VX + XW <= NW && XS + 2 <= NW, "wave shares");
     // staged FP64 halo of the centre plane: y halo (rho; FP32 flux: all five fields, which FP64
     // loads into the tile itself), x halo of five fields, corners of rho, mx, my
     static constexpr int HX = (F32 ? 5 : 1) * YH, HC = HX + 5 * XH, H = HC + 3 * CORN;
-    // where the arrays lie in LDS (the compiler's order, largest first)
-    static constexpr int DER = F32 ? LEAD * 8 : 0, C = F32 ? DER + 5 * TILE * B + H * 8 : DER + 5 * TILE * B;
-    static constexpr int LEAD_ = F32 ? 0 : C + 4 * TILE * B;
-    static constexpr int RING = F32 ? C + 4 * TILE * B : LEAD_ + LEAD * 8;
-    static constexpr int WZ = RING + 8 * HALO * B + (F32 ? 0 : H * 8), LVA = WZ + TILE * B, UXA = LVA + LV * B,
-                         LUA = UXA + LV * B, VYA = LUA + LU * B;
+};
+// The largest tile, whose arrays every tile uses, and where they lie in LDS (the compiler's order,
+// largest first)
+template <typename FT>
+struct Lay : Rows<FT, sizeof(FT) == 4 ? kTallRows : kShortRows> {
+    using G = Rows<FT, sizeof(FT) == 4 ? kTallRows : kShortRows>;
+    static constexpr int B = (int)sizeof(FT);
+    static constexpr int DER = G::F32 ? G::LEAD * 8 : 0;
+    static constexpr int C = DER + 5 * G::TILE * B + (G::F32 && G::H * 8 > 4 * G::TILE * B ? G::H * 8 : 0);
+    static constexpr int LEAD_ = G::F32 ? 0 : C + 4 * G::TILE * B;
+    static constexpr int RING = G::F32 ? DER + 9 * G::TILE * B + G::H * 8 : LEAD_ + G::LEAD * 8;
+    static constexpr int WZ = RING + 8 * G::HALO * B + (G::F32 ? 0 : G::H * 8), LVA = WZ + G::TILE * B,
+                         UXA = LVA + G::LV * B, LUA = UXA + G::LV * B, VYA = LUA + G::LU * B;
 };
 
 // 4 bytes a lane from src + off into 256 consecutive bytes of LDS.
@@ -50,46 +76,63 @@ __device__ __forceinline__ void dma4(const double *src, unsigned off, void *lds)
     __builtin_amdgcn_global_load_lds((const void GAS *)((const char GAS *)src + off), (lds_void *)lds, 4, 0, 0);
 }
 
+template <typename T>
+__device__ __forceinline__ T *uniform(T *p)
+{
+    const uint64_t a = (uint64_t)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a), hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+    return (T *)((uint64_t)hi << 32 | lo);
+}
+
 __device__ __forceinline__ int wrap(int a, int e)
 {
     const int r = a % e;
     return r < 0 ? r + e : r;
 }
 
-template <typename FT, int STAGE>
-__global__ void __launch_bounds__(NT, 2)
-batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles, int ntiles)
+// The arrays of a workgroup in LDS, each an object of its own: reads of one need not wait for
+// the DMA into another.
+template <typename FT>
+struct Shared {
+    double *lead, *h;
+    FT *c, *der, *lu, *lv, *ux, *vy, *ring, *wz;
+    unsigned *lx;
+};
+
+// Returns the lane's largest c + |u|, c + |v|, c + |w| of the result (bits; stage 3).
+template <typename FT, int STAGE, int ROWS>
+__device__ __forceinline__ unsigned long long stage_rows(BoxDev &B, const TileDev &tl, const Shared<FT> &sh)
 {
     using KK = K<FT>;
     using L = Lay<FT>;
-    constexpr bool F32 = L::F32;
-    __shared__ double s_lead[LEAD];                // leading plane, raw (cns_stage.hip's layout)
-    __shared__ double s_h[L::H];                   // centre plane's halo, raw
-    __shared__ FT s_c[4 * TILE];                   // centre plane: mx, my, mz, E
-    __shared__ FT der[VNF * TILE];                 // centre plane, derived
-    __shared__ FT s_lu[LU];                        // leading u: own rows, column c (0..39)
-    __shared__ FT s_lv[LV];                        // leading v: row r (0..R-1), column 4+c
-    __shared__ FT s_ux[LV];
-    __shared__ FT s_vy[LU];
-    __shared__ FT s_ring[8 * HALO];                // w of plane p on the halo columns, slot p % 8
-    __shared__ FT s_wz[TILE];
-    __shared__ unsigned s_lx[64];                  // a lane's column in a staged row of 32 cells
-    __shared__ unsigned long long s_red[NW];
-
-    const int ti = xcd_tile(blockIdx.x, gridDim.x);
-    if (ti >= ntiles) return;
-    const TileDev tl = tiles[ti];
-    if (tl.nz == 0) return;  // filler of an XCD's part of the list
-    BoxDev &B = boxes[__builtin_amdgcn_readfirstlane(tl.box)];
-    if (box_stopped(B)) return;  // uniform over the workgroup
+    using G = Rows<FT, ROWS>;
+    constexpr bool F32 = G::F32;
+    constexpr int BY = G::BY, R = G::R, NT = G::NT, NW = G::NW, TILE = G::TILE, XH = G::XH, HALO = G::HALO;
+    constexpr int LHY = G::LHY, LHX = G::LHX, LU = G::LU, LV = G::LV;
+    constexpr int XW = G::XW, YC = G::YC, XC = G::XC, CC = G::CC, VX = G::VX, XS = G::XS;
+    double *const s_lead = sh.lead;      // leading plane, raw (cns_stage.hip's layout)
+    double *const s_h = sh.h;            // centre plane's halo, raw
+    FT *const s_c = sh.c;                // centre plane: mx, my, mz, E
+    FT *const der = sh.der;              // centre plane, derived
+    FT *const s_lu = sh.lu;              // leading u: own rows, column c (0..39)
+    FT *const s_lv = sh.lv;              // leading v: row r (0..R-1), column 4+c
+    FT *const s_ux = sh.ux, *const s_vy = sh.vy, *const s_wz = sh.wz;
+    FT *const s_ring = sh.ring;          // w of plane p on the halo columns, slot p % 8
+    unsigned *const s_lx = sh.lx;        // a lane's column in a staged row of 32 cells
+    auto my_tid = []() {  // opaque_tid() of this many threads
+        unsigned t = threadIdx.x;
+        asm volatile("" : "+v"(t));
+        return t & ((1u << (32 - __builtin_clz(NT - 1))) - 1);
+    };
     const int x0 = __builtin_amdgcn_readfirstlane(tl.x0), y0 = __builtin_amdgcn_readfirstlane(tl.y0);
     const int kbeg = __builtin_amdgcn_readfirstlane(tl.z0), kend = kbeg + __builtin_amdgcn_readfirstlane(tl.nz);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int e = B.e;
+    // (scalars for certain: with two bodies in a kernel the compiler no longer proves it of all)
+    const int e = __builtin_amdgcn_readfirstlane(B.e);
     const int64_t e2 = (int64_t)e * e, e3 = e2 * e;
-    const double *cons = STAGE == 1 ? B.U : (STAGE == 2 ? B.S1 : B.S2);
-    const double *base = B.U;
-    double *out = STAGE == 1 ? B.S1 : (STAGE == 2 ? B.S2 : B.U);
+    const double *cons = uniform(STAGE == 1 ? B.U : (STAGE == 2 ? B.S1 : B.S2));
+    const double *base = uniform(B.U);
+    double *out = uniform(STAGE == 1 ? B.S1 : (STAGE == 2 ? B.S2 : B.U));
     const double dt = B.dt, pref = B.pref;
     const double ra = STAGE == 1 ? 0.0E0 : (STAGE == 2 ? ThreeQuarters : OneThird);
     const double rb = STAGE == 1 ? 1.0E0 : (STAGE == 2 ? OneQuarter : TwoThirds);
@@ -97,25 +140,24 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
     const FT dxi0 = (FT)B.dxi[0], dxi1 = (FT)B.dxi[1], dxi2 = (FT)B.dxi[2];
     const FT dxi0s = (FT)(B.dxi[0] * B.dxi[0]), dxi1s = (FT)(B.dxi[1] * B.dxi[1]), dxi2s = (FT)(B.dxi[2] * B.dxi[2]);
 
-    // Shares of the halo cells, one cell per lane: leading y halo, its ring and wz on waves 0..3;
-    // leading x halo, its ring and wz on waves 4, 5; centre y halo and its ux on waves 4..7;
-    // centre x halo on waves 0, 1; corners on wave 2; vy's x halo on 6, 7.
     auto wv = [&]() {
         int w = wave;
         asm volatile("" : "+s"(w));
         return w;
     };
     // Byte offsets within a plane.  Staging: own rows 2 wave, 2 wave + 1 and halo row `wave` of
-    // the tile (scalars) with the lane's column; the x halo's slot `wave` (waves 0..3) or the
-    // corners' (4, 5).
+    // the tile (scalars; eight waves) with the lane's column; the x halo's slot `wave` or, past
+    // those, the corners'.
     unsigned row8[2], hrow8, xh;
     {
         const unsigned tid = threadIdx.x, lane = tid & 63, half = (lane & 1) * 4;
         for (int j = 0; j < 2; j++) row8[j] = (unsigned)(wrap(y0 + 2 * wave + j, e) * e) * 8u;
-        hrow8 = (unsigned)(wrap(y0 - 4 + (wave < 4 ? wave : wave + BY), e) * e) * 8u;
+        const int hw = wave & 7;
+        hrow8 = (unsigned)(wrap(y0 - 4 + (hw < 4 ? hw : hw + BY), e) * e) * 8u;
         if (wave == 0) s_lx[lane] = (unsigned)wrap(x0 + (int)(lane >> 1), e) * 8u + half;
-        const int h = 32 * (wave & 3) + (int)(lane >> 1), c8 = h & 7, c = c8 < 4 ? c8 : c8 + TX;
-        const int r = wave < 4 ? (h >> 3) + 4 : ((h >> 3) & 7) + (((h >> 3) & 7) < 4 ? 0 : BY);
+        const bool xs = wave < XS;
+        const int h = 32 * (xs ? wave : (wave - XS) & 1) + (int)(lane >> 1), c8 = h & 7, c = c8 < 4 ? c8 : c8 + TX;
+        const int r = xs ? (h >> 3) + 4 : (h >> 3) + ((h >> 3) < 4 ? 0 : BY);
         xh = (unsigned)(wrap(y0 + r - 4, e) * e + wrap(x0 + c - 4, e)) * 8u + half;
     }
     __syncthreads();
@@ -125,36 +167,38 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
         unsigned own8;
     };
     auto cell = [&]() {
-        const unsigned tid = opaque_tid();
+        const unsigned tid = my_tid();
         const int i = x0 + (int)(tid & (TX - 1)), j = y0 + (int)(tid / TX);
         return Cell{i < e && j < e, (mul24(min(j, e - 1), e) + (unsigned)min(i, e - 1)) * 8u};
     };
     auto issue_centre = [&](int k) {  // halo of centre plane k
         const double *p = cons + k * e2;
         const int w = wv(), yr = w < 4 ? w : w + BY;
-        const unsigned lx = s_lx[opaque_tid() & 63];
+        const unsigned lx = s_lx[my_tid() & 63];
         const double *ph = (const double *)((const char *)p + hrow8);
-        dma4(ph, lx, s_h + 32 * w);
+        if (w < 8) {
+            dma4(ph, lx, s_h + 32 * w);
 #pragma unroll
-        for (int f = 1; f < 5; f++) {
-            if (F32)
-                dma4(ph + f * e3, lx, s_h + f * YH + 32 * w);
-            else
-                dma4(ph + f * e3, lx, s_c + (f - 1) * TILE + yr * PX + 4);
+            for (int f = 1; f < 5; f++) {
+                if (F32)
+                    dma4(ph + f * e3, lx, s_h + f * YH + 32 * w);
+                else
+                    dma4(ph + f * e3, lx, s_c + (f - 1) * TILE + yr * PX + 4);
+            }
         }
-        if (w < 4) {
+        if (w < XS) {
 #pragma unroll
-            for (int f = 0; f < 5; f++) dma4(p + f * e3, xh, s_h + L::HX + f * XH + 32 * w);
-        } else if (w < 6) {
+            for (int f = 0; f < 5; f++) dma4(p + f * e3, xh, s_h + G::HX + f * XH + 32 * w);
+        } else if (w < XS + 2) {
 #pragma unroll
-            for (int f = 0; f < 3; f++) dma4(p + f * e3, xh, s_h + L::HC + f * CORN + 32 * (w - 4));
+            for (int f = 0; f < 3; f++) dma4(p + f * e3, xh, s_h + G::HC + f * CORN + 32 * (w - XS));
         }
     };
     auto issue_lead = [&](int k) {  // leading plane of centre plane k
         const int kl = k + 4;
         const double *p = cons + (kl >= e ? kl - e : kl) * e2;  // k + 4 < 2 e
         const int w = wv();
-        const unsigned lx = s_lx[opaque_tid() & 63];
+        const unsigned lx = s_lx[my_tid() & 63];
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const double *pr = (const double *)((const char *)p + row8[j]);
@@ -162,10 +206,12 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
             for (int f = 0; f < 5; f++) dma4(pr + f * e3, lx, s_lead + f * NT + (2 * w + j) * TX);
         }
         const double *ph = (const double *)((const char *)p + hrow8);
-        dma4(ph, lx, s_lead + LHY + 32 * w);
-        dma4(ph + IMY * e3, lx, s_lead + LHY + YH + 32 * w);
-        dma4(ph + IMZ * e3, lx, s_lead + LHY + 2 * YH + 32 * w);
-        if (w < 4) {
+        if (w < 8) {
+            dma4(ph, lx, s_lead + LHY + 32 * w);
+            dma4(ph + IMY * e3, lx, s_lead + LHY + YH + 32 * w);
+            dma4(ph + IMZ * e3, lx, s_lead + LHY + 2 * YH + 32 * w);
+        }
+        if (w < XS) {
             dma4(p, xh, s_lead + LHX + 32 * w);
             dma4(p + IMX * e3, xh, s_lead + LHX + XH + 32 * w);
             dma4(p + IMZ * e3, xh, s_lead + LHX + 2 * XH + 32 * w);
@@ -219,7 +265,7 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
     // primitives of the leading plane: own cell into the windows' entry 8, u and v with their
     // halos into the lead tiles, w of the halo columns
     auto lead = [&]() {
-        const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
+        const unsigned tid = my_tid(), col = tid & (TX - 1), row = tid / TX;
         FT u, v;
         window(8, s_lead[tid], s_lead[RMX * NT + tid], s_lead[RMY * NT + tid], s_lead[RMZ * NT + tid],
                s_lead[RE * NT + tid], u, v);
@@ -232,8 +278,8 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
             s_lv[yr * TX + col] = (FT)(s_lead[LHY + YH + tid] * hinv);
             s_wz[mul24(yr, PX) + col + 4] = (FT)(s_lead[LHY + 2 * YH + tid] * hinv);
         }
-        if (w == 4 || w == 5) {
-            const unsigned xid = tid & 127, c8 = xid & 7;
+        if (w >= 4 && w < 4 + XW) {
+            const unsigned xid = tid - 256, c8 = xid & 7;
             const double hinv = 1.0E0 / s_lead[LHX + xid];
             const unsigned l = mul24(xid >> 3, PX) + (c8 < 4 ? c8 : c8 + TX);
             s_lu[l] = (FT)(s_lead[LHX + XH + xid] * hinv);
@@ -243,7 +289,7 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
 
     // ux, vy of the leading plane into the windows; wz on the halo columns (cns_stage.hip)
     auto lead_grads = [&](int k) {
-        const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
+        const unsigned tid = my_tid(), col = tid & (TX - 1), row = tid / TX;
         FT a[9], b[9];
         {
             const Taps<L::LUA, FT> p_lu(s_lu, mul24(row, PX) + col);
@@ -263,8 +309,8 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
         pin(wux[8], wvy[8]);
         FENCE();
         const int w = wv();
-        if (w < 6) {
-            const unsigned xid = tid & 127, c8 = xid & 7;
+        if (w < 4 + XW) {
+            const unsigned xid = tid - 256, c8 = xid & 7;
             const unsigned rc = w < 4 ? tid : YH + xid;
             const unsigned l = w < 4 ? mul24(row < 4 ? row : row + BY, PX) + col + 4
                                : mul24((xid >> 3) + 4, PX) + (c8 < 4 ? c8 : c8 + TX);
@@ -284,9 +330,9 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
         FT *const fl = (FT *)s_lead;
         FT *const lu[8] = {fl, fl + LU, fl + 2 * LU, fl + 3 * LU, s_lu, s_ux, s_vy, s_wz};
         FT *const lv[8] = {fl + 4 * LU, s_lv, der, der + LV, der + 2 * LV, der + 3 * LV, der + 4 * LV, der + 5 * LV};
-        const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
-        const unsigned xid = tid & 127, c8 = xid & 7, xcol = c8 < 4 ? c8 : c8 + TX, yrow = row < 4 ? row : row + BY;
-        const bool yl = wave < 4, halo = wave < 6;
+        const unsigned tid = my_tid(), col = tid & (TX - 1), row = tid / TX;
+        const unsigned xid = tid - 256, c8 = xid & 7, xcol = c8 < 4 ? c8 : c8 + TX, yrow = row < 4 ? row : row + BY;
+        const bool yl = wave < 4, halo = wave < 4 + XW;
         double cr[8], cx[8], cy[8], cz[8], cE[8], hr[8], hm[8], hz[8];
         {
             const int hy = yl ? (int)yrow : (int)(xid >> 3) + 4, hx = yl ? (int)col + 4 : (int)xcol;
@@ -358,7 +404,7 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
         // ---------------- phase 1: primitives of the leading plane, tiles of the centre plane
         lead();
         {
-            const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX, lane = tid & 63;
+            const unsigned tid = my_tid(), col = tid & (TX - 1), row = tid / TX, lane = tid & 63;
             const unsigned me = mul24(row + 4, PX) + col + 4;
             der[VU * TILE + me] = WU(4);
             der[VV * TILE + me] = WV(4);
@@ -385,8 +431,8 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
                 s_c[3 * TILE + l] = (FT)E;
             };
             const int w = wv();
-            if (w >= 4) {
-                const unsigned yrow = row - 8, l = mul24(yrow < 4 ? yrow : yrow + BY, PX) + col + 4, h = tid - YH;
+            if (w >= YC) {
+                const unsigned yrow = row - 2 * YC, l = mul24(yrow < 4 ? yrow : yrow + BY, PX) + col + 4, h = tid - 64 * YC;
                 if (F32) {
                     const double mx = s_h[YH + h], my = s_h[2 * YH + h], mz = s_h[3 * YH + h], E = s_h[4 * YH + h];
                     halo_cons(l, mx, my, mz, E);
@@ -395,17 +441,17 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
                     halo_prim(l, s_h[h], s_c[l], s_c[TILE + l], s_c[2 * TILE + l], s_c[3 * TILE + l]);
                 }
             }
-            if (w < 2) {
-                const unsigned c8 = tid & 7, l = mul24((tid >> 3) + 4, PX) + (c8 < 4 ? c8 : c8 + TX);
-                const double *h = s_h + L::HX;
-                const double mx = h[XH + tid], my = h[2 * XH + tid], mz = h[3 * XH + tid], E = h[4 * XH + tid];
+            if (w >= XC && w < XC + XW) {
+                const unsigned xid = tid - 64 * XC, c8 = xid & 7, l = mul24((xid >> 3) + 4, PX) + (c8 < 4 ? c8 : c8 + TX);
+                const double *h = s_h + G::HX + xid;
+                const double mx = h[XH], my = h[2 * XH], mz = h[3 * XH], E = h[4 * XH];
                 halo_cons(l, mx, my, mz, E);
-                halo_prim(l, h[tid], mx, my, mz, E);
+                halo_prim(l, h[0], mx, my, mz, E);
             }
-            if (w == 2) {  // u and v only
+            if (w == CC) {  // u and v only
                 const unsigned r8 = lane >> 3, c8 = lane & 7;
                 const unsigned l = mul24(r8 < 4 ? r8 : r8 + BY, PX) + (c8 < 4 ? c8 : c8 + TX);
-                const double *h = s_h + L::HC;
+                const double *h = s_h + G::HC;
                 const double cinv = 1.0E0 / h[lane];
                 der[VU * TILE + l] = (FT)(h[CORN + lane] * cinv);
                 der[VV * TILE + l] = (FT)(h[2 * CORN + lane] * cinv);
@@ -416,19 +462,22 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
         // ---------------- phase 2
         // Of the two waves of a SIMD the older wins every choice, and would wait at C while the
         // younger (4..7) runs alone: the younger goes first up to the end of the z terms.
-        if (wave >= 4) __builtin_amdgcn_s_setprio(1);
+        if (wave >= 8)
+            __builtin_amdgcn_s_setprio(2);
+        else if (wave >= 4)
+            __builtin_amdgcn_s_setprio(1);
         if (k + 1 < kend) issue_lead(k + 1);
         FT F[5], zf[5];
         lead_grads(k);
         {
-            const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
+            const unsigned tid = my_tid(), col = tid & (TX - 1), row = tid / TX;
             // ux, vy of the centre plane: own cells from the windows, the halos the mixed
             // derivatives read from the derived tiles (cpu/diffterm.cpp:77-151)
             s_ux[(row + 4) * TX + col] = wux[4];
             const int w = wv();
             FT a[9];
-            if (w >= 4) {
-                const unsigned yrow = row - 8, yr = yrow < 4 ? yrow : yrow + BY;
+            if (w >= YC) {
+                const unsigned yrow = row - 2 * YC, yr = yrow < 4 ? yrow : yrow + BY;
                 const Taps<L::DER, FT> p_u(d_u, mul24(yr, PX) + col);
 #pragma unroll
                 for (int m = 0; m < 9; m++)
@@ -437,8 +486,8 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
                 s_ux[yr * TX + col] = KD1(GA) * dxi0;
             }
             s_vy[mul24(row, PX) + col + 4] = wvy[4];
-            if (w >= 6) {
-                const unsigned xid = tid & 127, c8 = xid & 7, l = mul24(xid >> 3, PX) + (c8 < 4 ? c8 : c8 + TX);
+            if (w >= VX && w < VX + XW) {
+                const unsigned xid = tid - 64 * VX, c8 = xid & 7, l = mul24(xid >> 3, PX) + (c8 < 4 ? c8 : c8 + TX);
                 const Taps<L::DER, FT> p_v(d_v, l);
 #pragma unroll
                 for (int m = 0; m < 9; m++)
@@ -498,7 +547,7 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
             mz = uxz * dxi2 + vyz * dxi2;
             pin(zf[0], zf[1], zf[2], zf[3], zf[4], uz, vz, zx, zy, zz, zt, mz);
             FENCE();
-            const unsigned tid = opaque_tid();
+            const unsigned tid = my_tid();
             s_wz[mul24(tid / TX + 4, PX) + (tid & (TX - 1)) + 4] = wzc;
         }
         __builtin_amdgcn_s_setprio(0);
@@ -506,7 +555,7 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
         constexpr int Z = 4 * PX;
         {
             // from four rows above the own cell: every tap is a non-negative constant away
-            const unsigned tid = opaque_tid(), me4 = mul24(tid / TX, PX) + (tid & (TX - 1)) + 4;
+            const unsigned tid = my_tid(), me4 = mul24(tid / TX, PX) + (tid & (TX - 1)) + 4;
             const Taps<L::C, FT> s_m(s_c, me4);
             const Taps<L::DER, FT> s_d(der, me4);
             FT hs[5], A[12];
@@ -563,12 +612,12 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
         // ---------------- phase 3
         if (k + 1 < kend) issue_centre(k + 1);
         {   // held in the lead tile's own cells (read by the neighbours before C) until the update
-            const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
+            const unsigned tid = my_tid(), col = tid & (TX - 1), row = tid / TX;
             s_lv[(row + 4) * TX + col] = F[IENE];
         }
         {
             // diffterm's x and y terms, from the tiles, then its sums (cpu/diffterm.cpp:159-311)
-            const unsigned tid = opaque_tid(), col = tid & (TX - 1), row = tid / TX;
+            const unsigned tid = my_tid(), col = tid & (TX - 1), row = tid / TX;
             const unsigned me4 = mul24(row, PX) + col + 4;
             const Taps<L::DER, FT> s_d(der, me4);
             const Taps<L::WZ, FT> s_z(s_wz, me4);
@@ -725,16 +774,53 @@ batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles
 #undef WU
 #undef WV
 #undef WW
+    return cmax;
+}
+
+template <typename FT, int STAGE>
+__global__ void __launch_bounds__(Lay<FT>::NT, Lay<FT>::NW / 4)
+batch_stage_kernel(BoxDev *__restrict__ boxes, const TileDev *__restrict__ tiles, int ntiles)
+{
+    using L = Lay<FT>;
+    __shared__ double s_lead[L::LEAD];
+    __shared__ double s_h[L::H];
+    __shared__ FT s_c[4 * L::TILE];
+    __shared__ FT der[VNF * L::TILE];
+    __shared__ FT s_lu[L::LU];
+    __shared__ FT s_lv[L::LV];
+    __shared__ FT s_ux[L::LV];
+    __shared__ FT s_vy[L::LU];
+    __shared__ FT s_ring[8 * L::HALO];
+    __shared__ FT s_wz[L::TILE];
+    __shared__ unsigned s_lx[64];
+    __shared__ unsigned long long s_red[L::NW];
+
+    const int ti = xcd_tile(blockIdx.x, gridDim.x);
+    if (ti >= ntiles) return;
+    const TileDev tl = tiles[ti];
+    if (tl.nz == 0) return;  // filler of an XCD's part of the list
+    BoxDev &B = boxes[__builtin_amdgcn_readfirstlane(tl.box)];
+    if (box_stopped(B)) return;  // uniform over the workgroup
+    const Shared<FT> sh{s_lead, s_h, s_c, der, s_lu, s_lv, s_ux, s_vy, s_ring, s_wz, s_lx};
+    const int rows = L::F32 ? __builtin_amdgcn_readfirstlane(tl.rows) : kShortRows, waves = rows / 2;
+    unsigned long long cmax;
+    if (L::F32 && rows == kTallRows) {
+        cmax = stage_rows<FT, STAGE, L::BY>(B, tl, sh);
+    } else {
+        // (a wave that has ended no longer counts at the barriers)
+        if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= TX * kShortRows) return;
+        cmax = stage_rows<FT, STAGE, kShortRows>(B, tl, sh);
+    }
     if (STAGE == 3) {
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
             const unsigned long long v = __shfl_xor(cmax, off);
             cmax = cmax > v ? cmax : v;
         }
-        if ((threadIdx.x & 63) == 0) s_red[wave] = cmax;
+        if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = cmax;
         __syncthreads();
         if (threadIdx.x == 0) {
-            for (int w = 0; w < NW; w++) cmax = cmax > s_red[w] ? cmax : s_red[w];
+            for (int w = 0; w < waves; w++) cmax = cmax > s_red[w] ? cmax : s_red[w];
             atomicMax(&B.acc, courno_bits(__longlong_as_double((long long)cmax) / B.dx[0]));
         }
     }
@@ -747,9 +833,9 @@ hipError_t launch_batch_fused(BoxDev *boxes, const TileDev *tiles, int n, int st
     if (n <= 0) return hipSuccess;
 #define BATCH_STAGE(FT)                                                               \
     switch (stage) {                                                                  \
-    case 1: batch_stage_kernel<FT, 1><<<n, NT, 0, s>>>(boxes, tiles, n); break;       \
-    case 2: batch_stage_kernel<FT, 2><<<n, NT, 0, s>>>(boxes, tiles, n); break;       \
-    case 3: batch_stage_kernel<FT, 3><<<n, NT, 0, s>>>(boxes, tiles, n); break;       \
+    case 1: batch_stage_kernel<FT, 1><<<n, Lay<FT>::NT, 0, s>>>(boxes, tiles, n); break; \
+    case 2: batch_stage_kernel<FT, 2><<<n, Lay<FT>::NT, 0, s>>>(boxes, tiles, n); break; \
+    case 3: batch_stage_kernel<FT, 3><<<n, Lay<FT>::NT, 0, s>>>(boxes, tiles, n); break; \
     default: return hipErrorInvalidValue;                                             \
     }
     if (fp32) {

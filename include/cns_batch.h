@@ -75,7 +75,8 @@ int cns_batch_query(cns_batch *b, int n, const int *ids, long long *steps, doubl
                     double *courno, int *err);
 
 /* Tile shape used for boxes of a given edge: width 16, 32 or 64 cells and z run kz
- * (1..edge).  Tiles are 256/width cells high, 32-wide ones 16, whose kz is the longest run:
+ * (1..edge).  Tiles are 256/width cells high, 32-wide ones 16 (FP32 flux:
+ * 16 or 24, whichever cover the box best), whose kz is the longest run:
  * the work list splits every box so that the GPU's CUs end together.  Applies to boxes
  * admitted afterwards and rebuilds the work list; results do not depend on it.  The table
  * starts from built-in defaults; the package's autotuner measures and sets it. */

@@ -260,3 +260,19 @@ def test_autotune_table_loads_and_keeps_bits(device, tmp_path):
             eng.close()
         for a, b in zip(*out):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("edge", [9, 17, 23, 25, 33, 39, 41, 57])
+def test_fused_stage_row_heights_agree(device, monkeypatch, edge):
+    """FP32 flux covers a box's rows with 24- and 16-row tiles: at the edges where that cover
+    changes and where the last tile holds one row, the bits of the separate kernels."""
+    u = compact_sinusoid(edge, 40 + edge, mach=0.25, kmax=3).reshape(-1)
+    out = []
+    for hyp in ("1", "0"):
+        monkeypatch.setenv("CNS_BATCH_HYP", hyp)
+        eng = BatchEngine(1 << 30, fp32=True, max_boxes=2, tuning={})
+        i = eng.add(u, edge)
+        eng.step(3)
+        out.append((eng.read(i).cpu().numpy(), eng.query([i])[i]["dt"]))
+        eng.close()
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
