@@ -6,6 +6,8 @@
 // Every kernel keeps the reference's per-cell operation order; the library is
 // compiled with -ffp-contract=off, so results are bit-identical to the
 // reference cpu/ path (which g++ -O2 builds without FMA).
+#include <algorithm>
+
 #include "cns_kernels.h"
 #include "cns_fill.h"
 
@@ -113,30 +115,37 @@ ctoprim_kernel(Geom g, const double *__restrict__ u, double *__restrict__ q,
 
 // ------------------------------------------------------------------ RK update
 // cpu/advance.cpp:78-85 (phase 1), :110-119 (phase 2), :144-153 (phase 3).
+// HBM-bound at large boxes (256^3 0.67 ms, 4.7 TB/s).  All operands of a cell are loaded before its
+// first store: u and unew are read and written at the same places, so the compiler would keep loads
+// behind stores and a cell wait five times (64^3 14.0 -> 9.4 us, with one quotient a thread).
+template <int PHASE>
 __global__ void __launch_bounds__(kStreamBlock)
-rk_update_kernel(Geom g, int phase, double *__restrict__ u, double *__restrict__ unew,
-                 const double *__restrict__ d, const double *__restrict__ f,
-                 const double *__restrict__ dt_dev, double dt_host)
+rk_update_kernel(Geom g, double *__restrict__ u, double *__restrict__ unew, const double *__restrict__ d,
+                 const double *__restrict__ f, const double *__restrict__ dt_dev, double dt_host, FastDiv by_x)
 {
     const double dt = dt_dev ? dt_dev[0] : dt_host;
-    const int64_t total = (int64_t)g.n2 * g.p;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t row = e / g.x;
-        const int i = (int)(e - row * g.x);
-        if (i >= g.n0) continue;
-        const int k = (int)(row / g.n1);
-        const int j = (int)(row - (int64_t)k * g.n1);
-        const int64_t o = gidx(g, i + NG, j + NG, k + NG);
+    const unsigned in = blockIdx.x * kStreamBlock + threadIdx.x;  // of the plane
+    const int j = (int)by_x.div(in), i = (int)(in - (unsigned)j * by_x.d);
+    if (j >= g.n1 || i >= g.n0) return;
+    for (int k = blockIdx.y; k < g.n2; k += gridDim.y) {
+        const int64_t o = gidx(g, i + NG, j + NG, k + NG), e = (int64_t)k * g.p + in;
+        double a[NC], b[NC], x[NC], y[NC];
 #pragma unroll
         for (int l = 0; l < NC; l++) {
-            const int64_t go = l * g.cg + o, io = l * g.c + e;
-            if (phase == 1)
-                unew[go] = u[go] + dt * (d[io] + f[io]);
-            else if (phase == 2)
-                unew[go] = ThreeQuarters * u[go] + OneQuarter * (unew[go] + dt * (d[io] + f[io]));
+            a[l] = u[l * g.cg + o];
+            b[l] = PHASE == 1 ? 0.0 : unew[l * g.cg + o];
+            x[l] = d[l * g.c + e];
+            y[l] = f[l * g.c + e];
+        }
+#pragma unroll
+        for (int l = 0; l < NC; l++) {
+            const int64_t go = l * g.cg + o;
+            if (PHASE == 1)
+                unew[go] = a[l] + dt * (x[l] + y[l]);
+            else if (PHASE == 2)
+                unew[go] = ThreeQuarters * a[l] + OneQuarter * (b[l] + dt * (x[l] + y[l]));
             else
-                u[go] = OneThird * u[go] + TwoThirds * (unew[go] + dt * (d[io] + f[io]));
+                u[go] = OneThird * a[l] + TwoThirds * (b[l] + dt * (x[l] + y[l]));
         }
     }
 }
@@ -440,9 +449,18 @@ void step_dt_free(unsigned long long *acc, double *host)
 hipError_t launch_rk_update(const Geom &g, int phase, double *u, double *unew, const double *d,
                             const double *f, const double *dt_dev, double dt_host, hipStream_t s)
 {
-    const int64_t total = (int64_t)g.n2 * g.p;
-    rk_update_kernel<<<stream_grid(total, 4), kStreamBlock, 0, s>>>(g, phase, u, unew, d, f, dt_dev,
-                                                                     dt_host);
+    if (g.p > 0x7fffffff) return hipErrorInvalidValue;
+    // A thread takes one place of the plane in every (grid y)-th plane, so that its row and column
+    // cost one quotient by a launch constant in all.
+    const int64_t gx = (g.p + kStreamBlock - 1) / kStreamBlock, each = std::max<int64_t>(1, gx * g.n2 / 16384);
+    const dim3 grid((unsigned)gx, (unsigned)std::min<int64_t>(65535, (g.n2 + each - 1) / each));
+    const FastDiv by_x = fast_div((unsigned)g.x);
+    switch (phase) {
+    case 1: rk_update_kernel<1><<<grid, kStreamBlock, 0, s>>>(g, u, unew, d, f, dt_dev, dt_host, by_x); break;
+    case 2: rk_update_kernel<2><<<grid, kStreamBlock, 0, s>>>(g, u, unew, d, f, dt_dev, dt_host, by_x); break;
+    case 3: rk_update_kernel<3><<<grid, kStreamBlock, 0, s>>>(g, u, unew, d, f, dt_dev, dt_host, by_x); break;
+    default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 

@@ -22,7 +22,6 @@ static_assert(LEAD >= 4 * LU + LV && 5 * TILE >= 6 * LV && TILE >= LU && LV >= L
 enum { RRHO = 0, RMX, RMY, RMZ, RE, RNF };
 enum { VU = 0, VV, VW, VT, VP, VNF };
 
-typedef __attribute__((address_space(3))) double lds_double;
 // Taps are read one by one: the compiler otherwise pairs them into ds_read2_b64, which moves
 // 128 bytes per cycle where ds_read_b64 moves 240 (measured, eight waves).
 template <typename T>

@@ -7,11 +7,19 @@
 // is staged in LDS as a full 16 x (TX+8) tile (4 cells of halo on each side), loaded with
 // direct-to-LDS DMA (global_load_lds_dwordx4: each lane moves 16 bytes straight
 // into the tile, no registers involved) into one of two LDS buffers.  The loads of
-// plane k+1 are issued right after the barrier that opens plane k, so the whole
-// compute of plane k hides their latency; a plane costs one barrier (hypterm) or
+// plane k+1 are issued right after the last barrier of plane k, so that its
+// compute hides their latency; a plane costs one barrier (hypterm) or
 // two (diffterm), and there is no per-plane gather loop.  z neighbours of the
 // lane's own column come from 9-plane register windows whose leading values are
 // prefetched one plane ahead.
+//
+// What bounds them: with two workgroups of four waves on a CU, each wave's own chain of LDS
+// reads, FP64 arithmetic and barriers (at 256^3 diffterm moves 2.9 TB/s, hypterm 3.6).  What a wave must
+// not do is wait for memory: the next plane is waited for before the stores of this one join
+// the queue, diffterm's two buffers are two objects and its DMA starts behind its LDS stores
+// (the compiler waits for a DMA in flight at an access that might touch what it writes), and
+// taps are read one by one and once each (cns_stage_tile.h).  diffterm 258 -> 202 us at
+// 200x180x160 and 554 -> 462 us at 256^3, hypterm 251 -> 221 and 585 -> 528.
 //
 // diffterm reads wz = d(w)/dz on the cross halo as a precomputed field (wz_kernel
 // below, the reference's wz temporary of cpu/diffterm.cpp:127-151 over the ghosted
@@ -21,8 +29,9 @@
 // cpu/diffterm.cpp:22-320, cpu/advance.cpp:78-153); with -ffp-contract=off the
 // results are bit-identical to the reference cpu/ path and to the other kernels.
 #include <cstdlib>
+#include <type_traits>
 
-#include "cns_pipe_tile.h"
+#include "cns_stage_tile.h"
 
 namespace cns {
 
@@ -58,7 +67,7 @@ hypterm_pipe_kernel(Geom g, const double *__restrict__ cons, const double *__res
 
     const int t = xcd_tile(blockIdx.x, gridDim.x);
     const int bx = t % ntx, by = (t / ntx) % nty, bz = t / (ntx * nty);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;       // DMA issue
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // DMA issue
     const int col = threadIdx.x % S::TX, row = threadIdx.x / S::TX;  // the lane's cell
     const TileDma td{bx * S::TX, by * S::BY, g.g1 - 1, g.xg - 2, (unsigned)g.xg};
     const int gi = td.gi0 + col + 4, gj = td.gj0 + row + 4;
@@ -83,7 +92,7 @@ hypterm_pipe_kernel(Geom g, const double *__restrict__ cons, const double *__res
     }
 
     // first plane's tiles in flight while the windows fill
-    dma_plane_s<S, HNF>(src, (int64_t)(kbeg + NG) * pg, sm, td, wave, lane);
+    dma_plane_s<S, HNF>(src, (int64_t)(kbeg + NG) * pg, (lds_double *)sm, td, wave, lane);
 
     double wmx[9], wmy[9], wmz[9], wE[9], ww[9], wp[9];
     double nmx = 0, nmy = 0, nmz = 0, nE = 0, nw = 0, np = 0;
@@ -98,12 +107,12 @@ hypterm_pipe_kernel(Geom g, const double *__restrict__ cons, const double *__res
         nmx = c_mx[o]; nmy = c_my[o]; nmz = c_mz[o]; nE = c_E[o]; nw = q_w[o]; np = q_p[o];
     }
 
+    __builtin_amdgcn_s_waitcnt(0xF70);
     for (int k = kbeg; k < kend; k++) {
         const int cur = (k - kbeg) & 1;
-        const double *b = sm + cur * (HNF * TILE_);
-        plane_barrier();
+        __syncthreads();
         if (k + 1 < kend)
-            dma_plane_s<S, HNF>(src, (int64_t)(k + 1 + NG) * pg, sm + (cur ^ 1) * (HNF * TILE_), td, wave, lane);
+            dma_plane_s<S, HNF>(src, (int64_t)(k + 1 + NG) * pg, (lds_double *)sm + (cur ^ 1) * (HNF * TILE_), td, wave, lane);
 
         const int64_t zo = (int64_t)(k + NG) * pg + own;
         wmx[8] = nmx; wmy[8] = nmy; wmz[8] = nmz; wE[8] = nE; ww[8] = nw; wp[8] = np;
@@ -123,12 +132,70 @@ hypterm_pipe_kernel(Geom g, const double *__restrict__ cons, const double *__res
             }
         }
 
+        // (cells past the box are computed too, for nothing: no divergent branch around the taps)
+        double F[5];
+        {
+            // from four rows above the own cell: every tap is a non-negative constant away
+            const Taps<0> s_f(sm, (unsigned)(cur * (HNF * TILE_) + me - 4 * PX_));
+            constexpr int Z = 4 * PX_;
+            double hs[5], A[12];
+            // fields n, a, b, E, p and v of the tile at taps +o and -o
+            auto load = [&](int n, int a, int b, int v, int o) {
+                A[0] = s_f[n * TILE_ + Z + o]; A[1] = s_f[n * TILE_ + Z - o];
+                A[2] = s_f[a * TILE_ + Z + o]; A[3] = s_f[a * TILE_ + Z - o];
+                A[4] = s_f[b * TILE_ + Z + o]; A[5] = s_f[b * TILE_ + Z - o];
+                A[6] = s_f[HE * TILE_ + Z + o]; A[7] = s_f[HE * TILE_ + Z - o];
+                A[8] = s_f[HP * TILE_ + Z + o]; A[9] = s_f[HP * TILE_ + Z - o];
+                A[10] = s_f[v * TILE_ + Z + o]; A[11] = s_f[v * TILE_ + Z - o];
+            };
+#define XY(FIRST, C) \
+    hyp_tap<FIRST>(C, A[0], A[1], A[2], A[3], A[4], A[5], A[6], A[7], A[8], A[9], A[8], A[9], A[10], A[11], hs)
+#define ZT(FIRST, C, m)                                                                                        \
+    hyp_tap<FIRST>(C, wmz[4 + m], wmz[4 - m], wmx[4 + m], wmx[4 - m], wmy[4 + m], wmy[4 - m], wE[4 + m],       \
+                   wE[4 - m], wp[4 + m], wp[4 - m], wp[4 + m], wp[4 - m], ww[4 + m], ww[4 - m], hs)
+            load(HMX, HMY, HMZ, HU, 1);
+            XY(true, ALP);
+            load(HMX, HMY, HMZ, HU, 2);
+            XY(false, BET);
+            load(HMX, HMY, HMZ, HU, 3);
+            XY(false, GAM);
+            load(HMX, HMY, HMZ, HU, 4);
+            XY(false, DEL);
+            F[IRHO] = -(hs[0]) * dxi0;
+            F[IMX] = -(hs[1]) * dxi0;
+            F[IMY] = -(hs[2]) * dxi0;
+            F[IMZ] = -(hs[3]) * dxi0;
+            F[IENE] = -(hs[4]) * dxi0;
+            load(HMY, HMX, HMZ, HV, PX_);
+            XY(true, ALP);
+            load(HMY, HMX, HMZ, HV, 2 * PX_);
+            XY(false, BET);
+            load(HMY, HMX, HMZ, HV, 3 * PX_);
+            XY(false, GAM);
+            load(HMY, HMX, HMZ, HV, 4 * PX_);
+            XY(false, DEL);
+            F[IRHO] = F[IRHO] - hs[0] * dxi1;
+            F[IMY] = F[IMY] - hs[1] * dxi1;
+            F[IMX] = F[IMX] - hs[2] * dxi1;
+            F[IMZ] = F[IMZ] - hs[3] * dxi1;
+            F[IENE] = F[IENE] - hs[4] * dxi1;
+            ZT(true, ALP, 1);
+            ZT(false, BET, 2);
+            ZT(false, GAM, 3);
+            ZT(false, DEL, 4);
+            F[IRHO] = F[IRHO] - hs[0] * dxi2;
+            F[IMZ] = F[IMZ] - hs[1] * dxi2;
+            F[IMX] = F[IMX] - hs[2] * dxi2;
+            F[IMY] = F[IMY] - hs[3] * dxi2;
+            F[IENE] = F[IENE] - hs[4] * dxi2;
+            pin(F[0], F[1], F[2], F[3], F[4]);
+#undef XY
+#undef ZT
+        }
+        // The next plane has landed before the stores join the queue: the barrier that opens it
+        // need not wait for them.
+        __builtin_amdgcn_s_waitcnt(0xF70);
         if (active) {
-            const double *s_mx = b + HMX * TILE_, *s_my = b + HMY * TILE_, *s_mz = b + HMZ * TILE_,
-                         *s_E = b + HE * TILE_, *s_p = b + HP * TILE_, *s_u = b + HU * TILE_,
-                         *s_v = b + HV * TILE_;
-            double F[5];
-            hyp_flux<PX_>(s_mx, s_my, s_mz, s_E, s_p, s_u, s_v, me, wmx, wmy, wmz, wE, ww, wp, dxi0, dxi1, dxi2, F);
             if (RK) {
                 const double uc[5] = {rho_c, wmx[4], wmy[4], wmz[4], wE[4]};
                 double o[5];
@@ -186,13 +253,14 @@ diffterm_pipe_kernel(Geom g, const double *__restrict__ q, const double *__restr
                      double *__restrict__ difflux, double dxi0, double dxi1, double dxi2, double eta,
                      double alam, int kz, int ntx, int nty)
 {
-    __shared__ double sm[2 * DNF * S::TILE];
+    // two objects: reads of the one then need not wait for the DMA into the other
+    __shared__ __align__(16) double sm0[DNF * S::TILE], sm1[DNF * S::TILE];
     __shared__ double s_ux[S::R * S::TX];   // row r (0..15), column 4+c
     __shared__ double s_vy[S::BY * S::PX];  // row 4+r (r 0..7), column c (0..PX-1)
 
     const int t = xcd_tile(blockIdx.x, gridDim.x);
     const int bx = t % ntx, by = (t / ntx) % nty, bz = t / (ntx * nty);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;       // DMA issue
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // DMA issue
     const int col = threadIdx.x % S::TX, row = threadIdx.x / S::TX;  // the lane's cell
     const TileDma td{bx * S::TX, by * S::BY, g.g1 - 1, g.xg - 2, (unsigned)g.xg};
     const int gi = td.gi0 + col + 4, gj = td.gj0 + row + 4;
@@ -208,7 +276,7 @@ diffterm_pipe_kernel(Geom g, const double *__restrict__ q, const double *__restr
     const int meby = row * S::PX + col + 4;      // own cell in s_vy
     const double dxi0s = dxi0 * dxi0, dxi1s = dxi1 * dxi1, dxi2s = dxi2 * dxi2;
 
-    dma_plane_s<S, DNF>(src, (int64_t)(kbeg + NG) * pg, sm, td, wave, lane);
+    dma_plane_s<S, DNF>(src, (int64_t)(kbeg + NG) * pg, (lds_double *)sm0, td, wave, lane);
 
     // windows: plane k+m at [4+m]; ux and vy of the first 8 planes straight from
     // global memory (the same expressions as the per-plane path)
@@ -221,11 +289,21 @@ diffterm_pipe_kernel(Geom g, const double *__restrict__ q, const double *__restr
 #pragma unroll 1
     for (int m = 0; m < 8; m++) {
         const int64_t o = (int64_t)(kbeg + m) * pg + own;
-        double ux_ = 0.0, vy_ = 0.0;
-#define GUX(mm) q_u[o + (mm)]
-#define GVY(mm) q_v[o + (int64_t)(mm) * xg]
-        if (need_ux) ux_ = D1(GUX) * dxi0;
-        if (need_vy) vy_ = D1(GVY) * dxi1;
+        double a[9] = {}, b[9] = {};  // all loads of a plane at once
+        if (need_ux) {
+#pragma unroll
+            for (int i = 0; i < 9; i++)
+                if (i != 4) a[i] = q_u[o + i - 4];
+        }
+        if (need_vy) {
+#pragma unroll
+            for (int i = 0; i < 9; i++)
+                if (i != 4) b[i] = q_v[o + (int64_t)(i - 4) * xg];
+        }
+        FENCE();
+#define GUX(mm) a[4 + (mm)]
+#define GVY(mm) b[4 + (mm)]
+        const double ux_ = D1(GUX) * dxi0, vy_ = D1(GVY) * dxi1;
 #undef GUX
 #undef GVY
 #pragma unroll
@@ -247,147 +325,161 @@ diffterm_pipe_kernel(Geom g, const double *__restrict__ q, const double *__restr
         nt = q_t[o];
     }
 
-    for (int k = kbeg; k < kend; k++) {
-        const int cur = (k - kbeg) & 1;
-        const double *b = sm + cur * (DNF * S::TILE);
-        plane_barrier();
-        if (k + 1 < kend)
-            dma_plane_s<S, DNF>(src, (int64_t)(k + 1 + NG) * pg, sm + (cur ^ 1) * (DNF * S::TILE), td, wave, lane);
-        const double *s_cu = b + DCU * S::TILE, *s_cv = b + DCV * S::TILE, *s_cw = b + DCW * S::TILE,
-                     *s_ct = b + DCT * S::TILE, *s_wz = b + DWZ * S::TILE, *s_lu = b + DLU * S::TILE,
-                     *s_lv = b + DLV * S::TILE;
-
-        const int64_t zo = (int64_t)(k + NG) * pg + own;
-        wu[8] = s_lu[me];
-        wv[8] = s_lv[me];
+    auto plane = [&](int k, auto odd) {
+        const double *const b = decltype(odd)::value ? sm1 : sm0;
+        lds_double *const next = decltype(odd)::value ? (lds_double *)sm0 : (lds_double *)sm1;
+        __syncthreads();
         ww[8] = nw;
         wt[8] = nt;
-        if (inbox && k + 1 < kend) {
-            const int64_t o = zo + 5 * pg;
-            nw = q_w[o];
-            nt = q_t[o];
-        }
-
+        constexpr int T = S::TILE, P = S::PX, Z = 4 * P;
         // ---------------- phase B
         {
-#define LUX(mm) s_lu[me + (mm)]
-#define LVY(mm) s_lv[me + (mm) * S::PX]
+            double a[9];
+#define GA(mm) a[4 + (mm)]
             // leading plane: ux, vy of the own column (cpu/diffterm.cpp:77-81, :110-114)
-            wux[8] = D1(LUX) * dxi0;
-            wvy[8] = D1(LVY) * dxi1;
-#undef LUX
-#undef LVY
+            const Taps<0> p_l(b, (unsigned)(me - Z));
+            wu[8] = p_l[DLU * T + Z];
+            wv[8] = p_l[DLV * T + Z];
+#pragma unroll
+            for (int m = 0; m < 9; m++)
+                if (m != 4) a[m] = p_l[DLU * T + Z + m - 4];
+            wux[8] = D1(GA) * dxi0;
+#pragma unroll
+            for (int m = 0; m < 9; m++)
+                if (m != 4) a[m] = p_l[DLV * T + m * P];
+            wvy[8] = D1(GA) * dxi1;
             // centre plane, ux: the own rows from the window (ux of plane k, computed from
             // the same values four planes ago), the halo rows 0..3 and 12..15 from the tile
             s_ux[me64] = wux[4];
             {
                 const int rr = threadIdx.x / S::TX, r = rr < 4 ? rr : rr + S::BY, c = threadIdx.x % S::TX;
-                const int l = r * S::PX + c + 4;
-#define CUX(mm) s_cu[l + (mm)]
-                s_ux[r * S::TX + c] = D1(CUX) * dxi0;
-#undef CUX
+                const Taps<0> p_u(b, (unsigned)(DCU * T + r * P + c));
+#pragma unroll
+                for (int m = 0; m < 9; m++)
+                    if (m != 4) a[m] = p_u[m];
+                s_ux[r * S::TX + c] = D1(GA) * dxi0;
             }
             // centre plane, vy: the own cells from the window, the x-halo columns 0..3 and
             // 68..71 of rows 4..11 from the tile
             s_vy[meby] = wvy[4];
             if (threadIdx.x < 8 * S::BY) {
                 const int rr = threadIdx.x >> 3, cc = threadIdx.x & 7, c = cc < 4 ? cc : cc + S::TX;
-                const int l = (rr + 4) * S::PX + c;
-#define CVY(mm) s_cv[l + (mm) * S::PX]
-                s_vy[rr * S::PX + c] = D1(CVY) * dxi1;
-#undef CVY
+                const Taps<0> p_v(b, (unsigned)(DCV * T + rr * P + c));
+#pragma unroll
+                for (int m = 0; m < 9; m++)
+                    if (m != 4) a[m] = p_v[m * P];
+                s_vy[rr * P + c] = D1(GA) * dxi1;
             }
+#undef GA
         }
         __syncthreads();
+        // (in flight during phase B the next plane's loads would be waited for at its LDS stores)
+        if (k + 1 < kend) {
+            dma_plane_s<S, DNF>(src, (int64_t)(k + 1 + NG) * pg, next, td, wave, lane);
+            if (inbox) {
+                const int64_t o = (int64_t)(k + NG + 5) * pg + own;
+                nw = q_w[o];
+                nt = q_t[o];
+            }
+        }
 
-        // ---------------- phase C
+        // ---------------- phase C: z terms from the windows, x and y terms from the tiles, one
+        // tap pair of all of them at a time, then the reference's sums (cpu/diffterm.cpp:159-311)
+        double xu, xv, xw, xt, d2v, d2w, m1, m2, A[12];
+        double uzz = CENTER * wu[4], vzz = CENTER * wv[4], wzz = CENTER * ww[4], tzz = CENTER * wt[4], uz, vz, uxz, vyz;
+#define ZT(FIRST, C1, C2, m)                          \
+    tap<false>(uzz, C2 * (wu[4 + m] + wu[4 - m]));    \
+    tap<false>(vzz, C2 * (wv[4 + m] + wv[4 - m]));    \
+    tap<false>(wzz, C2 * (ww[4 + m] + ww[4 - m]));    \
+    tap<false>(tzz, C2 * (wt[4 + m] + wt[4 - m]));    \
+    tap<FIRST>(uz, C1 * (wu[4 + m] - wu[4 - m]));     \
+    tap<FIRST>(vz, C1 * (wv[4 + m] - wv[4 - m]));     \
+    tap<FIRST>(uxz, C1 * (wux[4 + m] - wux[4 - m]));  \
+    tap<FIRST>(vyz, C1 * (wvy[4 + m] - wvy[4 - m]))
+        ZT(true, ALP, OFF1, 1);
+        ZT(false, BET, OFF2, 2);
+        ZT(false, GAM, OFF3, 3);
+        ZT(false, DEL, OFF4, 4);
+#undef ZT
+        uzz = uzz * dxi2s;
+        vzz = vzz * dxi2s;
+        wzz = wzz * dxi2s;
+        tzz = tzz * dxi2s;
+        uz = uz * dxi2;
+        vz = vz * dxi2;
+        const Taps<0> s_d(b, (unsigned)(me - Z));
+        // u, v, w, T, wz of the tile at taps +o and -o, vy (x) or ux (y) in the last pair
+        auto load = [&](int o) {
+            A[0] = s_d[DCU * T + Z + o]; A[1] = s_d[DCU * T + Z - o];
+            A[2] = s_d[DCV * T + Z + o]; A[3] = s_d[DCV * T + Z - o];
+            A[4] = s_d[DCW * T + Z + o]; A[5] = s_d[DCW * T + Z - o];
+            A[6] = s_d[DCT * T + Z + o]; A[7] = s_d[DCT * T + Z - o];
+            A[8] = s_d[DWZ * T + Z + o]; A[9] = s_d[DWZ * T + Z - o];
+        };
+        // second differences of u, v, w, T; first of A[2 f] (d2v), w (d2w) and of the two mixed terms
+#define XY(FIRST, C1, C2, f)                         \
+    tap<false>(xu, C2 * (A[0] + A[1]));              \
+    tap<false>(xv, C2 * (A[2] + A[3]));              \
+    tap<false>(xw, C2 * (A[4] + A[5]));              \
+    tap<false>(xt, C2 * (A[6] + A[7]));              \
+    tap<FIRST>(d2v, C1 * (A[2 * f] - A[2 * f + 1])); \
+    tap<FIRST>(d2w, C1 * (A[4] - A[5]));             \
+    tap<FIRST>(m1, C1 * (A[10] - A[11]));            \
+    tap<FIRST>(m2, C1 * (A[8] - A[9]))
+#define XT(FIRST, C1, C2, m)                                  \
+    load(m);                                                  \
+    A[10] = s_m[4 + m]; A[11] = s_m[4 - m];                   \
+    XY(FIRST, C1, C2, 1)
+#define YT(FIRST, C1, C2, m)                                  \
+    load(m * P);                                              \
+    A[10] = s_n[(4 + m) * S::TX]; A[11] = s_n[(4 - m) * S::TX]; \
+    XY(FIRST, C1, C2, 0)
+        const Taps<0> s_m(s_vy, (unsigned)(meby - 4)), s_n(s_ux, (unsigned)(me64 - 4 * S::TX));
+        xu = CENTER * wu[4]; xv = CENTER * wv[4]; xw = CENTER * ww[4]; xt = CENTER * wt[4];
+        XT(true, ALP, OFF1, 1);
+        XT(false, BET, OFF2, 2);
+        XT(false, GAM, OFF3, 3);
+        XT(false, DEL, OFF4, 4);
+        const double uxx = xu * dxi0s, vxx = xv * dxi0s, wxx = xw * dxi0s, txx = xt * dxi0s;
+        const double vx = d2v * dxi0, wx = d2w * dxi0, vyx = m1 * dxi0, wzx = m2 * dxi0;
+        xu = CENTER * wu[4]; xv = CENTER * wv[4]; xw = CENTER * ww[4]; xt = CENTER * wt[4];
+        YT(true, ALP, OFF1, 1);
+        YT(false, BET, OFF2, 2);
+        YT(false, GAM, OFF3, 3);
+        YT(false, DEL, OFF4, 4);
+#undef XY
+#undef XT
+#undef YT
+        const double uyy = xu * dxi1s, vyy = xv * dxi1s, wyy = xw * dxi1s, tyy = xt * dxi1s;
+        const double uy = d2v * dxi1, wy = d2w * dxi1, uxy = m1 * dxi1, wzy = m2 * dxi1;
+        uxz = uxz * dxi2;
+        vyz = vyz * dxi2;
+        const double dmx = eta * (FourThirds * uxx + uyy + uzz + OneThird * (vyx + wzx));
+        const double dmy = eta * (vxx + FourThirds * vyy + vzz + OneThird * (uxy + wzy));
+        const double dmz = eta * (wxx + wyy + FourThirds * wzz + OneThird * (uxz + vyz));
+        const double ux = wux[4], vy = wvy[4], wz = s_d[DWZ * T + Z];
+        const double divu = TwoThirds * (ux + vy + wz);
+        const double tauxx = 2.E0 * ux - divu;
+        const double tauyy = 2.E0 * vy - divu;
+        const double tauzz = 2.E0 * wz - divu;
+        const double tauxy = uy + vx;
+        const double tauxz = uz + wx;
+        const double tauyz = vz + wy;
+        double mechwork = tauxx * ux + tauyy * vy + tauzz * wz + (tauxy * tauxy) + (tauxz * tauxz) + (tauyz * tauyz);
+        mechwork = eta * mechwork + dmx * wu[4] + dmy * wv[4] + dmz * ww[4];
+        double dE = alam * (txx + tyy + tzz) + mechwork;
+        pin(dE);
+        // The next plane has landed before the stores join the queue: the barrier that opens it
+        // need not wait for them.
+        __builtin_amdgcn_s_waitcnt(0xF70);
         if (active) {
-#define XS(a, mm) a[me + (mm)]
-#define YS(a, mm) a[me + (mm) * S::PX]
-#define CUx(mm) XS(s_cu, mm)
-#define CUy(mm) YS(s_cu, mm)
-#define CUz(mm) wu[4 + (mm)]
-#define CVx(mm) XS(s_cv, mm)
-#define CVy(mm) YS(s_cv, mm)
-#define CVz(mm) wv[4 + (mm)]
-#define CWx(mm) XS(s_cw, mm)
-#define CWy(mm) YS(s_cw, mm)
-#define CWz(mm) ww[4 + (mm)]
-#define CTx(mm) XS(s_ct, mm)
-#define CTy(mm) YS(s_ct, mm)
-#define CTz(mm) wt[4 + (mm)]
-#define VYx(mm) s_vy[meby + (mm)]
-#define WZx(mm) XS(s_wz, mm)
-#define UXy(mm) s_ux[me64 + (mm) * S::TX]
-#define WZy(mm) YS(s_wz, mm)
-#define UXz(mm) wux[4 + (mm)]
-#define VYz(mm) wvy[4 + (mm)]
-            // cpu/diffterm.cpp:159-187
-            const double uxx = D2(CUx) * dxi0s;
-            const double uyy = D2(CUy) * dxi1s;
-            const double uzz = D2(CUz) * dxi2s;
-            const double vyx = D1(VYx) * dxi0;
-            const double wzx = D1(WZx) * dxi0;
-            const double dmx = eta * (FourThirds * uxx + uyy + uzz + OneThird * (vyx + wzx));
-            // :198-226
-            const double vxx = D2(CVx) * dxi0s;
-            const double vyy = D2(CVy) * dxi1s;
-            const double vzz = D2(CVz) * dxi2s;
-            const double uxy = D1(UXy) * dxi1;
-            const double wzy = D1(WZy) * dxi1;
-            const double dmy = eta * (vxx + FourThirds * vyy + vzz + OneThird * (uxy + wzy));
-            // :237-265
-            const double wxx = D2(CWx) * dxi0s;
-            const double wyy = D2(CWy) * dxi1s;
-            const double wzz = D2(CWz) * dxi2s;
-            const double uxz = D1(UXz) * dxi2;
-            const double vyz = D1(VYz) * dxi2;
-            const double dmz = eta * (wxx + wyy + FourThirds * wzz + OneThird * (uxz + vyz));
-            // :276-311
-            const double txx = D2(CTx) * dxi0s;
-            const double tyy = D2(CTy) * dxi1s;
-            const double tzz = D2(CTz) * dxi2s;
-            const double ux = wux[4], vy = wvy[4], wz = s_wz[me];
-            const double uy = D1(CUy) * dxi1, uz = D1(CUz) * dxi2;
-            const double vx = D1(CVx) * dxi0, vz = D1(CVz) * dxi2;
-            const double wx = D1(CWx) * dxi0, wy = D1(CWy) * dxi1;
-            const double divu = TwoThirds * (ux + vy + wz);
-            const double tauxx = 2.E0 * ux - divu;
-            const double tauyy = 2.E0 * vy - divu;
-            const double tauzz = 2.E0 * wz - divu;
-            const double tauxy = uy + vx;
-            const double tauxz = uz + wx;
-            const double tauyz = vz + wy;
-            double mechwork = tauxx * ux + tauyy * vy + tauzz * wz + (tauxy * tauxy) + (tauxz * tauxz)
-                              + (tauyz * tauyz);
-            mechwork = eta * mechwork + dmx * wu[4] + dmy * wv[4] + dmz * ww[4];
             const int64_t fo = iidx(g, gi - NG, gj - NG, k);
             const int64_t c = g.c;
             difflux[fo] = 0.0E0;
             difflux[fo + IMX * c] = dmx;
             difflux[fo + IMY * c] = dmy;
             difflux[fo + IMZ * c] = dmz;
-            difflux[fo + IENE * c] = alam * (txx + tyy + tzz) + mechwork;
-#undef XS
-#undef YS
-#undef CUx
-#undef CUy
-#undef CUz
-#undef CVx
-#undef CVy
-#undef CVz
-#undef CWx
-#undef CWy
-#undef CWz
-#undef CTx
-#undef CTy
-#undef CTz
-#undef VYx
-#undef WZx
-#undef UXy
-#undef WZy
-#undef UXz
-#undef VYz
+            difflux[fo + IENE * c] = dE;
         }
 #pragma unroll
         for (int m = 0; m < 8; m++) {
@@ -398,6 +490,12 @@ diffterm_pipe_kernel(Geom g, const double *__restrict__ q, const double *__restr
             wux[m] = wux[m + 1];
             wvy[m] = wvy[m + 1];
         }
+    };
+    __builtin_amdgcn_s_waitcnt(0xF70);
+#pragma unroll 1
+    for (int k = kbeg; k < kend; k += 2) {
+        plane(k, std::false_type());
+        if (k + 1 < kend) plane(k + 1, std::true_type());
     }
 }
 
