@@ -292,6 +292,7 @@ struct cns_ctx {
     int device;
     // one device block: [0] Courant accumulator bits (zero between steps), [1] dt, [2] courno
     unsigned long long *d_acc;
+    bool fresh = true;  // d_acc is not yet zero
     double *d_dt, *d_courno;
     double *h_dt;  // dt and courno of cns_advance, written by the device (pinned)
     // Stage buffer of the fused step (ghosted, 5 comps): holds U^{1/3}, so that the
@@ -609,6 +610,7 @@ static int advance(cns_ctx *ctx, double *U, double *Unew, double *Q, double *D, 
 {
     if (!ctx || !U || !Unew || !Q || !D || !F) return fail(CNS_EINVAL, "NULL argument");
     const StepDt sd{ctx->d_acc, ctx->cfl, dt_dev ? dt_dev : ctx->d_dt, courno_dev ? courno_dev : ctx->d_courno, host};
+    HIPCHK(step_dt_begin(ctx->d_acc, ctx->fresh, t_stream));
     const int rc = enqueue_step(ctx, U, Unew, Q, D, F, sd, t_stream);
     // A step cut short may leave its maximum behind.
     if (rc) (void)launch_courno_reset(ctx->d_acc, 0.0, t_stream);

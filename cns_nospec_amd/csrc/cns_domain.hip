@@ -24,6 +24,7 @@ struct cns_domain {
     double dx[3], dxi[3];
     double cfl, eta, alam;
     unsigned long long *d_acc;  // Courant bits, zero between steps
+    bool fresh = true;          // d_acc is not yet zero
     double *d_dt, *d_courno;
     double *h_dt;               // dt and courno, written by the device (pinned)
     double *d_stage;  // U^{1/3} of every box (5 ghosted comps per box)
@@ -148,6 +149,7 @@ int cns_domain_advance(cns_domain *D, double *U, double *Unew, double *Q, double
     for (const void *p : {(const void *)U, (const void *)Unew, (const void *)Q, (const void *)Dd, (const void *)F})
         if (!pipe_aligned(p)) return fail(CNS_EINVAL, "domain arrays must be 16-byte aligned");
     hipStream_t s = current_stream();
+    CNS_HIPCHK(step_dt_begin(D->d_acc, D->fresh, s));
     const hipError_t e = enqueue_step(D, U, Unew, Q, Dd, F, s);
     if (e != hipSuccess) {
         // A step cut short may leave its maximum behind.

@@ -42,7 +42,10 @@ hipError_t launch_courno_reset(unsigned long long *acc, double init, hipStream_t
 hipError_t launch_ctoprim(const Geom &g, const double *u, double *q, unsigned long long *acc,
                           double dx0, double dx1, double dx2, hipStream_t s, bool full = true);
 
-// The device words and the pinned host words of a StepDt, acc zero.
+// The device words and the pinned host words of a StepDt.  step_dt_begin() before each step clears
+// acc while it is fresh, that is until a step has run outside a capture (a captured first step
+// takes the clearing launch with it: its graph may never run).
+hipError_t step_dt_begin(unsigned long long *acc, bool &fresh, hipStream_t s);
 hipError_t step_dt_alloc(unsigned long long **acc, double **dt, double **courno, double **host);
 void step_dt_free(unsigned long long *acc, double *host);
 // sd.dt = cfl / max(acc, 1e-50) and the Courant number; acc back to zero.

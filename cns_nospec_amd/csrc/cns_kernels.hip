@@ -7,6 +7,9 @@
 // compiled with -ffp-contract=off, so results are bit-identical to the
 // reference cpu/ path (which g++ -O2 builds without FMA).
 #include <algorithm>
+#include <bitset>
+#include <functional>
+#include <mutex>
 
 #include "cns_kernels.h"
 #include "cns_fill.h"
@@ -417,18 +420,54 @@ hipError_t launch_courno_to_dt(const StepDt &sd, hipStream_t s)
     return hipGetLastError();
 }
 
+// Pinned words for dt and courno of a context: one page for the process, in slots that are given
+// back, since pinning memory takes longer than all else of a context's creation.  More contexts
+// than slots pin their own.
+namespace {
+struct HostWords {
+    static constexpr int kSlots = 256;
+    std::mutex mu;
+    double *page = nullptr;
+    std::bitset<kSlots> used;
+};
+HostWords g_words;
+
+hipError_t host_words(double **out)
+{
+    std::lock_guard<std::mutex> lock(g_words.mu);
+    if (!g_words.page) {
+        const hipError_t e = hipHostMalloc((void **)&g_words.page, HostWords::kSlots * 2 * sizeof(double), hipHostMallocPortable);
+        if (e) {
+            g_words.page = nullptr;
+            return e;
+        }
+    }
+    for (int i = 0; i < HostWords::kSlots; i++)
+        if (!g_words.used[i]) {
+            g_words.used[i] = true;
+            *out = g_words.page + 2 * i;
+            return hipSuccess;
+        }
+    return hipHostMalloc((void **)out, 2 * sizeof(double), hipHostMallocPortable);
+}
+
+void host_words_free(double *p)
+{
+    std::lock_guard<std::mutex> lock(g_words.mu);
+    const std::less<const double *> before;
+    if (g_words.page && !before(p, g_words.page) && before(p, g_words.page + 2 * HostWords::kSlots))
+        g_words.used[(p - g_words.page) / 2] = false;
+    else
+        (void)hipHostFree(p);
+}
+}  // namespace
+
 hipError_t step_dt_alloc(unsigned long long **acc, double **dt, double **courno, double **host)
 {
     *host = nullptr;
     unsigned long long *blk = nullptr;
-    hipStream_t s = nullptr;
     hipError_t e = hipMalloc((void **)&blk, 4 * sizeof(double));
-    if (!e) e = hipHostMalloc((void **)host, 2 * sizeof(double), hipHostMallocDefault);
-    // A stream of its own: no other stream is waited for or made to wait.
-    if (!e) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-    if (!e) e = launch_courno_reset(blk, 0.0, s);
-    if (!e) e = hipStreamSynchronize(s);
-    if (s) (void)hipStreamDestroy(s);
+    if (!e) e = host_words(host);
     if (e) {
         (void)hipGetLastError();
         step_dt_free(blk, *host);
@@ -440,10 +479,21 @@ hipError_t step_dt_alloc(unsigned long long **acc, double **dt, double **courno,
     return hipSuccess;
 }
 
+hipError_t step_dt_begin(unsigned long long *acc, bool &fresh, hipStream_t s)
+{
+    if (!fresh) return hipSuccess;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(s, &st);
+    if (!e) e = launch_courno_reset(acc, 0.0, s);
+    if (!e && st == hipStreamCaptureStatusNone) fresh = false;
+    return e;
+}
+
+// (The device is idle once hipFree returns: nothing writes to the host words any more.)
 void step_dt_free(unsigned long long *acc, double *host)
 {
     if (acc) (void)hipFree(acc);
-    if (host) (void)hipHostFree(host);
+    if (host) host_words_free(host);
 }
 
 hipError_t launch_rk_update(const Geom &g, int phase, double *u, double *unew, const double *d,

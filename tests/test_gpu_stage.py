@@ -74,3 +74,44 @@ def test_courant_maximum_does_not_outlive_a_step(device, first):
         assert step(st, first, fresh(0.9)) == want_fast
         assert step(st, route, fresh(0.01)) == want_slow
     st.close()
+
+
+def test_many_contexts_and_a_first_step_that_is_captured(device):
+    """A context clears its Courant maximum with its first step, also when that one goes into a
+    graph that never runs, and more contexts than the pinned page has slots return their own dt."""
+    import torch
+    lay = BoxLayout((8, 6, 5))
+
+    def fresh(mach):
+        arrays = ops.allocate_variables(lay, device)
+        arrays[0].copy_(torch.from_numpy(sinusoid_state(lay, 5, mach=mach, kmax=2)).to(device))
+        return arrays
+
+    ref = ops.Stepper(lay)
+    want = {mach: ref.new_advance(*fresh(mach)) for mach in (0.9, 0.01)}
+    many = [ops.Stepper(lay) for _ in range(300)]
+    for i in (0, 255, 256, 299):
+        assert many[i].new_advance(*fresh(0.9)) == want[0.9]
+        assert many[i].new_advance(*fresh(0.01)) == want[0.01]
+    for st in many:
+        st.close()
+    st = ops.Stepper(lay)
+    arrays, dt = fresh(0.9), torch.zeros(1, dtype=torch.float64, device=device)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        st.advance_async(*arrays, dt)
+    del graph
+    assert st.new_advance(*fresh(0.01)) == want[0.01]
+    graph = torch.cuda.CUDAGraph()
+    start = arrays[0].clone()
+    with torch.cuda.graph(graph):
+        st.advance_async(*arrays, dt)
+    for _ in range(3):
+        arrays[0].copy_(start)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float(dt) == want[0.9]
+        assert st.new_advance(*fresh(0.01)) == want[0.01]
+    st.close()
+    ref.close()
