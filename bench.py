@@ -72,8 +72,26 @@ def step_algorithmic_bytes(n: int) -> float:
     return 8.0 * (99 * (n + 8) ** 3 + 70 * n ** 3)
 
 
+def stage_bytes(n: int) -> float:
+    """Per-launch algorithmic HBM bytes of the one-kernel RK stage that ``cns_advance`` runs
+    (profile kind ``hypterm_rk``), the mean of a step's three: the five conserved fields over
+    their halos (5g), the stage base in stages 2 and 3 (10c / 3), the result (5c), the
+    primitives of stage 2's result (6c / 3), D and F of stage 3 (10c / 3)."""
+    g3, n3 = (n + 8) ** 3, n ** 3
+    return 8.0 * (5 * g3 + 7 * n3 + 20 * n3 / 3)
+
+
+def step_min_bytes(n: int) -> float:
+    """What the launches of a ``cns_advance`` step of a large box must move (f64): the fill of
+    U with the Courant pass 10(g-c) + 5c, the fills after stages 1 (U^{1/3}) and 2 (Unew and
+    Q) 32(g-c), three stages."""
+    g3, n3 = (n + 8) ** 3, n ** 3
+    return 8.0 * (42 * (g3 - n3) + 5 * n3) + 3 * stage_bytes(n)
+
+
 def fused_step_min_bytes(n: int) -> float:
-    """What the fused composition itself must move per step (f64): fills 50(g-c)
+    """What the step composed of separate ctoprim, wz, diffterm and hypterm + update kernels
+    (arrays that are not 16-byte aligned) must move (f64): fills 50(g-c)
     (state shell in three stages, plus u, v, w, T and then all six primitives in
     stages 2 and 3), ctoprim + wz 10g (stage 1), wz 2g (stages 2 and 3), diffterm
     5g + 4c/4c/5c, fused hypterm + RK 3 x (5g + 17.33c): 94g + 15c in all."""
@@ -96,7 +114,7 @@ def step_traffic(kern: dict, edge: int):
     steps_kinds = {k: v for k, v in kern.items() if v[1] > 0}
     if not steps_kinds:
         return None
-    launches_per_step = {"fill": 3, "ctoprim": 1, "diffterm": 3, "hypterm_rk": 3, "wz": 2}
+    launches_per_step = {"fill_courno": 1, "fill": 2, "stage": 3}
     total = 0.0
     for kind, per_step in launches_per_step.items():
         b = read_traffic(kind, edge)
@@ -635,15 +653,15 @@ def main():
     if dom:
         ms_tot, cnt = kern[dom]
         avg_s = ms_tot / cnt / 1e3
-        nbytes = algorithmic_bytes(dom, args.edge)
+        nbytes = stage_bytes(args.edge) if dom == "hypterm_rk" else algorithmic_bytes(dom, args.edge)
         ach = nbytes / avg_s / 1e9
-        traffic = read_traffic(dom, args.edge)
+        traffic = read_traffic("stage" if dom == "hypterm_rk" else dom, args.edge)
         roof = {"bound": "hbm", "kernel": dom, "achieved": round(ach, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                 "traffic": traffic, "algorithmic_bytes": nbytes, "avg_ms": round(avg_s * 1e3, 4),
                 "traffic_vs_algorithmic": round(traffic / nbytes, 3) if traffic else None}
     step_bytes = step_algorithmic_bytes(args.edge)
-    fused_min = fused_step_min_bytes(args.edge)
+    fused_min = step_min_bytes(args.edge)
     measured_step = step_traffic(kern, args.edge)
     out = {
         "metric": METRIC,

@@ -28,12 +28,13 @@
 //   A
 // Before the first centre plane the windows and the ring are filled with eight planes at once.
 //
-// What bounds it: the vector arithmetic, about 1020 FP64 and 250 other instructions per
-// cell and plane at 4.5 cycles each (two waves per SIMD: 64 % of the cycles of a plane; the
-// rest is the latency of phase 1's divisions and the three barriers).  The time of a plane is
-// the same for one workgroup alone on the GPU and for 256.  512^3: 7.8 / 8.5 / 8.9 ms for stages
-// 1 / 2 / 3 against 11.4 / 12.8 / 11.4 ms of the fill-to-update chain of separate kernels;
-// 256^3 1.03 / 1.07 / 1.14 ms against 1.6 / 1.8 / 1.7 ms.
+// What bounds it: each wave's own chain.  A plane is 1120 to 1200 vector, 150 to 250 scalar and
+// 250 LDS instructions a wave (about 1020 FP64); a wave issues an FP64 instruction every 4.2 cycles at
+// best, 6.5 when it waits for the one before, two waves of a SIMD do not slow each other, and a
+// plane takes 14 to 17 thousand cycles: 45 % issuing, 25 % ready and not issued, 30 % in waits
+// and barriers.  More waves would need fewer registers than the windows hold.  512^3: 6.8 / 7.9 /
+// 8.2 ms for stages 1 / 2 / 3 (3.3 to 4.4 TB/s where a copy does 4.8) against 11.4 / 12.8 / 11.4 ms
+// of the fill-to-update chain of separate kernels; 256^3 0.91 / 1.04 / 1.06 ms against 1.6 / 1.8 / 1.7 ms.
 //   A register spilled in the loop costs far more than its instructions: the reload waits for
 // every DMA issued before it (stages 2 and 3 ran 13 ms at 512^3 with ten reloads per plane).
 // Hence one-plane products instead of u, v, w windows, indices formed anew where they are used,
@@ -74,6 +75,19 @@ struct StageArgs {
     Shell shell;
     double *fill_u;
 };
+
+// Stage 3 stores past the caches: its fifteen streams would push out the planes that the
+// neighbours read again, and nothing reads them before the next step (8.37 -> 8.22 ms at 512^3, 1.08
+// -> 1.06 at 256^3, 32.4 -> 31.8 us at 64^3).  What stages 1 and 2 store is read by the next one:
+// stored so it made stage 2 2 to 4 % slower.
+template <bool NT_>
+__device__ __forceinline__ void put(double *p, unsigned off, double v)
+{
+    if (NT_)
+        __builtin_nontemporal_store(v, &at(p, off));
+    else
+        at(p, off) = v;
+}
 
 template <bool STAGE1, bool LAST, bool QOUT, bool WRAP>
 __global__ void __launch_bounds__(NT, 2)
@@ -713,13 +727,13 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
 #pragma unroll
                 for (int l = 0; l < NC; l++) {
                     if (LAST) {
-                        at(dif + l * g.c + fk, int8) = D[l];
-                        at(flux + l * g.c + fk, int8) = F[l];
+                        put<true>(dif + l * g.c + fk, int8, D[l]);
+                        put<true>(flux + l * g.c + fk, int8, F[l]);
                     }
                     // STAGE1: cons + dt(D+F) (cpu/advance.cpp:82); then ra*base + rb*(cons + dt(D+F))
                     // (:114-116, :148-150)
                     o[l] = STAGE1 ? uc[l] + dt * (D[l] + F[l]) : ra * rkb[l] + rb * (uc[l] + dt * (D[l] + F[l]));
-                    at(out + l * cg + zk, own8) = o[l];
+                    put<LAST>(out + l * cg + zk, own8, o[l]);
                 }
                 // the x ghosts that are images of the cell
                 int i0 = gi0;
