@@ -42,7 +42,7 @@ typedef struct cns_domain cns_domain;
 
 /* A periodic domain of ncell[0] x ncell[1] x ncell[2] cells of size dx, cut into
  * boxes of max_grid_size^3 cells; cfl, eta, alam as cns_ctx_create.  Allocates the
- * domain's scratch (a stage buffer and the wz field, 6 ghosted components per box). */
+ * domain's scratch (a stage buffer, 5 ghosted components per box). */
 int cns_domain_create(cns_domain **d, const int ncell[3], int max_grid_size, const double dx[3],
                       double cfl, double eta, double alam);
 int cns_domain_destroy(cns_domain *d);
