@@ -505,7 +505,7 @@ diffterm_pipe_kernel(Geom g, const double *__restrict__ q, const double *__restr
 // runs within 1 % the shortest, which start their neighbours' planes closer in time.  Halving
 // until 2048 workgroups, as before, left a last round nearly empty or the runs at twice
 // the fill: diffterm 324 -> 272 us at 200x180x160, 76 -> 54 us at 130x97x61, 712 -> 655 us at
-// 256^3; hypterm 58 -> 39 us at 130x97x61.
+// 256^3; hypterm 58 -> 39 us at 130x97x61 (all before the planes stopped waiting for memory).
 // CNS_PIPE_KZ in the environment caps the run length (for measurements).
 int pipe_kz(const Geom &g, int64_t tiles, int slots, int warm)
 {
