@@ -51,6 +51,7 @@
 #include <type_traits>
 
 #include "cns_fill.h"
+#include "cns_runs.h"
 #include "cns_stage_tile.h"
 
 namespace cns {
@@ -772,21 +773,7 @@ stage_kernel(Geom g, const double *__restrict__ cons, StageArgs a, double dxi0, 
 constexpr int kCUs = 256;
 constexpr double kFill = 1.6;
 
-int stage_kz(const Geom &g, int64_t tiles)
-{
-    int best = g.n2;
-    double cost = 1e300;
-    for (int nz = 1; nz <= g.n2; nz++) {
-        const int kz = (g.n2 + nz - 1) / nz, runs = (g.n2 + kz - 1) / kz;
-        const int64_t rounds = (tiles * runs + kCUs - 1) / kCUs;
-        const double c = (double)rounds * (kz + kFill);
-        if (c < cost) {
-            cost = c;
-            best = kz;
-        }
-    }
-    return best;
-}
+int stage_kz(const Geom &g, int64_t tiles) { return stage_run(g.n2, tiles, kCUs, kFill); }
 
 }  // namespace
 

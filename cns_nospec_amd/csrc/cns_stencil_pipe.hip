@@ -31,6 +31,7 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "cns_runs.h"
 #include "cns_stage_tile.h"
 
 namespace cns {
@@ -513,17 +514,7 @@ int pipe_kz(const Geom &g, int64_t tiles, int slots, int warm)
         const char *e = getenv("CNS_PIPE_KZ");
         return e ? atoi(e) : 0;
     }();
-    const int most = cap >= 4 && cap < g.n2 ? cap : g.n2;
-    int best = most;
-    int64_t cost = INT64_MAX / 2;
-    for (int nz = (g.n2 + most - 1) / most; nz <= g.n2; nz++) {
-        const int kz = (g.n2 + nz - 1) / nz, runs = (g.n2 + kz - 1) / kz;
-        const int64_t c = (tiles * runs + slots - 1) / slots * (kz + warm);
-        if (c > cost + cost / 100) continue;
-        best = kz;
-        if (c < cost) cost = c;
-    }
-    return best;
+    return pipe_run(g.n2, cap >= 4 && cap < g.n2 ? cap : g.n2, tiles, slots, warm);
 }
 
 // The stencils run on 32 x 8 tiles, two workgroups per CU (512^3: diffterm
