@@ -536,7 +536,7 @@ static int enqueue_step(cns_ctx *ctx, double *U, double *Unew, double *Q, double
 {
     const Geom &g = ctx->g;
     const double *dt = sd.dt;
-    if (ctx->d_stage) {
+    if (ctx->d_stage && stage_pays(g)) {
         // Fused composition.  Stage results go to a buffer the stage does not read with halos:
         //   stage 1: U -> stage (U^{1/3});  stage 2: stage -> Unew (U^{2/3});
         //   stage 3: Unew -> U (U^{n+1}).
@@ -566,7 +566,7 @@ static int enqueue_step(cns_ctx *ctx, double *U, double *Unew, double *Q, double
         // Arrays that are not 16-byte aligned, or too large for its offsets: fill, ctoprim,
         // diffterm, and hypterm with the RK update of its cell applied in the same pass.
         TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, nullptr, s));
-            TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, U, Q, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
+        TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, U, Q, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
         HIPCHK(launch_courno_to_dt(sd, s));
         TIMED(ctx, CNS_PROF_DIFFTERM, s, stencil_diffterm(g, Q, D, ctx->dxi, ctx->eta, ctx->alam, ctx->d_wz, s));
         TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, U, Q, F, ctx->dxi, D, U, T, dt, 1, false, s));
@@ -582,7 +582,7 @@ static int enqueue_step(cns_ctx *ctx, double *U, double *Unew, double *Q, double
         TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, Unew, Q, F, ctx->dxi, D, U, U, dt, 3, true, s));
         return CNS_OK;
     }
-    // Unfused composition, kernel for kernel as the reference.
+    // Unfused composition, kernel for kernel as the reference (also for tall columns of a few cells).
     // cpu/advance.cpp:45-85: stage 1
     TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, U, nullptr, s));
     TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, U, Q, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));

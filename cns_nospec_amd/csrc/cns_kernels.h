@@ -104,6 +104,7 @@ hipError_t launch_fill_courno(const Geom &g, double *u, unsigned long long *acc,
 // interior, phases 2 and 3 read cons at wrapped rows and planes, and phase 3 fills the ghosts
 // of cons (which is not const then) and q.  Null: cons has its ghosts filled.
 bool stage_fits(const Geom &g);
+bool stage_pays(const Geom &g);   // whether a step of separate kernels would be slower
 bool stage_wraps(const Geom &g);  // whether a periodic box is stepped without fills between its stages
 hipError_t launch_stage(const Geom &g, const double *cons, const double *base, double *out, double *q, double *d,
                         double *f, const StepDt &sd, const double dxi[3], double eta, double alam, int phase,

@@ -782,6 +782,13 @@ bool stage_fits(const Geom &g)
     return g.pg < (1 << 29) && g.xg < (1 << 24) && g.g1 < (1 << 24);
 }
 
+// A tile of 32 x 16 cells costs its time however few of them the box has, so a tall column of a few
+// cells is stepped faster by the separate kernels, whose tiles are half as high: us a step with one
+// kernel a stage / separate kernels, 4 x 4 x 512 112 / 168, x 4096 395 / 337, x 20000 1689 / 1360;
+// 8 x 8 x 512 109 / 175, x 4096 401 / 393, x 20000 1747 / 1647; 16 x 8 x 20000 2053 / 2650, 12 x 12 x 20000
+// 2255 / 3806.
+bool stage_pays(const Geom &g) { return g.n0 > 8 || g.n1 > 8 || g.n2 < 16 * kCUs; }
+
 // Reading at wrapped addresses and storing the x ghosts beside the result costs a plane about
 // 1.5 % (scalar registers that no longer fit), two fill launches their time and two gaps: a step
 // with / without them takes 73 / 80 us at 16^3, 113 / 120 at 64^3, 466 / 480 at 128^3, 3.24 / 3.26

@@ -115,3 +115,35 @@ def test_many_contexts_and_a_first_step_that_is_captured(device):
         assert st.new_advance(*fresh(0.01)) == want[0.01]
     st.close()
     ref.close()
+
+
+@pytest.mark.parametrize("n,separate", [((8, 8, 4096), True), ((4, 5, 4099), True), ((8, 8, 4095), False),
+                                        ((9, 8, 4096), False), ((8, 9, 4096), False)])
+def test_tall_columns_take_the_separate_kernels(device, n, separate):
+    """Columns of up to 8 x 8 cells and at least 4096 planes are stepped kernel for kernel, their
+    neighbours by the stage kernel; both to the bits of the direct kernels."""
+    import torch
+    lay = BoxLayout(n)
+    U0 = torch.from_numpy(sinusoid_state(lay, 23, mach=0.2, kmax=2)).to(device)
+    got = {}
+    for impl in (_lib.CNS_IMPL_TILED, _lib.CNS_IMPL_DIRECT):
+        print(f"tall column n={n} impl={impl}", flush=True)
+        ops.set_stencil_impl(impl)
+        try:
+            arrays = ops.allocate_variables(lay, device)
+            arrays[0].copy_(U0)
+            st = ops.Stepper(lay)
+            st.set_fused(impl == _lib.CNS_IMPL_TILED)
+            st.profile(True)
+            dts = [st.new_advance(*arrays) for _ in range(2)]
+            kinds = {k for k, v in st.profile_read().items() if v[1] > 0}
+            got[impl] = (dts, kinds, [a.cpu().numpy() for a in arrays])
+            st.profile(False)
+            st.close()
+        finally:
+            ops.set_stencil_impl(_lib.CNS_IMPL_TILED)
+    (dts, kinds, arrays), (rdts, _, rarrays) = got[_lib.CNS_IMPL_TILED], got[_lib.CNS_IMPL_DIRECT]
+    assert ("diffterm" in kinds) == separate and ("hypterm_rk" in kinds) != separate
+    assert dts == rdts
+    for a, b, name in zip(arrays, rarrays, ("U", "Unew", "Q", "D", "F")):
+        assert np.array_equal(a, b), name
