@@ -5,6 +5,7 @@
 // halos are gathered, so no ghost storage and no fill pass exist.
 #pragma once
 
+#include "cns_batch_plan.h"
 #include "cns_common.h"
 
 namespace cns {
@@ -32,13 +33,6 @@ struct BoxDev {
 // A box that has reached its step target is skipped by every kernel of the step.
 __host__ __device__ inline bool box_stopped(const BoxDev &b) { return b.target > 0 && b.steps >= b.target; }
 
-struct TileDev {
-    int box;
-    short x0, y0, z0, nz;  // tile origin (cells) and z run
-    short ltx;             // log2 of the tile width (4, 5 or 6)
-    short rows;            // of a tile of the fused kernel
-};
-
 // Tile widths 16, 32, 64 (class 0, 1, 2); a box's tiles all have one width.
 constexpr int kTileClasses = 3;
 
@@ -59,7 +53,6 @@ hipError_t launch_batch_stage(BoxDev *boxes, const TileDev *tiles, const int sta
                               const int count[3], int stage, bool fp32, bool fused, bool staged_diff,
                               bool keep_centre, hipStream_t s);
 // Its class-1 launch (cns_batch_stage.hip).
-constexpr int kShortRows = 16, kTallRows = 24;
 hipError_t launch_batch_fused(BoxDev *boxes, const TileDev *tiles, int n, int stage, bool fp32, hipStream_t s);
 
 }  // namespace cns

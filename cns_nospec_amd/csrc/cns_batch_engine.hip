@@ -9,13 +9,11 @@
 // the dt finalize) is captured once into a hipGraph and replayed until the
 // resident set or the tile table changes.
 #include <algorithm>
-#include <climits>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <new>
-#include <queue>
 #include <vector>
 
 #include "cns_batch.h"
@@ -155,144 +153,6 @@ void destroy_graph(cns_batch *b)
     if (b->graph) (void)hipGraphDestroy(b->graph);
     b->exec = nullptr;
     b->graph = nullptr;
-}
-
-// The fused class's work list.  A CU holds one workgroup of the stage kernel, which takes
-// about planes + 1.5 plane times, and XCD x runs the x-th eighth of the list in order on its
-// 32 CUs.  So the list is made of eight equally long parts (dummy tiles fill them up): the z
-// runs of all boxes, longest first, each go whole (its tiles share halos) to the part with the
-// least work.  Long runs fill their windows less often, short ones end together: the boxes are
-// split in one of a few ways, the one whose slowest part is predicted to end first.
-//   Predicted / measured with 16-row tiles alone, 64 boxes of edges 16..96 (the work alone: 125
-// plane times of every CU): runs of 16 planes 140 / 2.86 ms a step (FP64), of 32 151 / 3.17, this
-// list 134 / 2.80; 40 boxes of 24..128 (233): runs of 16 in the boxes' order 5.12 ms (FP32 flux), of
-// 32 longest first 260 / 4.86, this list 248 / 4.64.
-constexpr int kXcds = 8, kCusPerXcd = 32;
-constexpr int kTallCost = 4, kShortCost = 3;  // of a plane
-constexpr size_t kMostSimulated = 1 << 14;  // tiles; a longer list's tail is short however it is split
-
-struct Split {
-    int run, last, eighths;  // runs of `run` planes, and of `last` for so many eighths:
-    bool boxes;              // of the work, the smallest boxes (or the last planes of every box)
-};
-constexpr Split kSplits[] = {{24, 0, 0, false}, {16, 0, 0, false}, {32, 0, 0, false}, {48, 0, 0, false},
-                             {64, 0, 0, false}, {48, 16, 3, true}, {32, 16, 2, true}, {24, 16, 2, true},
-                             {40, 8, 2, true},  {64, 12, 1, false}, {48, 8, 1, false}, {24, 8, 4, false}};
-
-struct FusedBox {
-    int id, e, kz;      // kz: longest run allowed
-    int nx, tall, low;  // tiles of a plane: nx times so many of kTallRows and of kShortRows rows
-    int cost() const { return nx * (kTallCost * tall + kShortCost * low); }
-    int tiles() const { return nx * (tall + low); }
-};
-
-// A box's rows in the fewest plane times: of FP32 flux a tall tile's plane takes 1.35 times a
-// short one's (cns_batch_stage.hip; edges 96 and 64 measured), e.g. 16 rows one short tile, 24 one
-// tall, 32 two short, 40 one of each.
-void tile_rows(FusedBox &b, bool fp32)
-{
-    int best = INT_MAX;
-    for (int tall = 0; tall <= (fp32 ? (b.e + kTallRows - 1) / kTallRows : 0); tall++) {
-        const int low = std::max(0, (b.e - tall * kTallRows + kShortRows - 1) / kShortRows);
-        const int cost = kTallCost * tall + kShortCost * low;
-        if (cost < best) {
-            best = cost;
-            b.tall = tall;
-            b.low = low;
-        }
-    }
-}
-
-struct Unit {
-    int box, z0, nz;  // index of the FusedBox
-};
-struct FusedPlan {
-    std::vector<Unit> part[kXcds];
-    int64_t end = 0;  // of the slowest part, in sixths of a short tile's plane time
-    size_t tiles = 0;
-};
-
-// `boxes`: largest first
-FusedPlan plan_runs(const std::vector<FusedBox> &boxes, const Split &sp, bool simulate)
-{
-    FusedPlan p;
-    std::vector<Unit> units;
-    int64_t all = 0, done = 0;
-    for (const FusedBox &b : boxes) all += (int64_t)b.cost() * b.e;
-    // planes z0 .. z1-1 of box b in even runs of about `run`, at most the box's kz
-    auto runs = [&](int b, int z0, int z1, int run) {
-        const int len = z1 - z0;
-        if (len <= 0) return;
-        const int n = std::max({1, (len + run / 2) / run, (len + boxes[b].kz - 1) / boxes[b].kz});
-        const int nz = (len + n - 1) / n;
-        for (int z = z0; z < z1; z += nz) units.push_back({b, z, std::min(nz, z1 - z)});
-    };
-    for (int b = 0; b < (int)boxes.size(); b++) {
-        const int e = boxes[b].e;
-        if (sp.boxes) {
-            runs(b, 0, e, 8 * done < (8 - sp.eighths) * all ? sp.run : sp.last);
-            done += (int64_t)boxes[b].cost() * e;
-        } else {
-            const int first = e - e * sp.eighths / 8;
-            runs(b, 0, first, sp.run);
-            runs(b, first, e, sp.last);
-        }
-    }
-    std::stable_sort(units.begin(), units.end(), [](const Unit &a, const Unit &b) { return a.nz > b.nz; });
-    int64_t load[kXcds] = {};
-    for (const Unit &u : units) {
-        const int x = (int)(std::min_element(load, load + kXcds) - load);
-        load[x] += (int64_t)boxes[u.box].cost() * (2 * u.nz + 3);
-        p.part[x].push_back(u);
-        p.tiles += (size_t)boxes[u.box].tiles();
-    }
-    for (int x = 0; simulate && x < kXcds; x++) {
-        std::priority_queue<int64_t, std::vector<int64_t>, std::greater<int64_t>> cu;
-        for (int i = 0; i < kCusPerXcd; i++) cu.push(0);
-        for (const Unit &u : p.part[x])
-            for (int t = 0; t < boxes[u.box].tiles(); t++) {
-                const int c = t < boxes[u.box].nx * boxes[u.box].tall ? kTallCost : kShortCost;
-                const int64_t end = cu.top() + c * (2 * u.nz + 3);
-                cu.pop();
-                cu.push(end);
-                p.end = std::max(p.end, end);
-            }
-    }
-    return p;
-}
-
-// Appends the list; returns the number of its real tiles.
-size_t fused_list(std::vector<FusedBox> &boxes, std::vector<TileDev> &out)
-{
-    std::stable_sort(boxes.begin(), boxes.end(), [](const FusedBox &a, const FusedBox &b) { return a.e > b.e; });
-    size_t most = 0;
-    for (const FusedBox &b : boxes) most += (size_t)b.tiles() * ((b.e + 11) / 12);
-    const bool simulate = most <= kMostSimulated;
-    FusedPlan best;
-    for (const Split &sp : kSplits) {
-        FusedPlan p = plan_runs(boxes, sp, simulate);
-        if (&sp == kSplits || p.end < best.end) best = std::move(p);
-        if (!simulate) break;
-    }
-    std::vector<TileDev> part[kXcds];
-    most = 0;
-    for (int x = 0; x < kXcds; x++) {
-        for (const Unit &u : best.part[x]) {
-            const FusedBox &b = boxes[u.box];
-            for (int y0 = 0, r = 0; r < b.tall + b.low; r++) {
-                const short rows = r < b.tall ? kTallRows : kShortRows;
-                for (int x0 = 0; x0 < b.e; x0 += 32)
-                    part[x].push_back({b.id, (short)x0, (short)y0, (short)u.z0, (short)u.nz, 5, rows});
-                y0 += rows;
-            }
-        }
-        most = std::max(most, part[x].size());
-    }
-    for (int x = 0; x < kXcds; x++) {
-        part[x].resize(most, {boxes[0].id, 0, 0, 0, 0, 5, 0});  // no planes: ends at once
-        out.insert(out.end(), part[x].begin(), part[x].end());
-    }
-    return best.tiles;
 }
 
 // Rebuild the work list and re-capture the step graph.
