@@ -41,7 +41,12 @@ struct Split {
 };
 constexpr Split kSplits[] = {{24, 0, 0, false}, {16, 0, 0, false}, {32, 0, 0, false}, {48, 0, 0, false},
                              {64, 0, 0, false}, {48, 16, 3, true}, {32, 16, 2, true}, {24, 16, 2, true},
-                             {40, 8, 2, true},  {64, 12, 1, false}, {48, 8, 1, false}, {24, 8, 4, false}};
+                             {40, 8, 2, true},  {64, 12, 1, false}, {48, 8, 1, false}, {24, 8, 4, false},
+                             {8, 0, 0, false},  {4, 0, 0, false},  {2, 0, 0, false}};
+// The last three are for boxes that leave most CUs idle (1 / 4 / 8 boxes of 48^3, FP32 flux, 89 / 138 / 213
+// us a step, in runs of 16 planes 357 / 362 / 365).  The shorter the runs, the more of the prediction rests on the
+// window fill, which for tall tiles is nearer 2.5 planes: they have to be an eighth better than the rest.
+constexpr int kShortRun = 16;
 
 struct FusedBox {
     int id, e, kz;      // kz: longest run allowed
@@ -216,7 +221,7 @@ inline size_t fused_list(std::vector<FusedBox> &boxes, std::vector<TileDev> &out
         std::vector<GroupRuns> runs = split_runs(boxes, groups, all, sp);
         if (std::find(tried.begin(), tried.end(), runs) != tried.end()) continue;
         FusedPlan p;
-        if (plan_runs(boxes, runs, best.end, simulate, p)) best = std::move(p);
+        if (plan_runs(boxes, runs, sp.run < kShortRun ? best.end - best.end / 8 : best.end, simulate, p)) best = std::move(p);
         if (!simulate) break;
         tried.push_back(std::move(runs));
     }

@@ -100,6 +100,7 @@ def test_run_lengths_are_those_of_the_plain_search(runs):
 LIST = r"""
 #include <chrono>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <functional>
 #include <queue>
@@ -164,7 +165,7 @@ static std::vector<TileDev> plain_list(std::vector<FusedBox> boxes)
     Plain best;
     for (const Split &sp : kSplits) {
         Plain p = plain_plan(boxes, sp);
-        if (&sp == kSplits || p.end < best.end) best = p;
+        if (&sp == kSplits || p.end < (sp.run < kShortRun ? best.end - best.end / 8 : best.end)) best = p;
         if (most > kMostSimulated) break;
     }
     std::vector<TileDev> part[kXcds], out;
@@ -238,6 +239,14 @@ int main(int, char **argv)
         printf("%g\n", fast / plain);
         return 0;
     }
+    if (!strcmp(argv[1], "few")) {
+        // tiles of n boxes of edge e
+        std::vector<FusedBox> boxes;
+        for (int i = 0; i < atoi(argv[2]); i++) boxes.push_back(box(i, atoi(argv[3]), 512, argv[4][0] == '1'));
+        std::vector<TileDev> out;
+        printf("%zu\n", fused_list(boxes, out));
+        return 0;
+    }
     int bad = 0;
     for (int t = 0; t < 400; t++) {
         const bool fp32 = t & 1, alike = t & 2, capped = t & 4;
@@ -279,3 +288,17 @@ def test_work_list_is_made_in_a_fraction_of_the_plain_search(work_list):
     """The list is made anew whenever a box comes or goes: of 4000 boxes of one edge in about a tenth of
     the time of the plain search (the limit leaves a factor of five for a busy machine)."""
     assert float(work_list("time")) < 0.5
+
+
+@pytest.mark.parametrize("n,e,fp32", [(1, 48, 1), (1, 32, 0), (4, 48, 1), (1, 64, 1), (2, 64, 0)])
+def test_few_boxes_are_split_until_they_use_the_gpu(work_list, n, e, fp32):
+    """Few boxes are cut into runs short enough to give many CUs one (runs of 16 planes gave one box
+    of 48^3 twelve workgroups and one of 32^3 four)."""
+    assert int(work_list("few", n, e, fp32)) >= 32
+
+
+@pytest.mark.parametrize("n,e,fp32", [(64, 96, 1), (64, 96, 0), (1000, 24, 1), (600, 17, 0), (16, 64, 0)])
+def test_boxes_that_fill_the_gpu_keep_long_runs(work_list, n, e, fp32):
+    """Runs of fewer than 16 planes (or a whole box) cost more window fills than they save here."""
+    rows = -(-e // 24) if fp32 else -(-e // 16)
+    assert int(work_list("few", n, e, fp32)) <= n * -(-e // 32) * (rows + 1) * max(1, -(-e // 12))
