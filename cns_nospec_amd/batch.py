@@ -248,7 +248,7 @@ def autotune(requests, fp32: bool, widths=WIDTHS, kzs=KZS, buckets=EDGE_BUCKETS,
         if not any(bk[0] <= e <= bk[1] for e in present):
             continue
         for kz in kzs:
-            if kz == choice[bk]:
+            if kz == base[1]:  # what the bucket had before its first trial
                 continue
             trial_choice = dict(choice)
             trial_choice[bk] = kz

@@ -302,3 +302,44 @@ def test_boxes_that_fill_the_gpu_keep_long_runs(work_list, n, e, fp32):
     """Runs of fewer than 16 planes (or a whole box) cost more window fills than they save here."""
     rows = -(-e // 24) if fp32 else -(-e // 16)
     assert int(work_list("few", n, e, fp32)) <= n * -(-e // 32) * (rows + 1) * max(1, -(-e // 12))
+
+
+@pytest.mark.parametrize("gain", [1.0, 1.02])
+def test_autotuner_does_not_time_a_replaced_choice_again(monkeypatch, gain):
+    """A bucket takes one trial of every other run length, also when one of them is the faster (gain: of
+    every trial of a bucket over the last)."""
+    from cns_nospec_amd import batch, serve
+
+    class Engine:
+        def __init__(self, *args, **kwargs):
+            self.table = {}
+
+        def add(self, u, e):
+            self.table[e] = None
+
+        def set_tile(self, e, w, kz):
+            self.table[e] = (w, kz)
+
+        def close(self):
+            pass
+
+    class Request:
+        def __init__(self, edge):
+            self.edge = edge
+
+    class State:
+        def reshape(self, n):
+            return self
+
+    seen = []
+
+    def rate(eng, cells, steps, reps):
+        seen.append(tuple(sorted(eng.table.items())))
+        return gain ** max(0, len(seen) - 4)
+
+    monkeypatch.setattr(batch, "BatchEngine", Engine)
+    monkeypatch.setattr(batch, "_rate", rate)
+    monkeypatch.setattr(serve, "request_state", lambda r: State())
+    table, log = batch.autotune([Request(16), Request(24)], True, widths=(16, 32), kzs=(8, 16), buckets=((8, 20), (21, 40)))
+    assert len(seen) == 2 * 2 + 2 * 1 and len(log) == len(seen) + 1
+    assert set(table.values()) == {(16, 16 if gain == 1.0 else 8)}
