@@ -101,9 +101,9 @@ __device__ __forceinline__ unsigned long long block_max_u64(unsigned long long v
 // Primitives of U into Q[0]; at admission (FRESH) also its Courant maximum into acc, and pref.
 template <typename FT, bool FRESH>
 __global__ void __launch_bounds__(kBatchThreads)
-batch_init_kernel(BoxDev *__restrict__ boxes, int b)
+batch_init_kernel(BoxDev *__restrict__ boxes, const int *__restrict__ ids)
 {
-    BoxDev &B = boxes[b];
+    BoxDev &B = boxes[ids[blockIdx.y]];
     const int e = B.e;
     const int64_t e3 = (int64_t)e * e * e;
     const double *U = B.U;
@@ -1085,20 +1085,24 @@ hipError_t stage_class(BoxDev *boxes, const TileDev *tiles, int n, int stage, Pa
 
 }  // namespace
 
-hipError_t launch_batch_init(BoxDev *boxes, int box, int e, bool fp32, bool fresh, hipStream_t s)
+hipError_t launch_batch_init(BoxDev *boxes, const int *ids, int n, int e, bool fp32, bool fresh, hipStream_t s)
 {
     const int64_t e3 = (int64_t)e * e * e;
-    int grid = (int)((e3 + kBatchThreads * 4 - 1) / (kBatchThreads * 4));
-    grid = grid < 1 ? 1 : (grid > 4096 ? 4096 : grid);
-    if (fp32 && fresh)
-        batch_init_kernel<float, true><<<grid, kBatchThreads, 0, s>>>(boxes, box);
-    else if (fp32)
-        batch_init_kernel<float, false><<<grid, kBatchThreads, 0, s>>>(boxes, box);
-    else if (fresh)
-        batch_init_kernel<double, true><<<grid, kBatchThreads, 0, s>>>(boxes, box);
-    else
-        batch_init_kernel<double, false><<<grid, kBatchThreads, 0, s>>>(boxes, box);
-    return hipGetLastError();
+    const int64_t blocks = (e3 + kBatchThreads * 4 - 1) / (kBatchThreads * 4);
+    for (; n > 0; n -= 65535, ids += 65535) {
+        const dim3 grid((unsigned)(blocks < 4096 ? blocks : 4096), (unsigned)(n < 65535 ? n : 65535));
+        if (fp32 && fresh)
+            batch_init_kernel<float, true><<<grid, kBatchThreads, 0, s>>>(boxes, ids);
+        else if (fp32)
+            batch_init_kernel<float, false><<<grid, kBatchThreads, 0, s>>>(boxes, ids);
+        else if (fresh)
+            batch_init_kernel<double, true><<<grid, kBatchThreads, 0, s>>>(boxes, ids);
+        else
+            batch_init_kernel<double, false><<<grid, kBatchThreads, 0, s>>>(boxes, ids);
+        const hipError_t rc = hipGetLastError();
+        if (rc != hipSuccess) return rc;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_batch_finalize(BoxDev *boxes, const int *ids, int n, int count_step, hipStream_t s)

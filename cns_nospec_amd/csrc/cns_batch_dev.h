@@ -38,8 +38,9 @@ constexpr int kTileClasses = 3;
 
 constexpr int kBatchThreads = 256;
 
-// Primitives of the box's U into Q[0]; fresh (admission): its Courant maximum and pref too.
-hipError_t launch_batch_init(BoxDev *boxes, int box, int e, bool fp32, bool fresh, hipStream_t s);
+// Primitives of the boxes' U into Q[0]; fresh (admission): their Courant maximum and pref too.  ids: n
+// box ids on the device; e: the largest edge.
+hipError_t launch_batch_init(BoxDev *boxes, const int *ids, int n, int e, bool fp32, bool fresh, hipStream_t s);
 hipError_t launch_batch_finalize(BoxDev *boxes, const int *box_ids, int nbox, int count_step,
                                  hipStream_t s);
 // One RK stage over the tile list: the list holds class 0, 1, 2 tiles in the

@@ -161,17 +161,39 @@ int rebuild(cns_batch *b, hipStream_t s)
     CNS_HIPCHK(hipStreamSynchronize(s));  // host staging is about to change
     std::vector<TileDev> cls[kTileClasses];
     std::vector<FusedBox> fboxes;
+    auto small = [&](const BoxHost &h) {
+        return b->fused() && h.e <= small_edge(b->fp32) && b->tile_of(h.e).first == 32;
+    };
+    size_t nsmall = 0, live = 0;
+    for (const BoxHost &h : b->hb) {
+        live += h.live;
+        nsmall += h.live && small(h);
+    }
+    const bool apart = small_apart(nsmall, live - nsmall);
+    auto width_of = [&](const BoxHost &h) { return apart && small(h) ? 16 : b->tile_of(h.e).first; };
+    auto in_fused = [&](const BoxHost &h) { return b->fused() && width_of(h) == 32; };
+    // Boxes that leave the fused class, which keeps no Q[0]
+    std::vector<int> stale;
+    int stale_e = 0;
+    for (int id = 0; id < (int)b->hb.size(); id++) {
+        const BoxHost &h = b->hb[id];
+        if (!h.live || !h.fused || in_fused(h)) continue;
+        stale.push_back(id);
+        stale_e = std::max(stale_e, h.e);
+    }
+    if (!stale.empty()) {
+        CNS_HIPCHK(hipMemcpyAsync(b->d_ids, stale.data(), stale.size() * sizeof(int), hipMemcpyHostToDevice, s));
+        CNS_HIPCHK(launch_batch_init(b->d_boxes, b->d_ids, (int)stale.size(), stale_e, b->fp32, false, s));
+        CNS_HIPCHK(hipStreamSynchronize(s));
+    }
     b->hids.clear();
     for (int id = 0; id < (int)b->hb.size(); id++) {
         BoxHost &h = b->hb[id];
         if (!h.live) continue;
         b->hids.push_back(id);
-        const auto t = b->tile_of(h.e);
-        const int w = t.first, c = width_class(w), kz = std::max(1, std::min(t.second, h.e));
-        const bool fused = b->fused() && c == 1;
-        if (h.fused && !fused) CNS_HIPCHK(launch_batch_init(b->d_boxes, id, h.e, b->fp32, false, s));
-        h.fused = fused;
-        if (fused) {
+        const int w = width_of(h), c = width_class(w), kz = std::max(1, std::min(b->tile_of(h.e).second, h.e));
+        h.fused = in_fused(h);
+        if (h.fused) {
             FusedBox fb{id, h.e, kz, (h.e + 31) / 32, 0, 0};
             tile_rows(fb, b->fp32);
             fboxes.push_back(fb);
@@ -368,7 +390,7 @@ int cns_batch_add(cns_batch *b, int edge, double dx, double cfl, double eta, dou
     int rc = CNS_OK;
     if (hipMemcpyAsync(b->d_boxes + id, &r, sizeof r, hipMemcpyHostToDevice, s) != hipSuccess ||
         hipMemcpyAsync(r.U, u0, 5 * e3 * sizeof(double), hipMemcpyDeviceToDevice, s) != hipSuccess ||
-        launch_batch_init(b->d_boxes, id, edge, b->fp32, true, s) != hipSuccess ||
+        launch_batch_init(b->d_boxes, b->d_iota + id, 1, edge, b->fp32, true, s) != hipSuccess ||
         launch_batch_finalize(b->d_boxes, b->d_iota + id, 1, 0, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
         rc = fail(CNS_EHIP, "initialising box %d failed: %s", id, hipGetErrorString(hipGetLastError()));

@@ -48,6 +48,19 @@ constexpr Split kSplits[] = {{24, 0, 0, false}, {16, 0, 0, false}, {32, 0, 0, fa
 // window fill, which for tall tiles is nearer 2.5 planes: they have to be an eighth better than the rest.
 constexpr int kShortRun = 16;
 
+// Small boxes.  A 32 x 16 tile of the one-kernel stage takes its time however few of its cells a box
+// has; the separate kernels' 16 x 16 tiles of four waves share a CU instead, but are nine launches a
+// step.  So boxes of at most small_edge() cells take 16-wide tiles where they are many: more than one a CU,
+// or two beside other boxes, whose stage goes on without them.  us a step with one kernel a stage / 16-wide
+// tiles, FP32 flux: 256 boxes of 8^3 190 / 170, 320 308 / 190, 1024 675 / 298; of 16^3 256 346 / 338, 320 499 /
+// 387, 1024 1308 / 931; beside 30 of 64^3 320 of 16^3 1597 / 1716, 512 1781 / 1783, 1024 2357 / 2159. FP64: 320 boxes
+// of 8^3 330 / 263, of 14^3 505 / 483, 1024 740 / 479 and 1309 / 1135; of 16^3 1459 / 1409, 320 562 / 611.
+constexpr int small_edge(bool fp32) { return fp32 ? 16 : 14; }
+constexpr bool small_apart(size_t small, size_t others)
+{
+    return small > (others ? 2 : 1) * (size_t)(kXcds * kCusPerXcd);
+}
+
 struct FusedBox {
     int id, e, kz;      // kz: longest run allowed
     int nx, tall, low;  // tiles of a plane: nx times so many of kTallRows and of kShortRows rows

@@ -77,9 +77,10 @@ int cns_batch_query(cns_batch *b, int n, const int *ids, long long *steps, doubl
 /* Tile shape used for boxes of a given edge: width 16, 32 or 64 cells and z run kz
  * (1..edge).  Tiles are 256/width cells high, 32-wide ones 16 (FP32 flux:
  * 16 or 24, whichever cover the box best), whose kz is the longest run:
- * the work list splits every box so that the GPU's CUs end together.  Applies to boxes
- * admitted afterwards and rebuilds the work list; results do not depend on it.  The table
- * starts from built-in defaults; the package's autotuner measures and sets it. */
+ * the work list splits every box so that the GPU's CUs end together.  Where hundreds of boxes of 32-wide
+ * edges up to 16 are resident, the engine takes 16-wide tiles for them.  Applies to every
+ * resident box from the next step on; results do not depend on it.  The table starts
+ * from built-in defaults; the package's autotuner measures and sets it. */
 int cns_batch_set_tile(cns_batch *b, int edge, int tile_width, int kz);
 int cns_batch_get_tile(cns_batch *b, int edge, int *tile_width, int *kz);
 

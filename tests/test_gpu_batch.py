@@ -276,3 +276,64 @@ def test_fused_stage_row_heights_agree(device, monkeypatch, edge):
         out.append((eng.read(i).cpu().numpy(), eng.query([i])[i]["dt"]))
         eng.close()
     assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+def test_tile_width_changes_between_steps_keep_the_bits(device, fp32):
+    """Boxes that move between the one-kernel stage, which keeps no primitives between stages, and
+    the separate kernels, which start from them, step to the bits of boxes that never moved."""
+    edges = (8, 16, 21, 40)
+    init = {e: compact_sinusoid(e, 70 + e, mach=0.25, kmax=3).reshape(-1) for e in edges}
+    stay = BatchEngine(1 << 30, fp32=fp32, max_boxes=4, tuning={e: (16, 5) for e in edges})
+    move = BatchEngine(1 << 30, fp32=fp32, max_boxes=4, tuning={})
+    a = {e: stay.add(init[e], e) for e in edges}
+    b = {e: move.add(init[e], e) for e in edges}
+    for widths in ((32, 32, 32, 32), (16, 32, 16, 64), (32, 16, 32, 32), (64, 16, 16, 16), (32, 32, 64, 32)):
+        for e, w in zip(edges, widths):
+            move.set_tile(e, w, 7)
+        print(f"tile widths {widths} fp32={fp32}", flush=True)
+        stay.step(2)
+        move.step(2)
+        for e in edges:
+            assert np.array_equal(stay.read(a[e]).cpu().numpy(), move.read(b[e]).cpu().numpy()), f"{widths}: edge {e}"
+    qa, qb = stay.query(a.values()), move.query(b.values())
+    assert [qa[a[e]] for e in edges] == [qb[b[e]] for e in edges]
+    stay.close()
+    move.close()
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+def test_many_small_boxes_come_and_go(device, monkeypatch, fp32):
+    """Small boxes change to 16-wide tiles when there are many of them and back when there are few,
+    alone and beside a large box, with the bits of an engine that runs the separate kernels throughout."""
+    edges = (8, 9, 13, 14, 16)
+    init = {e: compact_sinusoid(e, 30 + e, mach=0.2, kmax=3).reshape(-1) for e in (*edges, 40)}
+    engines = []
+    for hyp in ("1", "0"):
+        monkeypatch.setenv("CNS_BATCH_HYP", hyp)
+        monkeypatch.setenv("CNS_BATCH_HYP64", hyp)
+        engines.append(BatchEngine(2 << 30, fp32=fp32, max_boxes=1200, tuning={}))
+    ids = [[], []]
+
+    def populate(n, edge=None):
+        for eng, mine in zip(engines, ids):
+            while len(mine) > n:
+                eng.remove(mine.pop(len(mine) // 2)[0])
+            while len(mine) < n:
+                e = edge or edges[len(mine) % len(edges)]
+                mine.append((eng.add(init[e], e), e))
+
+    for n, big in ((12, 0), (700, 0), (100, 1), (1100, 0), (40, 0), (400, 0)):
+        populate(n)
+        if big:
+            populate(n + 1, 40)
+        print(f"small boxes {n}, large {big}, fp32={fp32}", flush=True)
+        for eng in engines:
+            eng.step(2)
+        got = [eng.query([i for i, _ in mine]) for eng, mine in zip(engines, ids)]
+        for k in range(0, len(ids[0]), 7):
+            (i, e), (j, f) = ids[0][k], ids[1][k]
+            assert e == f and got[0][i] == got[1][j]
+            assert np.array_equal(engines[0].read(i).cpu().numpy(), engines[1].read(j).cpu().numpy()), f"{n}: edge {e}"
+    for eng in engines:
+        eng.close()

@@ -247,6 +247,10 @@ int main(int, char **argv)
         printf("%zu\n", fused_list(boxes, out));
         return 0;
     }
+    if (!strcmp(argv[1], "small")) {
+        printf("%d %d %d\n", small_edge(false), small_edge(true), small_apart(atoi(argv[2]), atoi(argv[3])));
+        return 0;
+    }
     int bad = 0;
     for (int t = 0; t < 400; t++) {
         const bool fp32 = t & 1, alike = t & 2, capped = t & 4;
@@ -302,6 +306,12 @@ def test_boxes_that_fill_the_gpu_keep_long_runs(work_list, n, e, fp32):
     """Runs of fewer than 16 planes (or a whole box) cost more window fills than they save here."""
     rows = -(-e // 24) if fp32 else -(-e // 16)
     assert int(work_list("few", n, e, fp32)) <= n * -(-e // 32) * (rows + 1) * max(1, -(-e // 12))
+
+
+@pytest.mark.parametrize("small,others,apart", [(0, 0, 0), (256, 0, 0), (257, 0, 1), (257, 1, 0), (512, 9, 0), (513, 9, 1)])
+def test_small_boxes_take_narrow_tiles_where_they_are_many(work_list, small, others, apart):
+    """More than one small box a CU, or two beside other boxes."""
+    assert work_list("small", small, others).split() == ["14", "16", str(apart)]
 
 
 @pytest.mark.parametrize("gain", [1.0, 1.02])
