@@ -20,24 +20,33 @@ namespace {
 // What bounds it: at small boxes latency, so the index arithmetic is 32-bit with
 // precomputed quotients; at large ones the x ghosts, whose four-cell pieces touch
 // two 128-byte lines per row and component.
-struct Shell {
+//
+// N counts the cells: 32 bits, or 64 with ordinary division for the long thin boxes of the
+// free-standing fill that have 2^32 ghost cells or more.
+template <typename N>
+struct ShellOf {
     FastDiv g0, g1, n1, nbx, nby;
-    unsigned plane_rows, elems_a, total;  // rows of the ghost planes; cells of the full rows; all cells
+    N plane_rows, elems_a, total;  // rows of the ghost planes; cells of the full rows; all cells
 };
+using Shell = ShellOf<unsigned>;
 
-inline Shell make_shell(const Geom &g, const int nb[3])
+template <typename N = unsigned>
+inline ShellOf<N> make_shell(const Geom &g, const int nb[3])
 {
-    Shell h;
+    ShellOf<N> h;
     h.g0 = fast_div(g.g0);
     h.g1 = fast_div(g.g1);
     h.n1 = fast_div(g.n1);
     h.nbx = fast_div(nb[0]);
     h.nby = fast_div(nb[1]);
-    h.plane_rows = 2u * NG * g.g1;
-    h.elems_a = (h.plane_rows + 2u * NG * g.n2) * g.g0;
-    h.total = h.elems_a + 2u * NG * (unsigned)g.n1 * g.n2;
+    h.plane_rows = (N)(2 * NG) * g.g1;
+    h.elems_a = (h.plane_rows + (N)(2 * NG) * g.n2) * g.g0;
+    h.total = h.elems_a + (N)(2 * NG) * g.n1 * g.n2;
     return h;
 }
+
+__host__ __device__ __forceinline__ unsigned quotient(unsigned n, const FastDiv &by) { return by.div(n); }
+__host__ __device__ __forceinline__ uint64_t quotient(uint64_t n, const FastDiv &by) { return n / by.d; }
 
 inline int64_t shell_cells(const Geom &g)
 {
@@ -45,13 +54,14 @@ inline int64_t shell_cells(const Geom &g)
 }
 
 // Ghost cell e of the enumeration, as (i, j, k).
-__device__ __forceinline__ void shell_cell(const Geom &g, const Shell &h, unsigned e, int &i, int &j, int &k)
+template <typename N>
+__host__ __device__ __forceinline__ void shell_cell(const Geom &g, const ShellOf<N> &h, N e, int &i, int &j, int &k)
 {
     if (e < h.elems_a) {
-        unsigned r = h.g0.div(e);
+        N r = quotient(e, h.g0);
         i = (int)(e - r * g.g0);
         if (r < h.plane_rows) {
-            const int kk = (int)h.g1.div(r);
+            const int kk = (int)quotient(r, h.g1);
             j = (int)r - kk * g.g1;
             k = kk < NG ? kk : g.n2 + kk;
         } else {
@@ -61,7 +71,7 @@ __device__ __forceinline__ void shell_cell(const Geom &g, const Shell &h, unsign
             j = jj < NG ? jj : g.n1 + jj;
         }
     } else {
-        const unsigned e2 = e - h.elems_a, row = e2 / (2 * NG), kk = h.n1.div(row);
+        const N e2 = e - h.elems_a, row = e2 / (2 * NG), kk = quotient(row, h.n1);
         const int ii = (int)(e2 & (2 * NG - 1));
         i = ii < NG ? ii : g.n0 + ii;
         k = NG + (int)kk;
@@ -80,9 +90,9 @@ __device__ __forceinline__ int image(int a, int I, int n, int nb, int &dI)
 
 // Ghost cell e of box b of a set of nb[0] x nb[1] x nb[2] boxes (one box: its own images).  Q:
 // the components of q as well.  u_x: u's x ghosts of the interior rows too.
-template <bool Q>
-__device__ __forceinline__ void fill_cell(const Geom &g, const Shell &h, const BoxSet &bs, int nbx, int nby, int nbz,
-                                          unsigned e, unsigned b, double *u, double *q, bool u_x = true)
+template <bool Q, typename N>
+__device__ __forceinline__ void fill_cell(const Geom &g, const ShellOf<N> &h, const BoxSet &bs, int nbx, int nby, int nbz,
+                                          N e, unsigned b, double *u, double *q, bool u_x = true)
 {
     const unsigned r = h.nbx.div(b);
     const int K = (int)h.nby.div(r), J = (int)r - K * nby, I = (int)b - (int)r * nbx;

@@ -37,6 +37,16 @@ fill_kernel(Geom g, Shell h, BoxSet bs, int nbx, int nby, int nbz, double *__res
     if (e < h.total) fill_cell<Q>(g, h, bs, nbx, nby, nbz, e, blockIdx.y, u, q);
 }
 
+// 2^32 ghost cells of a box and more
+template <bool Q>
+__global__ void __launch_bounds__(kStreamBlock)
+fill_long_kernel(Geom g, ShellOf<uint64_t> h, BoxSet bs, int nbx, int nby, int nbz, double *__restrict__ u,
+                 double *__restrict__ q)
+{
+    for (uint64_t e = (uint64_t)blockIdx.x * kStreamBlock + threadIdx.x; e < h.total; e += (uint64_t)gridDim.x * kStreamBlock)
+        fill_cell<Q>(g, h, bs, nbx, nby, nbz, e, blockIdx.y, u, q);
+}
+
 // -------------------------------------------------------------------- courno
 __global__ void courno_reset_kernel(unsigned long long *acc, double init)
 {
@@ -357,8 +367,16 @@ diffterm_direct_kernel(Geom g, const double *__restrict__ q, double *__restrict_
 hipError_t launch_domain_fill(const Geom &g, const BoxSet &bs, const int nb[3], double *u, double *q, hipStream_t s)
 {
     const int64_t total = shell_cells(g);
-    if (bs.n != nb[0] * nb[1] * nb[2] || bs.n < 1 || bs.n > 65535 || total > 0xffffffffll - kStreamBlock)
-        return hipErrorInvalidValue;
+    if (bs.n != nb[0] * nb[1] * nb[2] || bs.n < 1 || bs.n > 65535) return hipErrorInvalidValue;
+    if (total > 0xffffffffll - kStreamBlock) {
+        const ShellOf<uint64_t> h = make_shell<uint64_t>(g, nb);
+        const dim3 grid(1u << 16, (unsigned)bs.n);
+        if (q)
+            fill_long_kernel<true><<<grid, kStreamBlock, 0, s>>>(g, h, bs, nb[0], nb[1], nb[2], u, q);
+        else
+            fill_long_kernel<false><<<grid, kStreamBlock, 0, s>>>(g, h, bs, nb[0], nb[1], nb[2], u, nullptr);
+        return hipGetLastError();
+    }
     const Shell h = make_shell(g, nb);
     const dim3 grid((unsigned)((total + kStreamBlock - 1) / kStreamBlock), (unsigned)bs.n);
     if (q)

@@ -61,3 +61,34 @@ def test_rk_update_equals_torch(device, n, phase):
     ops.rk_update(phase, lay.lo, lay.hi, NG, U, Unew, D, F, dt)
     torch.cuda.synchronize()
     assert torch.equal(U, u0) and torch.equal(Unew, w0)
+
+
+def test_fill_boundary_of_more_than_32_bits_of_ghost_cells(device):
+    """A long thin box whose ghost cells do not fit 32 bits (2^32 + 1152 of them; 193 GB): every ghost
+    cell holds its periodic image."""
+    import torch
+    torch.cuda.empty_cache()
+    n = (1 << 25, 4, 4)
+    lay = BoxLayout(n)
+    if torch.cuda.mem_get_info()[0] < lay.ghosted_len(NC) * 8 + (4 << 30):
+        pytest.skip("needs 198 GB of free GPU memory")
+    g = lay.dimg
+    U = torch.full((lay.ghosted_len(NC),), float("nan"), dtype=torch.float64, device=device)
+    v = U.view(NC, g[2], g[1], lay.xg)
+    x = torch.arange(n[0], dtype=torch.float64, device=device)
+    rows = {}
+    for l in range(NC):
+        for k in range(n[2]):
+            for j in range(n[1]):
+                rows[l, k, j] = 1e8 * (1 + j + n[1] * (k + n[2] * l))
+                torch.add(x, rows[l, k, j], out=v[l, NG + k, NG + j, NG:NG + n[0]])
+    print("fill_boundary of 2^25 x 4 x 4", flush=True)
+    ops.fill_boundary(U, lay.n, lay.dimg)
+    torch.cuda.synchronize()
+    want = torch.cat([x[-NG:], x, x[:NG]])
+    for l in range(NC):
+        for k in range(g[2]):
+            for j in range(g[1]):
+                assert torch.equal(v[l, k, j, :g[0]], want + rows[l, (k - NG) % n[2], (j - NG) % n[1]]), (l, k, j)
+    del U, v, x, want
+    torch.cuda.empty_cache()

@@ -10,11 +10,11 @@ from conftest import ROOT
 CSRC = os.path.join(ROOT, "cns_nospec_amd", "csrc")
 
 
-def compiled(tmp_path_factory, name, source):
+def compiled(tmp_path_factory, name, source, compiler=("g++", "-Wall", "-Werror")):
     folder = tmp_path_factory.mktemp(name)
     src, exe = folder / f"{name}.cpp", folder / name
     src.write_text(source)
-    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", f"-I{CSRC}", "-o", str(exe), str(src)], check=True)
+    subprocess.run([*compiler, "-std=c++17", "-O2", f"-I{CSRC}", "-o", str(exe), str(src)], check=True)
 
     def run(*args):
         return subprocess.run([str(exe), *map(str, args)], check=True, capture_output=True, text=True).stdout
@@ -312,6 +312,56 @@ def test_boxes_that_fill_the_gpu_keep_long_runs(work_list, n, e, fp32):
 def test_small_boxes_take_narrow_tiles_where_they_are_many(work_list, small, others, apart):
     """More than one small box a CU, or two beside other boxes."""
     assert work_list("small", small, others).split() == ["14", "16", str(apart)]
+
+
+# The enumeration of the ghost cells (cns_fill.h) in 32 and in 64 bits: every ghost cell of a box once,
+# in the same order; and the last cells of a box with more than 2^32 of them.
+SHELL = r"""
+#include <cstdio>
+#include <vector>
+#include "cns_fill.h"
+using namespace cns;
+
+int main()
+{
+    long bad = 0;
+    const int sizes[][3] = {{4, 4, 4}, {5, 4, 7}, {16, 16, 16}, {33, 9, 5}, {4, 61, 4}, {70, 4, 21}};
+    for (const auto &n : sizes) {
+        const Geom g = make_geom(n[0], n[1], n[2]);
+        const Shell h = make_shell(g, kOneBox);
+        const ShellOf<uint64_t> w = make_shell<uint64_t>(g, kOneBox);
+        std::vector<int> seen((size_t)g.g0 * g.g1 * g.g2);
+        bad += h.total != w.total || (int64_t)h.total != shell_cells(g);
+        for (unsigned e = 0; e < h.total; e++) {
+            int i, j, k, a, b, c;
+            shell_cell(g, h, e, i, j, k);
+            shell_cell(g, w, (uint64_t)e, a, b, c);
+            bad += i != a || j != b || k != c || i < 0 || j < 0 || k < 0 || i >= g.g0 || j >= g.g1 || k >= g.g2;
+            seen[((size_t)k * g.g1 + j) * g.g0 + i]++;
+        }
+        for (int k = 0; k < g.g2; k++)
+            for (int j = 0; j < g.g1; j++)
+                for (int i = 0; i < g.g0; i++) {
+                    const bool in = i >= NG && i < g.n0 + NG && j >= NG && j < g.n1 + NG && k >= NG && k < g.n2 + NG;
+                    bad += seen[((size_t)k * g.g1 + j) * g.g0 + i] != !in;
+                }
+    }
+    const Geom g = make_geom(1 << 25, 4, 4);
+    const ShellOf<uint64_t> w = make_shell<uint64_t>(g, kOneBox);
+    int i, j, k;
+    shell_cell(g, w, w.elems_a - 1, i, j, k);  // the last full row: the upper y ghosts of the last interior plane
+    bad += w.total != (1ull << 32) + 1152 || i != g.g0 - 1 || j != g.g1 - 1 || k != g.n2 + NG - 1;
+    shell_cell(g, w, w.total - 1, i, j, k);  // the upper x ghosts of the last interior row
+    bad += i != g.g0 - 1 || j != g.n1 + NG - 1 || k != g.n2 + NG - 1;
+    printf("%ld\n", bad);
+}
+"""
+
+
+def test_ghost_cells_are_enumerated_once_in_32_and_64_bits(tmp_path_factory):
+    from cns_nospec_amd import build
+    shell = compiled(tmp_path_factory, "shell", SHELL, (build.hipcc(), "-x", "hip", f"--offload-arch={build.ARCH}"))
+    assert int(shell()) == 0
 
 
 @pytest.mark.parametrize("gain", [1.0, 1.02])
