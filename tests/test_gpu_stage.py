@@ -147,3 +147,121 @@ def test_tall_columns_take_the_separate_kernels(device, n, separate):
     assert dts == rdts
     for a, b, name in zip(arrays, rarrays, ("U", "Unew", "Q", "D", "F")):
         assert np.array_equal(a, b), name
+
+
+NAMES = ("U", "Unew", "Q", "D", "F")
+
+
+def stepped(device, n, impl=_lib.CNS_IMPL_TILED, fused=True, off=(), steps=3):
+    """dt of each step and the arrays after it; `off`: arrays that begin 8 bytes past an alignment of 16."""
+    import torch
+    lay = BoxLayout(n)
+    arrays = [torch.zeros(a.numel() + 1, dtype=a.dtype, device=device)[1:] if name in off else a
+              for name, a in zip(NAMES, ops.allocate_variables(lay, device))]
+    arrays[0].copy_(torch.from_numpy(sinusoid_state(lay, 29, mach=0.25, kmax=3)).to(device))
+    ops.set_stencil_impl(impl)
+    st = ops.Stepper(lay)
+    try:
+        st.set_fused(fused)
+        return [st.new_advance(*arrays) for _ in range(steps)], [a.cpu().numpy() for a in arrays]
+    finally:
+        ops.set_stencil_impl(_lib.CNS_IMPL_TILED)
+        st.close()
+
+
+def same(a, b):
+    assert a[0] == b[0]
+    for x, y, name in zip(a[1], b[1], NAMES):
+        assert np.array_equal(x, y), name
+
+
+@pytest.mark.parametrize("tx", ["32", "64"])
+@pytest.mark.parametrize("off", [(name,) for name in NAMES] + [NAMES])
+def test_step_with_arrays_off_the_alignment(device, monkeypatch, off, tx):
+    """Arrays that are not all 16-byte aligned take the separate kernels: with Unew alone off it, stage 1
+    still takes the pipelined ones, with the update in hypterm's pass (32- and 64-wide tiles)."""
+    monkeypatch.setenv("CNS_HYP_TX", tx)
+    monkeypatch.setenv("CNS_DIFF_TX", tx)
+    n = (70, 33, 21)
+    print(f"step off alignment {off} tx={tx}", flush=True)
+    same(stepped(device, n, off=off), stepped(device, n, impl=_lib.CNS_IMPL_DIRECT, fused=False))
+
+
+@pytest.mark.parametrize("n", [(4, 4, 4), (20, 6, 5), (65, 17, 130), (129, 9, 31)])
+def test_wide_tiles_of_the_separate_kernels(device, monkeypatch, n):
+    """The 64-wide tiles of the pipelined stencils, which the unfused step runs on request."""
+    monkeypatch.setenv("CNS_HYP_TX", "64")
+    monkeypatch.setenv("CNS_DIFF_TX", "64")
+    print(f"wide tiles n={n}", flush=True)
+    same(stepped(device, n, fused=False), stepped(device, n, impl=_lib.CNS_IMPL_DIRECT, fused=False))
+
+
+@pytest.mark.parametrize("first", ["staged", "misaligned"])
+def test_courant_maximum_of_the_separate_fused_kernels(device, monkeypatch, first):
+    """The step that arrays off the alignment (or CNS_PIPE=0) take leaves the Courant maximum at zero
+    too, and finds it there after a stage-kernel step."""
+    import torch
+    lay = BoxLayout((20, 18, 9))
+
+    def fresh(mach, off=False):
+        arrays = ops.allocate_variables(lay, device)
+        if off:
+            arrays = [torch.zeros(a.numel() + 1, dtype=a.dtype, device=device)[1:] for a in arrays]
+        arrays[0].copy_(torch.from_numpy(sinusoid_state(lay, 5, mach=mach, kmax=2)).to(device))
+        return arrays
+
+    def step(st, route, mach):
+        print(f"courant maximum route={route}", flush=True)
+        monkeypatch.setenv("CNS_PIPE", "0" if route == "staged" else "1")
+        return st.new_advance(*fresh(mach, route == "misaligned"))
+
+    ref = ops.Stepper(lay)
+    want_fast, want_slow = step(ref, "stage", 0.9), step(ref, "stage", 0.01)
+    ref.close()
+    assert want_slow > want_fast
+    st = ops.Stepper(lay)
+    for route in (first, "stage", "staged", "misaligned", first):
+        assert step(st, route, 0.9) == want_fast
+        assert step(st, "stage", 0.01) == want_slow
+        assert step(st, "stage", 0.9) == want_fast
+        assert step(st, route, 0.01) == want_slow
+    st.close()
+
+
+@pytest.mark.parametrize("captured", [False, True])
+def test_first_step_does_not_take_what_the_memory_held(device, captured):
+    """A context's words come from memory that held a large finite number (blocks of their size, filled
+    and freed just before): its first step, eager or in a graph, gets the dt of the state."""
+    import ctypes as C
+    import torch
+    lay = BoxLayout((8, 6, 5))
+
+    def fresh():
+        arrays = ops.allocate_variables(lay, device)
+        arrays[0].copy_(torch.from_numpy(sinusoid_state(lay, 5, mach=0.01, kmax=2)).to(device))
+        torch.cuda.synchronize()
+        return arrays
+
+    ref = ops.Stepper(lay)
+    want = ref.new_advance(*fresh())
+    arrays, dt = fresh(), torch.zeros(1, dtype=torch.float64, device=device)
+    lib = _lib.load()  # (the HIP runtime is among its dependencies)
+    blocks = [C.c_void_p() for _ in range(64)]
+    for b in blocks:
+        assert lib.hipMalloc(C.byref(b), C.c_size_t(32)) == 0
+        assert lib.hipMemset(b, 0x43, C.c_size_t(32)) == 0  # 1.1e16 as a double
+    torch.cuda.synchronize()
+    for b in blocks:
+        assert lib.hipFree(b) == 0
+    st = ops.Stepper(lay)
+    if captured:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            st.advance_async(*arrays, dt)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float(dt) == want
+    else:
+        assert st.new_advance(*arrays) == want
+    st.close()
+    ref.close()
