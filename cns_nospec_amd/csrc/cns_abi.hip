@@ -197,20 +197,18 @@ hipError_t stencil_hypterm(const Geom &g, const double *cons, const double *q, d
     if (g_stencil_impl == CNS_IMPL_DIRECT)
         return launch_hypterm_direct(g, cons, q, flux, dxi[0], dxi[1], dxi[2], s);
     if (pipe_on({cons, q, flux}))
-        return launch_hypterm_pipe(g, cons, q, flux, dxi[0], dxi[1], dxi[2], nullptr, nullptr,
-                                   nullptr, nullptr, 0, true, s);
+        return launch_hypterm_pipe(g, cons, q, flux, dxi, s);
     return launch_hypterm_tiled(g, cons, q, flux, dxi[0], dxi[1], dxi[2], s);
 }
 
-// write_f: whether F must hold this stage's flux afterwards (only the last stage's
-// F is an output of the step; the register-staged kernel always stores it).
+// hypterm with the RK update of its cell in the same pass: stage 1 (base = cons) pipelined where its arrays
+// are aligned, without storing F, which stage 3 overwrites; else the register-staged kernel.
 hipError_t stencil_hypterm_rk(const Geom &g, const double *cons, const double *q, double *flux,
                               const double dxi[3], const double *d, const double *base, double *out,
-                              const double *dt, int phase, bool write_f, hipStream_t s)
+                              const double *dt, int phase, hipStream_t s)
 {
-    if (pipe_on({cons, q, flux, d, base, out}))
-        return launch_hypterm_pipe(g, cons, q, flux, dxi[0], dxi[1], dxi[2], d, base, out, dt, phase,
-                                   write_f, s);
+    if (phase == 1 && base == cons && pipe_on({cons, q, d, out}))
+        return launch_hypterm_pipe_rk1(g, cons, q, dxi, d, out, dt, s);
     return launch_hypterm_rk(g, cons, q, flux, dxi[0], dxi[1], dxi[2], d, base, out, dt, phase, s);
 }
 
@@ -569,17 +567,17 @@ static int enqueue_step(cns_ctx *ctx, double *U, double *Unew, double *Q, double
         TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, U, Q, ctx->d_acc, ctx->dx[0], ctx->dx[1], ctx->dx[2], s));
         HIPCHK(launch_courno_to_dt(sd, s));
         TIMED(ctx, CNS_PROF_DIFFTERM, s, stencil_diffterm(g, Q, D, ctx->dxi, ctx->eta, ctx->alam, ctx->d_wz, s));
-        TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, U, Q, F, ctx->dxi, D, U, T, dt, 1, false, s));
+        TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, U, Q, F, ctx->dxi, D, U, T, dt, 1, s));
 
         TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, T, nullptr, s));
         TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, T, Q, nullptr, 0.0, 0.0, 0.0, s));
         TIMED(ctx, CNS_PROF_DIFFTERM, s, stencil_diffterm(g, Q, D, ctx->dxi, ctx->eta, ctx->alam, ctx->d_wz, s));
-        TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, T, Q, F, ctx->dxi, D, U, Unew, dt, 2, false, s));
+        TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, T, Q, F, ctx->dxi, D, U, Unew, dt, 2, s));
 
         TIMED(ctx, CNS_PROF_FILL, s, launch_fill_boundary(g, Unew, nullptr, s));
         TIMED(ctx, CNS_PROF_CTOPRIM, s, launch_ctoprim(g, Unew, Q, nullptr, 0.0, 0.0, 0.0, s));
         TIMED(ctx, CNS_PROF_DIFFTERM, s, stencil_diffterm(g, Q, D, ctx->dxi, ctx->eta, ctx->alam, ctx->d_wz, s));
-        TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, Unew, Q, F, ctx->dxi, D, U, U, dt, 3, true, s));
+        TIMED(ctx, CNS_PROF_HYPTERM_RK, s, stencil_hypterm_rk(g, Unew, Q, F, ctx->dxi, D, U, U, dt, 3, s));
         return CNS_OK;
     }
     // Unfused composition, kernel for kernel as the reference (also for tall columns of a few cells).

@@ -38,9 +38,8 @@ hipError_t launch_domain_fill(const Geom &g, const BoxSet &bs, const int nb[3], 
 hipError_t launch_courno_reset(unsigned long long *acc, double init, hipStream_t s);
 
 // ctoprim over the ghosted box; acc != nullptr adds the Courant max reduction.
-// full = false stores only u, v, w and T (what diffterm reads), not rho and p.
 hipError_t launch_ctoprim(const Geom &g, const double *u, double *q, unsigned long long *acc,
-                          double dx0, double dx1, double dx2, hipStream_t s, bool full = true);
+                          double dx0, double dx1, double dx2, hipStream_t s);
 
 // The device words and the pinned host words of a StepDt.  step_dt_begin() before each step clears
 // acc while it is fresh, that is until a step has run outside a capture (a captured first step
@@ -76,16 +75,14 @@ hipError_t launch_diffterm_tiled(const Geom &g, const double *q, double *difflux
                                  double dxi1, double dxi2, double eta, double alam, hipStream_t s);
 
 // DMA-pipelined z-marching stencils (cns_stencil_pipe.hip).  Every array must be
-// 16-byte aligned (pipe_aligned).  hypterm: phase 0 is plain hypterm, 1..3 fuse the
-// RK stage update as launch_hypterm_rk (phase 1 with base == cons takes the direct
-// form); write_f = false skips storing flux (for a stage whose F is overwritten
-// later).  diffterm reads wz, a one-component ghosted array filled by launch_wz from
-// the same q.
+// 16-byte aligned (pipe_aligned).  diffterm reads wz, a one-component ghosted array filled by
+// launch_wz from the same q.
 bool pipe_aligned(const void *p);
-hipError_t launch_hypterm_pipe(const Geom &g, const double *cons, const double *q, double *flux,
-                               double dxi0, double dxi1, double dxi2, const double *d,
-                               const double *base, double *out, const double *dt_dev, int phase,
-                               bool write_f, hipStream_t s);
+hipError_t launch_hypterm_pipe(const Geom &g, const double *cons, const double *q, double *flux, const double dxi[3],
+                               hipStream_t s);
+// The same with stage 1's update in place of storing the flux: out = cons + dt (d + flux).
+hipError_t launch_hypterm_pipe_rk1(const Geom &g, const double *cons, const double *q, const double dxi[3],
+                                   const double *d, double *out, const double *dt_dev, hipStream_t s);
 hipError_t launch_wz(const Geom &g, const double *q, double *wz, double dxi2, hipStream_t s);
 hipError_t launch_diffterm_pipe(const Geom &g, const double *q, const double *wz, double *difflux,
                                 double dxi0, double dxi1, double dxi2, double eta, double alam,

@@ -72,7 +72,7 @@ __global__ void courno_to_dt_kernel(StepDt sd)
 template <bool COURNO>
 __global__ void __launch_bounds__(kStreamBlock)
 ctoprim_kernel(Geom g, const double *__restrict__ u, double *__restrict__ q,
-               unsigned long long *__restrict__ acc, double dx0, double dx1, double dx2, bool full)
+               unsigned long long *__restrict__ acc, double dx0, double dx1, double dx2)
 {
     const int64_t total = (int64_t)g.g2 * g.pg;
     const int64_t cg = g.cg;
@@ -85,11 +85,11 @@ ctoprim_kernel(Geom g, const double *__restrict__ u, double *__restrict__ q,
         const double rho = u[e];
         double qu, qv, qw, eint, p;
         ctoprim_cell(rho, u[e + cg], u[e + 2 * cg], u[e + 3 * cg], u[e + 4 * cg], qu, qv, qw, eint, p);
-        if (full) q[e] = rho;
+        q[e] = rho;
         q[e + cg] = qu;
         q[e + 2 * cg] = qv;
         q[e + 3 * cg] = qw;
-        if (full) q[e + 4 * cg] = p;
+        q[e + 4 * cg] = p;
         q[e + 5 * cg] = eint / CV;
         if (COURNO) {
             const int k = (int)(row / g.g1);
@@ -421,14 +421,14 @@ hipError_t launch_fill_courno(const Geom &g, double *u, unsigned long long *acc,
 }
 
 hipError_t launch_ctoprim(const Geom &g, const double *u, double *q, unsigned long long *acc,
-                          double dx0, double dx1, double dx2, hipStream_t s, bool full)
+                          double dx0, double dx1, double dx2, hipStream_t s)
 {
     const int64_t total = (int64_t)g.g2 * g.pg;
     const int grid = stream_grid(total, 8);
     if (acc)
-        ctoprim_kernel<true><<<grid, kStreamBlock, 0, s>>>(g, u, q, acc, dx0, dx1, dx2, full);
+        ctoprim_kernel<true><<<grid, kStreamBlock, 0, s>>>(g, u, q, acc, dx0, dx1, dx2);
     else
-        ctoprim_kernel<false><<<grid, kStreamBlock, 0, s>>>(g, u, q, nullptr, dx0, dx1, dx2, full);
+        ctoprim_kernel<false><<<grid, kStreamBlock, 0, s>>>(g, u, q, nullptr, dx0, dx1, dx2);
     return hipGetLastError();
 }
 

@@ -1,6 +1,5 @@
 // cns_pipe_tile.h -- pieces shared by the z-marching, DMA-staged stencil kernels (internal):
-// the difference sum, the XCD-aware tile order, direct-to-LDS loads of a haloed tile and the
-// stage update with its stores.
+// the difference sum, the XCD-aware tile order and direct-to-LDS loads of a haloed tile.
 #pragma once
 
 #include "cns_kernels.h"
@@ -66,26 +65,6 @@ __device__ __forceinline__ void dma_plane_s(const double *const (&src)[NF], int6
         const int n0 = (wave - f) & (S::NW - 1);
         dma_block_s<S>(src[f] + plane, buf + f * S::TILE, n0, t, lane);
         if (n0 + S::NW < S::NDMA) dma_block_s<S>(src[f] + plane, buf + f * S::TILE, n0 + S::NW, t, lane);
-    }
-}
-
-// The stage update of the cell and its stores (STAGE1: cons + dt(D+F), the reference's
-// form of cpu/advance.cpp:82; later stages ra*base + rb*(cons + dt(D+F)), which is
-// 3/4 base + 1/4(..) and 1/3 base + 2/3(..) of :114-116, :148-150).
-template <bool STAGE1, bool WRITE_F>
-__device__ __forceinline__ void rk_store(const double (&F)[5], const double (&uc)[5], const double (&rkd)[5],
-                                         const double (&rkb)[5], double ra, double rb, double dt,
-                                         double *flux, int64_t fo, int64_t c, double *out, int64_t zo,
-                                         int64_t cg, double (&o)[5])
-{
-    if (WRITE_F) {
-#pragma unroll
-        for (int l = 0; l < NC; l++) flux[l * c + fo] = F[l];
-    }
-#pragma unroll
-    for (int l = 0; l < NC; l++) {
-        o[l] = STAGE1 ? uc[l] + dt * (rkd[l] + F[l]) : ra * rkb[l] + rb * (uc[l] + dt * (rkd[l] + F[l]));
-        out[l * cg + zo] = o[l];
     }
 }
 

@@ -39,25 +39,20 @@ namespace cns {
 namespace {
 
 struct PipeRk {
-    const double *d;     // difflux (interior)
-    const double *base;  // U^n (ghosted), phases 2 and 3
-    double *out;         // result (ghosted); must not alias cons
-    const double *dt;    // device dt
-    int phase;           // 0: plain hypterm
+    const double *d;   // difflux (interior)
+    double *out;       // result (ghosted); must not alias cons
+    const double *dt;  // device dt
 };
 
 // ======================================================================= hypterm
 // LDS fields (centre plane): mx, my, mz, E, p, u, v.  Register windows: mx, my, mz,
-// E, w, p.  With RK the stage update of the cell is applied as in cns_stencil.hip,
-// with three savings of HBM traffic that leave every result bit-identical:
-//  * D_rho is not read: diffterm always stores 0.0 there (cpu/diffterm.cpp:63-68);
-//  * STAGE1: the base is cons itself, so the update is cons + dt*(D+F), the
-//    reference's own form (cpu/advance.cpp:82), without re-reading the base;
-//  * !WRITE_F: flux is not stored (stages 1 and 2 of a step, whose F the third
-//    stage overwrites).
+// E, w, p.  With RK the update of stage 1, cons + dt (D + F) (cpu/advance.cpp:82), takes the place of
+// storing F, which stage 3 overwrites: a step of which only Unew or F is not 16-byte aligned runs it
+// (cns_stencil.hip has the others).  D_rho is not read: diffterm always stores 0.0 there
+// (cpu/diffterm.cpp:63-68).
 enum { HMX = 0, HMY, HMZ, HE, HP, HU, HV, HNF };
 
-template <class S, bool RK, bool STAGE1, bool WRITE_F>
+template <class S, bool RK>
 __global__ void __launch_bounds__(S::NT, 2)
 hypterm_pipe_kernel(Geom g, const double *__restrict__ cons, const double *__restrict__ q,
                     double *__restrict__ flux, double dxi0, double dxi1, double dxi2, int kz,
@@ -82,15 +77,7 @@ hypterm_pipe_kernel(Geom g, const double *__restrict__ cons, const double *__res
     const double *const src[HNF] = {c_mx, c_my, c_mz, c_E, q_p, q_u, q_v};
     const int64_t own = (int64_t)gj * g.xg + gi;
     const int me = (row + 4) * PX_ + col + 4;
-    double dt = 0.0, ra = 0.0, rb = 1.0;
-    if (RK) {
-        // r = ra*base + rb*(cons + dt*(D+F)) with (ra, rb) = (0, 1), (3/4, 1/4), (1/3, 2/3):
-        // 0*base + 1*x is exactly x, so each phase keeps the reference's rounding
-        // (cpu/advance.cpp:82, :114-116, :148-150)
-        dt = rk.dt[0];
-        ra = rk.phase == 1 ? 0.0E0 : (rk.phase == 2 ? ThreeQuarters : OneThird);
-        rb = rk.phase == 1 ? 1.0E0 : (rk.phase == 2 ? OneQuarter : TwoThirds);
-    }
+    const double dt = RK ? rk.dt[0] : 0.0;
 
     // first plane's tiles in flight while the windows fill
     dma_plane_s<S, HNF>(src, (int64_t)(kbeg + NG) * pg, (lds_double *)sm, td, wave, lane);
@@ -122,15 +109,12 @@ hypterm_pipe_kernel(Geom g, const double *__restrict__ cons, const double *__res
             nmx = c_mx[o]; nmy = c_my[o]; nmz = c_mz[o]; nE = c_E[o]; nw = q_w[o]; np = q_p[o];
         }
         const int64_t fo = iidx(g, gi - NG, gj - NG, k);
-        double rkd[5], rkb[5], rho_c = 0.0;
+        double rkd[5], rho_c = 0.0;
         if (RK && active) {
             rho_c = cons[zo];
             rkd[IRHO] = 0.0E0;
 #pragma unroll
-            for (int l = 0; l < NC; l++) {
-                if (l != IRHO) rkd[l] = rk.d[l * g.c + fo];
-                if (!STAGE1) rkb[l] = rk.base[l * cg + zo];
-            }
+            for (int l = 1; l < NC; l++) rkd[l] = rk.d[l * g.c + fo];
         }
 
         // (cells past the box are computed too, for nothing: no divergent branch around the taps)
@@ -197,13 +181,13 @@ hypterm_pipe_kernel(Geom g, const double *__restrict__ cons, const double *__res
         // need not wait for them.
         __builtin_amdgcn_s_waitcnt(0xF70);
         if (active) {
-            if (RK) {
-                const double uc[5] = {rho_c, wmx[4], wmy[4], wmz[4], wE[4]};
-                double o[5];
-                rk_store<STAGE1, WRITE_F>(F, uc, rkd, rkb, ra, rb, dt, flux, fo, g.c, rk.out, zo, cg, o);
-            } else {
+            const double uc[5] = {rho_c, wmx[4], wmy[4], wmz[4], wE[4]};
 #pragma unroll
-                for (int l = 0; l < NC; l++) flux[l * g.c + fo] = F[l];
+            for (int l = 0; l < NC; l++) {
+                if (RK)
+                    rk.out[l * cg + zo] = uc[l] + dt * (rkd[l] + F[l]);
+                else
+                    flux[l * g.c + fo] = F[l];
             }
         }
 #pragma unroll
@@ -528,24 +512,15 @@ bool wide_tiles(const char *var)
 
 template <class S>
 hipError_t launch_hyp_pipe_shape(const Geom &g, const double *cons, const double *q, double *flux, double dxi0,
-                                 double dxi1, double dxi2, const double *d, const double *base, double *out,
-                                 const double *dt_dev, int phase, bool write_f, hipStream_t s)
+                                 double dxi1, double dxi2, const PipeRk &rk, hipStream_t s)
 {
     const int ntx = (g.n0 + S::TX - 1) / S::TX, nty = (g.n1 + S::BY - 1) / S::BY;
     const int kz = pipe_kz(g, (int64_t)ntx * nty, S::TX == 32 ? 512 : 256, 1);
     const int nb = ntx * nty * ((g.n2 + kz - 1) / kz);
-    PipeRk rk{d, base, out, dt_dev, phase};
-    const bool stage1 = phase == 1 && base == cons;
-#define HYP_PIPE(RK, S1, WF)                                                                              \
-    hypterm_pipe_kernel<S, RK, S1, WF><<<nb, S::NT, 0, s>>>(g, cons, q, flux, dxi0, dxi1, dxi2, kz, ntx, nty, \
-                                                            rk)
-    if (!phase)
-        HYP_PIPE(false, false, true);
-    else if (stage1)
-        write_f ? HYP_PIPE(true, true, true) : HYP_PIPE(true, true, false);
+    if (rk.out)
+        hypterm_pipe_kernel<S, true><<<nb, S::NT, 0, s>>>(g, cons, q, flux, dxi0, dxi1, dxi2, kz, ntx, nty, rk);
     else
-        write_f ? HYP_PIPE(true, false, true) : HYP_PIPE(true, false, false);
-#undef HYP_PIPE
+        hypterm_pipe_kernel<S, false><<<nb, S::NT, 0, s>>>(g, cons, q, flux, dxi0, dxi1, dxi2, kz, ntx, nty, rk);
     return hipGetLastError();
 }
 
@@ -565,16 +540,24 @@ hipError_t launch_diffterm_shape(const Geom &g, const double *q, const double *w
 
 bool pipe_aligned(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
-hipError_t launch_hypterm_pipe(const Geom &g, const double *cons, const double *q, double *flux,
-                               double dxi0, double dxi1, double dxi2, const double *d,
-                               const double *base, double *out, const double *dt_dev, int phase,
-                               bool write_f, hipStream_t s)
+static hipError_t launch_hyp_pipe(const Geom &g, const double *cons, const double *q, double *flux, const double dxi[3],
+                                  const PipeRk &rk, hipStream_t s)
 {
     if (wide_tiles("CNS_HYP_TX"))
-        return launch_hyp_pipe_shape<Shape<64>>(g, cons, q, flux, dxi0, dxi1, dxi2, d, base, out, dt_dev, phase,
-                                                write_f, s);
-    return launch_hyp_pipe_shape<Shape<32>>(g, cons, q, flux, dxi0, dxi1, dxi2, d, base, out, dt_dev, phase,
-                                            write_f, s);
+        return launch_hyp_pipe_shape<Shape<64>>(g, cons, q, flux, dxi[0], dxi[1], dxi[2], rk, s);
+    return launch_hyp_pipe_shape<Shape<32>>(g, cons, q, flux, dxi[0], dxi[1], dxi[2], rk, s);
+}
+
+hipError_t launch_hypterm_pipe(const Geom &g, const double *cons, const double *q, double *flux, const double dxi[3],
+                               hipStream_t s)
+{
+    return launch_hyp_pipe(g, cons, q, flux, dxi, PipeRk{}, s);
+}
+
+hipError_t launch_hypterm_pipe_rk1(const Geom &g, const double *cons, const double *q, const double dxi[3],
+                                   const double *d, double *out, const double *dt_dev, hipStream_t s)
+{
+    return launch_hyp_pipe(g, cons, q, nullptr, dxi, PipeRk{d, out, dt_dev}, s);
 }
 
 hipError_t launch_wz(const Geom &g, const double *q, double *wz, double dxi2, hipStream_t s)

@@ -178,7 +178,7 @@ def same(a, b):
 @pytest.mark.parametrize("tx", ["32", "64"])
 @pytest.mark.parametrize("off", [(name,) for name in NAMES] + [NAMES])
 def test_step_with_arrays_off_the_alignment(device, monkeypatch, off, tx):
-    """Arrays that are not all 16-byte aligned take the separate kernels: with Unew alone off it, stage 1
+    """Arrays that are not all 16-byte aligned take the separate kernels: with Unew or F off it, stage 1
     still takes the pipelined ones, with the update in hypterm's pass (32- and 64-wide tiles)."""
     monkeypatch.setenv("CNS_HYP_TX", tx)
     monkeypatch.setenv("CNS_DIFF_TX", tx)
