@@ -69,3 +69,43 @@ def test_error_summaries():
     assert e["mx"]["rel_l2"] == pytest.approx(1e-7, rel=1e-6)
     w = bench.worst_errors([e, bench.field_errors(b, b)])
     assert w["mx"]["rel_l2"] == pytest.approx(1e-7, rel=1e-6)
+
+
+@pytest.mark.parametrize("n,wraps", [(16, True), (64, True), (384, True), (416, False), (512, False)])
+def test_step_minimum_is_the_sum_of_the_launches_it_takes(n, wraps):
+    """The step that runs: the fill of U with the Courant pass and three stages, and fills after stages 1
+    and 2 where the box is too large to be read at periodic addresses."""
+    g, c, w = (n + 8) ** 3, n ** 3, (n + 8) * n * n
+    start = 10 * (g - c) + 5 * c  # U's ghosts; the state once
+    if wraps:
+        s1 = 5 * g + 5 * c + 5 * (w - c)  # U over its halos; the result with its x ghosts
+        s2 = 5 * w + 5 * c + 5 * c + 6 * c + 5 * (w - c)  # rows and x halos, base; result, primitives, x ghosts
+        s3 = 5 * w + 5 * c + 5 * c + 10 * c + 2 * 5 * (g - w) + 2 * 6 * (g - c)  # base; U, D, F; ghosts of Unew and Q
+        fills = 0
+    else:
+        s1 = 5 * g + 5 * c
+        s2 = 5 * g + 5 * c + 5 * c + 6 * c
+        s3 = 5 * g + 5 * c + 5 * c + 10 * c
+        fills = 2 * 5 * (g - c) + 2 * 11 * (g - c)
+    assert bench.step_wraps(n) == wraps
+    assert bench.stage_bytes(n) == pytest.approx(8 * (s1 + s2 + s3) / 3, rel=1e-12)
+    assert bench.step_min_bytes(n) == pytest.approx(8 * (start + s1 + s2 + s3 + fills), rel=1e-12)
+
+
+def test_wrap_rule_is_the_library_s():
+    """step_wraps restates stage_wraps of cns_stage.hip: the same line, in the same units."""
+    import os
+    src = open(os.path.join(bench.ROOT, "cns_nospec_amd", "csrc", "cns_stage.hip")).read()
+    assert "((g.n0 + TX - 1) / TX) * ((g.n1 + BY - 1) / BY) * g.n2 <= 512 * kCUs" in src
+    assert "constexpr int kCUs = 256;" in src
+
+
+@pytest.mark.parametrize("edge,fills", [(64, 0), (512, 2)])
+def test_measured_step_traffic(edge, fills):
+    """The traffic of a step adds up the launches that the box's step has, and exceeds what they must move."""
+    t = bench.read_traffic
+    want = t("fill_courno", edge) + 3 * t("stage", edge) + (fills * t("fill", edge) if fills else 0)
+    got = bench.step_traffic({"hypterm_rk": (1.0, 3)}, edge)
+    assert got == pytest.approx(want, rel=1e-12)
+    assert t("stage", edge) > bench.stage_bytes(edge) and got > bench.step_min_bytes(edge)
+    assert bench.step_traffic({"hypterm_rk": (1.0, 3)}, 7) is None
