@@ -5,9 +5,9 @@
 // does not fit is refused, never an out-of-memory fault) and nothing is
 // allocated while stepping.  Box records (BoxDev) live in a device array indexed
 // by box id.  The work list holds every resident box's tiles, grouped by tile-
-// width class; a step (3 RK stages x {wz, diffterm, hypterm+update} per class, then
-// the dt finalize) is captured once into a hipGraph and replayed until the
-// resident set or the tile table changes.
+// width class; a step (3 RK stages, each one launch for the 32-wide class and {wz, diffterm,
+// hypterm+update} for every other, then the dt finalize) is captured once into a hipGraph
+// and replayed until the resident set or the tile table changes.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -86,8 +86,9 @@ struct BoxHost {
 int width_class(int w) { return w == 16 ? 0 : (w == 32 ? 1 : (w == 64 ? 2 : -1)); }
 
 // Default tile: 32-wide columns, so that all boxes share one width class and an RK stage is
-// one launch of the fused kernel, whose work list chooses the z runs.
-std::pair<int, int> default_tile(int e) { return {32, e}; }
+// one launch of the fused kernel, whose work list chooses the z runs; the separate kernels take runs
+// of 16 planes (of 8 or 32 they are 2 to 3 % slower, of whole boxes they leave CUs idle).
+std::pair<int, int> default_tile(int e, bool fused) { return {32, fused ? e : std::min(e, 16)}; }
 
 }  // namespace
 
@@ -132,7 +133,7 @@ struct cns_batch {
     std::pair<int, int> tile_of(int e) const
     {
         auto it = tune.find(e);
-        return it != tune.end() ? it->second : default_tile(e);
+        return it != tune.end() ? it->second : default_tile(e, fused());
     }
 };
 

@@ -33,7 +33,9 @@ struct TileDev {
 constexpr int kShortRows = 16, kTallRows = 24;  // tiles of the fused kernel (tall: FP32 flux only)
 constexpr int kXcds = 8, kCusPerXcd = 32;
 constexpr int kTallCost = 4, kShortCost = 3;  // of a plane
-constexpr size_t kMostSimulated = 1 << 14;  // tiles; a longer list's tail is short however it is split
+// Tiles, counted at runs of 12 planes, up to which the splits are compared; a longer list takes the first of
+// them: its tail is short however it is split, and the comparison would cost the host more than that.
+constexpr size_t kMostSimulated = 1 << 14;
 
 struct Split {
     int run, last, eighths;  // runs of `run` planes, and of `last` for so many eighths:

@@ -136,11 +136,12 @@ int cns_ctx_create(cns_ctx **ctx, const int ncells[3], const double dx[3],
 int cns_ctx_destroy(cns_ctx *ctx);
 
 /* Selects how cns_advance composes a stage.  fused = 1 (the default set by
- * cns_ctx_create): fill, ctoprim, diffterm, then hypterm with the RK update of each
- * cell applied in the same pass; the context then owns one ghosted 5-component
- * stage buffer (the U^{1/3} state), allocated here or at creation.  fused = 0:
- * kernel for kernel as the reference (separate hypterm and update launches), and
- * the stage buffer is released.  Both give bit-identical results.  No
+ * cns_ctx_create): one kernel a stage where every array is 16-byte aligned (tall columns
+ * of up to 8 x 8 cells take the composition of fused = 0), else fill, ctoprim, diffterm,
+ * then hypterm with the RK update of each cell applied in the same pass; the context then
+ * owns one ghosted 5-component stage buffer (the U^{1/3} state), allocated here or at
+ * creation.  fused = 0: kernel for kernel as the reference (separate hypterm and update
+ * launches), and the stage buffer is released.  All give bit-identical results.  No
  * counterpart in the reference. */
 int cns_ctx_set_fused(cns_ctx *ctx, int fused);
 
@@ -169,7 +170,11 @@ int cns_advance_async(cns_ctx *ctx, double *U, double *Unew, double *Q, double *
  * cns_ctx_profile_read() waits for the recorded launches and returns, per kernel
  * kind, the summed milliseconds and the number of launches.  Must not be on
  * while a step is being captured into a graph.  No counterpart in the
- * reference (whose timers are host gettimeofday, cpu/advance.cpp:53-73). */
+ * reference (whose timers are host gettimeofday, cpu/advance.cpp:53-73).
+ * HYPTERM_RK is a launch that ends in the stage update: the one-kernel stage (the whole
+ * stage), or hypterm with the update where the step runs separate kernels.  FILL_CTOPRIM
+ * is the launch that opens a step of one-kernel stages: the ghost fill of U with the
+ * Courant maximum. */
 #define CNS_PROF_FILL 0
 #define CNS_PROF_CTOPRIM 1
 #define CNS_PROF_DIFFTERM 2

@@ -337,3 +337,16 @@ def test_many_small_boxes_come_and_go(device, monkeypatch, fp32):
             assert np.array_equal(engines[0].read(i).cpu().numpy(), engines[1].read(j).cpu().numpy()), f"{n}: edge {e}"
     for eng in engines:
         eng.close()
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("var", [None, "CNS_BATCH_DIFF", "CNS_BATCH_HYP"])
+def test_default_tiles(device, monkeypatch, fp32, var):
+    """Without a table the work list of the one-kernel stage chooses the runs of 32-wide tiles; the
+    separate kernels take runs of 16 planes."""
+    if var:
+        monkeypatch.setenv(var, "0")
+        monkeypatch.setenv(var + "64", "0")
+    eng = BatchEngine(1 << 28, fp32=fp32, max_boxes=2, tuning={})
+    assert eng.get_tile(96) == (32, 16 if var else 96) and eng.get_tile(12) == (32, 12)
+    eng.close()
