@@ -36,6 +36,8 @@ constexpr int kTallCost = 4, kShortCost = 3;  // of a plane
 // Tiles, counted at runs of 12 planes, up to which the splits are compared; a longer list takes the first of
 // them: its tail is short however it is split, and the comparison would cost the host more than that.
 constexpr size_t kMostSimulated = 1 << 14;
+// Tiles of a list at most: a launch has fewer than 2^32 threads, 768 a tile.
+constexpr size_t kMostListed = 1 << 22;
 
 struct Split {
     int run, last, eighths;  // runs of `run` planes, and of `last` for so many eighths:
@@ -217,6 +219,10 @@ inline bool plan_runs(const std::vector<FusedBox> &boxes, const std::vector<Grou
 inline size_t fused_list(std::vector<FusedBox> &boxes, std::vector<TileDev> &out)
 {
     std::stable_sort(boxes.begin(), boxes.end(), [](const FusedBox &a, const FusedBox &b) { return a.e > b.e; });
+    size_t capped = 0;  // tiles that the caps of the runs alone ask for
+    for (const FusedBox &b : boxes) capped += (size_t)b.tiles() * ((b.e + b.kz - 1) / b.kz);
+    if (capped > kMostListed)
+        for (FusedBox &b : boxes) b.kz = b.e;
     std::vector<BoxGroup> groups;
     size_t most = 0;
     int64_t all = 0;

@@ -247,6 +247,15 @@ int main(int, char **argv)
         printf("%zu\n", fused_list(boxes, out));
         return 0;
     }
+    if (!strcmp(argv[1], "long")) {
+        // tiles of n boxes of edge e in runs of one plane
+        std::vector<FusedBox> boxes;
+        for (int i = 0; i < atoi(argv[2]); i++) boxes.push_back(box(i, atoi(argv[3]), 1, true));
+        std::vector<TileDev> out;
+        fused_list(boxes, out);
+        printf("%zu\n", out.size());
+        return 0;
+    }
     if (!strcmp(argv[1], "small")) {
         printf("%d %d %d\n", small_edge(false), small_edge(true), small_apart(atoi(argv[2]), atoi(argv[3])));
         return 0;
@@ -312,6 +321,13 @@ def test_boxes_that_fill_the_gpu_keep_long_runs(work_list, n, e, fp32):
 def test_small_boxes_take_narrow_tiles_where_they_are_many(work_list, small, others, apart):
     """More than one small box a CU, or two beside other boxes."""
     assert work_list("small", small, others).split() == ["14", "16", str(apart)]
+
+
+def test_a_list_of_short_runs_fits_one_launch(work_list):
+    """Boxes that fill the GPU's memory with runs capped at one plane: a launch has fewer than 2^32 threads,
+    768 of them a tile, so the caps give way; fewer boxes keep them."""
+    assert int(work_list("long", 45000, 33)) * 768 < 1 << 32
+    assert int(work_list("long", 1000, 33)) >= 1000 * 4 * 33
 
 
 # The enumeration of the ghost cells (cns_fill.h) in 32 and in 64 bits: every ghost cell of a box once,
