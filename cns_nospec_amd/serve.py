@@ -177,10 +177,9 @@ class BatchServer:
         self.engine = BatchEngine(hbm_budget, fp32=fp32, max_boxes=max_boxes)
         self.max_chunk = max_chunk
         # Admission also stops once the resident boxes hold this many cells (0: only
-        # the HBM budget limits it).  The engine's rate falls as its resident footprint
-        # grows (every step touches every resident box): on the request mix 3.5 G
-        # cell-steps/s at 113 M cells, 3.2 G at 490 M, 3.0 G at 960 M; a 2000-request
-        # burst runs 10 % faster with 128 M cells resident than with all that fit.
+        # the HBM budget limits it).  More resident boxes hardly raise the rate and make each
+        # wait longer: a 2000-request burst runs at 6.18 / 6.19 / 6.22 G cell-steps/s with 128 /
+        # 256 / 384 M cells resident, its mean latency 40.6 / 43.3 / 45.5 s.
         self.max_resident_cells = max_resident_cells
         self.keep = set(keep_states)
         self.progress_every = progress_every
