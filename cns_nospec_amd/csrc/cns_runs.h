@@ -7,7 +7,7 @@ namespace cns {
 
 // Calls f(kz) for the lengths that n planes have when cut into 1, 2, .. n even runs, at most
 // `most` planes long, longest first and each once: about 2 sqrt(n) of them.  (Trying every number of
-// runs cost a launch 8 ns a plane: of 400000 planes hypterm's was 3.1 ms, 2.3 of them its kernel's.)
+// runs cost a launch 8 ns a plane: for 400000 planes 3.1 ms, where hypterm's kernel takes 2.05.)
 template <typename F>
 inline void each_run_length(int n, int most, F f)
 {
